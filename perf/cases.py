@@ -76,15 +76,17 @@ def draw(rng):
     if kind == "mobilenet":
         return dict(kind=kind, batch=_log_int(rng, 2, 250))
     if kind == "residual":
-        return dict(kind=kind, bits=bits, batch=batch, size=4 * rng.randint(4, 14), c=16 * rng.randint(1, 8))
+        return dict(kind=kind, bits=bits, batch=batch, size=4 * rng.randint(4, 14), c=16 * rng.randint(3, 8))
     case = dict(kind=kind, bits=bits, requant=rng.choice(["bn", "bn", "mult"]), batch=batch)
     if kind == "linear":
         case.update(k=_channels(rng, 32, 4096), n=_channels(rng, 10, 4096))
         return case
     case.update(h=_log_int(rng, 7, 64), w=_log_int(rng, 7, 64))
     if kind == "conv":
-        case.update(ci=_channels(rng, 3, 256), co=_channels(rng, 8, 256), kx=3, ky=3, stride=rng.choice([1, 1, 2]), pt=1,
-                    pb=1, pl=1, pr=1)
+        ci = _channels(rng, 3, 256)
+        while ci in (16, 32):  # whole tiles of pixels only at these: the listed layers and the networks have them
+            ci = _channels(rng, 3, 256)
+        case.update(ci=ci, co=_channels(rng, 8, 256), kx=3, ky=3, stride=rng.choice([1, 1, 2]), pt=1, pb=1, pl=1, pr=1)
         if rng.random() < 0.15:
             case.update(kx=5, ky=5, pt=2, pb=2, pl=2, pr=2)
         elif rng.random() < 0.15:
