@@ -253,8 +253,10 @@ void igemm_kernel(ConvGeom g, EpiArgs e)
 #pragma unroll
     for (int i = 0; i < RA; i++) {
       const int m = m0 + (tid >> 2) + RPP * i;
+      // (a row past the last pixel: with SUB the tap's offset is added to poff before the range check, so 0xffffffff
+      // alone would wrap to an address in front of the input; every tap of such a row is out of range)
       poff[i] = 0xffffffffu;
-      pinv[i] = 0;
+      pinv[i] = SUB ? ~0u : 0u;
       if (m < g.M) {
         const int b = (int)fastdiv((unsigned)m, g.d_howo), rem = m - b * g.HoWo;
         const int oy = (int)fastdiv((unsigned)rem, g.d_wo), ox = rem - oy * g.Wo;
