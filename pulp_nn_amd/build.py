@@ -5,6 +5,7 @@
 import os
 import subprocess
 import sys
+import tempfile
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
@@ -12,7 +13,7 @@ LIBDIR = os.path.join(HERE, "lib")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
-    "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared",
+    "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wall", "-Wno-unused-function",
 ]
@@ -22,19 +23,36 @@ def lib_path(bn_bits):
     return os.path.join(LIBDIR, "libpulpnn_hip%d.so" % bn_bits)
 
 
-def build(bn_bits, verbose=False):
-    os.makedirs(LIBDIR, exist_ok=True)
-    out = lib_path(bn_bits)
-    cmd = [HIPCC] + FLAGS + ["-DPULPNN_BN_BITS=%d" % bn_bits, os.path.join(CSRC, "pulp_nn_hip.hip"), "-o", out]
+# translation units of the library: the host layer with most kernels, and kernel families compiled beside it
+UNITS = ("conv", "dwpw", "depthwise", "dw_mfma", "pulp_nn_hip")
+
+
+def _run(cmd, what, verbose):
     if verbose:
         print(" ".join(cmd), flush=True)
     res = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     # the host pass warns that it does not know the packed-fp32 feature: harmless
     log = "\n".join(l for l in res.stdout.splitlines() if "packed-fp32-ops" not in l)
     if res.returncode != 0:
-        raise RuntimeError("hipcc failed:\n" + log)
+        raise RuntimeError("%s failed:\n" % what + log)
     if verbose and log.strip():
         print(log)
+
+
+def compile_unit(bn_bits, unit, obj, verbose=False):
+    _run([HIPCC] + FLAGS + ["-c", "-DPULPNN_BN_BITS=%d" % bn_bits, os.path.join(CSRC, unit + ".hip"), "-o", obj], "hipcc", verbose)
+    return obj
+
+
+def build(bn_bits, verbose=False, pool=None):
+    """Compiles the units side by side (on `pool` if given) and links them into one shared object."""
+    from concurrent.futures import ThreadPoolExecutor
+    os.makedirs(LIBDIR, exist_ok=True)
+    out = lib_path(bn_bits)
+    with tempfile.TemporaryDirectory() as tmp, ThreadPoolExecutor(4) as own:
+        jobs = [(pool or own).submit(compile_unit, bn_bits, u, os.path.join(tmp, u + ".o"), verbose) for u in UNITS]
+        objs = [j.result() for j in jobs]
+        _run([HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC"] + objs + ["-o", out], "link", verbose)
     return out
 
 
@@ -81,9 +99,9 @@ def build_demo(verbose=False):
 
 def build_all(verbose=False):
     from concurrent.futures import ThreadPoolExecutor
-    with ThreadPoolExecutor(4) as ex:
-        libs = [ex.submit(build, b, verbose) for b in (32, 64)]
-        tools = [ex.submit(build_tool, t, verbose) for t in TOOLS]
+    with ThreadPoolExecutor(2) as ex, ThreadPoolExecutor(6) as units:
+        libs = [ex.submit(build, b, verbose, units) for b in (32, 64)]
+        tools = [units.submit(build_tool, t, verbose) for t in TOOLS]
         out = [f.result() for f in libs] + [f.result() for f in tools]
     return out + [build_demo(verbose)]
 

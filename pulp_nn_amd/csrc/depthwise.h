@@ -152,97 +152,6 @@ __device__ __forceinline__ int dw_tap_first(const unsigned (&span)[NS], unsigned
   else return __builtin_amdgcn_sdot4((int)dw_window<O, NS>(span), (int)wA, start, true);
 }
 
-// 3x3 depthwise, stride S (1 or 2) in both directions, left padding PL (0 or 1).
-template <int S, int PL, int MODE>
-__global__ __launch_bounds__(256) void dw3x3_kernel(DwGeom g, EpiArgs e)
-{
-  extern __shared__ unsigned dw_lds[];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-
-  int id = dw_xcd_remap(blockIdx.x, g.total);
-  const int cg = id % g.cgroups;
-  id /= g.cgroups;
-  const int band = id % g.bands;
-  const int b = id / g.bands;
-  const int c0 = cg * DW_CG;
-  const int oy0 = band * g.RB;
-  const int rows = min(g.RB, g.Ho - oy0);
-
-  const uint8_t *img = g.in + (long long)b * g.CH * g.H * g.W;
-  dw_stage(g, dw_lds, img, c0, oy0 * S - g.pt);
-
-  // per-lane channel constants
-  const int ch = c0 + lane;
-  const bool ch_ok = ch < g.CH;
-  unsigned wA[3], wB[3];  // (K0,K1,K2,0) and (0,K0,K1,K2) per filter row
-  int corr = 0;
-  bn_t kk = 0, ll = 0;
-  if (ch_ok) {
-    int wsum = 0;
-#pragma unroll
-    for (int i = 0; i < 3; i++) {
-      const int8_t *p = g.wt + (long long)ch * 9 + 3 * i;
-      const unsigned k0 = (uint8_t)p[0], k1 = (uint8_t)p[1], k2 = (uint8_t)p[2];
-      wA[i] = k0 | (k1 << 8) | (k2 << 16);
-      wB[i] = wA[i] << 8;
-      wsum += (int)p[0] + (int)p[1] + (int)p[2];
-    }
-    corr = 128 * wsum + (g.bias ? (int)g.bias[ch] : 0);
-    if (MODE == EPI_BN) {
-      kk = e.k[ch];
-      ll = e.lambda[ch];
-    }
-  } else {
-#pragma unroll
-    for (int i = 0; i < 3; i++) wA[i] = wB[i] = 0;
-  }
-  __syncthreads();
-
-  // dwords per input row needed for 4 outputs: window j starts at byte
-  // (4 - PL) + S*j of the span that begins one dword left of output column 4*xg*S
-  constexpr int O0 = 4 - PL;
-  constexpr int NS = (O0 + 3 * S + 2) / 4 + 1;
-  const int xgroups = (g.Wo + 3) >> 2;
-  const int items = rows * xgroups;
-  const unsigned *lbase = dw_lds + lane * g.CSD + (g.LP >> 2) - 1;
-  uint8_t *obase = g.out + (((long long)b * g.Ho + oy0) * g.Wo) * g.CH + c0;
-
-  for (int it = wave; it < items; it += 4) {
-    const int r = it / xgroups, xg = it - r * xgroups;
-    int acc[4] = {corr, corr, corr, corr};
-#pragma unroll
-    for (int i = 0; i < 3; i++) {
-      const unsigned *p = lbase + (r * S + i) * g.LWD + xg * S;
-      unsigned span[NS];
-#pragma unroll
-      for (int d = 0; d < NS; d++) span[d] = p[d];
-      dw_tap<O0, NS>(span, wA[i], wB[i], acc[0]);
-      dw_tap<O0 + S, NS>(span, wA[i], wB[i], acc[1]);
-      dw_tap<O0 + 2 * S, NS>(span, wA[i], wB[i], acc[2]);
-      dw_tap<O0 + 3 * S, NS>(span, wA[i], wB[i], acc[3]);
-    }
-    unsigned packed = 0;
-#pragma unroll
-    for (int j = 0; j < 4; j++)
-      packed |= (unsigned)requant<MODE>(acc[j], kk, ll, e.mult, e.shift) << (8 * j);
-    // lane now holds 4 pixels of its channel; after the transpose it holds 4
-    // channels (those of its quad) of pixel 4*xg + (lane & 3)
-    packed = quad_transpose4x4(packed, lane);
-    const int ox = 4 * xg + (lane & 3);
-    const int cq = lane & ~3;
-    if (ox < g.Wo) {
-      uint8_t *o = obase + ((long long)r * g.Wo + ox) * g.CH + cq;
-      if (g.out_vec4 && c0 + cq + 3 < g.CH) {
-        *(unsigned *)o = packed;
-      } else {
-#pragma unroll
-        for (int c = 0; c < 4; c++)
-          if (c0 + cq + c < g.CH) o[c] = (uint8_t)(packed >> (8 * c));
-      }
-    }
-  }
-}
-
 // One group of 4 output columns of one channel per lane, walked down the rows of a band.
 struct DwColumn {
   const unsigned *p;  // LDS: first dword of the window in the first staged row
@@ -811,126 +720,5 @@ __global__ __launch_bounds__(256) void dw_generic_kernel(DwGeom g, EpiArgs e)
       for (int fx = 0; fx < g.kx; fx++)
         acc += (int)p[fy * rowbytes + fx] * (int)wp[fy * g.kx + fx];
     if (ch_ok) obase[((long long)r * g.Wo + ox) * g.CH] = (uint8_t)requant<MODE>(acc, kk, ll, e.mult, e.shift);
-  }
-}
-
-// HWC -> CHW layout change with optional zero rows above and below each plane:
-// the glue between a conv / pointwise output and a depthwise input (the
-// reference leaves this step to the application).  out is [C][pad_t+H+pad_b][W].
-__global__ __launch_bounds__(256) void hwc_to_chw_kernel(const uint8_t *in, uint8_t *out, int H, int W, int C,
-                                                         int pad_t, int pad_b, int tiles_p, int tiles_c)
-{
-  // tile: 64 pixels x 64 channels through LDS
-  __shared__ uint8_t tile[64][65];
-  int id = blockIdx.x;
-  const int tc = id % tiles_c;
-  id /= tiles_c;
-  const int tp = id % tiles_p;
-  const int b = id / tiles_p;
-  const int HW = H * W;
-  const int Hp = pad_t + H + pad_b;
-  const uint8_t *src = in + (long long)b * HW * C;
-  uint8_t *dst = out + (long long)b * C * Hp * W;
-  const int p0 = tp * 64, c0 = tc * 64;
-  const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-  for (int i = ty; i < 64; i += 4) {
-    const int p = p0 + i, c = c0 + tx;
-    tile[i][tx] = (p < HW && c < C) ? src[(long long)p * C + c] : 0;
-  }
-  __syncthreads();
-  for (int i = ty; i < 64; i += 4) {
-    const int c = c0 + i, p = p0 + tx;
-    if (c < C && p < HW) dst[((long long)c * Hp + pad_t) * W + p] = tile[tx][i];
-  }
-  // zero rows
-  if (tp == 0 && (pad_t | pad_b)) {
-    for (int i = ty; i < 64; i += 4) {
-      const int c = c0 + i;
-      if (c >= C) continue;
-      for (int x = tx; x < pad_t * W; x += 64) dst[(long long)c * Hp * W + x] = 0;
-      for (int x = tx; x < pad_b * W; x += 64) dst[((long long)c * Hp + pad_t + H) * W + x] = 0;
-    }
-  }
-}
-
-// 4x4 byte transpose inside one lane: r[i] = bytes of pixel i (4 channels) ->
-// t[j] = bytes of channel j (4 pixels).
-__device__ __forceinline__ void transpose4x4_bytes(const unsigned (&r)[4], unsigned (&t)[4])
-{
-  // __builtin_amdgcn_perm(hi, lo, sel): selector 0-3 picks bytes of lo, 4-7 bytes of hi
-  const unsigned a0 = __builtin_amdgcn_perm(r[1], r[0], 0x05010400);  // p0c0 p1c0 p0c1 p1c1
-  const unsigned a1 = __builtin_amdgcn_perm(r[1], r[0], 0x07030602);  // p0c2 p1c2 p0c3 p1c3
-  const unsigned b0 = __builtin_amdgcn_perm(r[3], r[2], 0x05010400);  // p2c0 p3c0 p2c1 p3c1
-  const unsigned b1 = __builtin_amdgcn_perm(r[3], r[2], 0x07030602);
-  t[0] = __builtin_amdgcn_perm(b0, a0, 0x05040100);
-  t[1] = __builtin_amdgcn_perm(b0, a0, 0x07060302);
-  t[2] = __builtin_amdgcn_perm(b1, a1, 0x05040100);
-  t[3] = __builtin_amdgcn_perm(b1, a1, 0x07060302);
-}
-
-// Fast HWC -> CHW for C % 16 == 0, H*W % 4 == 0 and 16-byte aligned maps: a tile of
-// 256 pixels x 64 channels goes through LDS; reads are 16 bytes per lane (64 contiguous
-// bytes per pixel), writes are one dword of 4 pixels per lane, 256 contiguous bytes per
-// channel and store instruction.
-template <bool NT>
-__global__ __launch_bounds__(256) void hwc_to_chw_fast_kernel(const uint8_t *in, uint8_t *out, int H, int W, int C,
-                                                              int pad_t, int pad_b, int tiles_p, int tiles_c)
-{
-  constexpr int P = 80;  // LDS row pitch in bytes (16-byte aligned rows)
-  __shared__ __attribute__((aligned(16))) uint8_t tile[256 * P];
-  int id = blockIdx.x;
-  const int tc = id % tiles_c;
-  id /= tiles_c;
-  const int tp = id % tiles_p;
-  const int b = id / tiles_p;
-  const int HW = H * W;
-  const int Hp = pad_t + H + pad_b;
-  const uint8_t *src = in + (long long)b * HW * C;
-  uint8_t *dst = out + (long long)b * C * Hp * W;
-  const int p0 = tp * 256, c0 = tc * 64;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  {
-    const int chunk = tid & 3, c = c0 + 16 * chunk;
-    v4i v[4];
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const int p = min(p0 + (tid >> 2) + 64 * i, HW - 1);
-      v[i] = *(const v4i *)(src + (long long)p * C + min(c, C - 16));
-    }
-#pragma unroll
-    for (int i = 0; i < 4; i++) *(v4i *)&tile[((tid >> 2) + 64 * i) * P + 16 * chunk] = v[i];
-  }
-  __syncthreads();
-  const int cw = c0 + 16 * wave;  // this wave's 16 channels
-  const int p = p0 + 4 * lane;    // this lane's 4 pixels
-  if (cw < C && p < HW) {
-    unsigned rows[4][4];
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const v4i r = *(const v4i *)&tile[(4 * lane + i) * P + 16 * wave];
-      rows[i][0] = (unsigned)r.x;
-      rows[i][1] = (unsigned)r.y;
-      rows[i][2] = (unsigned)r.z;
-      rows[i][3] = (unsigned)r.w;
-    }
-    uint8_t *o = dst + ((long long)cw * Hp + pad_t) * W + p;
-    const long long plane = (long long)Hp * W;
-#pragma unroll
-    for (int d = 0; d < 4; d++) {
-      const unsigned r[4] = {rows[0][d], rows[1][d], rows[2][d], rows[3][d]};
-      unsigned t[4];
-      transpose4x4_bytes(r, t);
-#pragma unroll
-      for (int j = 0; j < 4; j++) store4<NT>(o + (4 * d + j) * plane, (int)t[j]);
-    }
-  }
-  // zero rows
-  if (tp == 0 && (pad_t | pad_b)) {
-    for (int i = wave; i < 64; i += 4) {
-      const int c = c0 + i;
-      if (c >= C) continue;
-      for (int x = lane; x < pad_t * W; x += 64) dst[(long long)c * Hp * W + x] = 0;
-      for (int x = lane; x < pad_b * W; x += 64) dst[((long long)c * Hp + pad_t + H) * W + x] = 0;
-    }
   }
 }

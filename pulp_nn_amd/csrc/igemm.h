@@ -42,7 +42,6 @@
 #include "requant.h"
 
 enum { GATHER_CHUNK16 = 0, GATHER_BYTES = 1, GATHER_UNIFORM = 2, GATHER_SUBTAP = 3 };
-enum { EPI_OUT32 = 3 };  // linear_out_32: int32 accumulators + int32 bias, no requantisation
 
 // Division of a 32-bit unsigned number by a divisor fixed for the launch, as a multiply-high, an add and
 // two shifts (Granlund & Montgomery); the host computes the constants.  The compiler's expansion of a

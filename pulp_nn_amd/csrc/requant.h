@@ -25,6 +25,7 @@ typedef int32_t bn_t;
 #endif
 
 enum { EPI_BN = 0, EPI_MULT = 1, EPI_RAW = 2 };
+enum { EPI_OUT32 = 3 };  // linear_out_32: int32 accumulators + int32 bias, no requantisation
 
 // Scalar (per launch) epilogue parameters.
 struct EpiArgs {
