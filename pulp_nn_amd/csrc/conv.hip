@@ -332,11 +332,10 @@ void conv_common(const char *fn, bool pointwise, const uint8_t *in, const int8_t
     return set_error(PULP_NN_HIP_ERR_ARGUMENT, fn, "out_shift out of range or null k/lambda");
   const long long M = (long long)g_batch * dim_out_x * dim_out_y;
   if (M > 0x7fffffffLL) return set_error(PULP_NN_HIP_ERR_ARGUMENT, fn, "batch too large");
-  if (kx == 1 && ky == 1 && sx == 1 && sy == 1 && pt == 0 && pl == 0 && dim_out_x == dim_in_x &&
-      dim_out_y == dim_in_y && try_pw_stream(mode, in, w, bias, out, M, ch_out, ch_in, e, g_stream)) {
-    check_launch(fn);
-    return;
-  }
+  if (kx == 1 && ky == 1 && sx == 1 && sy == 1 && pt == 0 && pl == 0 && dim_out_x == dim_in_x && dim_out_y == dim_in_y &&
+      (try_pw_stream(mode, in, w, bias, out, M, ch_out, ch_in, e, g_stream) ||
+       launch_pw_any(mode, in, w, bias, out, M, ch_out, ch_in, e, num_cus(), g_stream)))
+    return check_launch(fn);
   ConvGeom g;
   g.in = in;
   g.w = w;
@@ -368,6 +367,16 @@ void conv_common(const char *fn, bool pointwise, const uint8_t *in, const int8_t
     if (g.N <= 16) launch_smallk<16>(mode, rows, g, e, g_stream);
     else launch_smallk<32>(mode, rows, g, e, g_stream);
   } else {
+    // Channel counts that are not whole 16-byte chunks: from a band of the input in LDS (conv_band.h).  So are layers of
+    // few output channels, which leave most of the tiled kernel's 128 x 64 tile empty and its many waves waiting for each
+    // other (kernel times, tiled / band: 8x38x9 240 -> 32 s2 21.9 / 12.6 us; 2x8x13 48 -> 16 5x5 14.2 / 7.2; 31x19 80 -> 16
+    // 10.6 / 6.8; 23x14 144 -> 35 12.0 / 8.8; but 133x16x28 176 -> 128 28.6 / 34.2, 252x12x29 64 -> 40 s2 7.3 / 8.4).
+    const bool whole16 = ch_in % 16 == 0 && aligned(in, 16) && aligned(w, 16);
+    const bool few = ch_in == 16 || ch_in == 32 ? false : ch_in % 64 == 0 ? g.N <= 32 : g.N <= 64;
+    if (!whole16 || few) {
+      const ConvLayer L = {in, w, bias, out, (int)g_batch, dim_in_y, dim_in_x, ch_in, dim_out_y, dim_out_x, ch_out, kx, ky, pt, pl, sx, sy};
+      if (launch_conv_band(mode, L, e, num_cus(), g_stream)) return check_launch(fn);
+    }
     launch_igemm(mode, g, e, g_stream);
   }
   check_launch(fn);

@@ -81,6 +81,16 @@ struct DwLayer {
   uint8_t *out;
   int B, CH, H, W, Ho, Wo, kx, ky, pt, pl, sx, sy;
 };
+struct ConvLayer {
+  const uint8_t *in;
+  const int8_t *w;
+  const int8_t *bias;
+  uint8_t *out;
+  int B, H, W, Ci, Ho, Wo, N, kx, ky, pt, pl, sx, sy;
+};
+bool launch_conv_band(int mode, const ConvLayer &L, const EpiArgs &e, int cus, hipStream_t s);
+bool launch_pw_any(int mode, const uint8_t *in, const int8_t *w, const int8_t *bias, uint8_t *out, long long M, int N, int K,
+                   const EpiArgs &e, int cus, hipStream_t s);
 bool launch_dw_mfma(int mode, const DwLayer &L, const EpiArgs &e, int cus, hipStream_t s);
 
 #pragma GCC visibility pop
