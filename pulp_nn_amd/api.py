@@ -1,12 +1,28 @@
-"""ctypes binding of libpulpnn_hip{32,64}.so (the C ABI declared in include/)."""
+"""Python binding of libpulpnn_hip{32,64}.so (the C ABI declared in include/): the library is loaded with ctypes, the
+layer functions are called through csrc/pybind_fast.cpp (argument conversion in C)."""
 import ctypes as C
+import importlib.machinery
+import importlib.util
 import os
 
-from .build import lib_path
+from .build import fast_path, lib_path
 
 _U16, _I8, _INT, _PTR = C.c_uint16, C.c_int8, C.c_int, C.c_void_p
 
-_CONV_ARGS = [_PTR] * 7 + [_U16] * 16 + [_INT, _INT]
+
+def _load_fast():
+    """The extension module, or None if it has not been built (PulpNN() then says so)."""
+    path = fast_path()
+    if not os.path.exists(path):
+        return None
+    import torch  # noqa: F401  (the extension resolves its tensor type against the loaded torch)
+    loader = importlib.machinery.ExtensionFileLoader("_pulpnn_fast", path)
+    mod = importlib.util.module_from_spec(importlib.util.spec_from_loader("_pulpnn_fast", loader))
+    loader.exec_module(mod)
+    return mod
+
+
+_fast = _load_fast()
 
 
 class HipBlock(C.Structure):
@@ -15,8 +31,6 @@ class HipBlock(C.Structure):
                 ("dw_out_mult", _U16), ("dw_out_shift", _U16), ("dw_flag_relu", _I8), ("dw_flag_batch_norm", _I8),
                 ("pw_weight", _PTR), ("pw_bias", _PTR), ("pw_k", _PTR), ("pw_lambda", _PTR),
                 ("pw_out_mult", _U16), ("pw_out_shift", _U16), ("pw_flag_relu", _I8), ("pw_flag_batch_norm", _I8)]
-
-_DW_ARGS = [_PTR] * 8 + [_U16] * 16 + [_I8, _I8]
 
 CONV_NAMES = ("pulp_nn_conv_Ho_parallel", "pulp_nn_conv_Co_parallel", "pulp_nn_conv_HoWo_parallel",
               "pulp_nn_pointwise_HoWo_parallel", "pulp_nn_pointwise_Ho_parallel", "pulp_nn_pointwise_Co_parallel")
@@ -44,44 +58,46 @@ def _ptr(x):
     return x.data_ptr()
 
 
-class PulpNN:
+FAST_NAMES = CONV_NAMES + DW_NAMES + (
+    "pulp_nn_linear", "pulp_nn_linear_out_32", "pulp_nn_maxpool", "pulp_nn_avgpool", "pulp_nn_add", "pulp_nn_depthwise_3x3_s1",
+    "pulp_nn_hip_hwc_to_chw", "pulp_nn_hip_depthwise_hwc", "pulp_nn_hip_dw_pw_hwc", "pulp_nn_hip_dw_pw_chain_hwc",
+    "pulp_nn_hip_set_batch", "pulp_nn_hip_last_error")
+
+
+class PulpNN(_fast.Base if _fast else object):
     """One loaded library (32- or 64-bit batch-norm parameters).
 
     With check=True (default) every layer call raises PulpNNError if the library
-    rejected it; the C functions themselves return void like the reference's."""
+    rejected it; the C functions themselves return void like the reference's.
+
+    The layer functions are methods of the base class, with the reference's names and argument lists (the four or so
+    scalars of the added entry points in parentheses): pulp_nn_conv_{Ho,Co,HoWo}_parallel,
+    pulp_nn_pointwise_{HoWo,Ho,Co}_parallel, pulp_nn_depthwise_generic, pulp_nn_depthwise_generic_less_4_weights,
+    pulp_nn_depthwise_3x3_s1, pulp_nn_linear, pulp_nn_linear_out_32, pulp_nn_maxpool, pulp_nn_avgpool, pulp_nn_add;
+    set_batch(n);
+    hwc_to_chw(x, out, dim_x, dim_y, ch, pad_top=0, pad_bottom=0);
+    depthwise_hwc(x, bias, out, wt, k, lam, out_mult, out_shift, dim_in_x, dim_in_y, ch, dim_out_x, dim_out_y, stride,
+    flag_relu, flag_batch_norm): 3x3 depthwise, padding 1, HWC in and out (the layout change fused in); PulpNNError
+    (unsupported) for geometries without a fused kernel;
+    dw_pw_hwc(x, out, dim_in_x, dim_in_y, ch, dim_out_x, dim_out_y, ch_out, stride, dw_wt, dw_bias, dw_k, dw_lam, dw_mult,
+    dw_shift, dw_relu, dw_bn, pw_w, pw_bias, pw_k, pw_lam, pw_mult, pw_shift, pw_relu, pw_bn): 3x3 depthwise (padding 1,
+    HWC in) and the pointwise layer behind it in one launch; PulpNNError (unsupported) likewise."""
 
     def __init__(self, bn_bits=32, check=True):
         if bn_bits not in (32, 64):
             raise ValueError("bn_bits must be 32 or 64")
         path = lib_path(bn_bits)
-        if not os.path.exists(path):
-            raise ImportError("%s is missing: build it with `python -m pulp_nn_amd.build` "
-                              "(there is no CPU fallback)" % path)
+        for need in (path, fast_path()):
+            if not os.path.exists(need) or _fast is None:
+                raise ImportError("%s is missing: build it with `python -m pulp_nn_amd.build` "
+                                  "(there is no CPU fallback)" % need)
         self.bn_bits = bn_bits
-        self.check = check
+        self.check = bool(check)
         self.path = path
         L = self._lib = C.CDLL(path)
-        bn_scalar = C.c_int64 if bn_bits == 64 else C.c_int32
-        for n in CONV_NAMES:
-            getattr(L, n).argtypes, getattr(L, n).restype = _CONV_ARGS, None
-        for n in DW_NAMES:
-            getattr(L, n).argtypes, getattr(L, n).restype = _DW_ARGS, None
-        L.pulp_nn_linear.argtypes = [_PTR] * 6 + [_U16, _I8, _U16, _U16, _INT, _INT]
-        L.pulp_nn_linear.restype = None
-        L.pulp_nn_linear_out_32.argtypes = [_PTR] * 4 + [_U16, _U16]
-        L.pulp_nn_linear_out_32.restype = None
+        self._bind(bn_bits, {n: C.cast(getattr(L, n), _PTR).value for n in FAST_NAMES})
         L.pulp_nn_matmul.argtypes = [_PTR, _PTR, _U16, _U16, _U16, _U16, _PTR, _PTR, _PTR, _PTR, _PTR, _INT, _INT]
         L.pulp_nn_matmul.restype = _PTR
-        L.pulp_nn_maxpool.argtypes = [_PTR, _PTR] + [_U16] * 13
-        L.pulp_nn_maxpool.restype = None
-        L.pulp_nn_avgpool.argtypes = [_PTR, _PTR, bn_scalar, _U16, bn_scalar] + [_U16] * 13 + [_INT]
-        L.pulp_nn_avgpool.restype = None
-        L.pulp_nn_add.argtypes = [_PTR] * 3 + [_U16] * 6
-        L.pulp_nn_add.restype = None
-        L.pulp_nn_depthwise_3x3_s1.argtypes = [_PTR, _PTR, _INT, _INT, _INT, _INT, _INT, _PTR, _I8, _U16, _PTR, _PTR,
-                                               _INT, _INT, _PTR]
-        L.pulp_nn_depthwise_3x3_s1.restype = None
-        L.pulp_nn_hip_set_batch.argtypes = [C.c_uint]
         L.pulp_nn_hip_get_batch.restype = C.c_uint
         L.pulp_nn_hip_set_stream.argtypes = [_PTR]
         L.pulp_nn_hip_get_stream.restype = _PTR
@@ -91,13 +107,6 @@ class PulpNN:
         L.pulp_nn_hip_last_error.restype = _INT
         L.pulp_nn_hip_last_error_string.restype = C.c_char_p
         L.pulp_nn_hip_bn_bits.restype = _INT
-        L.pulp_nn_hip_hwc_to_chw.argtypes = [_PTR, _PTR] + [C.c_uint] * 5
-        L.pulp_nn_hip_hwc_to_chw.restype = None
-        L.pulp_nn_hip_depthwise_hwc.argtypes = [_PTR] * 6 + [_U16] * 8 + [_I8, _I8]
-        L.pulp_nn_hip_depthwise_hwc.restype = None
-        L.pulp_nn_hip_dw_pw_hwc.argtypes = ([_PTR] * 2 + [_U16] * 7 + [_PTR] * 4 + [_U16] * 2 + [_I8] * 2 + [_PTR] * 4 +
-                                            [_U16] * 2 + [_I8] * 2)
-        L.pulp_nn_hip_dw_pw_hwc.restype = None
         L.pulp_nn_hip_dw_pw_chain_hwc.argtypes = [_PTR] * 2 + [_U16] * 3 + [C.c_uint, C.POINTER(HipBlock)]
         L.pulp_nn_hip_dw_pw_chain_hwc.restype = None
         _U64 = C.c_uint64
@@ -111,9 +120,6 @@ class PulpNN:
         assert L.pulp_nn_hip_bn_bits() == bn_bits
 
     # -- added entry points ------------------------------------------------
-    def set_batch(self, n):
-        self._lib.pulp_nn_hip_set_batch(int(n))
-
     def get_batch(self):
         return int(self._lib.pulp_nn_hip_get_batch())
 
@@ -155,24 +161,6 @@ class PulpNN:
             self._raise()
         return res
 
-    def hwc_to_chw(self, x, out, dim_x, dim_y, ch, pad_top=0, pad_bottom=0):
-        self._call("pulp_nn_hip_hwc_to_chw", _ptr(x), _ptr(out), dim_x, dim_y, ch, pad_top, pad_bottom)
-
-    def depthwise_hwc(self, x, bias, out, wt, k, lam, out_mult, out_shift, dim_in_x, dim_in_y, ch, dim_out_x,
-                      dim_out_y, stride, flag_relu, flag_batch_norm):
-        """3x3 depthwise, padding 1, HWC in and out (the layout change fused in).  Raises
-        PulpNNError (unsupported) for geometries without a fused kernel."""
-        self._call("pulp_nn_hip_depthwise_hwc", _ptr(x), _ptr(bias), _ptr(out), _ptr(wt), _ptr(k), _ptr(lam), out_mult,
-                   out_shift, dim_in_x, dim_in_y, ch, dim_out_x, dim_out_y, stride, flag_relu, flag_batch_norm)
-
-    def dw_pw_hwc(self, x, out, dim_in_x, dim_in_y, ch, dim_out_x, dim_out_y, ch_out, stride, dw_wt, dw_bias, dw_k, dw_lam,
-                  dw_mult, dw_shift, dw_relu, dw_bn, pw_w, pw_bias, pw_k, pw_lam, pw_mult, pw_shift, pw_relu, pw_bn):
-        """3x3 depthwise (padding 1, HWC in) and the pointwise layer behind it in one launch.  Raises
-        PulpNNError (unsupported) for geometries without a fused kernel."""
-        self._call("pulp_nn_hip_dw_pw_hwc", _ptr(x), _ptr(out), dim_in_x, dim_in_y, ch, dim_out_x, dim_out_y, ch_out, stride,
-                   _ptr(dw_wt), _ptr(dw_bias), _ptr(dw_k), _ptr(dw_lam), dw_mult, dw_shift, dw_relu, dw_bn,
-                   _ptr(pw_w), _ptr(pw_bias), _ptr(pw_k), _ptr(pw_lam), pw_mult, pw_shift, pw_relu, pw_bn)
-
     def dw_pw_chain_hwc(self, x, out, dim_x, dim_y, ch, blocks):
         """Several depthwise + pointwise blocks of one shape (stride 1, ch channels throughout) in one launch.
         blocks: a list of tuples (dw_wt, dw_bias, dw_k, dw_lam, dw_mult, dw_shift, dw_relu, dw_bn, pw_w, pw_bias,
@@ -209,65 +197,9 @@ class PulpNN:
         self._call("pulp_nn_hip_calib_conv_static", _ptr(x), _ptr(bias), _ptr(w), _ptr(k), dim_in_x, dim_in_y, ch_in,
                    dim_out_x, dim_out_y, ch_out, kx, ky, pad_top, pad_left, stride_x, stride_y, _ptr(result))
 
-    # -- the reference API ---------------------------------------------------
-    def _conv(self, name, pIn, pIm2Col, bias, pOut, pWeight, k, lam, *scalars):
-        assert len(scalars) == 18, "expected out_mult .. flag_batch_norm"
-        self._call(name, _ptr(pIn), _ptr(pIm2Col), _ptr(bias), _ptr(pOut), _ptr(pWeight), _ptr(k), _ptr(lam),
-                   *[int(s) & 0xFFFF for s in scalars[:16]], int(scalars[16]), int(scalars[17]))
-
-    def _dw(self, name, Im_in, bufferC, bias, Im_out, wt, bufferB, k, lam, *scalars):
-        assert len(scalars) == 18, "expected out_mult .. FLAG_BATCH_NORM"
-        f8 = lambda v: ((int(v) + 128) & 0xFF) - 128
-        self._call(name, _ptr(Im_in), _ptr(bufferC), _ptr(bias), _ptr(Im_out), _ptr(wt), _ptr(bufferB), _ptr(k),
-                   _ptr(lam), *[int(s) & 0xFFFF for s in scalars[:16]], f8(scalars[16]), f8(scalars[17]))
-
-    def pulp_nn_linear(self, pIn, bias, pOut, pWeights, k, lam, out_mult, out_shift, dim_vec, num_o_neurons,
-                       flag_relu, flag_batch_norm):
-        self._call("pulp_nn_linear", _ptr(pIn), _ptr(bias), _ptr(pOut), _ptr(pWeights), _ptr(k), _ptr(lam),
-                   int(out_mult) & 0xFFFF, int(out_shift), int(dim_vec), int(num_o_neurons), int(flag_relu),
-                   int(flag_batch_norm))
-
-    def pulp_nn_linear_out_32(self, pIn, bias, pOut, pWeights, dim_vec, num_o_neurons):
-        self._call("pulp_nn_linear_out_32", _ptr(pIn), _ptr(bias), _ptr(pOut), _ptr(pWeights), int(dim_vec),
-                   int(num_o_neurons))
-
+    # -- the reference's inner two-pixel matmul (the layer functions are the base class's) ----
     def pulp_nn_matmul(self, pWeight, pIn, ch_out, num_col_im2col, out_shift, out_mult, k, lam, bias, pOut, pOut2,
                        flag_relu, flag_batch_norm):
         return self._call("pulp_nn_matmul", _ptr(pWeight), _ptr(pIn), int(ch_out), int(num_col_im2col),
                           int(out_shift) & 0xFFFF, int(out_mult) & 0xFFFF, _ptr(k), _ptr(lam), _ptr(bias), _ptr(pOut),
                           _ptr(pOut2), int(flag_relu), int(flag_batch_norm))
-
-    def pulp_nn_maxpool(self, Im_in, Im_out, *scalars):
-        assert len(scalars) == 13
-        self._call("pulp_nn_maxpool", _ptr(Im_in), _ptr(Im_out), *[int(s) & 0xFFFF for s in scalars])
-
-    def pulp_nn_avgpool(self, Im_in, Im_out, lam, out_shift, out_add, *scalars):
-        assert len(scalars) == 14
-        self._call("pulp_nn_avgpool", _ptr(Im_in), _ptr(Im_out), int(lam), int(out_shift) & 0xFFFF, int(out_add),
-                   *[int(s) & 0xFFFF for s in scalars[:13]], int(scalars[13]))
-
-    def pulp_nn_add(self, in1, in2, out, out_mult1, out_mult2, out_shift, dim_h, dim_w, ch):
-        self._call("pulp_nn_add", _ptr(in1), _ptr(in2), _ptr(out), int(out_mult1) & 0xFFFF, int(out_mult2) & 0xFFFF,
-                   int(out_shift) & 0xFFFF, int(dim_h), int(dim_w), int(ch))
-
-    def pulp_nn_depthwise_3x3_s1(self, In_Img, Out_Img, R, C_, CH, p_l, p_r, Kernel, out_shift, out_mult, kappa, lam,
-                                 flag_relu, flag_batch_norm, memory_chan=None):
-        self._call("pulp_nn_depthwise_3x3_s1", _ptr(In_Img), _ptr(Out_Img), int(R), int(C_), int(CH), int(p_l),
-                   int(p_r), _ptr(Kernel), int(out_shift), int(out_mult) & 0xFFFF, _ptr(kappa), _ptr(lam),
-                   int(flag_relu), int(flag_batch_norm), _ptr(memory_chan))
-
-
-def _make_forwarders():
-    for n in CONV_NAMES:
-        def f(self, *a, _n=n):
-            return self._conv(_n, *a)
-        f.__name__ = n
-        setattr(PulpNN, n, f)
-    for n in DW_NAMES:
-        def f(self, *a, _n=n):
-            return self._dw(_n, *a)
-        f.__name__ = n
-        setattr(PulpNN, n, f)
-
-
-_make_forwarders()

@@ -77,6 +77,23 @@ def build_tool(name="mfma_ceiling", verbose=False):
     return tool_path(name)
 
 
+def fast_path():
+    return os.path.join(LIBDIR, "_pulpnn_fast.so")
+
+
+def build_fast(verbose=False):
+    """The Python front end's call path (csrc/pybind_fast.cpp): a CPython extension module, host code only."""
+    import sysconfig
+    from torch.utils import cpp_extension
+    os.makedirs(LIBDIR, exist_ok=True)
+    libs = cpp_extension.library_paths()
+    cmd = (["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-I", sysconfig.get_paths()["include"]] +
+           ["-I" + d for d in cpp_extension.include_paths()] + [os.path.join(CSRC, "pybind_fast.cpp"), "-o", fast_path()] +
+           ["-L" + d for d in libs] + ["-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10"] + ["-Wl,-rpath," + d for d in libs])
+    _run(cmd, "g++", verbose)
+    return fast_path()
+
+
 def demo_path():
     return os.path.join(LIBDIR, "capi_demo")
 
@@ -101,7 +118,7 @@ def build_all(verbose=False):
     from concurrent.futures import ThreadPoolExecutor
     with ThreadPoolExecutor(2) as ex, ThreadPoolExecutor(6) as units:
         libs = [ex.submit(build, b, verbose, units) for b in (32, 64)]
-        tools = [units.submit(build_tool, t, verbose) for t in TOOLS]
+        tools = [units.submit(build_fast, verbose)] + [units.submit(build_tool, t, verbose) for t in TOOLS]
         out = [f.result() for f in libs] + [f.result() for f in tools]
     return out + [build_demo(verbose)]
 

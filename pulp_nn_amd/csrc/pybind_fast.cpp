@@ -1,0 +1,522 @@
+// The Python front end's call path: argument conversion and the call itself in C, for one loaded library.
+//
+// A layer of a few MB takes the GPU 4 to 7 us.  Through ctypes a call costs 3.5 us of argument conversion (25 Python
+// objects, six of them tensors asked for their address) before hipLaunchKernel is reached; here it is a few tenths of a
+// microsecond.  `Base` is the base class of api.PulpNN: its methods take the reference's argument lists.  `Plan` is a
+// list of such calls with their arguments converted once, for a chain of layers on buffers that its owner keeps: a run
+// is one Python call, and only the chain's input is converted per run.
+//
+// The entry points are looked up by ctypes (api.py loads the library) and handed over as addresses, so this module does
+// not link against either library.
+#define PY_SSIZE_T_CLEAN
+#include <Python.h>
+#include <structmember.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <stdint.h>
+#include <string.h>
+
+#include <string>
+#include <vector>
+
+#include "../../include/pulp_nn_hip.h"
+
+namespace {
+
+typedef unsigned short u16;
+typedef signed char i8;
+
+enum Kind { CONV, DW, LINEAR, LINEAR32, MAXPOOL, AVGPOOL, ADD, DW3, HWC2CHW, DWHWC, DWPW, CHAIN, NKIND };
+
+// argument types in order: p = tensor / address / None, i = integer; names for keyword calls (null: positional only);
+// the last `optional` arguments default to zero / null
+struct KindInfo {
+  const char *spec;
+  const char *names;
+  int optional;
+};
+const KindInfo kinds[NKIND] = {
+    {"pppppppiiiiiiiiiiiiiiiiii", nullptr, 0},
+    {"ppppppppiiiiiiiiiiiiiiiiii", nullptr, 0},
+    {"ppppppiiiiii", "pIn bias pOut pWeights k lam out_mult out_shift dim_vec num_o_neurons flag_relu flag_batch_norm", 0},
+    {"ppppii", "pIn bias pOut pWeights dim_vec num_o_neurons", 0},
+    {"ppiiiiiiiiiiiii", nullptr, 0},
+    {"ppiiiiiiiiiiiiiiiii", nullptr, 0},
+    {"pppiiiiii", "in1 in2 out out_mult1 out_mult2 out_shift dim_h dim_w ch", 0},
+    {"ppiiiiipiippiip", "In_Img Out_Img R C_ CH p_l p_r Kernel out_shift out_mult kappa lam flag_relu flag_batch_norm memory_chan", 1},
+    {"ppiiiii", "x out dim_x dim_y ch pad_top pad_bottom", 2},
+    {"ppppppiiiiiiiiii", "x bias out wt k lam out_mult out_shift dim_in_x dim_in_y ch dim_out_x dim_out_y stride flag_relu flag_batch_norm", 0},
+    {"ppiiiiiiippppiiiippppiiii",
+     "x out dim_in_x dim_in_y ch dim_out_x dim_out_y ch_out stride dw_wt dw_bias dw_k dw_lam dw_mult dw_shift dw_relu dw_bn pw_w pw_bias pw_k "
+     "pw_lam pw_mult pw_shift pw_relu pw_bn",
+     0},
+    {nullptr, nullptr, 0},
+};
+
+// entry points by index: the two families with several names first
+enum Fn {
+  F_CONV_HO, F_CONV_CO, F_CONV_HOWO, F_PW_HOWO, F_PW_HO, F_PW_CO, F_DW_GENERIC, F_DW_LESS4, F_LINEAR, F_LINEAR32, F_MAXPOOL,
+  F_AVGPOOL, F_ADD, F_DW3, F_HWC2CHW, F_DWHWC, F_DWPW, F_CHAIN, F_SET_BATCH, F_LAST_ERROR, NFN
+};
+const char *fn_names[NFN] = {
+    "pulp_nn_conv_Ho_parallel", "pulp_nn_conv_Co_parallel", "pulp_nn_conv_HoWo_parallel", "pulp_nn_pointwise_HoWo_parallel",
+    "pulp_nn_pointwise_Ho_parallel", "pulp_nn_pointwise_Co_parallel", "pulp_nn_depthwise_generic",
+    "pulp_nn_depthwise_generic_less_4_weights", "pulp_nn_linear", "pulp_nn_linear_out_32", "pulp_nn_maxpool", "pulp_nn_avgpool",
+    "pulp_nn_add", "pulp_nn_depthwise_3x3_s1", "pulp_nn_hip_hwc_to_chw", "pulp_nn_hip_depthwise_hwc", "pulp_nn_hip_dw_pw_hwc",
+    "pulp_nn_hip_dw_pw_chain_hwc", "pulp_nn_hip_set_batch", "pulp_nn_hip_last_error"};
+const Kind fn_kind[F_SET_BATCH] = {CONV, CONV, CONV, CONV, CONV, CONV, DW, DW, LINEAR, LINEAR32, MAXPOOL, AVGPOOL, ADD, DW3, HWC2CHW, DWHWC, DWPW, CHAIN};
+
+struct Base {
+  PyObject_HEAD
+  void *fn[NFN];
+  int bits;
+  char check;
+};
+
+struct Args {
+  void *p[10];
+  int64_t s[20];
+};
+
+// tensor / address / None -> device address
+bool to_ptr(PyObject *o, void **out)
+{
+  if (o == Py_None) {
+    *out = nullptr;
+    return true;
+  }
+  if (THPVariable_Check(o)) {
+    const at::Tensor &t = THPVariable_Unpack(o);
+    if (!t.is_cuda()) {
+      PyErr_SetString(PyExc_ValueError, "PULP-NN HIP kernels take device tensors");
+      return false;
+    }
+    if (!t.is_contiguous()) {
+      PyErr_SetString(PyExc_ValueError, "tensor must be contiguous");
+      return false;
+    }
+    *out = t.data_ptr();
+    return true;
+  }
+  if (PyLong_Check(o)) {
+    *out = PyLong_AsVoidPtr(o);
+    return *out || !PyErr_Occurred();
+  }
+  PyErr_Format(PyExc_TypeError, "expected a tensor, an address or None, not %.100s", Py_TYPE(o)->tp_name);
+  return false;
+}
+
+bool to_int(PyObject *o, int64_t *out)
+{
+  if (PyLong_CheckExact(o)) {
+    *out = (int64_t)PyLong_AsUnsignedLongLongMask(o);
+    return true;
+  }
+  PyObject *n = PyNumber_Long(o);  // what int() accepts
+  if (!n) return false;
+  *out = (int64_t)PyLong_AsUnsignedLongLongMask(n);
+  Py_DECREF(n);
+  return true;
+}
+
+bool parse(Kind kind, PyObject *const *args, Py_ssize_t n, Args *a)
+{
+  const char *spec = kinds[kind].spec;
+  const Py_ssize_t want = (Py_ssize_t)strlen(spec);
+  if (n > want || n < want - kinds[kind].optional) {
+    PyErr_Format(PyExc_AssertionError, "expected %zd arguments, got %zd", want, n);
+    return false;
+  }
+  int np = 0, ns = 0;
+  for (Py_ssize_t i = 0; i < want; i++) {
+    if (spec[i] == 'p') {
+      a->p[np] = nullptr;
+      if (i < n && !to_ptr(args[i], &a->p[np])) return false;
+      np++;
+    } else {
+      a->s[ns] = 0;
+      if (i < n && !to_int(args[i], &a->s[ns])) return false;
+      ns++;
+    }
+  }
+  return true;
+}
+
+#define U(i) (u16) a.s[i]
+#define I(i) (int)a.s[i]
+#define B8(i) (i8) a.s[i]
+typedef void *P;
+
+void invoke(const Base *b, int f, const Args &a, const pulp_nn_hip_block *blocks, unsigned n_blocks)
+{
+  void *fn = b->fn[f];
+  void *const *p = a.p;
+  switch (fn_kind[f]) {
+    case CONV:
+      ((void (*)(P, P, P, P, P, P, P, u16, u16, u16, u16, u16, u16, u16, u16, u16, u16, u16, u16, u16, u16, u16, u16, int, int))fn)(
+          p[0], p[1], p[2], p[3], p[4], p[5], p[6], U(0), U(1), U(2), U(3), U(4), U(5), U(6), U(7), U(8), U(9), U(10), U(11), U(12),
+          U(13), U(14), U(15), I(16), I(17));
+      break;
+    case DW:
+      ((void (*)(P, P, P, P, P, P, P, P, u16, u16, u16, u16, u16, u16, u16, u16, u16, u16, u16, u16, u16, u16, u16, u16, i8, i8))fn)(
+          p[0], p[1], p[2], p[3], p[4], p[5], p[6], p[7], U(0), U(1), U(2), U(3), U(4), U(5), U(6), U(7), U(8), U(9), U(10), U(11),
+          U(12), U(13), U(14), U(15), B8(16), B8(17));
+      break;
+    case LINEAR:
+      ((void (*)(P, P, P, P, P, P, u16, i8, u16, u16, int, int))fn)(p[0], p[1], p[2], p[3], p[4], p[5], U(0), B8(1), U(2), U(3), I(4), I(5));
+      break;
+    case LINEAR32: ((void (*)(P, P, P, P, u16, u16))fn)(p[0], p[1], p[2], p[3], U(0), U(1)); break;
+    case MAXPOOL:
+      ((void (*)(P, P, u16, u16, u16, u16, u16, u16, u16, u16, u16, u16, u16, u16, u16))fn)(
+          p[0], p[1], U(0), U(1), U(2), U(3), U(4), U(5), U(6), U(7), U(8), U(9), U(10), U(11), U(12));
+      break;
+    case AVGPOOL:
+      if (b->bits == 64)
+        ((void (*)(P, P, int64_t, u16, int64_t, u16, u16, u16, u16, u16, u16, u16, u16, u16, u16, u16, u16, u16, int))fn)(
+            p[0], p[1], a.s[0], U(1), a.s[2], U(3), U(4), U(5), U(6), U(7), U(8), U(9), U(10), U(11), U(12), U(13), U(14), U(15), I(16));
+      else
+        ((void (*)(P, P, int32_t, u16, int32_t, u16, u16, u16, u16, u16, u16, u16, u16, u16, u16, u16, u16, u16, int))fn)(
+            p[0], p[1], I(0), U(1), I(2), U(3), U(4), U(5), U(6), U(7), U(8), U(9), U(10), U(11), U(12), U(13), U(14), U(15), I(16));
+      break;
+    case ADD: ((void (*)(P, P, P, u16, u16, u16, u16, u16, u16))fn)(p[0], p[1], p[2], U(0), U(1), U(2), U(3), U(4), U(5)); break;
+    case DW3:
+      ((void (*)(P, P, int, int, int, int, int, P, i8, u16, P, P, int, int, P))fn)(p[0], p[1], I(0), I(1), I(2), I(3), I(4), p[2], B8(5), U(6),
+                                                                              p[3], p[4], I(7), I(8), p[5]);
+      break;
+    case HWC2CHW:
+      ((void (*)(P, P, unsigned, unsigned, unsigned, unsigned, unsigned))fn)(p[0], p[1], (unsigned)a.s[0], (unsigned)a.s[1], (unsigned)a.s[2],
+                                                                          (unsigned)a.s[3], (unsigned)a.s[4]);
+      break;
+    case DWHWC:
+      ((void (*)(P, P, P, P, P, P, u16, u16, u16, u16, u16, u16, u16, u16, i8, i8))fn)(p[0], p[1], p[2], p[3], p[4], p[5], U(0), U(1), U(2), U(3),
+                                                                                  U(4), U(5), U(6), U(7), B8(8), B8(9));
+      break;
+    case DWPW:
+      ((void (*)(P, P, u16, u16, u16, u16, u16, u16, u16, P, P, P, P, u16, u16, i8, i8, P, P, P, P, u16, u16, i8, i8))fn)(
+          p[0], p[1], U(0), U(1), U(2), U(3), U(4), U(5), U(6), p[2], p[3], p[4], p[5], U(7), U(8), B8(9), B8(10), p[6], p[7], p[8], p[9], U(11),
+          U(12), B8(13), B8(14));
+      break;
+    case CHAIN:
+      ((void (*)(P, P, u16, u16, u16, unsigned, const pulp_nn_hip_block *))fn)(p[0], p[1], U(0), U(1), U(2), n_blocks, blocks);
+      break;
+    default: break;
+  }
+}
+
+int last_error(const Base *b) { return ((int (*)(void))b->fn[F_LAST_ERROR])(); }
+
+// keyword arguments -> their places
+bool place_keywords(Kind kind, PyObject *const *args, Py_ssize_t n, PyObject *kw, std::vector<PyObject *> *out)
+{
+  const char *names = kinds[kind].names;
+  if (!names) {
+    PyErr_SetString(PyExc_TypeError, "this function takes no keyword arguments");
+    return false;
+  }
+  std::vector<std::string> list;
+  for (const char *s = names; *s;) {
+    const char *e = strchr(s, ' ');
+    list.emplace_back(s, e ? (size_t)(e - s) : strlen(s));
+    s = e ? e + 1 : s + strlen(s);
+  }
+  out->assign(list.size(), nullptr);
+  for (Py_ssize_t i = 0; i < n && i < (Py_ssize_t)list.size(); i++) (*out)[i] = args[i];
+  for (Py_ssize_t j = 0; j < PyTuple_GET_SIZE(kw); j++) {
+    const char *key = PyUnicode_AsUTF8(PyTuple_GET_ITEM(kw, j));
+    size_t i = 0;
+    while (i < list.size() && list[i] != key) i++;
+    if (i == list.size() || (*out)[i]) {
+      PyErr_Format(PyExc_TypeError, "unexpected or repeated argument '%s'", key);
+      return false;
+    }
+    (*out)[i] = args[n + j];
+  }
+  while (!out->empty() && !out->back() && (int)(list.size() - out->size()) < kinds[kind].optional) out->pop_back();
+  for (size_t i = 0; i < out->size(); i++)
+    if (!(*out)[i]) {
+      if (i + kinds[kind].optional < list.size()) {
+        PyErr_Format(PyExc_TypeError, "missing argument '%s'", list[i].c_str());
+        return false;
+      }
+      (*out)[i] = Py_None;
+    }
+  return true;
+}
+
+template <int F>
+PyObject *method(PyObject *self, PyObject *const *args, Py_ssize_t n, PyObject *kw)
+{
+  Base *b = (Base *)self;
+  Args a;
+  std::vector<PyObject *> placed;
+  if (kw && PyTuple_GET_SIZE(kw)) {
+    if (!place_keywords(fn_kind[F], args, n, kw, &placed)) return nullptr;
+    // (an omitted optional argument in the middle: zero)
+    static PyObject *zero = PyLong_FromLong(0);
+    for (size_t i = 0; i < placed.size(); i++)
+      if (placed[i] == Py_None && kinds[fn_kind[F]].spec[i] == 'i') placed[i] = zero;
+    args = placed.data();
+    n = (Py_ssize_t)placed.size();
+  }
+  if (!b->fn[F]) {
+    PyErr_SetString(PyExc_RuntimeError, "library not bound");
+    return nullptr;
+  }
+  if (!parse(fn_kind[F], args, n, &a)) return nullptr;
+  int err;
+  Py_BEGIN_ALLOW_THREADS
+  invoke(b, F, a, nullptr, 0);
+  err = b->check ? last_error(b) : 0;
+  Py_END_ALLOW_THREADS
+  if (err) return PyObject_CallMethod(self, "_raise", nullptr);
+  Py_RETURN_NONE;
+}
+
+PyObject *set_batch(PyObject *self, PyObject *arg)
+{
+  int64_t v;
+  if (!to_int(arg, &v)) return nullptr;
+  ((void (*)(unsigned))((Base *)self)->fn[F_SET_BATCH])((unsigned)v);
+  Py_RETURN_NONE;
+}
+
+// _bind(bits, {name: address})
+PyObject *bind(PyObject *self, PyObject *args)
+{
+  Base *b = (Base *)self;
+  PyObject *d;
+  if (!PyArg_ParseTuple(args, "iO!", &b->bits, &PyDict_Type, &d)) return nullptr;
+  for (int f = 0; f < NFN; f++) {
+    PyObject *v = PyDict_GetItemString(d, fn_names[f]);
+    if (!v) return PyErr_Format(PyExc_KeyError, "%s", fn_names[f]);
+    b->fn[f] = PyLong_AsVoidPtr(v);
+    if (PyErr_Occurred()) return nullptr;
+  }
+  Py_RETURN_NONE;
+}
+
+#define M(F, NAME) {NAME, (PyCFunction)(void (*)(void))method<F>, METH_FASTCALL | METH_KEYWORDS, nullptr}
+PyMethodDef base_methods[] = {
+    M(F_CONV_HO, "pulp_nn_conv_Ho_parallel"),
+    M(F_CONV_CO, "pulp_nn_conv_Co_parallel"),
+    M(F_CONV_HOWO, "pulp_nn_conv_HoWo_parallel"),
+    M(F_PW_HOWO, "pulp_nn_pointwise_HoWo_parallel"),
+    M(F_PW_HO, "pulp_nn_pointwise_Ho_parallel"),
+    M(F_PW_CO, "pulp_nn_pointwise_Co_parallel"),
+    M(F_DW_GENERIC, "pulp_nn_depthwise_generic"),
+    M(F_DW_LESS4, "pulp_nn_depthwise_generic_less_4_weights"),
+    M(F_LINEAR, "pulp_nn_linear"),
+    M(F_LINEAR32, "pulp_nn_linear_out_32"),
+    M(F_MAXPOOL, "pulp_nn_maxpool"),
+    M(F_AVGPOOL, "pulp_nn_avgpool"),
+    M(F_ADD, "pulp_nn_add"),
+    M(F_DW3, "pulp_nn_depthwise_3x3_s1"),
+    M(F_HWC2CHW, "hwc_to_chw"),
+    M(F_DWHWC, "depthwise_hwc"),
+    M(F_DWPW, "dw_pw_hwc"),
+    {"set_batch", set_batch, METH_O, nullptr},
+    {"_bind", bind, METH_VARARGS, nullptr},
+    {nullptr, nullptr, 0, nullptr}};
+PyMemberDef base_members[] = {{"check", T_BOOL, offsetof(Base, check), 0, "raise PulpNNError when the library rejects a call"},
+                              {nullptr, 0, 0, 0, nullptr}};
+PyTypeObject BaseType = {PyVarObject_HEAD_INIT(nullptr, 0)};
+
+// ---- Plan ---------------------------------------------------------------------------------------------------------------
+
+struct Call {
+  int f;
+  Args a;
+  unsigned inputs;  // bit i: pointer i is the chain's input
+  std::vector<pulp_nn_hip_block> blocks;
+};
+// what the plan was made from: dict[key] was value (null: absent)
+struct Guard {
+  PyObject *dict, *key, *value;
+};
+struct Plan {
+  PyObject_HEAD
+  PyObject *nn;      // Base
+  PyObject *keep;    // the argument tuples: whatever owns the addresses
+  std::vector<Call> *calls;
+  std::vector<Guard> *guards;
+  unsigned batch;
+};
+
+int fn_index(const char *name)
+{
+  for (int f = 0; f < F_SET_BATCH; f++)
+    if (!strcmp(fn_names[f], name)) return f;
+  return -1;
+}
+
+bool block_from(PyObject *t, pulp_nn_hip_block *b)
+{
+  if (!PyTuple_Check(t) || PyTuple_GET_SIZE(t) != 16) {
+    PyErr_SetString(PyExc_TypeError, "a block is a tuple of 16");
+    return false;
+  }
+  void *p[8];
+  int64_t s[8];
+  for (int half = 0, np = 0, ns = 0; half < 2; half++)
+    for (int i = 0; i < 8; i++) {
+      PyObject *o = PyTuple_GET_ITEM(t, 8 * half + i);
+      if (i < 4 ? !to_ptr(o, &p[np++]) : !to_int(o, &s[ns++])) return false;
+    }
+  *b = pulp_nn_hip_block{(const i8 *)p[0], (const i8 *)p[1], p[2], p[3], (u16)s[0], (u16)s[1], (i8)s[2], (i8)s[3],
+                         (const i8 *)p[4], (const i8 *)p[5], p[6], p[7], (u16)s[4], (u16)s[5], (i8)s[6], (i8)s[7]};
+  return true;
+}
+
+// Plan(nn, batch, [(entry point, arguments), ...], input, [(dict, (key, ...)), ...]): `input` is the object that stands for the
+// chain's input in the arguments.  The chain entry point's arguments are (x, out, dim_x, dim_y, ch, [block, ...]).  The
+// pairs name the entries the calls were made from: run() does nothing once one of them has changed.
+int plan_init(PyObject *self, PyObject *args, PyObject *)
+{
+  Plan *pl = (Plan *)self;
+  PyObject *nn, *list, *input, *from;
+  if (pl->nn) {
+    PyErr_SetString(PyExc_RuntimeError, "already initialised");
+    return -1;
+  }
+  if (!PyArg_ParseTuple(args, "O!IO!OO!", &BaseType, &nn, &pl->batch, &PyList_Type, &list, &input, &PyList_Type, &from)) return -1;
+  Py_INCREF(nn);
+  pl->nn = nn;
+  Py_INCREF(list);
+  pl->keep = list;
+  pl->calls = new std::vector<Call>();
+  pl->guards = new std::vector<Guard>();
+  for (Py_ssize_t i = 0; i < PyList_GET_SIZE(from); i++) {
+    PyObject *dict, *keys;
+    if (!PyArg_ParseTuple(PyList_GET_ITEM(from, i), "O!O!", &PyDict_Type, &dict, &PyTuple_Type, &keys)) return -1;
+    for (Py_ssize_t j = 0; j < PyTuple_GET_SIZE(keys); j++) {
+      const Guard g = {dict, PyTuple_GET_ITEM(keys, j), PyDict_GetItem(dict, PyTuple_GET_ITEM(keys, j))};
+      Py_INCREF(g.dict);
+      Py_INCREF(g.key);
+      Py_XINCREF(g.value);
+      pl->guards->push_back(g);
+    }
+  }
+  for (Py_ssize_t i = 0; i < PyList_GET_SIZE(list); i++) {
+    const char *name;
+    PyObject *a;
+    if (!PyArg_ParseTuple(PyList_GET_ITEM(list, i), "sO!", &name, &PyTuple_Type, &a)) return -1;
+    Call c = {};
+    c.f = fn_index(name);
+    if (c.f < 0) {
+      PyErr_Format(PyExc_ValueError, "unknown entry point %s", name);
+      return -1;
+    }
+    std::vector<PyObject *> v;
+    const Py_ssize_t n = fn_kind[c.f] == CHAIN ? 5 : PyTuple_GET_SIZE(a);
+    const char *spec = fn_kind[c.f] == CHAIN ? "ppiii" : kinds[fn_kind[c.f]].spec;
+    if (PyTuple_GET_SIZE(a) < n || (Py_ssize_t)strlen(spec) != n) {
+      PyErr_Format(PyExc_ValueError, "wrong number of arguments for %s", name);
+      return -1;
+    }
+    int np = 0, ns = 0;
+    for (Py_ssize_t j = 0; j < n; j++) {
+      PyObject *o = PyTuple_GET_ITEM(a, j);
+      if (spec[j] == 'p') {
+        if (o == input) c.inputs |= 1u << np;
+        else if (!to_ptr(o, &c.a.p[np])) return -1;
+        np++;
+      } else if (!to_int(o, &c.a.s[ns++])) {
+        return -1;
+      }
+    }
+    if (fn_kind[c.f] == CHAIN) {
+      PyObject *blocks = PyTuple_GetItem(a, 5);
+      if (!blocks || !PyList_Check(blocks)) return -1;
+      for (Py_ssize_t j = 0; j < PyList_GET_SIZE(blocks); j++) {
+        pulp_nn_hip_block b;
+        if (!block_from(PyList_GET_ITEM(blocks, j), &b)) return -1;
+        c.blocks.push_back(b);
+      }
+    }
+    pl->calls->push_back(c);
+  }
+  return 0;
+}
+
+// run(x): queues every call with x as the chain's input; raises like the calls themselves would.  False, with nothing
+// queued, if what the plan was made from has changed.
+PyObject *plan_run(PyObject *self, PyObject *x)
+{
+  Plan *pl = (Plan *)self;
+  Base *b = (Base *)pl->nn;
+  for (const Guard &g : *pl->guards) {
+    PyObject *v = PyDict_GetItem(g.dict, g.key);
+    if (v == g.value) continue;
+    if (!v || !g.value || !PyLong_CheckExact(v) || !PyLong_CheckExact(g.value)) Py_RETURN_FALSE;
+    const int eq = PyObject_RichCompareBool(v, g.value, Py_EQ);
+    if (eq < 0) return nullptr;
+    if (!eq) Py_RETURN_FALSE;
+  }
+  void *in;
+  if (!to_ptr(x, &in)) return nullptr;
+  int err = 0;
+  Py_BEGIN_ALLOW_THREADS
+  ((void (*)(unsigned))b->fn[F_SET_BATCH])(pl->batch);
+  for (const Call &c : *pl->calls) {
+    if (c.inputs) {
+      Args a = c.a;
+      for (int i = 0; i < 10; i++)
+        if (c.inputs >> i & 1) a.p[i] = in;
+      invoke(b, c.f, a, c.blocks.data(), (unsigned)c.blocks.size());
+    } else {
+      invoke(b, c.f, c.a, c.blocks.data(), (unsigned)c.blocks.size());
+    }
+    if (b->check && (err = last_error(b))) break;
+  }
+  Py_END_ALLOW_THREADS
+  if (err) return PyObject_CallMethod(pl->nn, "_raise", nullptr);
+  Py_RETURN_TRUE;
+}
+
+void plan_dealloc(PyObject *self)
+{
+  Plan *pl = (Plan *)self;
+  Py_XDECREF(pl->nn);
+  Py_XDECREF(pl->keep);
+  if (pl->guards)
+    for (Guard &g : *pl->guards) {
+      Py_XDECREF(g.dict);
+      Py_XDECREF(g.key);
+      Py_XDECREF(g.value);
+    }
+  delete pl->guards;
+  delete pl->calls;
+  Py_TYPE(self)->tp_free(self);
+}
+
+PyMethodDef plan_methods[] = {{"run", plan_run, METH_O, nullptr}, {nullptr, nullptr, 0, nullptr}};
+PyTypeObject PlanType = {PyVarObject_HEAD_INIT(nullptr, 0)};
+
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "_pulpnn_fast", nullptr, -1, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__pulpnn_fast(void)
+{
+  BaseType.tp_name = "_pulpnn_fast.Base";
+  BaseType.tp_basicsize = sizeof(Base);
+  BaseType.tp_flags = Py_TPFLAGS_DEFAULT | Py_TPFLAGS_BASETYPE;
+  BaseType.tp_new = PyType_GenericNew;
+  BaseType.tp_methods = base_methods;
+  BaseType.tp_members = base_members;
+  PlanType.tp_name = "_pulpnn_fast.Plan";
+  PlanType.tp_basicsize = sizeof(Plan);
+  PlanType.tp_flags = Py_TPFLAGS_DEFAULT;
+  PlanType.tp_new = PyType_GenericNew;
+  PlanType.tp_init = plan_init;
+  PlanType.tp_dealloc = plan_dealloc;
+  PlanType.tp_methods = plan_methods;
+  if (PyType_Ready(&BaseType) < 0 || PyType_Ready(&PlanType) < 0) return nullptr;
+  PyObject *m = PyModule_Create(&module);
+  if (!m) return nullptr;
+  Py_INCREF(&BaseType);
+  PyModule_AddObject(m, "Base", (PyObject *)&BaseType);
+  Py_INCREF(&PlanType);
+  PyModule_AddObject(m, "Plan", (PyObject *)&PlanType);
+  return m;
+}

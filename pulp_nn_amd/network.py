@@ -33,6 +33,7 @@ sets it to floor(log2(max |acc * k|)) - 7 over the batch it is given, computed o
 """
 import numpy as np
 
+from . import api
 from .api import PulpNNError
 
 CONV_LIKE = ("conv", "pointwise", "depthwise", "linear")
@@ -78,8 +79,32 @@ def infer_shapes(layers, input_shape):
     return shapes
 
 
+class _Recorder:
+    """Stands in for PulpNN: collects the calls of a walk over the table instead of making them."""
+    _NAMES = {"hwc_to_chw": "pulp_nn_hip_hwc_to_chw", "depthwise_hwc": "pulp_nn_hip_depthwise_hwc",
+              "dw_pw_hwc": "pulp_nn_hip_dw_pw_hwc", "dw_pw_chain_hwc": "pulp_nn_hip_dw_pw_chain_hwc"}
+
+    def __init__(self):
+        self.calls = []
+
+    def set_batch(self, n):
+        pass
+
+    def __getattr__(self, name):
+        def call(*args):
+            if name == "hwc_to_chw":
+                args += (0,) * (7 - len(args))   # pad_top, pad_bottom
+            self.calls.append((self._NAMES.get(name, name), args))
+        return call
+
+
 class Runner:
-    """Uploads the parameters once, owns the activation buffers and queues the chain."""
+    """Uploads the parameters once, owns the activation buffers and queues the chain.
+
+    The first run() walks the table in Python and learns which geometries have a fused kernel; the second lays the calls
+    out as a plan (api's extension module), and from then on a run() is one call that queues them, 2 us a launch instead of
+    9.  A plan belongs to the table and the buffers it was made from: a changed shift, flag, choice or buffer makes run()
+    walk again."""
 
     def __init__(self, nn, layers, input_shape, batch, fused=True, fuse_blocks="auto", chain_blocks=True):
         import torch
@@ -118,6 +143,8 @@ class Runner:
                 H, W, Cc = self.shapes[L["in"]]
                 self.chw[L["name"]] = torch.empty((batch, Cc, H, W), dtype=torch.uint8, device="cuda")
         self._calib = None
+        self._plan = None        # (choices, objects, plan, result tensor, launches)
+        self._walked = None      # the choices of the last walk
 
     # -- one layer ------------------------------------------------------------------------
     def _requant_args(self, L, P):
@@ -126,8 +153,8 @@ class Runner:
             raise ValueError("layer %s has no out_shift: run calibrate() first" % L["name"])
         return P.get("k"), P.get("lam"), L.get("mult", 0), L.get("shift", 0) or 0, relu, bn
 
-    def _queue(self, i, tensors):
-        L, P, nn = self.layers[i], self.params[i], self.nn
+    def _queue(self, i, tensors, nn=None):
+        L, P, nn = self.layers[i], self.params[i], nn or self.nn
         op, out = L["op"], self.act[L["name"]]
         if op == "add":
             a, b = tensors[L["in"][0]], tensors[L["in"][1]]
@@ -188,7 +215,37 @@ class Runner:
 
     def run(self, x):
         """x: device tensor batch,H,W,C uint8.  Queues every layer; returns the last layer's tensor."""
-        self.nn.set_batch(self.batch)
+        choices = self._choices()
+        if self._plan is None and self._walked == choices and self.layers:
+            self._lay_out_plan(choices)
+        if self._plan is not None:
+            made_with, objects, plan, out, launches = self._plan
+            if made_with == choices and all(a is b for a, b in zip(objects, self._objects())) and plan.run(x):
+                self.launches = launches
+                return out
+            self._plan = None
+        out = self._walk(x, self.nn)
+        self._walked = self._choices()
+        return out
+
+    def _choices(self):
+        return (len(self.layers), self.batch, self.fused, self.fuse_blocks, self.chain_blocks, len(self.unfused),
+                len(self.unfused_blocks), len(self.unchained), tuple(self.block_choice.items()))
+
+    def _objects(self):
+        return self.nn, self.layers, self.params, self.act, self.chw
+
+    def _lay_out_plan(self, choices):
+        """The calls of a walk (the last one has met every geometry without a kernel), and the entries they are made from."""
+        marker, rec = object(), _Recorder()
+        out = self._walk(marker, rec)
+        scalars = {"add": ("m1", "m2", "shift"), "avgpool": ("lam", "shift", "add", "requant"), "maxpool": (), "linear_out_32": ()}
+        made_from = [(L, scalars.get(L["op"], ("shift", "mult", "relu", "bn"))) for L in self.layers]
+        made_from += [(P, tuple(P)) for P in self.params] + [(d, tuple(d)) for d in (self.act, self.chw)]
+        self._plan = (choices, self._objects(), api._fast.Plan(self.nn, self.batch, rec.calls, marker, made_from), out, self.launches)
+
+    def _walk(self, x, nn):
+        nn.set_batch(self.batch)
         tensors = {"input": x}
         out = x
         self.launches = 0
@@ -196,16 +253,16 @@ class Runner:
         while i < len(self.layers):
             L = self.layers[i]
             n = self._chain_length(i) if self.chain_blocks else 0
-            if n >= 2 and self._queue_chain(i, n, tensors):
+            if n >= 2 and self._queue_chain(i, n, tensors, nn):
                 last = self.layers[i + 2 * n - 1]["name"]
                 out = tensors[last] = self.act[last]
                 i += 2 * n
                 continue
-            if self._block_fusable(i) and self._queue_block(i, tensors):
+            if self._block_fusable(i) and self._queue_block(i, tensors, nn):
                 out = tensors[self.layers[i + 1]["name"]] = self.act[self.layers[i + 1]["name"]]
                 i += 2
                 continue
-            out = tensors[L["name"]] = self._queue(i, tensors)
+            out = tensors[L["name"]] = self._queue(i, tensors, nn)
             self.launches += 2 if (L["op"] == "depthwise" and (not self.fused or i in self.unfused)) else 1
             i += 1
         return out
@@ -261,8 +318,8 @@ class Runner:
             n += 1
         return n
 
-    def _queue_chain(self, i, n, tensors):
-        nn = self.nn
+    def _queue_chain(self, i, n, tensors, nn=None):
+        nn = nn or self.nn
         H, W, Cc = self.shapes[self.layers[i]["in"]]
         blocks = []
         for j in range(n):
@@ -280,8 +337,8 @@ class Runner:
         self.launches += 1
         return True
 
-    def _queue_block(self, i, tensors):
-        L, P, N, Q, nn = self.layers[i], self.params[i], self.layers[i + 1], self.params[i + 1], self.nn
+    def _queue_block(self, i, tensors, nn=None):
+        L, P, N, Q, nn = self.layers[i], self.params[i], self.layers[i + 1], self.params[i + 1], nn or self.nn
         H, W, Cc = self.shapes[L["in"]]
         Ho, Wo, Co = self.shapes[N["name"]]
         k1, l1, m1, s1, r1, b1 = self._requant_args(L, P)
