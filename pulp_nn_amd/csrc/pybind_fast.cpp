@@ -16,6 +16,7 @@
 #include <stdint.h>
 #include <string.h>
 
+#include <exception>
 #include <string>
 #include <vector>
 
@@ -80,7 +81,7 @@ struct Args {
 
 // tensor / address / None -> device address
 bool to_ptr(PyObject *o, void **out)
-{
+try {
   if (o == Py_None) {
     *out = nullptr;
     return true;
@@ -103,6 +104,9 @@ bool to_ptr(PyObject *o, void **out)
     return *out || !PyErr_Occurred();
   }
   PyErr_Format(PyExc_TypeError, "expected a tensor, an address or None, not %.100s", Py_TYPE(o)->tp_name);
+  return false;
+} catch (const std::exception &e) {  // a tensor without storage (a fake or a functional one) has no address
+  if (!PyErr_Occurred()) PyErr_SetString(PyExc_RuntimeError, e.what());
   return false;
 }
 
@@ -323,10 +327,12 @@ PyTypeObject BaseType = {PyVarObject_HEAD_INIT(nullptr, 0)};
 
 // ---- Plan ---------------------------------------------------------------------------------------------------------------
 
+// Addresses are asked for at each run, as a call by itself would: a tensor may have been given other storage since.
 struct Call {
   int f;
   Args a;
-  unsigned inputs;  // bit i: pointer i is the chain's input
+  PyObject *owner[10];  // what pointer i belongs to; null: the chain's input
+  PyObject *block_list;  // the chain entry point's
   std::vector<pulp_nn_hip_block> blocks;
 };
 // what the plan was made from: dict[key] was value (null: absent)
@@ -414,19 +420,24 @@ int plan_init(PyObject *self, PyObject *args, PyObject *)
       return -1;
     }
     int np = 0, ns = 0;
+    for (PyObject *&o : c.owner) o = Py_None;
     for (Py_ssize_t j = 0; j < n; j++) {
       PyObject *o = PyTuple_GET_ITEM(a, j);
       if (spec[j] == 'p') {
-        if (o == input) c.inputs |= 1u << np;
-        else if (!to_ptr(o, &c.a.p[np])) return -1;
-        np++;
+        if (o != input && !to_ptr(o, &c.a.p[np])) return -1;
+        c.owner[np++] = o == input ? nullptr : o;
       } else if (!to_int(o, &c.a.s[ns++])) {
         return -1;
       }
     }
     if (fn_kind[c.f] == CHAIN) {
       PyObject *blocks = PyTuple_GetItem(a, 5);
-      if (!blocks || !PyList_Check(blocks)) return -1;
+      if (!blocks) return -1;
+      if (!PyList_Check(blocks)) {
+        PyErr_SetString(PyExc_TypeError, "the blocks are a list");
+        return -1;
+      }
+      c.block_list = blocks;
       for (Py_ssize_t j = 0; j < PyList_GET_SIZE(blocks); j++) {
         pulp_nn_hip_block b;
         if (!block_from(PyList_GET_ITEM(blocks, j), &b)) return -1;
@@ -452,20 +463,17 @@ PyObject *plan_run(PyObject *self, PyObject *x)
     if (eq < 0) return nullptr;
     if (!eq) Py_RETURN_FALSE;
   }
-  void *in;
-  if (!to_ptr(x, &in)) return nullptr;
+  for (Call &c : *pl->calls) {
+    for (int i = 0; i < 10; i++)
+      if (c.owner[i] != Py_None && !to_ptr(c.owner[i] ? c.owner[i] : x, &c.a.p[i])) return nullptr;
+    for (size_t i = 0; i < c.blocks.size(); i++)
+      if (!block_from(PyList_GET_ITEM(c.block_list, i), &c.blocks[i])) return nullptr;
+  }
   int err = 0;
   Py_BEGIN_ALLOW_THREADS
   ((void (*)(unsigned))b->fn[F_SET_BATCH])(pl->batch);
   for (const Call &c : *pl->calls) {
-    if (c.inputs) {
-      Args a = c.a;
-      for (int i = 0; i < 10; i++)
-        if (c.inputs >> i & 1) a.p[i] = in;
-      invoke(b, c.f, a, c.blocks.data(), (unsigned)c.blocks.size());
-    } else {
-      invoke(b, c.f, c.a, c.blocks.data(), (unsigned)c.blocks.size());
-    }
+    invoke(b, c.f, c.a, c.blocks.data(), (unsigned)c.blocks.size());
     if (b->check && (err = last_error(b))) break;
   }
   Py_END_ALLOW_THREADS

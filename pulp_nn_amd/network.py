@@ -233,14 +233,17 @@ class Runner:
                 len(self.unfused_blocks), len(self.unchained), tuple(self.block_choice.items()))
 
     def _objects(self):
-        return self.nn, self.layers, self.params, self.act, self.chw
+        return (self.nn, self.layers, self.params, self.act, self.chw, *self.layers)
 
     def _lay_out_plan(self, choices):
         """The calls of a walk (the last one has met every geometry without a kernel), and the entries they are made from."""
         marker, rec = object(), _Recorder()
         out = self._walk(marker, rec)
         scalars = {"add": ("m1", "m2", "shift"), "avgpool": ("lam", "shift", "add", "requant"), "maxpool": (), "linear_out_32": ()}
-        made_from = [(L, scalars.get(L["op"], ("shift", "mult", "relu", "bn"))) for L in self.layers]
+        shape = {"add": (), "linear": (), "linear_out_32": (), "pointwise": (), "maxpool": ("kernel", "strides", "pads"),
+                 "avgpool": ("kernel", "strides")}
+        made_from = [(L, ("op", "in") + shape.get(L["op"], ("strides", "pads")) +
+                      scalars.get(L["op"], ("shift", "mult", "relu", "bn"))) for L in self.layers]
         made_from += [(P, tuple(P)) for P in self.params] + [(d, tuple(d)) for d in (self.act, self.chw)]
         self._plan = (choices, self._objects(), api._fast.Plan(self.nn, self.batch, rec.calls, marker, made_from), out, self.launches)
 

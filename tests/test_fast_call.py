@@ -52,3 +52,24 @@ def test_plan_notices_changed_entries(nn):
     assert plan.run(0) is False
     with pytest.raises(ValueError):
         api._fast.Plan(nn, 1, [("pulp_nn_nothing", ())], marker, [])
+
+
+@pytest.mark.gpu
+def test_plan_asks_for_addresses_at_each_run(nn):
+    """A chain's buffer that has other storage than when the plan was made: the run uses the new one.  A tensor without an
+    address: an exception, at the call, at the plan and at the run."""
+    marker = object()
+    a, b, x, y = (torch.full((64,), v, dtype=torch.uint8, device="cuda") for v in (3, 5, 10, 20))
+    out = torch.zeros(64, dtype=torch.uint8, device="cuda")
+    nn.use_torch_stream()
+    plan = api._fast.Plan(nn, 1, [("pulp_nn_add", (marker, a, out, 1, 1, 0, 1, 1, 64))], marker, [])
+    assert plan.run(x) is True
+    assert (out.cpu() == 13).all()
+    a.set_(b)
+    assert plan.run(y) is True
+    assert (out.cpu() == 25).all()
+    none = torch.zeros(64, dtype=torch.uint8, device="cuda").to_sparse()
+    for refused in (lambda: nn.pulp_nn_add(none, a, out, 1, 1, 0, 1, 1, 64), lambda: plan.run(none),
+                    lambda: api._fast.Plan(nn, 1, [("pulp_nn_add", (marker, none, out, 1, 1, 0, 1, 1, 64))], marker, [])):
+        with pytest.raises((RuntimeError, ValueError)):
+            refused()
