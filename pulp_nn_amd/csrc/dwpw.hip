@@ -92,16 +92,20 @@ void dwpw_common(const char *fn, const unsigned char *Im_in, unsigned char *Im_o
   if (g.KT == 1) hipLaunchKernelGGL((dwpw_fused_kernel<WB, RR, SS, NW, TM, 1>), grid, block, lds, g_stream, g);      \
   else if (g.KT == 2) hipLaunchKernelGGL((dwpw_fused_kernel<WB, RR, SS, NW, TM, 2>), grid, block, lds, g_stream, g); \
   else hipLaunchKernelGGL((dwpw_fused_kernel<WB, RR, SS, NW, TM, 4>), grid, block, lds, g_stream, g);
-#define DWPW_CHAIN_KP(WB, RR, NW, TM)                                                                                     \
-  if (g.KT == 1) hipLaunchKernelGGL((dwpw_fused_kernel<WB, RR, 1, NW, TM, 1, true>), grid, block, lds, g_stream, g);      \
-  else if (g.KT == 2) hipLaunchKernelGGL((dwpw_fused_kernel<WB, RR, 1, NW, TM, 2, true>), grid, block, lds, g_stream, g); \
-  else hipLaunchKernelGGL((dwpw_fused_kernel<WB, RR, 1, NW, TM, 4, true>), grid, block, lds, g_stream, g);
+#define DWPW_CHAIN_KP(WB, RR, NW, TM, NT)                                                                                     \
+  if (g.KT == 1) hipLaunchKernelGGL((dwpw_fused_kernel<WB, RR, 1, NW, TM, 1, true, NT>), grid, block, lds, g_stream, g);      \
+  else if (g.KT == 2) hipLaunchKernelGGL((dwpw_fused_kernel<WB, RR, 1, NW, TM, 2, true, NT>), grid, block, lds, g_stream, g); \
+  else hipLaunchKernelGGL((dwpw_fused_kernel<WB, RR, 1, NW, TM, 4, true, NT>), grid, block, lds, g_stream, g);
+  // Stage-2 blocks of 64 pixels x 32 channels instead of 32 x 64: each weight fragment then goes to one wave of the tile,
+  // not to two.
+  const bool wide_px = g.BM % 64 == 0 && C >= 64;
   if (n_blocks > 1) {
     // (stride 1 only; the widest planes never fit the LDS of a chained launch)
-    if (W == 32) { DWPW_CHAIN_KP(32, 4, 4, 2) }
-    else if (W == 16) { DWPW_CHAIN_KP(16, 4, 8, 2) }
-    else if (W == 8) { DWPW_CHAIN_KP(8, 4, 8, 2) }
-    else if (W == 4) { DWPW_CHAIN_KP(4, 4, 8, 2) }
+    if (W == 32) { DWPW_CHAIN_KP(32, 4, 4, 2, 4) }
+    else if (W == 16) { DWPW_CHAIN_KP(16, 4, 8, 2, 4) }
+    else if (W == 8 && wide_px) { DWPW_CHAIN_KP(8, 4, 8, 4, 2) }
+    else if (W == 8) { DWPW_CHAIN_KP(8, 4, 8, 2, 4) }
+    else if (W == 4) { DWPW_CHAIN_KP(4, 4, 8, 2, 4) }
     else return set_error(PULP_NN_HIP_ERR_UNSUPPORTED, fn, "blocks of this width cannot be chained");
     check_launch(fn);
     return;

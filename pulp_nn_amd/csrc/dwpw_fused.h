@@ -29,6 +29,13 @@
 // there, and only the last block's output leaves the chip.  The blocks' parameters are an array in the kernel
 // arguments.  The weight fragments of a wave's first stage-2 block of the next block are requested behind the
 // MFMAs of its last one in this block: they travel during the epilogue, the barrier and the next depthwise stage.
+//
+// What bounds a chain is one workgroup per compute unit at two waves per SIMD: of the 14000 cycles a block of 64 pixels x
+// 256 channels takes, the depthwise stage's vector instructions are 6000, the multiplication and the requests for the next
+// weights 4400, the epilogue 3000.  It was 19500: the nine filter bytes, k, lambda and the pointwise constants were fetched
+// when they were needed (2000 cycles a block in two waits), and blocks of 32 pixels x 64 channels had each weight fragment
+// fetched by two waves and its 128-byte lines twice by each (the requests alone held a wave up for 5500 cycles).  With 64
+// pixels x 32 channels a fragment goes to one wave.  Five blocks of 8 x 8 x 256: 48 -> 36 us at batch 256, 43 -> 32 at batch 1.
 #pragma once
 #include "depthwise.h"
 #include "igemm.h"
@@ -72,11 +79,13 @@ __host__ __device__ static inline int dwpw_const_bytes(int nch) { return nch * (
 // is 16*TMB pixels x 64 channels.  KP: K slices whose weight fragments a wave holds at once (a pass over K).
 // The requantisation branches of both layers are run-time switches: one kernel per geometry, not nine.
 // CHAIN: g.nblocks blocks back to back; otherwise the one block g.blk[0], with nothing of the chain's loop left.
-template <int WB, int R, int S, int NWV, int TMB, int KP, bool CHAIN = false>
+// NT: weight fragments of a stage-2 block, 16 channels each (a lane ends up with 4*NT consecutive channels).
+template <int WB, int R, int S, int NWV, int TMB, int KP, bool CHAIN = false, int NT = 4>
 __global__ __launch_bounds__(64 * NWV) void dwpw_fused_kernel(DwPwGeom g)
 {
   constexpr int DWPW_WAVES = NWV;
   constexpr int BP = 16 * TMB;          // pixels of a stage-2 block
+  constexpr int BN = 16 * NT;           // ... and its channels
   constexpr int RD = WB / 4;            // dwords per input row (per channel, after the transpose)
   constexpr int WO = (WB - 1) / S + 1;  // output columns
   constexpr int XG = WO / 4;            // groups of 4 output columns
@@ -95,11 +104,11 @@ __global__ __launch_bounds__(64 * NWV) void dwpw_fused_kernel(DwPwGeom g)
   const bool narrow = g.C < 64;                 // rows of C bytes instead of 64-byte K slices
 
   const int MB = g.BM / BP;                     // pixel blocks of the tile
-  const int NBT = (g.Co + 63) / 64;             // channel blocks of the layer
+  const int NBT = (g.Co + BN - 1) / BN;         // channel blocks of the layer
   const int nb_per = (NBT + g.nsplit - 1) / g.nsplit;
   const int nb_lo = part * nb_per, nb_hi = min(NBT, nb_lo + nb_per);
   const int nblk = MB * max(nb_hi - nb_lo, 0);  // blocks of this workgroup, dealt to the waves in turn
-  const int nch = max(nb_hi - nb_lo, 0) * 64;
+  const int nch = max(nb_hi - nb_lo, 0) * BN;
   int *c_bias = (int *)(dwpw_lds + dwpw_lds_bytes(g.BM, g.C));
   bn_t *c_k = (bn_t *)(c_bias + nch), *c_l = c_k + nch;
   // the output of a block that another block follows: [tile pixel][Co + DWPW_YPAD] bytes, the next block's HWC input
@@ -107,45 +116,70 @@ __global__ __launch_bounds__(64 * NWV) void dwpw_fused_kernel(DwPwGeom g)
   typedef unsigned v4u __attribute__((ext_vector_type(4)));
   const v4i ones = {0x01010101, 0x01010101, 0x01010101, 0x01010101};
 
-  // weight fragment t of channel block nb: row i of the fragment is channel nb*64 + (i/4)*16 + 4*t + i%4, so that a
-  // lane ends up with 16 consecutive channels (the order igemm.h uses)
-  auto load_w = [&](const int8_t *pw_w, v4i (&wf)[KP][4], int nb, int kt0) {
+  // weight fragment t of channel block nb: row i of the fragment is channel nb*BN + (i/4)*4*NT + 4*t + i%4, so that a
+  // lane ends up with 4*NT consecutive channels (the order igemm.h uses).  The K slices of a fragment are requested one
+  // after the other: two of them are the halves of the same 128-byte lines.
+  auto load_w = [&](const int8_t *pw_w, v4i (&wf)[KP][NT], int nb, int kt0) {
     const __amdgpu_buffer_rsrc_t rsrc_w = __builtin_amdgcn_make_buffer_rsrc((void *)pw_w, 0, (unsigned)g.Co * (unsigned)g.C, 0x00020000);
 #pragma unroll
-    for (int kk = 0; kk < KP; kk++)
+    for (int t = 0; t < NT; t++)
 #pragma unroll
-      for (int t = 0; t < 4; t++) {
-        const int n = nb * 64 + (l16 >> 2) * 16 + 4 * t + (l16 & 3);
+      for (int kk = 0; kk < KP; kk++) {
+        const int n = nb * BN + (l16 >> 2) * (4 * NT) + 4 * t + (l16 & 3);
         const int kb = 64 * (kt0 + kk) + 16 * lgrp;
         const unsigned off = (n < g.Co && kb < g.C && kt0 + kk < g.KT) ? (unsigned)(n * g.C + kb) : 0xffffffffu;
         const v4u v = __builtin_amdgcn_raw_buffer_load_b128(rsrc_w, off, 0, 0);
         wf[kk][t] = (v4i){(int)v.x, (int)v.y, (int)v.z, (int)v.w};
       }
   };
-  v4i wf[KP][4];
+  v4i wf[KP][NT];
   int wf_nb = -1;  // channel block whose first-pass fragments wf holds
   const int nblocks = CHAIN ? g.nblocks : 1;
+
+  // Everything a block needs from memory besides the activations is requested one block ahead (the first block's at
+  // once): the pointwise layer's per-channel constants of this workgroup's channel blocks, which go to LDS behind the
+  // activation operand, and the filter and constants of the channel this lane takes in its first depthwise item.
+  constexpr int NCI = (1024 + 64 * DWPW_WAVES - 1) / (64 * DWPW_WAVES);  // at most 1024 output channels
+  int cb_[NCI];
+  bn_t ck_[NCI], cl_[NCI];
+  auto load_consts = [&](const DwPwBlock &P) {
+#pragma unroll
+    for (int q = 0; q < NCI; q++) {
+      const int c = tid + q * 64 * DWPW_WAVES, n = nb_lo * BN + c;
+      const bool ok = c < nch && n < g.Co;
+      cb_[q] = (P.pw_bias && ok) ? (int)P.pw_bias[n] : 0;
+      ck_[q] = (P.mode_pw == EPI_BN && ok) ? P.e_pw.k[n] : (bn_t)0;
+      cl_[q] = (P.mode_pw == EPI_BN && ok) ? P.e_pw.lambda[n] : (bn_t)0;
+    }
+  };
+  int dw_w[3], dw_b;  // the nine filter bytes, bias
+  bn_t dw_k, dw_l;
+  auto load_dw = [&](const DwPwBlock &P, int ch) {
+    typedef int i32_u __attribute__((aligned(1)));
+    const int8_t *p = P.dw_wt + (long long)ch * 9;
+    dw_w[0] = *(const i32_u *)p;
+    dw_w[1] = *(const i32_u *)(p + 4);
+    dw_w[2] = (int)p[8];
+    dw_b = P.dw_bias ? (int)P.dw_bias[ch] : 0;
+    dw_k = dw_l = 0;
+    if (P.mode_dw == EPI_BN) {
+      dw_k = P.e_dw.k[ch];
+      dw_l = P.e_dw.lambda[ch];
+    }
+  };
+  const int CGN = g.C >= 64 ? g.C / 64 : 1;  // channel groups
+  const int LG = g.C >= 64 ? 1 : 64 / g.C;   // row groups inside a wave (fewer than 64 channels)
+  auto item_ch = [&](int it) { return g.C >= 64 ? (it % CGN) * 64 + lane : lane % g.C; };
+  load_dw(g.blk[0], item_ch(wave));
+  load_consts(g.blk[0]);
 #pragma unroll 1
   for (int j = 0; j < nblocks; j++) {
     const DwPwBlock &P = g.blk[CHAIN ? j : 0];
     const bool first = !CHAIN || j == 0, last = !CHAIN || j == nblocks - 1;
 
     // ---- stage 2 set-up ------------------------------------------------------------------------------------
-    // The pointwise layer's per-channel constants of this workgroup's channel blocks go to LDS (behind the
-    // activation operand), where every stage-2 block's epilogue reads them.  Their loads are issued first and the
-    // weight fragments' behind them: loads complete in order, so the wait for the constants leaves the fragments
-    // in flight.
-    constexpr int NCI = (1024 + 64 * DWPW_WAVES - 1) / (64 * DWPW_WAVES);  // at most 1024 output channels
-    int cb_[NCI];
-    bn_t ck_[NCI], cl_[NCI];
-#pragma unroll
-    for (int q = 0; q < NCI; q++) {
-      const int c = tid + q * 64 * DWPW_WAVES, n = nb_lo * 64 + c;
-      const bool ok = c < nch && n < g.Co;
-      cb_[q] = (P.pw_bias && ok) ? (int)P.pw_bias[n] : 0;
-      ck_[q] = (P.mode_pw == EPI_BN && ok) ? P.e_pw.k[n] : (bn_t)0;
-      cl_[q] = (P.mode_pw == EPI_BN && ok) ? P.e_pw.lambda[n] : (bn_t)0;
-    }
+    // (loads complete in order, and the weight fragments' are issued behind the constants': the wait for the constants
+    // leaves the fragments in flight)
     // this wave's first stage-2 block: its weight fragments are requested now (first block of the launch; for the
     // others the request went out behind the MFMAs of the block before)
     if (first && wave < nblk) {
@@ -164,15 +198,13 @@ __global__ __launch_bounds__(64 * NWV) void dwpw_fused_kernel(DwPwGeom g)
 
     // ---- stage 1: depthwise into LDS ---------------------------------------------------------------------
     {
-      const int CGN = g.C >= 64 ? g.C / 64 : 1;  // channel groups
-      const int LG = g.C >= 64 ? 1 : 64 / g.C;   // row groups inside a wave (fewer than 64 channels)
       const int item_px = R * LG * WO;
       const int nitems = (g.BM / item_px) * CGN;
       const unsigned sel1 = quad_sel1(lane), sel2 = quad_sel2(lane);
       for (int it = wave; it < nitems; it += DWPW_WAVES) {
-        const int cg = it % CGN, seg = it / CGN;
+        const int seg = it / CGN;
         const int lg = g.C >= 64 ? 0 : lane / g.C;
-        const int ch = g.C >= 64 ? cg * 64 + lane : lane % g.C;
+        const int ch = item_ch(it);
         const int mi = m0 + seg * item_px;  // first pixel of the item (all of it in one image)
         if (mi >= g.M) break;
         const int b = (int)fastdiv((unsigned)mi, g.d_howo);
@@ -201,22 +233,13 @@ __global__ __launch_bounds__(64 * NWV) void dwpw_fused_kernel(DwPwGeom g)
         for (int r = 0; r < NIN; r++)
 #pragma unroll
           for (int d = 0; d < RD; d++) row[r][d] = quad_transpose4x4_perm(row[r][d], sel1, sel2) ^ 0x80808080u;
-        unsigned wA[3], wB[3];
-        int wsum = 0;
-#pragma unroll
-        for (int i = 0; i < 3; i++) {
-          const int8_t *p = P.dw_wt + (long long)ch * 9 + 3 * i;
-          const unsigned k0 = (uint8_t)p[0], k1 = (uint8_t)p[1], k2 = (uint8_t)p[2];
-          wA[i] = k0 | (k1 << 8) | (k2 << 16);
-          wB[i] = wA[i] << 8;
-          wsum += (int)p[0] + (int)p[1] + (int)p[2];
-        }
-        const int corr = 128 * wsum + (P.dw_bias ? (int)P.dw_bias[ch] : 0);
-        bn_t kk = 0, ll = 0;
-        if (P.mode_dw == EPI_BN) {
-          kk = P.e_dw.k[ch];
-          ll = P.e_dw.lambda[ch];
-        }
+        if (it != wave) load_dw(P, ch);
+        const unsigned w0 = (unsigned)dw_w[0], w1 = (unsigned)dw_w[1], w2 = (unsigned)dw_w[2];
+        const unsigned wA[3] = {w0 & 0xffffffu, __builtin_amdgcn_alignbyte(w1, w0, 3) & 0xffffffu, (w1 >> 16) | ((w2 & 255u) << 16)};
+        const unsigned wB[3] = {wA[0] << 8, wA[1] << 8, wA[2] << 8};
+        const int wsum = __builtin_amdgcn_sdot4((int)w0, 0x01010101, __builtin_amdgcn_sdot4((int)w1, 0x01010101, dw_w[2], false), false);
+        const int corr = 128 * wsum + dw_b;
+        const bn_t kk = dw_k, ll = dw_l;
         const int dw_mult = P.e_dw.mult, dw_shift = P.e_dw.shift;
         const bool fastq = (P.mode_dw == EPI_BN) ? __all(bn_k_small(kk)) : (dw_shift >= 16);
         // after the quad transpose this lane holds channels (ch & ~3) .. + 3 of pixel column 4*xg + lane%4:
@@ -271,11 +294,15 @@ __global__ __launch_bounds__(64 * NWV) void dwpw_fused_kernel(DwPwGeom g)
     // narrow rows: chunk lgrp of a row if it exists, else chunk 0 (multiplied by zero weights)
     const int nar_off = l16 * g.C + ((16 * lgrp < g.C) ? 16 * lgrp : 0);
     const int pw_mult = P.e_pw.mult, pw_shift = P.e_pw.shift;
+    if (!last) {
+      load_dw(g.blk[CHAIN ? j + 1 : 0], item_ch(wave));
+      load_consts(g.blk[CHAIN ? j + 1 : 0]);
+    }
     for (int blk = wave; blk < nblk; blk += DWPW_WAVES) {
       const int mb = blk % MB, nb = nb_lo + blk / MB;
-      v4i acc[4][TMB], wacc[4];
+      v4i acc[NT][TMB], wacc[NT];
 #pragma unroll
-      for (int t = 0; t < 4; t++) {
+      for (int t = 0; t < NT; t++) {
         wacc[t] = (v4i){0, 0, 0, 0};
 #pragma unroll
         for (int s = 0; s < TMB; s++) acc[t][s] = (v4i){0, 0, 0, 0};
@@ -297,7 +324,7 @@ __global__ __launch_bounds__(64 * NWV) void dwpw_fused_kernel(DwPwGeom g)
 #pragma unroll
             for (int s = 0; s < TMB; s++) af[s] = *(const v4i *)(ab + s * sstep);
 #pragma unroll
-            for (int t = 0; t < 4; t++) {
+            for (int t = 0; t < NT; t++) {
 #pragma unroll
               for (int s = 0; s < TMB; s++) acc[t][s] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wf[kk][t], af[s], acc[t][s], 0, 0, 0);
               wacc[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wf[kk][t], ones, wacc[t], 0, 0, 0);
@@ -313,19 +340,19 @@ __global__ __launch_bounds__(64 * NWV) void dwpw_fused_kernel(DwPwGeom g)
         load_w(g.blk[CHAIN ? j + 1 : 0].pw_w, wf, wf_nb, 0);
       }
       // epilogue: acc[t][s][r] = channel cb + 4*t + r of pixel m0 + mb*BP + 16*s + l16; wacc[t][r] = sum of that channel's weights
-      const int cb = nb * 64 + lgrp * 16;
+      const int cb = nb * BN + lgrp * 4 * NT;
       const bool acc24 = g.C <= 256;  // |acc| <= K * 255 * 128 + 128 < 2^23
-      unsigned packed[TMB][4];
+      unsigned packed[TMB][NT];
       auto requantise = [&](auto md) {
         constexpr int MODE_PW = decltype(md)::value;
 #pragma unroll
-        for (int t = 0; t < 4; t++) {
+        for (int t = 0; t < NT; t++) {
           int corr[4];
           bn_t kk[4], ll[4];
           bool ks = true;
 #pragma unroll
           for (int r = 0; r < 4; r++) {
-            const int c = cb + 4 * t + r - nb_lo * 64;  // channel inside this workgroup's range (constants past Co are zero)
+            const int c = cb + 4 * t + r - nb_lo * BN;  // channel inside this workgroup's range (constants past Co are zero)
             kk[r] = (MODE_PW == EPI_BN) ? c_k[c] : (bn_t)0;
             ll[r] = (MODE_PW == EPI_BN) ? c_l[c] : (bn_t)0;
             ks = ks && bn_k_small(kk[r]);
@@ -348,9 +375,12 @@ __global__ __launch_bounds__(64 * NWV) void dwpw_fused_kernel(DwPwGeom g)
       for (int s = 0; s < TMB; s++) {
         const int pl = mb * BP + 16 * s + l16;  // tile-local pixel
         if (m0 + pl < g.M && cb < g.Co) {
-          const v4i v = {(int)packed[s][0], (int)packed[s][1], (int)packed[s][2], (int)packed[s][3]};
-          if (last) *(v4i *)(g.out + (long long)(m0 + pl) * g.Co + cb) = v;
-          else *(v4i *)(ylds + pl * (g.Co + DWPW_YPAD) + cb) = v;
+          typedef int vnt __attribute__((ext_vector_type(NT)));
+          vnt v;
+#pragma unroll
+          for (int t = 0; t < NT; t++) v[t] = (int)packed[s][t];
+          if (last) *(vnt *)(g.out + (long long)(m0 + pl) * g.Co + cb) = v;
+          else *(vnt *)(ylds + pl * (g.Co + DWPW_YPAD) + cb) = v;
         }
       }
     }

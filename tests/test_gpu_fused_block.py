@@ -128,6 +128,9 @@ CHAINS = [
     (5, 16, 16, 64, 2),
     (4, 8, 8, 128, 8),       # the most blocks one launch takes
     (9, 8, 8, 64, 1),        # a single block through the chain entry point
+    (3, 8, 8, 384, 2),       # 64-pixel x 32-channel blocks of the pointwise stage: two passes over K
+    (2, 8, 8, 192, 3),       # ... three K slices
+    (3, 4, 8, 128, 2),       # tiles of 32 pixels: blocks of 32 pixels x 64 channels
 ]
 
 
