@@ -267,9 +267,7 @@ __device__ __forceinline__ void dw3x3_column(DwColumn c)
 // 3x3 depthwise, fast variant for W % 4 == 0 and a 16-byte aligned input.
 //
 // LDS holds the band exactly as it lies in memory (rows of W bytes back to back,
-// no column padding), so staging is a linear copy: each wave copies the
-// contiguous run of each of its 16 channels with one 16-byte load per lane, all
-// loads in flight before the first LDS write.  The columns left of 0 and right
+// no column padding), so staging is a linear copy.  The columns left of 0 and right
 // of W-1 are supplied in the compute phase instead: a wave works on one group of
 // 4 output columns at a time and walks down the rows of the band, so whether a
 // dword of the 3-dword window lies outside the row is decided once per column
@@ -289,7 +287,7 @@ __device__ __forceinline__ void dw3x3_column(DwColumn c)
 template <int S, int PL, int MODE, bool FULL, bool DMA = false>
 __global__ __launch_bounds__(64 * DW_WAVES) void dw3x3_lin_kernel(DwGeom g, EpiArgs e)
 {
-  static_assert(!DMA || FULL, "LDS-direct staging only for whole 64-channel groups");
+  static_assert(DMA && FULL, "whole 64-channel groups, staged by LDS-direct loads");
   constexpr int NWV = DW_WAVES, CPW = DW_CG / NWV;  // waves, channels staged per wave
   extern __shared__ unsigned dw_lds[];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -305,12 +303,9 @@ __global__ __launch_bounds__(64 * DW_WAVES) void dw3x3_lin_kernel(DwGeom g, EpiA
   const int rows = min(g.RB, g.Ho - oy0);
   const int iy_start = oy0 * S - g.pt;
   const int LWD = g.LWD;  // = W / 4
-  const int dummy = DW_CG * g.CSD;  // one spare dword behind the tile: target of masked-off writes
 
   // ---- stage -----------------------------------------------------------------
   const int r_lo = max(0, -iy_start), r_hi = min(g.NR, g.H - iy_start);  // rows of the band inside the image
-  const int run_len = max(r_hi - r_lo, 0) * g.W;                        // bytes per channel
-  const bool two = run_len + 12 > 64 * 16;  // a run may need more than 64 chunks
   if constexpr (DMA) {
     // Lane l fetches the 16-byte chunk l of a channel's band (dwords 4l .. 4l+3).  Dwords [lo_d, hi_d) lie inside
     // the image; a chunk wholly outside is requested out of range (zeros); a chunk that straddles the first or last
@@ -341,40 +336,6 @@ __global__ __launch_bounds__(64 * DW_WAVES) void dw3x3_lin_kernel(DwGeom g, EpiA
       if (act4) __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_in, (lds_ptr_t)dst, 16, (int)voff4, soff, 0, 0);
       if (q1 >= 0) fix(dst, soff, q1);
       if (q2 >= 0 && q2 != q1) fix(dst, soff, q2);
-    }
-  } else {
-    v4i ld[CPW][2];
-    int mis[CPW];
-#pragma unroll
-    for (int cc = 0; cc < CPW; cc++) {
-      const long long pl_ = min((long long)b * g.CH + min(c0 + wave + NWV * cc, g.CH - 1), g.planes - 1);
-      const uint8_t *g0 = g.in + (pl_ * g.H + min(max(iy_start + r_lo, 0), g.H - 1)) * g.W;
-      mis[cc] = (int)((uintptr_t)g0 & 15);
-      const int last = max(((run_len + mis[cc] + 15) >> 4) - 1, 0);
-      // lanes past the end of the run re-read its last chunk (masked off below)
-      ld[cc][0] = *(const v4i *)(g0 - mis[cc] + 16 * min(lane, last));
-      if (two) ld[cc][1] = *(const v4i *)(g0 - mis[cc] + 16 * min(lane + 64, last));
-    }
-#pragma unroll
-    for (int cc = 0; cc < CPW; cc++) {
-      const int c = wave + NWV * cc;
-      const int dst = c * g.CSD + r_lo * LWD;
-      const unsigned keep = (c0 + c < g.CH && (long long)b * g.CH + c0 + c < g.planes) ? 0xFFFFFFFFu : 0u;
-#pragma unroll
-      for (int t = 0; t < 2; t++) {
-        if (t == 1 && !two) break;
-        const int o = 16 * (lane + 64 * t) - mis[cc];  // byte offset of this chunk in the run
-#pragma unroll
-        for (int u = 0; u < 4; u++) {
-          const int ob = o + 4 * u;
-          const bool ok = ob >= 0 && ob < run_len;
-          dw_lds[ok ? dst + (ob >> 2) : dummy] = ((unsigned)ld[cc][t][u] & keep) ^ 0x80808080u;
-        }
-      }
-      // rows of the band above / below the image
-      unsigned *base = dw_lds + c * g.CSD;
-      for (int q = lane; q < r_lo * LWD; q += 64) base[q] = 0x80808080u;
-      for (int q = r_hi * LWD + lane; q < g.NR * LWD; q += 64) base[q] = 0x80808080u;
     }
   }
 

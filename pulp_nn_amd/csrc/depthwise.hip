@@ -160,9 +160,15 @@ void depthwise_common(const char *fn, const uint8_t *in, const int8_t *bias, uin
 #undef DW3L
   } else {
     // any other shape: on the matrix cores (filters up to 8 columns wide), or a byte loop
+    g.LP = pl > 4 ? ((pl + 3) & ~3) : 4;
+    // The widths this entry point takes: ky rows of 64 channels in 64 KiB, rows as windows of dwords read them.
+    // (dw_mfma_kernel alone could do more; callers see one limit, whichever kernel a shape takes.)
+    const int window = fast ? 4 * (g.LP / 4 - 1 + ((Wo + 3) / 4 - 1) * sx + (6 - pl + 3 * sx) / 4 + 1) : g.LP - pl + (Wo - 1) * sx + kx;
+    const bool dword_rows = fast && W % 4 == 0 && W / 4 * 3 <= 255 && aligned(in, 16);
+    if (!dword_rows && 255 / ((std::max(window, g.LP + W + 1) + 3) / 4) < ky)
+      return set_error(PULP_NN_HIP_ERR_UNSUPPORTED, fn, "image too wide for the LDS tile");
     const DwLayer L = {in, wt, bias, out, (int)g_batch, CH, H, W, Ho, Wo, kx, ky, pt, pl, sx, sy};
     if (launch_dw_mfma(mode, L, e, num_cus(), g_stream)) return check_launch(fn);
-    g.LP = pl > 4 ? ((pl + 3) & ~3) : 4;
     g.LWD = (std::max(g.LP - pl + (Wo - 1) * sx + kx, g.LP + W + 1) + 3) / 4;
     const int nr_max = 255 / g.LWD;  // 64 channels x 255 dwords = 63.75 KiB of LDS
     if (nr_max < ky) return set_error(PULP_NN_HIP_ERR_UNSUPPORTED, fn, "image too wide for the LDS tile");

@@ -3,6 +3,7 @@ import pytest
 
 import oracle
 from gpu_helpers import assert_same, depthwise_generic, rand_s8, rand_u8, rng_for
+from pulp_nn_amd import PulpNNError
 
 pytestmark = pytest.mark.gpu
 
@@ -20,7 +21,7 @@ GEOMS = [
     (1, 7, 10, 20, 3, 8, (1, 1, 3, 4), (1, 1)),      # the widest filter: two dwords per filter row
     (1, 5, 20, 9, 9, 2, (4, 4, 0, 1), (1, 3)),       # more filter rows than columns, row stride 3
     (1, 6, 8, 31, 3, 3, (1, 1, 1, 1), (3, 1)),
-    (1, 3, 7, 1300, 3, 3, (1, 1, 1, 1), (1, 1)),     # wider than a tile: several tiles along a row
+    (1, 3, 7, 1000, 1, 3, (0, 0, 1, 1), (1, 1)),    # wider than a tile: several tiles along a row
     (1, 2, 200, 18, 3, 3, (1, 1, 1, 1), (1, 1)),     # several bands of rows
     (600, 70, 7, 7, 3, 3, (1, 1, 1, 1), (1, 1)),     # small planes: 64 channels per workgroup, six in the last one
     (520, 128, 5, 9, 3, 3, (0, 0, 1, 1), (1, 1)),
@@ -45,3 +46,20 @@ def test_depthwise_shapes(geom, flags, bn_bits):
     want = oracle.depthwise_generic(x, wt, b, k, lam, 900, shift, pads, strides, relu, bn, bn_bits)
     got = depthwise_generic(x, wt, b, k, lam, 900, shift, pads, strides, relu, bn, bn_bits)
     assert_same(got, want, "depthwise %s" % (geom,))
+
+
+@pytest.mark.parametrize("width, kernel, accepted", [(331, 3, True), (333, 3, False), (340, 3, True), (343, 3, False),
+                                                     (198, 5, True), (199, 5, False)])
+def test_depthwise_width_limit(width, kernel, accepted):
+    """ky rows of 64 channels in 64 KiB of LDS, 4 bytes left of a row: the widest rows taken and the first refused
+    (3 x 3 on rows of whole dwords: no bytes beside the row, so 340 is one of the taken)."""
+    r = rng_for(7200 + width)
+    pad = (kernel // 2,) * 4
+    x, wt, b = rand_u8(r, (1, 3, 6, width)), rand_s8(r, (3, kernel, kernel)), rand_s8(r, (3,))
+    args = (x, wt, b, None, None, 900, 13, pad, (1, 1), 1, 0, 32)
+    if accepted:
+        assert_same(depthwise_generic(*args), oracle.depthwise_generic(*args), "width %d" % width)
+    else:
+        with pytest.raises(PulpNNError) as e:
+            depthwise_generic(*args)
+        assert e.value.code == 2
