@@ -6,7 +6,7 @@
 #include "igemm.h"
 #include "igemm_patch.h"
 #include "igemm_ring.h"
-#include "linear_skinny.h"
+#include "linear_any.h"
 #include "pw_stream.h"
 #include "smallk.h"
 
@@ -216,6 +216,18 @@ void launch_smallk(int mode, bool rows, ConvGeom &g, const EpiArgs &e, hipStream
 }
 
 
+template <bool ANY>
+void launch_skinny(int mode, const SkinnyGeom &g, const EpiArgs &e, dim3 grid, hipStream_t s)
+{
+  const dim3 block(256);
+  switch (mode) {
+    case EPI_BN: hipLaunchKernelGGL((ANY ? linear_skinny_any_kernel<EPI_BN> : linear_skinny_kernel<EPI_BN>), grid, block, 0, s, g, e); break;
+    case EPI_MULT: hipLaunchKernelGGL((ANY ? linear_skinny_any_kernel<EPI_MULT> : linear_skinny_kernel<EPI_MULT>), grid, block, 0, s, g, e); break;
+    case EPI_RAW: hipLaunchKernelGGL((ANY ? linear_skinny_any_kernel<EPI_RAW> : linear_skinny_kernel<EPI_RAW>), grid, block, 0, s, g, e); break;
+    default: hipLaunchKernelGGL((ANY ? linear_skinny_any_kernel<EPI_OUT32> : linear_skinny_kernel<EPI_OUT32>), grid, block, 0, s, g, e); break;
+  }
+}
+
 // Launches one instantiation; raises its dynamic-LDS limit above the default 64 KB as needed.
 template <auto KERN>
 bool launch_pw(const PwGeom &g, const EpiArgs &e, dim3 grid, dim3 block, size_t lds, hipStream_t s)
@@ -387,20 +399,17 @@ void linear_common(const char *fn, int mode, const uint8_t *in, const int8_t *bi
 {
   if (!in || !out || !w) return set_error(PULP_NN_HIP_ERR_ARGUMENT, fn, "null pointer");
   if (!dim_vec || !num_o_neurons) return set_error(PULP_NN_HIP_ERR_ARGUMENT, fn, "zero dimension");
-  // few rows: a workgroup per 16 neurons streams their weights once, no staging and no K-slice barriers
-  if (rows <= 256 && dim_vec % 16 == 0 && aligned(in, 16) && aligned(w, 16) && aligned(out, 4)) {
+  // few rows: a workgroup per 16 neurons streams their weights once, no staging and no K-slice barriers; rows that are
+  // not whole aligned 16-byte chunks by unaligned loads (shorter than one chunk: the tiled kernel)
+  if (rows <= 256 && dim_vec >= 16) {
     const int rblocks = (rows + 63) / 64, ngroups = (num_o_neurons + 15) / 16;
     // K in four parts and a workgroup per block of rows while that still leaves CUs without work
     const bool spread = ngroups * rblocks <= 2 * num_cus();
     const int kparts = spread ? 4 : (rblocks == 1 ? 4 : (rblocks == 2 ? 2 : 1));
-    SkinnyGeom sg = {in, w, bias, out, rows, (int)num_o_neurons, (int)dim_vec, kparts};
-    const dim3 grid(ngroups, spread ? rblocks : 1), block(256);
-    switch (mode) {
-      case EPI_BN: hipLaunchKernelGGL(linear_skinny_kernel<EPI_BN>, grid, block, 0, g_stream, sg, e); break;
-      case EPI_MULT: hipLaunchKernelGGL(linear_skinny_kernel<EPI_MULT>, grid, block, 0, g_stream, sg, e); break;
-      case EPI_RAW: hipLaunchKernelGGL(linear_skinny_kernel<EPI_RAW>, grid, block, 0, g_stream, sg, e); break;
-      default: hipLaunchKernelGGL(linear_skinny_kernel<EPI_OUT32>, grid, block, 0, g_stream, sg, e); break;
-    }
+    const SkinnyGeom sg = {in, w, bias, out, rows, (int)num_o_neurons, (int)dim_vec, kparts};
+    const dim3 grid(ngroups, spread ? rblocks : 1);
+    if (dim_vec % 16 == 0 && aligned(in, 16) && aligned(w, 16) && aligned(out, 4)) launch_skinny<false>(mode, sg, e, grid, g_stream);
+    else launch_skinny<true>(mode, sg, e, grid, g_stream);
     check_launch(fn);
     return;
   }
