@@ -28,30 +28,10 @@
 #pragma once
 #include <type_traits>
 
+#include "dw_mfma_geom.h"
 #include "igemm.h"
 #include "memops.h"
 #include "requant.h"
-
-struct DwmGeom {
-  const uint8_t *in;
-  const int8_t *wt;
-  const int8_t *bias;  // may be null
-  uint8_t *out;
-  int B, CH, H, W, Ho, Wo;
-  int kx, ky, pt, pl, sx, sy;
-  long long in_bytes;   // bytes of the whole input tensor
-  int wt_bytes;         // ... and of all filters
-  int ND, rND;          // dwords of an input row behind 16 output columns; 65536 / ND + 1
-  int RB, NR;           // output rows per tile, input rows behind them
-  int XT;               // groups of 16 output columns per tile
-  int pitch, CS;        // LDS bytes per staged row and per channel
-  int Q;                // 16-byte chunks staged per row
-  int w_off, c_off, o_off;  // LDS offsets: filter rows, per-channel constants, output tile
-  int nper, cpar;       // staging: slots (row, chunk) a pass covers, channels side by side
-  // tile index -> (channels, columns, rows, image); thread -> channel; slot -> row; unit -> row; pixel -> row; filter row -> channel
-  FastDiv d_cb, d_xt, d_band, d_nper, d_q, d_xg, d_wt, d_ky;
-  int cblocks, xtiles, bands, total;
-};
 
 typedef v4i v4i_u __attribute__((aligned(1)));
 typedef int i32_u __attribute__((aligned(1)));
@@ -71,12 +51,9 @@ __global__ __launch_bounds__(256) void dw_mfma_kernel(DwmGeom g, EpiArgs e)
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l16 = lane & 15, lgrp = lane >> 4;
-  // channels vary fastest: the pieces of a pixel's line that different workgroups write meet in one L2
-  const unsigned id = (unsigned)xcd_remap(blockIdx.x, g.total);
-  const unsigned t1 = fastdiv(id, g.d_cb), t2 = fastdiv(t1, g.d_xt), b = fastdiv(t2, g.d_band);
-  const int c0 = (int)(id - t1 * g.cblocks) * CB, xg0 = (int)(t1 - t2 * g.xtiles) * g.XT, oy0 = (int)(t2 - b * g.bands) * g.RB;
-  const int ncb = min(CB, g.CH - c0);
-  const int rows = min(g.RB, g.Ho - oy0), wt = min(16 * g.XT, g.Wo - 16 * xg0);
+  const DwmTile tile = dwm_tile<CB>(g, (unsigned)xcd_remap(blockIdx.x, g.total));
+  const unsigned b = tile.b;
+  const int c0 = tile.c0, xg0 = tile.xg0, oy0 = tile.oy0, ncb = tile.ncb, rows = tile.rows, wt = tile.wt;
   const int plane = g.H * g.W;
   const uint8_t *img = g.in + ((long long)b * g.CH + c0) * plane;
 
@@ -94,7 +71,7 @@ __global__ __launch_bounds__(256) void dw_mfma_kernel(DwmGeom g, EpiArgs e)
       const int row = (int)fastdiv((unsigned)slot, g.d_q), q = slot - row * g.Q;
       const int x = x0 + 16 * q, iy = iy0 + row;
       const bool row_ok = (unsigned)iy < (unsigned)g.H;
-      const int base = row_ok ? iy * g.W + x : 0;
+      const int base = dwm_load_base(g, iy, x);
       if (cpi < g.cpar && slot < slots) {
         // bytes of the chunk inside the image
         unsigned mask[4];
@@ -129,12 +106,8 @@ __global__ __launch_bounds__(256) void dw_mfma_kernel(DwmGeom g, EpiArgs e)
       }
     }
   };
-  {
-    const long long first = (img - g.in) + (long long)max(iy0, 0) * g.W + x0;
-    const long long last = (img - g.in) + (long long)(ncb - 1) * plane + (long long)min(iy0 + g.NR - 1, g.H - 1) * g.W + x0 + 16 * g.Q;
-    if (first < 0 || last > g.in_bytes) stage(std::true_type{});
-    else stage(std::false_type{});
-  }
+  if (dwm_edge(g, tile, img - g.in, iy0, x0)) stage(std::true_type{});
+  else stage(std::false_type{});
 
   // ---- filter rows (8 bytes each, bytes past kx zero) and per-channel constants -> LDS ------------------------
   for (int t = tid; t < CB * g.ky; t += 256) {
@@ -279,11 +252,10 @@ __global__ __launch_bounds__(256) void dw_mfma_kernel(DwmGeom g, EpiArgs e)
   {
     constexpr int NCH = CB / 16;
     const int px = rows * wt, ch = 16 * (tid % NCH), n = ncb - ch;
-    const bool whole = g.xtiles == 1;  // the tile is one run of pixels
     uint8_t *ob = g.out + ((long long)b * g.Ho * g.Wo + (long long)oy0 * g.Wo + 16 * xg0) * g.CH + c0 + ch;
     if (n > 0)
       for (int p = tid / NCH; p < px; p += 256 / NCH) {
-        const int y = whole ? 0 : (int)fastdiv((unsigned)p, g.d_wt);
+        const int y = dwm_out_row(g, tile, p);
         const int *src = (const int *)(dwm_lds + g.o_off + p * PP + ch);
         const v4i v = {src[0], src[1], src[2], src[3]};
         uint8_t *dst = ob + (long long)(p + y * (g.Wo - wt)) * g.CH;

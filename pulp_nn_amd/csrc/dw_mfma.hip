@@ -1,7 +1,5 @@
-// Host side of dw_mfma.h: tile shape and launch.
+// Host side of dw_mfma.h: launch (the tile's shape: dw_mfma_geom.h).
 #include "dw_mfma.h"
-
-#include <algorithm>
 
 #include "host.h"
 
@@ -21,74 +19,10 @@ void launch_mode(int mode, const DwmGeom &g, const EpiArgs &e, size_t lds, hipSt
 template <int CB>
 bool launch_cb(int mode, const DwLayer &L, const EpiArgs &e, int cus, hipStream_t s)
 {
-  const long long plane = (long long)L.H * L.W;
-  if (L.kx > 8 || L.kx * L.ky > 256 || L.sx > 4 || L.pl > 64 || plane * CB > (1 << 29) || (long long)L.B * L.CH * plane < 16) return false;
-  DwmGeom g = {};
-  g.in = L.in;
-  g.wt = L.wt;
-  g.bias = L.bias;
-  g.out = L.out;
-  g.B = L.B;
-  g.CH = L.CH;
-  g.H = L.H;
-  g.W = L.W;
-  g.Ho = L.Ho;
-  g.Wo = L.Wo;
-  g.kx = L.kx;
-  g.ky = L.ky;
-  g.pt = L.pt;
-  g.pl = L.pl;
-  g.sx = L.sx;
-  g.sy = L.sy;
-  g.in_bytes = L.B * L.CH * plane;
-  g.wt_bytes = L.CH * L.kx * L.ky;
-  g.ND = (15 * L.sx + L.kx + 3) / 4;
-  g.rND = 65536 / g.ND + 1;
-  const int nm = (L.ky * g.ND + 15) / 16;
-  if (nm > 5) return false;
-  g.cblocks = (L.CH + CB - 1) / CB;
-  const int xg = (L.Wo + 15) / 16;
-  const int fixed = CB * L.ky * 8 + CB * (4 + 2 * (int)sizeof(bn_t));
-  auto shape = [&](int xt, int rb) {
-    g.XT = xt;
-    g.RB = rb;
-    g.NR = (rb - 1) * L.sy + L.ky;
-    g.Q = ((xt - 1) * 16 * L.sx + 4 * g.ND + 15) / 16;
-    g.pitch = 16 * (g.Q | 1);  // an odd number of 16-byte chunks: the rows of a tile start in different banks
-    g.CS = g.NR * g.pitch;
-    g.xtiles = (xg + xt - 1) / xt;
-    g.bands = (L.Ho + rb - 1) / rb;
-    return CB * g.CS + fixed + rb * std::min(16 * xt, L.Wo) * (CB + 4);
-  };
-  // Rows of the full width, all rows of the plane, unless that takes more than 32 KB of LDS (four workgroups of a
-  // compute unit cover each other's load, multiply and store phases) ...
-  constexpr int LDS = CB == 16 ? 32 * 1024 : 48 * 1024;
-  int xt = xg, rb = L.Ho;
-  while (xt > 1 && shape(xt, 1) > LDS) xt = (xt + 1) / 2;
-  if (shape(xt, 1) > 64 * 1024) return false;
-  while (rb > 1 && shape(xt, rb) > LDS) rb--;
-  // ... and fewer rows while that leaves compute units without a workgroup and a tile still fills an MFMA
-  auto count = [&] { return (long long)L.B * g.cblocks * ((xg + xt - 1) / xt) * ((L.Ho + rb - 1) / rb); };
-  while (rb * xt > 16 && rb > 1 && count() < 2ll * cus) rb = (rb + 1) / 2;
-  rb = (L.Ho + (L.Ho + rb - 1) / rb - 1) / ((L.Ho + rb - 1) / rb);  // rows spread evenly over the bands
-  const int lds_bytes = shape(xt, rb);
-  const long long total = (long long)L.B * g.cblocks * g.xtiles * g.bands;
-  if (total > 0x7fffffffLL) return false;
-  g.total = (int)total;
-  g.w_off = CB * g.CS;
-  g.c_off = g.w_off + CB * L.ky * 8;
-  g.o_off = (g.c_off + CB * (4 + 2 * (int)sizeof(bn_t)) + 15) & ~15;
-  g.d_cb = fastdiv_make((unsigned)g.cblocks);
-  g.d_xt = fastdiv_make((unsigned)g.xtiles);
-  g.d_band = fastdiv_make((unsigned)g.bands);
-  g.nper = std::min(g.NR * g.Q, 256);
-  g.cpar = 256 / g.nper;
-  g.d_nper = fastdiv_make((unsigned)g.nper);
-  g.d_ky = fastdiv_make((unsigned)L.ky);
-  g.d_q = fastdiv_make((unsigned)g.Q);
-  g.d_xg = fastdiv_make((unsigned)g.XT);
-  g.d_wt = fastdiv_make((unsigned)std::min(16 * xt, L.Wo));
-  const size_t lds = (size_t)lds_bytes + 32;
+  DwmGeom g;
+  int nm;
+  size_t lds;
+  if (!dwm_shape<CB>(L, cus, (int)sizeof(bn_t), &g, &nm, &lds)) return false;
   if (nm == 1) launch_mode<CB, 1>(mode, g, e, lds, s);
   else if (nm == 2) launch_mode<CB, 2>(mode, g, e, lds, s);
   else if (nm == 3) launch_mode<CB, 3>(mode, g, e, lds, s);

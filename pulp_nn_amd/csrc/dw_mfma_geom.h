@@ -1,0 +1,157 @@
+// Tile shape of dw_mfma_kernel and the arithmetic that says which bytes a tile reads and writes.  Plain C++: the kernel
+// and its launcher use it, and a host program can walk the same numbers.
+#pragma once
+#include <stdint.h>
+
+#include <algorithm>
+
+#include "fastdiv.h"
+
+struct DwLayer {
+  const uint8_t *in;
+  const int8_t *wt;
+  const int8_t *bias;
+  uint8_t *out;
+  int B, CH, H, W, Ho, Wo, kx, ky, pt, pl, sx, sy;
+};
+
+struct DwmGeom {
+  const uint8_t *in;
+  const int8_t *wt;
+  const int8_t *bias;  // may be null
+  uint8_t *out;
+  int B, CH, H, W, Ho, Wo;
+  int kx, ky, pt, pl, sx, sy;
+  long long in_bytes;   // bytes of the whole input tensor
+  int wt_bytes;         // ... and of all filters
+  int ND, rND;          // dwords of an input row behind 16 output columns; 65536 / ND + 1
+  int RB, NR;           // output rows per tile, input rows behind them
+  int XT;               // groups of 16 output columns per tile
+  int pitch, CS;        // LDS bytes per staged row and per channel
+  int Q;                // 16-byte chunks staged per row
+  int w_off, c_off, o_off;  // LDS offsets: filter rows, per-channel constants, output tile
+  int nper, cpar;       // staging: slots (row, chunk) a pass covers, channels side by side
+  // tile index -> (channels, columns, rows, image); thread -> channel; slot -> row; unit -> row; pixel -> row; filter row -> channel
+  FastDiv d_cb, d_xt, d_band, d_nper, d_q, d_xg, d_wt, d_ky;
+  int cblocks, xtiles, bands, total;
+};
+
+// One tile: CB channels from c0 on (ncb of them exist), output rows oy0 .. oy0 + rows - 1 of image b, output columns
+// 16 * xg0 .. 16 * xg0 + wt - 1.
+struct DwmTile {
+  int c0, ncb, xt, xg0, oy0, rows, wt;
+  unsigned b;
+};
+template <int CB>
+PULPNN_HD DwmTile dwm_tile(const DwmGeom &g, unsigned id)
+{
+  // channels vary fastest: the pieces of a pixel's line that different workgroups write meet in one L2
+  const unsigned t1 = fastdiv(id, g.d_cb), t2 = fastdiv(t1, g.d_xt), b = fastdiv(t2, g.d_band);
+  DwmTile t;
+  t.b = b;
+  t.c0 = (int)(id - t1 * g.cblocks) * CB;
+  t.xt = (int)(t1 - t2 * g.xtiles);
+  t.xg0 = t.xt * g.XT;
+  t.oy0 = (int)(t2 - b * g.bands) * g.RB;
+  t.ncb = CB < g.CH - t.c0 ? CB : g.CH - t.c0;
+  t.rows = g.RB < g.Ho - t.oy0 ? g.RB : g.Ho - t.oy0;
+  t.wt = 16 * g.XT < g.Wo - 16 * t.xg0 ? 16 * g.XT : g.Wo - 16 * t.xg0;
+  return t;
+}
+
+// Whether a 16-byte load of the tile may leave the tensor (before: bytes of the tensor in front of the tile's first plane).
+PULPNN_HD bool dwm_edge(const DwmGeom &g, const DwmTile &t, long long before, int iy0, int x0)
+{
+  const int plane = g.H * g.W, iy_last = iy0 + g.NR - 1 < g.H - 1 ? iy0 + g.NR - 1 : g.H - 1;
+  const long long first = before + (long long)(iy0 > 0 ? iy0 : 0) * g.W + x0;
+  const long long last = before + (long long)(t.ncb - 1) * plane + (long long)iy_last * g.W + x0 + 16 * g.Q;
+  return first < 0 || last > g.in_bytes;
+}
+
+// Bytes from the tile's first plane to the load of chunk column x in row iy of channel c (a row outside the image: the
+// start of the plane, masked off).
+PULPNN_HD int dwm_load_base(const DwmGeom &g, int iy, int x) { return (unsigned)iy < (unsigned)g.H ? iy * g.W + x : 0; }
+
+// Row of the tile's pixel p, counted row by row.
+PULPNN_HD int dwm_out_row(const DwmGeom &g, const DwmTile &, int p)
+{
+  return g.xtiles == 1 ? 0 : (int)fastdiv((unsigned)p, g.d_wt);  // (one column tile: a single run of pixels)
+}
+
+// Tile shape for CB channels per workgroup; bn_bytes: bytes of a batch-norm parameter.  nm: MFMAs per (channel, 16 units);
+// lds: dynamic LDS of the launch.  False for a layer the kernel does not take.
+template <int CB>
+bool dwm_shape(const DwLayer &L, int cus, int bn_bytes, DwmGeom *out, int *nm_out, size_t *lds_out)
+{
+  const long long plane = (long long)L.H * L.W;
+  if (L.kx > 8 || L.kx * L.ky > 256 || L.sx > 4 || L.pl > 64 || plane * CB > (1 << 29) || (long long)L.B * L.CH * plane < 16) return false;
+  DwmGeom &g = *out;
+  g = DwmGeom{};
+  g.in = L.in;
+  g.wt = L.wt;
+  g.bias = L.bias;
+  g.out = L.out;
+  g.B = L.B;
+  g.CH = L.CH;
+  g.H = L.H;
+  g.W = L.W;
+  g.Ho = L.Ho;
+  g.Wo = L.Wo;
+  g.kx = L.kx;
+  g.ky = L.ky;
+  g.pt = L.pt;
+  g.pl = L.pl;
+  g.sx = L.sx;
+  g.sy = L.sy;
+  g.in_bytes = L.B * L.CH * plane;
+  g.wt_bytes = L.CH * L.kx * L.ky;
+  g.ND = (15 * L.sx + L.kx + 3) / 4;
+  g.rND = 65536 / g.ND + 1;
+  const int nm = (L.ky * g.ND + 15) / 16;
+  if (nm > 5) return false;
+  g.cblocks = (L.CH + CB - 1) / CB;
+  const int xg = (L.Wo + 15) / 16;
+  const int fixed = CB * L.ky * 8 + CB * (4 + 2 * bn_bytes);
+  auto shape = [&](int xt, int rb) {
+    g.XT = xt;
+    g.RB = rb;
+    g.NR = (rb - 1) * L.sy + L.ky;
+    g.Q = ((xt - 1) * 16 * L.sx + 4 * g.ND + 15) / 16;
+    g.pitch = 16 * (g.Q | 1);  // an odd number of 16-byte chunks: the rows of a tile start in different banks
+    g.CS = g.NR * g.pitch;
+    g.xtiles = (xg + xt - 1) / xt;
+    g.bands = (L.Ho + rb - 1) / rb;
+    return CB * g.CS + fixed + rb * std::min(16 * xt, L.Wo) * (CB + 4);
+  };
+  // Rows of the full width, all rows of the plane, unless that takes more than 32 KB of LDS (four workgroups of a
+  // compute unit cover each other's load, multiply and store phases) ...
+  constexpr int LDS = CB == 16 ? 32 * 1024 : 48 * 1024;
+  int xt = xg, rb = L.Ho;
+  while (xt > 1 && shape(xt, 1) > LDS) xt = (xt + 1) / 2;
+  if (shape(xt, 1) > 64 * 1024) return false;
+  while (rb > 1 && shape(xt, rb) > LDS) rb--;
+  // ... and fewer rows while that leaves compute units without a workgroup and a tile still fills an MFMA
+  auto count = [&] { return (long long)L.B * g.cblocks * ((xg + xt - 1) / xt) * ((L.Ho + rb - 1) / rb); };
+  while (rb * xt > 16 && rb > 1 && count() < 2ll * cus) rb = (rb + 1) / 2;
+  rb = (L.Ho + (L.Ho + rb - 1) / rb - 1) / ((L.Ho + rb - 1) / rb);  // rows spread evenly over the bands
+  const int lds_bytes = shape(xt, rb);
+  const long long total = (long long)L.B * g.cblocks * g.xtiles * g.bands;
+  if (total > 0x7fffffffLL) return false;
+  g.total = (int)total;
+  g.w_off = CB * g.CS;
+  g.c_off = g.w_off + CB * L.ky * 8;
+  g.o_off = (g.c_off + CB * (4 + 2 * bn_bytes) + 15) & ~15;
+  g.d_cb = fastdiv_make((unsigned)g.cblocks);
+  g.d_xt = fastdiv_make((unsigned)g.xtiles);
+  g.d_band = fastdiv_make((unsigned)g.bands);
+  g.nper = std::min(g.NR * g.Q, 256);
+  g.cpar = 256 / g.nper;
+  g.d_nper = fastdiv_make((unsigned)g.nper);
+  g.d_ky = fastdiv_make((unsigned)L.ky);
+  g.d_q = fastdiv_make((unsigned)g.Q);
+  g.d_xg = fastdiv_make((unsigned)g.XT);
+  g.d_wt = fastdiv_make((unsigned)std::min(16 * xt, L.Wo));
+  *nm_out = nm;
+  *lds_out = (size_t)lds_bytes + 32;
+  return true;
+}

@@ -12,6 +12,7 @@
 #include <atomic>
 #include <mutex>
 
+#include "dw_mfma_geom.h"
 #include "requant.h"
 
 #pragma GCC visibility push(hidden)
@@ -74,13 +75,6 @@ void linear_common(const char *fn, int mode, const uint8_t *in, const int8_t *bi
 
 // ---- kernels with a launcher of their own: false, with nothing queued, for a geometry the kernel does not take ---
 
-struct DwLayer {
-  const uint8_t *in;
-  const int8_t *wt;
-  const int8_t *bias;
-  uint8_t *out;
-  int B, CH, H, W, Ho, Wo, kx, ky, pt, pl, sx, sy;
-};
 struct ConvLayer {
   const uint8_t *in;
   const int8_t *w;

@@ -38,32 +38,11 @@
 #pragma once
 #include <type_traits>
 
+#include "fastdiv.h"
 #include "memops.h"
 #include "requant.h"
 
 enum { GATHER_CHUNK16 = 0, GATHER_BYTES = 1, GATHER_UNIFORM = 2, GATHER_SUBTAP = 3 };
-
-// Division of a 32-bit unsigned number by a divisor fixed for the launch, as a multiply-high, an add and
-// two shifts (Granlund & Montgomery); the host computes the constants.  The compiler's expansion of a
-// 32-bit division is some 40 instructions, and a tile's set-up divides several times per lane.
-struct FastDiv {
-  unsigned mul, sh1, sh2;
-};
-static inline FastDiv fastdiv_make(unsigned d)
-{
-  FastDiv f;
-  unsigned l = 0;
-  while ((1ull << l) < d) l++;  // ceil(log2(d))
-  f.mul = (unsigned)(((1ull << 32) * ((1ull << l) - d)) / d + 1);
-  f.sh1 = l < 1 ? l : 1;
-  f.sh2 = l > 1 ? l - 1 : 0;
-  return f;
-}
-__device__ __forceinline__ unsigned fastdiv(unsigned n, const FastDiv &f)
-{
-  const unsigned t = __umulhi(n, f.mul);
-  return (t + ((n - t) >> f.sh1)) >> f.sh2;
-}
 
 struct ConvGeom {
   const uint8_t *in;
