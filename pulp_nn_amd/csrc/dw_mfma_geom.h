@@ -31,8 +31,9 @@ struct DwmGeom {
   int Q;                // 16-byte chunks staged per row
   int w_off, c_off, o_off;  // LDS offsets: filter rows, per-channel constants, output tile
   int nper, cpar;       // staging: slots (row, chunk) a pass covers, channels side by side
-  // tile index -> (channels, columns, rows, image); thread -> channel; slot -> row; unit -> row; pixel -> row; filter row -> channel
-  FastDiv d_cb, d_xt, d_band, d_nper, d_q, d_xg, d_wt, d_ky;
+  // tile index -> (channels, columns, rows, image); thread -> channel; slot -> row; unit -> row; pixel -> row (of a tile
+  // of full width, of the last one along a row); filter row -> channel
+  FastDiv d_cb, d_xt, d_band, d_nper, d_q, d_xg, d_wt, d_wt_last, d_ky;
   int cblocks, xtiles, bands, total;
 };
 
@@ -73,9 +74,10 @@ PULPNN_HD bool dwm_edge(const DwmGeom &g, const DwmTile &t, long long before, in
 PULPNN_HD int dwm_load_base(const DwmGeom &g, int iy, int x) { return (unsigned)iy < (unsigned)g.H ? iy * g.W + x : 0; }
 
 // Row of the tile's pixel p, counted row by row.
-PULPNN_HD int dwm_out_row(const DwmGeom &g, const DwmTile &, int p)
+PULPNN_HD int dwm_out_row(const DwmGeom &g, const DwmTile &t, int p)
 {
-  return g.xtiles == 1 ? 0 : (int)fastdiv((unsigned)p, g.d_wt);  // (one column tile: a single run of pixels)
+  if (g.xtiles == 1) return 0;  // (one column tile: a single run of pixels)
+  return (int)fastdiv((unsigned)p, t.xt + 1 == g.xtiles ? g.d_wt_last : g.d_wt);
 }
 
 // Tile shape for CB channels per workgroup; bn_bytes: bytes of a batch-norm parameter.  nm: MFMAs per (channel, 16 units);
@@ -151,6 +153,7 @@ bool dwm_shape(const DwLayer &L, int cus, int bn_bytes, DwmGeom *out, int *nm_ou
   g.d_q = fastdiv_make((unsigned)g.Q);
   g.d_xg = fastdiv_make((unsigned)g.XT);
   g.d_wt = fastdiv_make((unsigned)std::min(16 * xt, L.Wo));
+  g.d_wt_last = fastdiv_make((unsigned)(L.Wo - 16 * xt * (g.xtiles - 1)));
   *nm_out = nm;
   *lds_out = (size_t)lds_bytes + 32;
   return true;

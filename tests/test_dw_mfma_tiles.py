@@ -45,3 +45,10 @@ def test_usual_layers(walk):
         layers.append(layer(r.choice([1, 2, 33, 256]), r.randint(1, 200), r.randint(k, 70), r.randint(16, 70), k, k, (k // 2,) * 4, (s, s),
                             bn_bytes=r.choice([4, 8])))
     check(walk, layers)
+
+
+def test_narrow_last_column_tile(walk):
+    """Several column tiles and several rows per tile: the last tile's rows are shorter, in LDS too."""
+    check(walk, [layer(600, 16, 6, 340, 3, 3, (1, 1, 1, 111), (1, 1)), layer(64, 16, 40, 320, 3, 3, (1, 1, 1, 131), (1, 1)),
+                 layer(600, 24, 8, 336, 3, 3, (1, 1, 0, 100), (1, 1), bn_bytes=8)])
+    assert walk([layer(600, 16, 6, 340, 3, 3, (1, 1, 1, 111), (1, 1))]) == ["ok 3600"]  # two column tiles, two rows each

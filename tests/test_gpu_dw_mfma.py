@@ -22,6 +22,8 @@ GEOMS = [
     (1, 5, 20, 9, 9, 2, (4, 4, 0, 1), (1, 3)),       # more filter rows than columns, row stride 3
     (1, 6, 8, 31, 3, 3, (1, 1, 1, 1), (3, 1)),
     (1, 3, 7, 1000, 1, 3, (0, 0, 1, 1), (1, 1)),    # wider than a tile: several tiles along a row
+    (600, 16, 6, 340, 3, 3, (1, 1, 1, 111), (1, 1)),  # two column tiles of two rows, the second one narrower
+    (400, 33, 5, 336, 3, 3, (1, 1, 0, 90), (1, 1)),
     (1, 2, 200, 18, 3, 3, (1, 1, 1, 1), (1, 1)),     # several bands of rows
     (600, 70, 7, 7, 3, 3, (1, 1, 1, 1), (1, 1)),     # small planes: 64 channels per workgroup, six in the last one
     (520, 128, 5, 9, 3, 3, (0, 0, 1, 1), (1, 1)),
