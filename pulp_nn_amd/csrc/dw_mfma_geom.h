@@ -105,7 +105,7 @@ bool dwm_shape(const DwLayer &L, int cus, int bn_bytes, DwmGeom *out, int *nm_ou
   g.pl = L.pl;
   g.sx = L.sx;
   g.sy = L.sy;
-  g.in_bytes = L.B * L.CH * plane;
+  g.in_bytes = (long long)L.B * L.CH * plane;
   g.wt_bytes = L.CH * L.kx * L.ky;
   g.ND = (15 * L.sx + L.kx + 3) / 4;
   g.rND = 65536 / g.ND + 1;

@@ -52,3 +52,8 @@ def test_narrow_last_column_tile(walk):
     check(walk, [layer(600, 16, 6, 340, 3, 3, (1, 1, 1, 111), (1, 1)), layer(64, 16, 40, 320, 3, 3, (1, 1, 1, 131), (1, 1)),
                  layer(600, 24, 8, 336, 3, 3, (1, 1, 0, 100), (1, 1), bn_bytes=8)])
     assert walk([layer(600, 16, 6, 340, 3, 3, (1, 1, 1, 111), (1, 1))]) == ["ok 3600"]  # two column tiles, two rows each
+
+
+def test_more_planes_than_an_int_counts(walk):
+    """batch x channels past 2^31: 105 GB and 107 GB of input, which the card holds."""
+    check(walk, [layer(2097152, 1024, 7, 7, 3, 3, (1, 1, 1, 1), (1, 1)), layer(4300000, 1000, 5, 5, 3, 3, (1, 1, 1, 1), (1, 1))])
