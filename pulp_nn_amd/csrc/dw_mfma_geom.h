@@ -65,8 +65,10 @@ PULPNN_HD bool dwm_edge(const DwmGeom &g, const DwmTile &t, long long before, in
 {
   const int plane = g.H * g.W, iy_last = iy0 + g.NR - 1 < g.H - 1 ? iy0 + g.NR - 1 : g.H - 1;
   const long long first = before + (long long)(iy0 > 0 ? iy0 : 0) * g.W + x0;
-  const long long last = before + (long long)(t.ncb - 1) * plane + (long long)iy_last * g.W + x0 + 16 * g.Q;
-  return first < 0 || last > g.in_bytes;
+  const long long last_plane = before + (long long)(t.ncb - 1) * plane;
+  const long long last = last_plane + (long long)iy_last * g.W + x0 + 16 * g.Q;
+  // (a row outside the image loads from the start of its plane, which in a plane of fewer than 16 bytes reaches past it)
+  return first < 0 || last > g.in_bytes || last_plane + 16 > g.in_bytes;
 }
 
 // Bytes from the tile's first plane to the load of chunk column x in row iy of channel c (a row outside the image: the

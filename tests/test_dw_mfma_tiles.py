@@ -57,3 +57,18 @@ def test_narrow_last_column_tile(walk):
 def test_more_planes_than_an_int_counts(walk):
     """batch x channels past 2^31: 105 GB and 107 GB of input, which the card holds."""
     check(walk, [layer(2097152, 1024, 7, 7, 3, 3, (1, 1, 1, 1), (1, 1)), layer(4300000, 1000, 5, 5, 3, 3, (1, 1, 1, 1), (1, 1))])
+
+
+def test_tiny_planes_with_wide_padding(walk):
+    """Planes of fewer than 16 bytes: a row outside the image must not load past the last one."""
+    layers = [layer(1, 2, 1, 14, 1, 2, (3, 3, 5, 5), (1, 1)), layer(2, 10, 3, 5, 8, 3, (8, 2, 7, 2), (1, 4)),
+              layer(5, 24, 1, 9, 1, 2, (6, 1, 62, 7), (1, 2)), layer(2, 3, 1, 4, 5, 2, (5, 5, 25, 8), (3, 4))]
+    r = random.Random(2)
+    while len(layers) < 8000:
+        H, W, kx, ky = r.choice([1, 1, 2, 2, 3, 4, 5, 8]), r.randint(1, 20), r.randint(1, 8), r.randint(1, 8)
+        pads = [r.randint(0, 8) for _ in range(4)]
+        if r.random() < 0.2:
+            pads[r.choice([0, 2])] = r.randint(0, 64)
+        if H + pads[0] + pads[1] >= ky and W + pads[2] + pads[3] >= kx:
+            layers.append(layer(r.choice([1, 2, 5]), r.randint(1, 40), H, W, kx, ky, pads, (r.randint(1, 4), r.randint(1, 5))))
+    check(walk, layers, taken=False)

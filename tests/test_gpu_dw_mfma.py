@@ -20,6 +20,9 @@ GEOMS = [
     (1, 8, 17, 40, 7, 7, (3, 3, 3, 3), (2, 2)),      # five
     (1, 7, 10, 20, 3, 8, (1, 1, 3, 4), (1, 1)),      # the widest filter: two dwords per filter row
     (1, 5, 20, 9, 9, 2, (4, 4, 0, 1), (1, 3)),       # more filter rows than columns, row stride 3
+    (1, 2, 1, 14, 2, 1, (3, 3, 5, 5), (1, 1)),       # 14 bytes a plane, rows that all lie in the padding
+    (3, 24, 1, 9, 2, 1, (6, 1, 7, 7), (1, 2)),
+    (2, 10, 3, 5, 3, 8, (8, 2, 7, 2), (1, 4)),
     (1, 6, 8, 31, 3, 3, (1, 1, 1, 1), (3, 1)),
     (1, 3, 7, 1000, 1, 3, (0, 0, 1, 1), (1, 1)),    # wider than a tile: several tiles along a row
     (600, 16, 6, 340, 3, 3, (1, 1, 1, 111), (1, 1)),  # two column tiles of two rows, the second one narrower
