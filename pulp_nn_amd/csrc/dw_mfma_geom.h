@@ -116,21 +116,24 @@ bool dwm_shape(const DwLayer &L, int cus, int bn_bytes, DwmGeom *out, int *nm_ou
   g.cblocks = (L.CH + CB - 1) / CB;
   const int xg = (L.Wo + 15) / 16;
   const int fixed = CB * L.ky * 8 + CB * (4 + 2 * bn_bytes);
-  auto shape = [&](int xt, int rb) {
+  // LDS of a tile, in 64 bits: a tall output at a large row stride would reach over more input rows than an int counts
+  // (the fields are what they should be for tiles that fit)
+  auto shape = [&](int xt, int rb) -> long long {
+    const long long nr = (rb - 1) * (long long)L.sy + L.ky;
     g.XT = xt;
     g.RB = rb;
-    g.NR = (rb - 1) * L.sy + L.ky;
+    g.NR = (int)nr;
     g.Q = ((xt - 1) * 16 * L.sx + 4 * g.ND + 15) / 16;
     g.pitch = 16 * (g.Q | 1);  // an odd number of 16-byte chunks: the rows of a tile start in different banks
-    g.CS = g.NR * g.pitch;
+    g.CS = (int)(nr * g.pitch);
     g.xtiles = (xg + xt - 1) / xt;
     g.bands = (L.Ho + rb - 1) / rb;
-    return CB * g.CS + fixed + rb * std::min(16 * xt, L.Wo) * (CB + 4);
+    return CB * nr * g.pitch + fixed + (long long)rb * std::min(16 * xt, L.Wo) * (CB + 4);
   };
   // Rows of the full width, all rows of the plane, unless that takes more than 32 KB of LDS (four workgroups of a
   // compute unit cover each other's load, multiply and store phases) ...
   constexpr int LDS = CB == 16 ? 32 * 1024 : 48 * 1024;
-  int xt = xg, rb = L.Ho;
+  int xt = xg, rb = std::min(L.Ho, LDS / (CB + 4));
   while (xt > 1 && shape(xt, 1) > LDS) xt = (xt + 1) / 2;
   if (shape(xt, 1) > 64 * 1024) return false;
   while (rb > 1 && shape(xt, rb) > LDS) rb--;
@@ -138,7 +141,7 @@ bool dwm_shape(const DwLayer &L, int cus, int bn_bytes, DwmGeom *out, int *nm_ou
   auto count = [&] { return (long long)L.B * g.cblocks * ((xg + xt - 1) / xt) * ((L.Ho + rb - 1) / rb); };
   while (rb * xt > 16 && rb > 1 && count() < 2ll * cus) rb = (rb + 1) / 2;
   rb = (L.Ho + (L.Ho + rb - 1) / rb - 1) / ((L.Ho + rb - 1) / rb);  // rows spread evenly over the bands
-  const int lds_bytes = shape(xt, rb);
+  const long long lds_bytes = shape(xt, rb);
   const long long total = (long long)L.B * g.cblocks * g.xtiles * g.bands;
   if (total > 0x7fffffffLL) return false;
   g.total = (int)total;

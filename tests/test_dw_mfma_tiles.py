@@ -72,3 +72,13 @@ def test_tiny_planes_with_wide_padding(walk):
         if H + pads[0] + pads[1] >= ky and W + pads[2] + pads[3] >= kx:
             layers.append(layer(r.choice([1, 2, 5]), r.randint(1, 40), H, W, kx, ky, pads, (r.randint(1, 4), r.randint(1, 5))))
     check(walk, layers, taken=False)
+
+
+def test_row_stride_far_past_the_image(walk):
+    """Output rows whose input rows reach further than an int counts: the tile is sized by what it would take."""
+    r = random.Random(3)
+    layers = [layer(1, 16, 8, 16, 3, 3, (1, 1, 1, 1), (1, 60000), out_hw=(2000, 16))]
+    for _ in range(300):
+        layers.append(layer(r.choice([1, 4]), r.randint(1, 70), r.randint(1, 60), r.randint(16, 60), 3, 3, (1, 1, 1, 1),
+                            (r.choice([1, 2]), r.randint(1, 65535)), out_hw=(r.choice([100, 1000, 30000]) + r.randint(0, 99), r.randint(1, 80))))
+    check(walk, layers)
