@@ -23,25 +23,8 @@
 #pragma once
 #include <type_traits>
 
+#include "conv_band_geom.h"
 #include "igemm.h"
-
-struct BandGeom {
-  const uint8_t *in;
-  const int8_t *w;
-  const int8_t *bias;  // may be null
-  uint8_t *out;
-  int N, K, H, W, Ci, Ho, Wo;
-  int kx, ky, pt, pl, sx, sy;
-  int CG, CP;          // 16-byte chunks per pixel, LDS bytes per pixel
-  int NK;              // MFMA steps: ceil(kx * ky * CG / 4)
-  int R, PC;           // output rows and columns per workgroup (R == 1 if PC < Wo)
-  int IW, NR;          // input columns and rows behind them
-  int WN;              // waves along the channels (1, 2 or 4 of four)
-  int mode;
-  int tab_off, c_off;  // LDS offsets: tap table, per-channel constants
-  int nblocks, xtiles, bands, total;
-  FastDiv d_nb, d_xt, d_band, d_cg, d_iw, d_pc, d_kx;
-};
 
 typedef v4i v4i_b __attribute__((aligned(1)));
 typedef v2i v2i_b __attribute__((aligned(1)));

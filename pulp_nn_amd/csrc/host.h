@@ -12,6 +12,7 @@
 #include <atomic>
 #include <mutex>
 
+#include "conv_band_geom.h"
 #include "dw_mfma_geom.h"
 #include "requant.h"
 
@@ -75,13 +76,6 @@ void linear_common(const char *fn, int mode, const uint8_t *in, const int8_t *bi
 
 // ---- kernels with a launcher of their own: false, with nothing queued, for a geometry the kernel does not take ---
 
-struct ConvLayer {
-  const uint8_t *in;
-  const int8_t *w;
-  const int8_t *bias;
-  uint8_t *out;
-  int B, H, W, Ci, Ho, Wo, N, kx, ky, pt, pl, sx, sy;
-};
 bool launch_conv_band(int mode, const ConvLayer &L, const EpiArgs &e, int cus, hipStream_t s);
 bool launch_pw_any(int mode, const uint8_t *in, const int8_t *w, const int8_t *bias, uint8_t *out, long long M, int N, int K,
                    const EpiArgs &e, int cus, hipStream_t s);

@@ -1,0 +1,54 @@
+"""The tile shapes of conv_band_kernel walked on the host (tests/host/conv_band_walk.cpp): everything a tile stages and reads
+inside the LDS it asks for, every output computed once."""
+import os
+import random
+import subprocess
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+
+@pytest.fixture(scope="module")
+def walk(tmp_path_factory):
+    exe = str(tmp_path_factory.mktemp("walk") / "conv_band_walk")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-fsanitize=undefined", "-fno-sanitize-recover=all",
+                    os.path.join(HERE, "host", "conv_band_walk.cpp"), "-o", exe], check=True)
+
+    def run(layers):
+        text = "\n".join(" ".join(map(str, l)) for l in layers)
+        res = subprocess.run([exe], input=text, stdout=subprocess.PIPE, stderr=subprocess.PIPE, text=True, timeout=100)
+        said = res.stdout.split("\n")[:-1]
+        assert res.returncode == 0, "layer %s: %s" % (layers[len(said)], res.stderr)
+        for l, s in zip(layers, said):
+            assert s.startswith("ok") or s == "no", "layer %s: %s" % (l, s)
+        return said
+    return run
+
+
+def layer(B, H, W, Ci, Ho, Wo, N, kx, ky, pt=0, pl=0, sx=1, sy=1, bn_bytes=4, cus=256):
+    return B, H, W, Ci, Ho, Wo, N, kx, ky, pt, pl, sx, sy, bn_bytes, cus
+
+
+def test_usual_layers(walk):
+    r = random.Random(1)
+    layers = []
+    for _ in range(4000):
+        k, s, H, W = r.choice([1, 3, 3, 5, 7]), r.choice([1, 1, 2]), r.randint(7, 70), r.randint(7, 70)
+        layers.append(layer(r.choice([1, 2, 33, 256]), H, W, r.randint(3, 300), (H - 1) // s + 1, (W - 1) // s + 1, r.randint(1, 300), k, k,
+                            k // 2, k // 2, s, s, bn_bytes=r.choice([4, 8])))
+    said = walk(layers)
+    assert sum(s != "no" for s in said) > 3500
+
+
+def test_lds_past_an_int(walk):
+    """Strides and filters whose staged input would take more bytes than an int counts: not taken, or in tiles that fit."""
+    layers = [layer(1, 60, 60, 57, 15292, 50, 6, 4, 1, sx=34257, sy=35775), layer(1, 60, 60, 53, 11955, 1, 10, 4, 2, sx=1, sy=37077),
+              layer(1, 60, 60, 19, 50314, 6, 2, 2, 5, sx=3, sy=63415), layer(1, 500, 500, 12, 6, 38, 77, 1974, 474, sx=4, sy=62959)]
+    r = random.Random(2)
+    for _ in range(4000):
+        big = r.random() < 0.3
+        kx, ky = (r.randint(1, 9000), r.randint(1, 9000)) if big else (r.randint(1, 5), r.randint(1, 5))
+        layers.append(layer(r.choice([1, 3]), r.randint(1, 500), r.randint(1, 500), r.randint(1, 60), r.randint(1, 65535), r.randint(1, 65535),
+                            r.randint(1, 100), kx, ky, 1, 1, r.randint(1, 65535), r.randint(1, 65535)))
+    walk(layers)
