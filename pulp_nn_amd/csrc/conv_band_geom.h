@@ -61,7 +61,7 @@ inline bool band_shape(const ConvLayer &L, int cus, int bn_bytes, BandGeom *out,
   if (L.kx == 1 && L.ky == 1 && L.sx == 1 && L.sy == 1 && !L.pt && !L.pl && L.Ho == L.H && L.Wo == L.W) {
     // pointwise: the batch is one row of pixels
     const long long m = (long long)B * L.H * L.W;
-    if (m > 0x7fffffffLL) return false;
+    if (m > 0x7fffffffLL - 1024) return false;  // (a tile's pixels are counted past the last one)
     g.H = g.Ho = B = 1;
     g.W = g.Wo = (int)m;
   }
@@ -101,7 +101,7 @@ inline bool band_shape(const ConvLayer &L, int cus, int bn_bytes, BandGeom *out,
   }
   g.xtiles = (g.Wo + pc - 1) / pc;
   // a row split evenly, rows spread evenly over the bands
-  if (g.xtiles > 1) pc = (g.Wo + g.xtiles - 1) / g.xtiles;
+  if (g.xtiles > 1) pc = (int)(((long long)g.Wo + g.xtiles - 1) / g.xtiles);
   g.bands = (g.Ho + r - 1) / r;
   r = (g.Ho + g.bands - 1) / g.bands;
   const long long lds = lds_for(r, pc);

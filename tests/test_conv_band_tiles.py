@@ -52,3 +52,8 @@ def test_lds_past_an_int(walk):
         layers.append(layer(r.choice([1, 3]), r.randint(1, 500), r.randint(1, 500), r.randint(1, 60), r.randint(1, 65535), r.randint(1, 65535),
                             r.randint(1, 100), kx, ky, 1, 1, r.randint(1, 65535), r.randint(1, 65535)))
     walk(layers)
+
+
+def test_pointwise_up_to_the_largest_batch(walk):
+    """As many pixels as the entry point takes (an int), and a few less."""
+    walk([layer(m, 1, 1, 20, 1, 1, 24, 1, 1) for m in (2 ** 31 - 1, 2 ** 31 - 16, 2 ** 31 - 600, 2 ** 31 - 5000, 65535 * 32767)])
