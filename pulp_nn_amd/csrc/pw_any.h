@@ -15,26 +15,7 @@
 #include <type_traits>
 
 #include "conv_band.h"
-
-struct PwAnyGeom {
-  const uint8_t *in;   // [M][K]
-  const int8_t *w;     // [N][K]
-  const int8_t *bias;  // may be null
-  uint8_t *out;        // [M][N]
-  int M, N, K;
-  int NB, nblk;        // channels per block (a multiple of 4 unless nblk == 1), blocks
-  int nt;              // write the output with non-temporal stores
-  int units;           // 16-pixel units
-  int nwg;             // workgroups per block of channels
-  FastDiv d_cpr, d_cpr_last;  // division by the 16-byte pieces of a pixel (of a block, of the last block)
-};
-
-// LDS: weights, k and lambda, corr, then a private output tile per wave (16 rows of 64 * NP + 20 bytes)
-#define PW_ANY_OROW(np) (64 * (np) + 20)
-static inline int pw_any_lds(int ks, int np, int nw)
-{
-  return np * 64 * (ks * 64 + 4 + 2 * (int)sizeof(bn_t)) + nw * 16 * PW_ANY_OROW(np) + 16;
-}
+#include "pw_any_geom.h"
 
 template <int KS, int NP, int MODE, int NW>
 __global__ __launch_bounds__(64 * NW) void pw_any_kernel(PwAnyGeom g, EpiArgs e)
@@ -56,10 +37,8 @@ __global__ __launch_bounds__(64 * NW) void pw_any_kernel(PwAnyGeom g, EpiArgs e)
   const int wg = g.nblk > 1 ? ((int)blockIdx.x >> 3) / g.nblk * 8 + ((int)blockIdx.x & 7) : (int)blockIdx.x;
   const int n0 = blk * g.NB, nb = min(g.NB, g.N - n0);
 
-  const int ub0 = (int)((long long)g.units * wg / g.nwg), nu = (int)((long long)g.units * (wg + 1) / g.nwg) - ub0;
-  const int u_beg = nu * wave / NW, u_end = nu * (wave + 1) / NW;
-  const int px_end = min((ub0 + u_end) * 16, g.M);
-  int px = (ub0 + u_beg) * 16;
+  int px, px_end;
+  pw_any_run(g, wg, wave, NW, &px, &px_end);
   int koff[KS];
 #pragma unroll
   for (int ks = 0; ks < KS; ks++) {
