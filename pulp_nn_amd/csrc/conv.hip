@@ -7,6 +7,7 @@
 #include "igemm_patch.h"
 #include "igemm_ring.h"
 #include "linear_any.h"
+#include "pw_any_geom.h"
 #include "pw_stream.h"
 #include "smallk.h"
 
@@ -278,7 +279,7 @@ bool launch_pw_stream_ks(int mode, int ks, bool wide, const PwGeom &g, const Epi
 bool try_pw_stream(int mode, const uint8_t *in, const int8_t *w, const int8_t *bias, void *out, long long M, int N,
                    int K, const EpiArgs &e, hipStream_t s)
 {
-  if (K > 256 || (K % 16) || !aligned(in, 16) || !aligned(w, 16) || !aligned(out, 16) || M < 2048) return false;
+  if (K > 256 || (K % 16) || !aligned(in, 16) || !aligned(w, 16) || !aligned(out, 16) || M < 2048 || M > PW_MOST_PIXELS) return false;
   if (!(N == 16 || N == 32 || N == 64 || N == 128 || N == 192 || N == 256)) return false;
   if (mode == EPI_OUT32) return false;
   const int tn = N == 16 ? 1 : (N == 32 ? 2 : 4);

@@ -7,6 +7,10 @@
 
 #include "fastdiv.h"
 
+// Most pixels of a layer that pw_any_kernel and pw_stream_kernel take: a run's counter goes up to three steps (of 16 and of 32
+// pixels) past its end.
+static constexpr long long PW_MOST_PIXELS = 0x7fffffffLL - 128;
+
 struct PwAnyGeom {
   const uint8_t *in;   // [M][K]
   const int8_t *w;     // [N][K]
@@ -41,7 +45,7 @@ PULPNN_HD void pw_any_run(const PwAnyGeom &g, int wg, int wave, int nw, int *px,
 inline bool pw_any_shape(long long M, int N, int K, int cus, int bn_bytes, PwAnyGeom *out, int *ks_out, int *np_out)
 {
   if (K > 512 || N < 16 || M * K < 16 || (long long)N * K < 16) return false;
-  if (M > 0x7fffffffLL - 64) return false;  // (the pixel counter goes up to three steps past the end)
+  if (M > PW_MOST_PIXELS) return false;
   PwAnyGeom &g = *out;
   g = PwAnyGeom{};
   g.M = (int)M;

@@ -22,9 +22,10 @@ static std::string check(long long M, int N, int K, int bn_bytes, int cus)
       pw_any_run(g, wg, wave, nw, &px, &px_end);
       if (px >= px_end) continue;
       if (px != next) return "run starts at pixel " + std::to_string(px) + ", the one before ended at " + std::to_string(next);
-      // the run's last step asks for the pixels of two steps ahead, and its counter goes one step past the end
+      // the run's last step asks for the pixels of two steps ahead, and its counter goes one step past the end (steps of 32 in
+      // pw_stream_kernel, which has the same limit)
       const long long last = px + (px_end - 1ll - px) / 16 * 16;
-      if (last + 32 + 15 > 0x7fffffffll) return "pixel counter past an int: " + std::to_string(last);
+      if (last + 3 * 32 + 15 > 0x7fffffffll) return "pixel counter past an int: " + std::to_string(last);
       next = px_end;
       runs++;
     }
