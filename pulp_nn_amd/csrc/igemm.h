@@ -39,6 +39,7 @@
 #include <type_traits>
 
 #include "fastdiv.h"
+#include "igemm_gather.h"
 #include "memops.h"
 #include "requant.h"
 
@@ -231,28 +232,11 @@ void igemm_kernel(ConvGeom g, EpiArgs e)
 #pragma unroll
     for (int i = 0; i < RA; i++) {
       const int m = m0 + (tid >> 2) + RPP * i;
-      // (a row past the last pixel: with SUB the tap's offset is added to poff before the range check, so 0xffffffff
-      // alone would wrap to an address in front of the input; every tap of such a row is out of range)
-      poff[i] = 0xffffffffu;
-      pinv[i] = SUB ? ~0u : 0u;
-      if (m < g.M) {
-        const int b = (int)fastdiv((unsigned)m, g.d_howo), rem = m - b * g.HoWo;
-        const int oy = (int)fastdiv((unsigned)rem, g.d_wo), ox = rem - oy * g.Wo;
-        poff[i] = (unsigned)b * (unsigned)g.in_img + (unsigned)((oy * g.sy * g.W + ox * g.sx) * g.Ci) +
-                  (SUB ? (16u * ck) & (unsigned)(g.Ci - 1) : 16u * ck);
-        if (SUB) pinv[i] = ~0u << (g.kx * g.ky);  // taps past the filter (the tail of the last K slice)
-        for (int fy_ = 0, t = 0; fy_ < g.ky; fy_++)
-          for (int fx_ = 0; fx_ < g.kx; fx_++, t++) {
-            const int iy = oy * g.sy - g.pt + fy_, ix = ox * g.sx - g.pl + fx_;
-            if ((unsigned)iy >= (unsigned)g.H || (unsigned)ix >= (unsigned)g.W) pinv[i] |= 1u << t;
-          }
-      }
+      igemm_row_gather<SUB>(g, m, ck, &poff[i], &pinv[i]);
     }
   }
-  // GATHER_SUBTAP: which of the slice's taps this lane's chunk belongs to, and 65536 / kx rounded up
-  // (t * that >> 16 == t / kx for the tap numbers that occur: t < 32, kx <= 32)
+  // GATHER_SUBTAP: which of the slice's taps this lane's chunk belongs to
   [[maybe_unused]] const int sub_h = SUB ? (16 * ck) >> g.ci_shift : 0;
-  [[maybe_unused]] const int sub_rkx = g.rkx;
   // (fy, fx, ci) of byte k = 16*ck of the current K slice
   int kpos = 16 * ck;
   int ci = 0, tap = 0, fy = 0, fx = 0;
@@ -303,12 +287,9 @@ void igemm_kernel(ConvGeom g, EpiArgs e)
       typedef unsigned v4u __attribute__((ext_vector_type(4)));
       // tap of this lane's chunk: taps per slice * slice + (16 * ck) / Ci; at most 31
       const int t = (u_slice << (6 - g.ci_shift)) + sub_h;
-      const int tfy = (t * sub_rkx) >> 16, tfx = t - tfy * g.kx;
-      const unsigned toff = (unsigned)((tfy * g.W + tfx) * g.Ci);
 #pragma unroll
       for (int i = 0; i < RA; i++) {
-        const unsigned oob = (unsigned)__builtin_amdgcn_sbfe((int)pinv[i], t, 1);
-        const v4u v = __builtin_amdgcn_raw_buffer_load_b128(rsrc_a, (poff[i] + toff) | oob, 0, 0);
+        const v4u v = __builtin_amdgcn_raw_buffer_load_b128(rsrc_a, igemm_sub_offset(g, poff[i], pinv[i], t), 0, 0);
         R.a[i] = (v4i){(int)v.x, (int)v.y, (int)v.z, (int)v.w};
       }
       // weight bytes past the end of a row (K is not a multiple of 64) belong to the next row: out of range instead
