@@ -17,6 +17,7 @@
 #include <string.h>
 
 #include <exception>
+#include <new>
 #include <string>
 #include <vector>
 
@@ -332,8 +333,8 @@ struct Call {
   int f;
   Args a;
   PyObject *owner[10];  // what pointer i belongs to; null: the chain's input
-  PyObject *block_list;  // the chain entry point's
-  std::vector<pulp_nn_hip_block> blocks;
+  PyObject *blocks;  // the chain entry point's, a tuple
+  size_t n_blocks;
 };
 // what the plan was made from: dict[key] was value (null: absent)
 struct Guard {
@@ -431,17 +432,20 @@ int plan_init(PyObject *self, PyObject *args, PyObject *)
       }
     }
     if (fn_kind[c.f] == CHAIN) {
-      PyObject *blocks = PyTuple_GetItem(a, 5);
-      if (!blocks) return -1;
-      if (!PyList_Check(blocks)) {
+      PyObject *list_of = PyTuple_GetItem(a, 5);
+      if (!list_of) return -1;
+      if (!PyList_Check(list_of)) {
         PyErr_SetString(PyExc_TypeError, "the blocks are a list");
         return -1;
       }
-      c.block_list = blocks;
-      for (Py_ssize_t j = 0; j < PyList_GET_SIZE(blocks); j++) {
+      c.blocks = PyList_AsTuple(list_of);
+      if (!c.blocks) return -1;
+      c.n_blocks = (size_t)PyTuple_GET_SIZE(c.blocks);
+      for (size_t j = 0; j < c.n_blocks; j++) {
         pulp_nn_hip_block b;
-        if (!block_from(PyList_GET_ITEM(blocks, j), &b)) return -1;
-        c.blocks.push_back(b);
+        if (block_from(PyTuple_GET_ITEM(c.blocks, j), &b)) continue;
+        Py_DECREF(c.blocks);
+        return -1;
       }
     }
     pl->calls->push_back(c);
@@ -463,17 +467,31 @@ PyObject *plan_run(PyObject *self, PyObject *x)
     if (eq < 0) return nullptr;
     if (!eq) Py_RETURN_FALSE;
   }
-  for (Call &c : *pl->calls) {
-    for (int i = 0; i < 10; i++)
-      if (c.owner[i] != Py_None && !to_ptr(c.owner[i] ? c.owner[i] : x, &c.a.p[i])) return nullptr;
-    for (size_t i = 0; i < c.blocks.size(); i++)
-      if (!block_from(PyList_GET_ITEM(c.block_list, i), &c.blocks[i])) return nullptr;
+  // A run's addresses are its own: another thread may enter while this one queues without the interpreter lock.
+  std::vector<Args> args;
+  std::vector<pulp_nn_hip_block> blocks;
+  try {
+    args.reserve(pl->calls->size());
+    for (const Call &c : *pl->calls) {
+      args.push_back(c.a);
+      for (int i = 0; i < 10; i++)
+        if (c.owner[i] != Py_None && !to_ptr(c.owner[i] ? c.owner[i] : x, &args.back().p[i])) return nullptr;
+      for (size_t i = 0; i < c.n_blocks; i++) {
+        blocks.emplace_back();
+        if (!block_from(PyTuple_GET_ITEM(c.blocks, i), &blocks.back())) return nullptr;
+      }
+    }
+  } catch (const std::bad_alloc &) {
+    return PyErr_NoMemory();
   }
   int err = 0;
   Py_BEGIN_ALLOW_THREADS
   ((void (*)(unsigned))b->fn[F_SET_BATCH])(pl->batch);
-  for (const Call &c : *pl->calls) {
-    invoke(b, c.f, c.a, c.blocks.data(), (unsigned)c.blocks.size());
+  const pulp_nn_hip_block *next = blocks.data();
+  for (size_t j = 0; j < args.size(); j++) {
+    const Call &c = (*pl->calls)[j];
+    invoke(b, c.f, args[j], next, (unsigned)c.n_blocks);
+    next += c.n_blocks;
     if (b->check && (err = last_error(b))) break;
   }
   Py_END_ALLOW_THREADS
@@ -492,6 +510,8 @@ void plan_dealloc(PyObject *self)
       Py_XDECREF(g.key);
       Py_XDECREF(g.value);
     }
+  if (pl->calls)
+    for (Call &c : *pl->calls) Py_XDECREF(c.blocks);
   delete pl->guards;
   delete pl->calls;
   Py_TYPE(self)->tp_free(self);
