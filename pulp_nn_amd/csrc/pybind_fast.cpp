@@ -454,7 +454,8 @@ int plan_init(PyObject *self, PyObject *args, PyObject *)
 }
 
 // run(x): queues every call with x as the chain's input; raises like the calls themselves would.  False, with nothing
-// queued, if what the plan was made from has changed.
+// queued, if what the plan was made from has changed.  Where the library has no kernel for a call on these addresses
+// (code 2): the call's index, with the calls in front of it queued and none from it on.
 PyObject *plan_run(PyObject *self, PyObject *x)
 {
   Plan *pl = (Plan *)self;
@@ -485,16 +486,23 @@ PyObject *plan_run(PyObject *self, PyObject *x)
     return PyErr_NoMemory();
   }
   int err = 0;
+  size_t j = 0;
   Py_BEGIN_ALLOW_THREADS
   ((void (*)(unsigned))b->fn[F_SET_BATCH])(pl->batch);
   const pulp_nn_hip_block *next = blocks.data();
-  for (size_t j = 0; j < args.size(); j++) {
+  for (; j < args.size(); j++) {
     const Call &c = (*pl->calls)[j];
     invoke(b, c.f, args[j], next, (unsigned)c.n_blocks);
     next += c.n_blocks;
     if (b->check && (err = last_error(b))) break;
   }
   Py_END_ALLOW_THREADS
+  if (err == PULP_NN_HIP_ERR_UNSUPPORTED) {
+    PyObject *r = PyObject_CallMethod(pl->nn, "clear_error", nullptr);
+    if (!r) return nullptr;
+    Py_DECREF(r);
+    return PyLong_FromSize_t(j);
+  }
   if (err) return PyObject_CallMethod(pl->nn, "_raise", nullptr);
   Py_RETURN_TRUE;
 }

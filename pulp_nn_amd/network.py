@@ -85,7 +85,7 @@ class _Recorder:
               "dw_pw_hwc": "pulp_nn_hip_dw_pw_hwc", "dw_pw_chain_hwc": "pulp_nn_hip_dw_pw_chain_hwc"}
 
     def __init__(self):
-        self.calls = []
+        self.calls, self.at, self.calls_at = [], None, []
 
     def set_batch(self, n):
         pass
@@ -95,6 +95,7 @@ class _Recorder:
             if name == "hwc_to_chw":
                 args += (0,) * (7 - len(args))   # pad_top, pad_bottom
             self.calls.append((self._NAMES.get(name, name), args))
+            self.calls_at.append(self.at)
         return call
 
 
@@ -143,7 +144,10 @@ class Runner:
                 H, W, Cc = self.shapes[L["in"]]
                 self.chw[L["name"]] = torch.empty((batch, Cc, H, W), dtype=torch.uint8, device="cuda")
         self._calib = None
-        self._plan = None        # (choices, objects, plan, result tensor, launches)
+        self._forget()
+
+    def _forget(self):
+        self._plan = None        # (choices, objects, plan, result tensor, launches, [(layer, launches) before a call])
         self._walked = None      # the choices of the last walk
 
     # -- one layer ------------------------------------------------------------------------
@@ -219,10 +223,15 @@ class Runner:
         if self._plan is None and self._walked == choices and self.layers:
             self._lay_out_plan(choices)
         if self._plan is not None:
-            made_with, objects, plan, out, launches = self._plan
-            if made_with == choices and all(a is b for a, b in zip(objects, self._objects())) and plan.run(x):
-                self.launches = launches
-                return out
+            made_with, objects, plan, out, launches, calls_at = self._plan
+            if made_with == choices and all(a is b for a, b in zip(objects, self._objects())):
+                done = plan.run(x)
+                if done is True:
+                    self.launches = launches
+                    return out
+                if done is not False:   # no kernel for a call on this input (its alignment): the walk takes other layers from there
+                    self._plan = None
+                    return self._walk(x, self.nn, *calls_at[done])
             self._plan = None
         out = self._walk(x, self.nn)
         self._walked = self._choices()
@@ -245,15 +254,19 @@ class Runner:
         made_from = [(L, ("op", "in") + shape.get(L["op"], ("strides", "pads")) +
                       scalars.get(L["op"], ("shift", "mult", "relu", "bn"))) for L in self.layers]
         made_from += [(P, tuple(P)) for P in self.params] + [(d, tuple(d)) for d in (self.act, self.chw)]
-        self._plan = (choices, self._objects(), api._fast.Plan(self.nn, self.batch, rec.calls, marker, made_from), out, self.launches)
+        self._plan = (choices, self._objects(), api._fast.Plan(self.nn, self.batch, rec.calls, marker, made_from), out, self.launches,
+                      rec.calls_at)
 
-    def _walk(self, x, nn):
+    def _walk(self, x, nn, first=0, launches=0):
+        """Queues the layers from `first` on, the ones before it being queued in `launches` launches."""
         nn.set_batch(self.batch)
-        tensors = {"input": x}
+        tensors = {"input": x, **{L["name"]: self.act[L["name"]] for L in self.layers[:first]}}
         out = x
-        self.launches = 0
-        i = 0
+        self.launches = launches
+        i = first
         while i < len(self.layers):
+            if isinstance(nn, _Recorder):
+                nn.at = (i, self.launches)
             L = self.layers[i]
             n = self._chain_length(i) if self.chain_blocks else 0
             if n >= 2 and self._queue_chain(i, n, tensors, nn):

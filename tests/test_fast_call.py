@@ -1,11 +1,13 @@
 """The extension module behind the Python front end (csrc/pybind_fast.cpp), as far as it goes without a GPU: argument
 counts, keywords, rejected calls, and plans that notice what they were made from has changed."""
 import ctypes
+import types
 
+import numpy as np
 import pytest
 import torch
 
-from pulp_nn_amd import api
+from pulp_nn_amd import api, network
 
 pytestmark = pytest.mark.skipif(api._fast is None, reason="extension not built")
 
@@ -77,37 +79,39 @@ def test_plan_asks_for_addresses_at_each_run(nn):
             refused()
 
 
+POINTERS = dict({n: 7 for n in api.CONV_NAMES}, **{n: 8 for n in api.DW_NAMES}, pulp_nn_linear=6, pulp_nn_linear_out_32=4, pulp_nn_maxpool=2,
+                pulp_nn_avgpool=2, pulp_nn_add=3, pulp_nn_depthwise_3x3_s1=2, pulp_nn_hip_hwc_to_chw=2, pulp_nn_hip_depthwise_hwc=6,
+                pulp_nn_hip_dw_pw_hwc=2)
+
+
 class FakeLibrary:
-    """The entry points as Python functions: pulp_nn_add and the chain record the addresses they get, the others do nothing."""
+    """The entry points as Python functions that note the pointers they are given (their leading arguments)."""
 
     def __init__(self):
-        self.seen, self.error, self.on_add, self.batch = [], 0, None, None
-        nothing = ctypes.CFUNCTYPE(None)(lambda: None)
-        add = ctypes.CFUNCTYPE(None, *[ctypes.c_void_p] * 3, *[ctypes.c_uint16] * 6)(self._add)
-        chain = ctypes.CFUNCTYPE(None, *[ctypes.c_void_p] * 2, *[ctypes.c_uint16] * 3, ctypes.c_uint, ctypes.POINTER(api.HipBlock))(self._chain)
-        last_error = ctypes.CFUNCTYPE(ctypes.c_int)(lambda: self.error)
-        set_batch = ctypes.CFUNCTYPE(None, ctypes.c_uint)(lambda n: setattr(self, "batch", n))
-        self.keep = dict.fromkeys(api.FAST_NAMES, nothing)
-        self.keep.update(pulp_nn_add=add, pulp_nn_hip_dw_pw_chain_hwc=chain, pulp_nn_hip_last_error=last_error, pulp_nn_hip_set_batch=set_batch)
+        self.seen, self.error, self.batch = [], 0, None
+        self.on_call = lambda n, name, pointers: None   # n: how many calls there have been
+        chain = ctypes.CFUNCTYPE(None, *[ctypes.c_void_p] * 2, *[ctypes.c_uint16] * 3, ctypes.c_uint, ctypes.POINTER(api.HipBlock))
+        self.keep = {n: ctypes.CFUNCTYPE(None, *[ctypes.c_void_p] * k)(self._noter(n)) for n, k in POINTERS.items()}
+        note = self._noter("pulp_nn_hip_dw_pw_chain_hwc")
+        self.keep.update(
+            pulp_nn_hip_dw_pw_chain_hwc=chain(lambda x, out, w, h, c, n, blocks: note(x, out, *(blocks[i].dw_wt for i in range(n)))),
+            pulp_nn_hip_last_error=ctypes.CFUNCTYPE(ctypes.c_int)(lambda: self.error),
+            pulp_nn_hip_clear_error=ctypes.CFUNCTYPE(None)(lambda: setattr(self, "error", 0)),
+            pulp_nn_hip_set_batch=ctypes.CFUNCTYPE(None, ctypes.c_uint)(lambda n: setattr(self, "batch", n)))
 
-    def _add(self, a, b, out, m1, m2, shift, h, w, ch):
-        self.seen.append((a, b, out))
-        if self.on_add:
-            self.on_add(len(self.seen), a)
+    def _noter(self, name):
+        def note(*pointers):
+            self.error = 0
+            self.seen.append((name,) + pointers)
+            self.on_call(len(self.seen), name, pointers)
+        return note
 
-    def _chain(self, x, out, w, h, c, n, blocks):
-        self.seen.append((x, out) + tuple(blocks[i].dw_wt for i in range(n)))
-
-    def bound(self):
-        nn = api.PulpNN.__new__(api.PulpNN)
-        nn._bind(32, {n: ctypes.cast(f, ctypes.c_void_p).value for n, f in self.keep.items()})
-        nn.check = True
-        nn._raise = self._raise
+    def bound(self, cls=api.PulpNN):
+        nn = cls.__new__(cls)
+        nn._bind(32, {n: ctypes.cast(self.keep[n], ctypes.c_void_p).value for n in api.FAST_NAMES})
+        nn.check, nn.bn_bits = True, 32
+        nn._lib = types.SimpleNamespace(**self.keep, pulp_nn_hip_last_error_string=lambda: b"fake")
         return nn
-
-    def _raise(self):
-        code, self.error = self.error, 0
-        raise api.PulpNNError(code, "fake")
 
 
 def test_runs_of_one_plan_do_not_share_addresses():
@@ -118,8 +122,88 @@ def test_runs_of_one_plan_do_not_share_addresses():
     calls = [("pulp_nn_add", (marker, 1, 2, 1, 1, 1, 1, 1, 1)), ("pulp_nn_add", (3, marker, 4, 1, 1, 1, 1, 1, 1)),
              ("pulp_nn_hip_dw_pw_chain_hwc", (marker, 5, 1, 1, 1, [block, block]))]
     plan = api._fast.Plan(lib.bound(), 6, calls, marker, [])
-    lib.on_add = lambda n, a: plan.run(2000) if n == 1 else None
+    lib.on_call = lambda n, name, pointers: plan.run(2000) if n == 1 else None
     assert plan.run(1000) is True
     inner = [(2000, 1, 2), (3, 2000, 4), (2000, 5, 7, 7)]
-    assert lib.seen == [(1000, 1, 2)] + inner + [(3, 1000, 4), (1000, 5, 7, 7)]
+    assert [c[1:] for c in lib.seen] == [(1000, 1, 2)] + inner + [(3, 1000, 4), (1000, 5, 7, 7)]
     assert lib.batch == 6
+
+
+def test_plan_stops_at_a_call_without_a_kernel():
+    """Code 2 is an answer, not an exception: the index of the call, for the caller to go on from."""
+    lib = FakeLibrary()
+    marker = object()
+    plan = api._fast.Plan(lib.bound(), 1, [("pulp_nn_add", (marker, i, 2, 1, 1, 1, 1, 1, 1)) for i in range(3)], marker, [])
+
+    def fail(code, when):
+        def on_call(n, name, pointers):
+            lib.error = code if when(n, *pointers) else 0
+        lib.on_call = on_call
+
+    fail(2, lambda n, a, b, out: b == 1 and a % 4)
+    assert plan.run(1001) == 1 and len(lib.seen) == 2 and lib.error == 0
+    lib.seen.clear()
+    assert plan.run(1000) is True and len(lib.seen) == 3
+    fail(1, lambda n, a, b, out: True)
+    with pytest.raises(api.PulpNNError):
+        plan.run(1000)
+
+
+def bare_runner(nn, layers, input_shape, batch=1):
+    """A runner whose tensors are addresses: the table's walk and its plan, without a GPU."""
+    r = network.Runner.__new__(network.Runner)
+    r.nn, r.layers, r.batch, r.fused, r.unfused = nn, layers, batch, True, set()
+    r.fuse_blocks, r.unfused_blocks, r.launches, r.block_choice, r.chain_blocks, r.unchained = "auto", set(), 0, {}, True, set()
+    r.shapes = network.infer_shapes(layers, input_shape)
+    address = iter(range(0x10000, 0x7fffffff, 0x1000))
+    r.params = [{k: next(address) for k in ("w", "bias", "k", "lam") if L.get(k) is not None} for L in layers]
+    r.act = {L["name"]: next(address) for L in layers}
+    r.chw = {L["name"]: next(address) for L in layers if L["op"] == "depthwise"}
+    r._forget()
+    return r
+
+
+def small_table():
+    """Depthwise + pointwise twice (a chain), a depthwise layer, two layers that read the input as well, a linear layer."""
+    def bn(n):
+        return dict(bias=np.zeros(n, np.int8), k=np.ones(n), lam=np.zeros(n), relu=1, bn=1, mult=0, shift=5)
+
+    def dw(name, src):
+        return dict(bn(64), op="depthwise", name=name, **{"in": src}, w=np.zeros((64, 3, 3), np.int8), pads=[1, 1, 1, 1], strides=[1, 1])
+
+    def pw(name, src):
+        return dict(bn(64), op="pointwise", name=name, **{"in": src}, w=np.zeros((64, 1, 1, 64), np.int8))
+
+    return [dw("d1", "input"), pw("p1", "d1"), dw("d2", "p1"), pw("p2", "d2"), dw("d3", "p2"),
+            dict(op="add", name="sum", **{"in": ("d3", "input")}, m1=1, m2=1, shift=1),
+            dict(op="maxpool", name="pool", **{"in": "sum"}, kernel=[2, 2], strides=[2, 2], out_hw=[4, 4]),
+            dict(bn(10), op="linear", name="fc", **{"in": "pool"}, w=np.zeros((10, 4 * 4 * 64), np.int8))]
+
+
+def test_runner_falls_back_from_its_plan():
+    """An input for which the library has no kernel (here: at an odd address) takes the layers that a walk takes for it, also
+    once there is a plan; what has been queued is not queued again."""
+    def odd_is_refused(lib):
+        def on_call(n, name, pointers):
+            if name in ("pulp_nn_hip_dw_pw_chain_hwc", "pulp_nn_hip_depthwise_hwc", "pulp_nn_hip_dw_pw_hwc") and pointers[0] % 4:
+                lib.error = 2
+                lib.seen.pop()
+        lib.on_call = on_call
+
+    whole, tail, behind = small_table(), small_table()[4:], small_table()[4:]
+    tail[0]["in"] = behind[0]["in"] = "input"
+    behind.insert(0, dict(op="add", name="twice", **{"in": ("input", "input")}, m1=1, m2=1, shift=1))
+    behind[2]["in"] = ("d3", "twice")
+    for table in (whole, tail, behind):   # the refused call is the first one, or not
+        runs = []
+        for xs in ((0x100, 0x200, 0x300, 0x301), (0x301,)):
+            lib = FakeLibrary()
+            odd_is_refused(lib)
+            r = bare_runner(lib.bound(), table, (8, 8, 64))
+            for x in xs:
+                lib.seen.clear()
+                out = r.run(x)
+            assert out == r.act["fc"]
+            runs.append((list(lib.seen), r.launches))
+        assert runs[0] == runs[1] and len(set(runs[0][0])) == len(runs[0][0])
+        assert any(name == "pulp_nn_depthwise_generic" for name, *_ in runs[0][0])

@@ -224,3 +224,45 @@ def test_maxpool_padded(case):
     got, xin_after = maxpool(x, kernel, strides, out_hw, pads)
     assert_same(got, oracle.maxpool(x, kernel, strides, pads, out_hw=out_hw), "padded maxpool")
     assert_same(xin_after, x, "maxpool input must stay intact")
+
+
+def test_plan_falls_back_and_takes_new_inputs():
+    """A runner with a plan: another input, an input at an odd address (no fused kernel takes it: the layers go separately
+    from there on), a changed shift; each against the oracle."""
+    r = rng_for(22700)
+    B, C = 4, 64
+
+    def bn(n, shift=12):
+        return dict(bias=rand_s8(r, (n,)), k=r.integers(256, 1025, n), lam=r.integers(-2 ** 16, 2 ** 16 + 1, n), relu=1, bn=1, shift=shift)
+
+    def dw(name, src):
+        return dict(op="depthwise", name=name, **{"in": src}, w=rand_s8(r, (C, 3, 3)), pads=(1, 1, 1, 1), strides=(1, 1), **bn(C))
+
+    def pw(name, src):
+        return dict(op="pointwise", name=name, **{"in": src}, w=rand_s8(r, (C, 1, 1, C)), **bn(C, 15))
+
+    layers = [dw("d1", "input"), pw("p1", "d1"), dw("d2", "p1"), pw("p2", "d2"), dict(op="add", name="sum", **{"in": ("p2", "input")}, m1=1, m2=1, shift=1),
+              dict(op="linear", name="fc", **{"in": "sum"}, w=rand_s8(r, (10, 8 * 8 * C)), **bn(10, 20))]
+    L = nn(32)
+    L.use_torch_stream()
+    runner = network.Runner(L, layers, (8, 8, C), B)
+
+    def check(x, xd, tag):
+        want = net_oracle.forward(layers, runner.shapes, x, 32, keep=True)
+        out = runner.run(xd)
+        L.sync()
+        assert_same(out.cpu().numpy().reshape(B, 10), want["fc"].reshape(B, 10), tag)
+
+    xs = [rand_u8(r, (B, 8, 8, C)) for _ in range(4)]
+    for i, x in enumerate(xs[:3]):
+        check(x, torch.from_numpy(x).cuda(), "input %d" % i)
+    fused = runner.launches
+    odd = torch.zeros(xs[3].size + 1, dtype=torch.uint8, device="cuda")[1:].view(xs[3].shape)
+    odd.copy_(torch.from_numpy(xs[3]))
+    for _ in range(3):
+        check(xs[3], odd, "odd address")
+    assert runner.launches > fused
+    layers[1]["shift"] = 14
+    for x in xs[:2]:
+        check(x, torch.from_numpy(x).cuda(), "changed shift")
+    L.set_batch(1)
