@@ -203,3 +203,18 @@ class PulpNN(_fast.Base if _fast else object):
         return self._call("pulp_nn_matmul", _ptr(pWeight), _ptr(pIn), int(ch_out), int(num_col_im2col),
                           int(out_shift) & 0xFFFF, int(out_mult) & 0xFFFF, _ptr(k), _ptr(lam), _ptr(bias), _ptr(pOut),
                           _ptr(pOut2), int(flag_relu), int(flag_batch_norm))
+
+
+def _methods():
+    """{name: attribute} of what a run over a table calls, as PulpNN has it."""
+    names = ("set_batch", "hwc_to_chw", "depthwise_hwc", "dw_pw_hwc", "dw_pw_chain_hwc", "_call", "__getattribute__",
+             *(n for n in FAST_NAMES if "_hip_" not in n))
+    return {n: next(vars(c)[n] for c in PulpNN.__mro__ if n in vars(c)) for n in names}
+
+
+_METHODS = _methods() if _fast else None
+
+
+def plain(nn):
+    """Whether nn's layer methods are PulpNN's own, so that a plan, which calls the library directly, does what they would do."""
+    return _fast is not None and _fast.plain(nn, _METHODS)

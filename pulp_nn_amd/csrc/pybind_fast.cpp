@@ -525,10 +525,29 @@ void plan_dealloc(PyObject *self)
   Py_TYPE(self)->tp_free(self);
 }
 
+// plain(nn, {name: attribute}): whether nn is a library object on which every name is found with that attribute, that is, no
+// subclass and no attribute of the object itself overrides one.
+PyObject *plain(PyObject *, PyObject *const *args, Py_ssize_t n)
+{
+  if (n != 2 || !PyDict_Check(args[1])) {
+    PyErr_SetString(PyExc_TypeError, "plain(object, {name: attribute})");
+    return nullptr;
+  }
+  if (!PyObject_TypeCheck(args[0], &BaseType)) Py_RETURN_FALSE;
+  PyObject *key, *value, **own = _PyObject_GetDictPtr(args[0]);
+  for (Py_ssize_t pos = 0; PyDict_Next(args[1], &pos, &key, &value);)
+    if (_PyType_Lookup(Py_TYPE(args[0]), key) != value) Py_RETURN_FALSE;
+  if (own && *own)
+    for (Py_ssize_t pos = 0; PyDict_Next(*own, &pos, &key, &value);)
+      if (PyDict_GetItem(args[1], key)) Py_RETURN_FALSE;
+  Py_RETURN_TRUE;
+}
+
+PyMethodDef module_methods[] = {{"plain", (PyCFunction)(void (*)(void))plain, METH_FASTCALL, nullptr}, {nullptr, nullptr, 0, nullptr}};
 PyMethodDef plan_methods[] = {{"run", plan_run, METH_O, nullptr}, {nullptr, nullptr, 0, nullptr}};
 PyTypeObject PlanType = {PyVarObject_HEAD_INIT(nullptr, 0)};
 
-PyModuleDef module = {PyModuleDef_HEAD_INIT, "_pulpnn_fast", nullptr, -1, nullptr};
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "_pulpnn_fast", nullptr, -1, module_methods};
 
 }  // namespace
 

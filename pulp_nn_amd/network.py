@@ -219,6 +219,9 @@ class Runner:
 
     def run(self, x):
         """x: device tensor batch,H,W,C uint8.  Queues every layer; returns the last layer's tensor."""
+        if not api.plain(self.nn):   # a layer method is overridden, or nn only wraps a library: its methods are called
+            self._forget()
+            return self._walk(x, self.nn)
         choices = self._choices()
         if self._plan is None and self._walked == choices and self.layers:
             self._lay_out_plan(choices)

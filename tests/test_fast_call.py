@@ -207,3 +207,49 @@ def test_runner_falls_back_from_its_plan():
             runs.append((list(lib.seen), r.launches))
         assert runs[0] == runs[1] and len(set(runs[0][0])) == len(runs[0][0])
         assert any(name == "pulp_nn_depthwise_generic" for name, *_ in runs[0][0])
+
+
+@pytest.mark.parametrize("how", ["subclass", "attribute", "class attribute", "chain", "wrapper"])
+def test_overridden_methods_are_called_at_every_run(how, monkeypatch):
+    """Tracing or logging put over a layer method, before the runner is made or once it has a plan; an object that only wraps
+    a library."""
+    lib, log = FakeLibrary(), []
+    name = "dw_pw_chain_hwc" if how == "chain" else "pulp_nn_add"
+    original = getattr(api.PulpNN, name)
+
+    def traced(self, *args):
+        log.append(args[0])
+        return original(self, *args)
+
+    if how == "wrapper":
+        real = lib.bound()
+
+        class Wrapper:
+            def __getattr__(self, n):
+                return getattr(real, n) if n != name else lambda *args: traced(real, *args)
+        nn = Wrapper()
+    else:
+        nn = lib.bound(type("Traced", (api.PulpNN,), {name: traced}) if how == "subclass" else api.PulpNN)
+    r = bare_runner(nn, small_table(), (8, 8, 64))
+    if how not in ("subclass", "wrapper"):
+        for x in (0x100, 0x200, 0x300):
+            r.run(x)
+        assert not log
+    if how == "attribute":
+        nn.pulp_nn_add = lambda *args: traced(nn, *args)
+    elif how in ("class attribute", "chain"):
+        monkeypatch.setattr(api.PulpNN, name, traced, raising=False)
+    runs = []
+    for x in (0x400, 0x500, 0x600):
+        log.clear()
+        lib.seen.clear()
+        r.run(x)
+        assert log == ([x] if how == "chain" else [r.act["d3"]])
+        runs.append([c[1:] for c in lib.seen])
+    assert [len(s) for s in runs] == [5] * 3
+    if how == "attribute":               # and away again
+        del nn.pulp_nn_add
+        for x in (0x400, 0x500, 0x600):
+            log.clear()
+            r.run(x)
+            assert not log
