@@ -336,9 +336,14 @@ struct Call {
   PyObject *blocks;  // the chain entry point's, a tuple
   size_t n_blocks;
 };
-// what the plan was made from: dict[key] was value (null: absent)
+// what the plan was made from: dict[key] was value (null: absent); items: what a list held, which may change in place
 struct Guard {
-  PyObject *dict, *key, *value;
+  PyObject *dict, *key, *value, *items;
+};
+// a dictionary of which every entry counts, with as many of them as there were (guards of these follow each other)
+struct Whole {
+  PyObject *dict;
+  Py_ssize_t size;
 };
 struct Plan {
   PyObject_HEAD
@@ -346,6 +351,7 @@ struct Plan {
   PyObject *keep;    // the argument tuples: whatever owns the addresses
   std::vector<Call> *calls;
   std::vector<Guard> *guards;
+  std::vector<Whole> *wholes;
   unsigned batch;
 };
 
@@ -374,9 +380,51 @@ bool block_from(PyObject *t, pulp_nn_hip_block *b)
   return true;
 }
 
-// Plan(nn, batch, [(entry point, arguments), ...], input, [(dict, (key, ...)), ...]): `input` is the object that stands for the
-// chain's input in the arguments.  The chain entry point's arguments are (x, out, dim_x, dim_y, ch, [block, ...]).  The
-// pairs name the entries the calls were made from: run() does nothing once one of them has changed.
+// the same value: the same object, or an equal int
+int same(PyObject *a, PyObject *b)
+{
+  if (a == b) return 1;
+  if (!a || !b || !PyLong_CheckExact(a) || !PyLong_CheckExact(b)) return 0;
+  return PyObject_RichCompareBool(a, b, Py_EQ);
+}
+
+// 1 if the entry is what it was, 0 if not, -1 with an exception set
+int unchanged(const Guard &g)
+{
+  PyObject *v = PyDict_GetItem(g.dict, g.key);
+  const int eq = same(v, g.value);
+  if (eq != 1 || !g.items) return eq;
+  if (PyList_GET_SIZE(v) != PyTuple_GET_SIZE(g.items)) return 0;
+  for (Py_ssize_t i = 0; i < PyList_GET_SIZE(v); i++) {
+    const int e = same(PyList_GET_ITEM(v, i), PyTuple_GET_ITEM(g.items, i));
+    if (e != 1) return e;
+  }
+  return 1;
+}
+
+bool add_guard(Plan *pl, PyObject *dict, PyObject *key, PyObject *value)
+{
+  Guard g = {dict, key, value, nullptr};
+  if (value && PyList_Check(value) && !(g.items = PyList_AsTuple(value))) return false;
+  Py_INCREF(g.dict);
+  Py_INCREF(g.key);
+  Py_XINCREF(g.value);
+  pl->guards->push_back(g);
+  return true;
+}
+
+// a value that cannot change in place, or a list, whose items are kept
+bool is_scalar(PyObject *v)
+{
+  if (v == Py_None || PyLong_Check(v) || PyFloat_Check(v) || PyUnicode_Check(v) || PyTuple_Check(v) || PyList_Check(v)) return true;
+  return PyNumber_Check(v) && Py_TYPE(v)->tp_hash != PyObject_HashNotImplemented && !THPVariable_Check(v);  // (numpy's scalars)
+}
+
+// Plan(nn, batch, [(entry point, arguments), ...], input, [(dict, which), ...]): `input` is the object that stands
+// for the chain's input in the arguments.  The chain entry point's arguments are (x, out, dim_x, dim_y, ch, [block, ...]).  The
+// pairs name the entries the calls were made from, as a tuple of keys, None (all of the dictionary's, and that there are no
+// others) or a set (the same; the values of other keys than these have to be numbers, texts, tuples or lists, not arrays, which
+// change in place): run() does nothing once one of them has changed, a list's items included.
 int plan_init(PyObject *self, PyObject *args, PyObject *)
 {
   Plan *pl = (Plan *)self;
@@ -392,16 +440,29 @@ int plan_init(PyObject *self, PyObject *args, PyObject *)
   pl->keep = list;
   pl->calls = new std::vector<Call>();
   pl->guards = new std::vector<Guard>();
+  pl->wholes = new std::vector<Whole>();
   for (Py_ssize_t i = 0; i < PyList_GET_SIZE(from); i++) {
-    PyObject *dict, *keys;
-    if (!PyArg_ParseTuple(PyList_GET_ITEM(from, i), "O!O!", &PyDict_Type, &dict, &PyTuple_Type, &keys)) return -1;
-    for (Py_ssize_t j = 0; j < PyTuple_GET_SIZE(keys); j++) {
-      const Guard g = {dict, PyTuple_GET_ITEM(keys, j), PyDict_GetItem(dict, PyTuple_GET_ITEM(keys, j))};
-      Py_INCREF(g.dict);
-      Py_INCREF(g.key);
-      Py_XINCREF(g.value);
-      pl->guards->push_back(g);
+    PyObject *dict, *keys, *key, *value;
+    if (!PyArg_ParseTuple(PyList_GET_ITEM(from, i), "O!O", &PyDict_Type, &dict, &keys)) return -1;
+    if (keys == Py_None || PyAnySet_Check(keys)) {
+      for (Py_ssize_t pos = 0; PyDict_Next(dict, &pos, &key, &value);) {
+        const int object = keys == Py_None ? 1 : PySet_Contains(keys, key);
+        if (object < 0 || !add_guard(pl, dict, key, value)) return -1;
+        if (!object && !is_scalar(value)) {
+          PyErr_Format(PyExc_TypeError, "%R is a %.100s, which may change in place", key, Py_TYPE(value)->tp_name);
+          return -1;
+        }
+      }
+      Py_INCREF(dict);
+      pl->wholes->push_back(Whole{dict, PyDict_Size(dict)});
+      continue;
     }
+    if (!PyTuple_Check(keys)) {
+      PyErr_SetString(PyExc_TypeError, "the keys are a tuple, a set or None");
+      return -1;
+    }
+    for (Py_ssize_t j = 0; j < PyTuple_GET_SIZE(keys); j++)
+      if (!add_guard(pl, dict, PyTuple_GET_ITEM(keys, j), PyDict_GetItem(dict, PyTuple_GET_ITEM(keys, j)))) return -1;
   }
   for (Py_ssize_t i = 0; i < PyList_GET_SIZE(list); i++) {
     const char *name;
@@ -460,13 +521,12 @@ PyObject *plan_run(PyObject *self, PyObject *x)
 {
   Plan *pl = (Plan *)self;
   Base *b = (Base *)pl->nn;
+  for (const Whole &w : *pl->wholes)
+    if (PyDict_Size(w.dict) != w.size) Py_RETURN_FALSE;
   for (const Guard &g : *pl->guards) {
-    PyObject *v = PyDict_GetItem(g.dict, g.key);
-    if (v == g.value) continue;
-    if (!v || !g.value || !PyLong_CheckExact(v) || !PyLong_CheckExact(g.value)) Py_RETURN_FALSE;
-    const int eq = PyObject_RichCompareBool(v, g.value, Py_EQ);
-    if (eq < 0) return nullptr;
-    if (!eq) Py_RETURN_FALSE;
+    const int is = unchanged(g);
+    if (is < 0) return nullptr;
+    if (!is) Py_RETURN_FALSE;
   }
   // A run's addresses are its own: another thread may enter while this one queues without the interpreter lock.
   std::vector<Args> args;
@@ -517,7 +577,11 @@ void plan_dealloc(PyObject *self)
       Py_XDECREF(g.dict);
       Py_XDECREF(g.key);
       Py_XDECREF(g.value);
+      Py_XDECREF(g.items);
     }
+  if (pl->wholes)
+    for (Whole &w : *pl->wholes) Py_DECREF(w.dict);
+  delete pl->wholes;
   if (pl->calls)
     for (Call &c : *pl->calls) Py_XDECREF(c.blocks);
   delete pl->guards;

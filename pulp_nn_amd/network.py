@@ -36,6 +36,7 @@ import numpy as np
 from . import api
 from .api import PulpNNError
 
+_ARRAYS = frozenset(("w", "bias", "bias32", "k", "lam"))   # of a layer: uploaded once, not read by run()
 CONV_LIKE = ("conv", "pointwise", "depthwise", "linear")
 
 
@@ -104,8 +105,8 @@ class Runner:
 
     The first run() walks the table in Python and learns which geometries have a fused kernel; the second lays the calls
     out as a plan (api's extension module), and from then on a run() is one call that queues them, 2 us a launch instead of
-    9.  A plan belongs to the table and the buffers it was made from: a changed shift, flag, choice or buffer makes run()
-    walk again."""
+    9.  A plan belongs to the table and the buffers it was made from: a changed entry of a layer, of its parameters or of the
+    buffers, a list changed in place, a changed choice makes run() walk again."""
 
     def __init__(self, nn, layers, input_shape, batch, fused=True, fuse_blocks="auto", chain_blocks=True):
         import torch
@@ -146,9 +147,10 @@ class Runner:
         self._calib = None
         self._forget()
 
-    def _forget(self):
+    def _forget(self, plannable=True):
         self._plan = None        # (choices, objects, plan, result tensor, launches, [(layer, launches) before a call])
         self._walked = None      # the choices of the last walk
+        self._plannable = plannable
 
     # -- one layer ------------------------------------------------------------------------
     def _requant_args(self, L, P):
@@ -223,7 +225,7 @@ class Runner:
             self._forget()
             return self._walk(x, self.nn)
         choices = self._choices()
-        if self._plan is None and self._walked == choices and self.layers:
+        if self._plan is None and self._plannable and self._walked == choices and self.layers:
             self._lay_out_plan(choices)
         if self._plan is not None:
             made_with, objects, plan, out, launches, calls_at = self._plan
@@ -241,24 +243,22 @@ class Runner:
         return out
 
     def _choices(self):
-        return (len(self.layers), self.batch, self.fused, self.fuse_blocks, self.chain_blocks, len(self.unfused),
-                len(self.unfused_blocks), len(self.unchained), tuple(self.block_choice.items()))
+        return (len(self.layers), len(self.params), self.batch, self.fused, self.fuse_blocks, self.chain_blocks, tuple(self.unfused),
+                tuple(self.unfused_blocks), tuple(self.unchained), tuple(self.block_choice.items()))
 
     def _objects(self):
-        return (self.nn, self.layers, self.params, self.act, self.chw, *self.layers)
+        return (self.nn, self.layers, self.params, self.act, self.chw, self.shapes, *self.layers, *self.params)
 
     def _lay_out_plan(self, choices):
         """The calls of a walk (the last one has met every geometry without a kernel), and the entries they are made from."""
         marker, rec = object(), _Recorder()
         out = self._walk(marker, rec)
-        scalars = {"add": ("m1", "m2", "shift"), "avgpool": ("lam", "shift", "add", "requant"), "maxpool": (), "linear_out_32": ()}
-        shape = {"add": (), "linear": (), "linear_out_32": (), "pointwise": (), "maxpool": ("kernel", "strides", "pads"),
-                 "avgpool": ("kernel", "strides")}
-        made_from = [(L, ("op", "in") + shape.get(L["op"], ("strides", "pads")) +
-                      scalars.get(L["op"], ("shift", "mult", "relu", "bn"))) for L in self.layers]
-        made_from += [(P, tuple(P)) for P in self.params] + [(d, tuple(d)) for d in (self.act, self.chw)]
-        self._plan = (choices, self._objects(), api._fast.Plan(self.nn, self.batch, rec.calls, marker, made_from), out, self.launches,
-                      rec.calls_at)
+        made_from = [(L, _ARRAYS) for L in self.layers] + [(d, None) for d in (*self.params, self.act, self.chw, self.shapes)]
+        try:
+            plan = api._fast.Plan(self.nn, self.batch, rec.calls, marker, made_from)
+        except TypeError:   # (an entry that may change in place without a trace: no plan)
+            return self._forget(plannable=False)
+        self._plan = (choices, self._objects(), plan, out, self.launches, rec.calls_at)
 
     def _walk(self, x, nn, first=0, launches=0):
         """Queues the layers from `first` on, the ones before it being queued in `launches` launches."""

@@ -253,3 +253,57 @@ def test_overridden_methods_are_called_at_every_run(how, monkeypatch):
             log.clear()
             r.run(x)
             assert not log
+
+
+def test_runner_notices_every_change():
+    """Whatever run() reads of the table, the parameters and the buffers: after a change, in place or not, and one run later
+    the calls are those of a runner that has just been made."""
+    def changes():
+        yield lambda r: r.layers[0]["pads"].__setitem__(0, 2)
+        yield lambda r: r.layers[2]["strides"].__setitem__(slice(None), [2, 2])
+        yield lambda r: r.layers[6]["kernel"].__setitem__(1, 3)
+        yield lambda r: r.layers[4].update(shift=7)
+        yield lambda r: r.layers[4].update(mult=np.int32(3))
+        yield lambda r: r.layers[5].update(m2=2)
+        yield lambda r: r.layers[6].update(pads=(0, 1, 0, 0))     # a key that was absent
+        yield lambda r: r.params[7].pop("bias")
+        yield lambda r: r.params[1].update(bias=0x99)
+        yield lambda r: r.params.__setitem__(3, dict(r.params[3], w=0x98))
+        yield lambda r: r.act.update(sum=0x97)
+        yield lambda r: r.shapes.update(fc=(1, 1, 9))
+        yield lambda r: setattr(r, "fused", False)
+        yield lambda r: r.unchained.add(0)
+
+    def calls_of(r, lib):
+        lib.seen.clear()
+        r.run(0x100)
+        return list(lib.seen)
+
+    for i, change in enumerate(changes()):
+        lib = FakeLibrary()
+        original = network.Runner._walk
+        r = bare_runner(lib.bound(), small_table(), (8, 8, 64))
+        walks = []
+        r._walk = lambda *a, **k: (walks.append(a[1]), original(r, *a, **k))[1]
+        for _ in range(3):
+            before = calls_of(r, lib)
+        walks.clear()
+        assert calls_of(r, lib) == before and not walks, "change %d: the plan runs" % i
+        change(r)
+        after = calls_of(r, lib)
+        assert walks and walks[0] is r.nn, "change %d was not noticed" % i
+        assert calls_of(r, lib) == after and calls_of(r, lib) == after, "change %d" % i
+
+
+def test_runner_keeps_no_plan_of_entries_that_change_without_a_trace():
+    lib = FakeLibrary()
+    r = bare_runner(lib.bound(), small_table(), (8, 8, 64))
+    r.layers[6]["kernel"] = np.array([2, 2])
+    for _ in range(4):
+        r.run(0x100)
+    assert r._plan is None
+    r = bare_runner(lib.bound(), small_table(), (8, 8, 64))
+    r.layers[4]["shift"] = np.int64(5)                            # immutable: a plan
+    for _ in range(4):
+        r.run(0x100)
+    assert r._plan is not None
