@@ -81,21 +81,26 @@ def infer_shapes(layers, input_shape):
 
 
 class _Recorder:
-    """Stands in for PulpNN: collects the calls of a walk over the table instead of making them."""
+    """Stands in for a PulpNN during a walk over the table: makes the calls and keeps those that the library took, with
+    `input` in the place of the chain's input, and the layer each belongs to."""
     _NAMES = {"hwc_to_chw": "pulp_nn_hip_hwc_to_chw", "depthwise_hwc": "pulp_nn_hip_depthwise_hwc",
               "dw_pw_hwc": "pulp_nn_hip_dw_pw_hwc", "dw_pw_chain_hwc": "pulp_nn_hip_dw_pw_chain_hwc"}
 
-    def __init__(self):
-        self.calls, self.at, self.calls_at = [], None, []
+    def __init__(self, nn, x):
+        self.nn, self.x, self.input = nn, x, object()
+        self.calls, self.calls_at, self.at = [], [], None
 
     def set_batch(self, n):
-        pass
+        self.nn.set_batch(n)
 
     def __getattr__(self, name):
+        method = getattr(self.nn, name)
+
         def call(*args):
+            method(*args)
             if name == "hwc_to_chw":
                 args += (0,) * (7 - len(args))   # pad_top, pad_bottom
-            self.calls.append((self._NAMES.get(name, name), args))
+            self.calls.append((self._NAMES.get(name, name), tuple(self.input if a is self.x else a for a in args)))
             self.calls_at.append(self.at)
         return call
 
@@ -103,9 +108,8 @@ class _Recorder:
 class Runner:
     """Uploads the parameters once, owns the activation buffers and queues the chain.
 
-    The first run() walks the table in Python and learns which geometries have a fused kernel; the second lays the calls
-    out as a plan (api's extension module), and from then on a run() is one call that queues them, 2 us a launch instead of
-    9.  A plan belongs to the table and the buffers it was made from: a changed entry of a layer, of its parameters or of the
+    The first run() walks the table in Python, learns which geometries have a fused kernel and lays the calls it made out as a
+    plan (api's extension module); from then on a run() is one call that queues them, 2 us a launch instead of 9.  A plan belongs to the table and the buffers it was made from: a changed entry of a layer, of its parameters or of the
     buffers, a list changed in place, a changed choice makes run() walk again."""
 
     def __init__(self, nn, layers, input_shape, batch, fused=True, fuse_blocks="auto", chain_blocks=True):
@@ -149,7 +153,6 @@ class Runner:
 
     def _forget(self, plannable=True):
         self._plan = None        # (choices, objects, plan, result tensor, launches, [(layer, launches) before a call])
-        self._walked = None      # the choices of the last walk
         self._plannable = plannable
 
     # -- one layer ------------------------------------------------------------------------
@@ -224,11 +227,9 @@ class Runner:
         if not api.plain(self.nn):   # a layer method is overridden, or nn only wraps a library: its methods are called
             self._forget()
             return self._walk(x, self.nn)
-        choices = self._choices()
-        if self._plan is None and self._plannable and self._walked == choices and self.layers:
-            self._lay_out_plan(choices)
-        if self._plan is not None:
-            made_with, objects, plan, out, launches, calls_at = self._plan
+        choices, laid_out = self._choices(), self._plan
+        if laid_out is not None:
+            made_with, objects, plan, out, launches, calls_at = laid_out
             if made_with == choices and all(a is b for a, b in zip(objects, self._objects())):
                 done = plan.run(x)
                 if done is True:
@@ -238,8 +239,11 @@ class Runner:
                     self._plan = None
                     return self._walk(x, self.nn, *calls_at[done])
             self._plan = None
-        out = self._walk(x, self.nn)
-        self._walked = self._choices()
+        if not self._plannable or not self.layers or any(x is t for d in (self.act, self.chw) for t in d.values()):
+            return self._walk(x, self.nn)
+        rec = _Recorder(self.nn, x)
+        out = self._walk(x, rec)
+        self._lay_out_plan(rec, out)
         return out
 
     def _choices(self):
@@ -249,16 +253,14 @@ class Runner:
     def _objects(self):
         return (self.nn, self.layers, self.params, self.act, self.chw, self.shapes, *self.layers, *self.params)
 
-    def _lay_out_plan(self, choices):
-        """The calls of a walk (the last one has met every geometry without a kernel), and the entries they are made from."""
-        marker, rec = object(), _Recorder()
-        out = self._walk(marker, rec)
+    def _lay_out_plan(self, rec, out):
+        """The calls of a walk and the entries they were made from."""
         made_from = [(L, _ARRAYS) for L in self.layers] + [(d, None) for d in (*self.params, self.act, self.chw, self.shapes)]
         try:
-            plan = api._fast.Plan(self.nn, self.batch, rec.calls, marker, made_from)
-        except TypeError:   # (an entry that may change in place without a trace: no plan)
+            plan = api._fast.Plan(self.nn, self.batch, rec.calls, rec.input, made_from)
+        except Exception:   # (an entry that may change in place without a trace, for one: no plan, the calls are made)
             return self._forget(plannable=False)
-        self._plan = (choices, self._objects(), plan, out, self.launches, rec.calls_at)
+        self._plan = (self._choices(), self._objects(), plan, out, self.launches, rec.calls_at)
 
     def _walk(self, x, nn, first=0, launches=0):
         """Queues the layers from `first` on, the ones before it being queued in `launches` launches."""
