@@ -210,6 +210,13 @@ void invoke(const Base *b, int f, const Args &a, const pulp_nn_hip_block *blocks
 
 int last_error(const Base *b) { return ((int (*)(void))b->fn[F_LAST_ERROR])(); }
 
+// whether __init__ has looked the entry points up (all of them or none)
+bool bound(const Base *b)
+{
+  if (!b->fn[F_LAST_ERROR]) PyErr_SetString(PyExc_RuntimeError, "library not bound");
+  return b->fn[F_LAST_ERROR] != nullptr;
+}
+
 // keyword arguments -> their places
 bool place_keywords(Kind kind, PyObject *const *args, Py_ssize_t n, PyObject *kw, std::vector<PyObject *> *out)
 {
@@ -263,10 +270,7 @@ PyObject *method(PyObject *self, PyObject *const *args, Py_ssize_t n, PyObject *
     args = placed.data();
     n = (Py_ssize_t)placed.size();
   }
-  if (!b->fn[F]) {
-    PyErr_SetString(PyExc_RuntimeError, "library not bound");
-    return nullptr;
-  }
+  if (!bound(b)) return nullptr;
   if (!parse(fn_kind[F], args, n, &a)) return nullptr;
   int err;
   Py_BEGIN_ALLOW_THREADS
@@ -280,6 +284,7 @@ PyObject *method(PyObject *self, PyObject *const *args, Py_ssize_t n, PyObject *
 PyObject *set_batch(PyObject *self, PyObject *arg)
 {
   int64_t v;
+  if (!bound((Base *)self)) return nullptr;
   if (!to_int(arg, &v)) return nullptr;
   ((void (*)(unsigned))((Base *)self)->fn[F_SET_BATCH])((unsigned)v);
   Py_RETURN_NONE;
@@ -291,12 +296,14 @@ PyObject *bind(PyObject *self, PyObject *args)
   Base *b = (Base *)self;
   PyObject *d;
   if (!PyArg_ParseTuple(args, "iO!", &b->bits, &PyDict_Type, &d)) return nullptr;
+  void *fn[NFN];
   for (int f = 0; f < NFN; f++) {
     PyObject *v = PyDict_GetItemString(d, fn_names[f]);
     if (!v) return PyErr_Format(PyExc_KeyError, "%s", fn_names[f]);
-    b->fn[f] = PyLong_AsVoidPtr(v);
+    fn[f] = PyLong_AsVoidPtr(v);
     if (PyErr_Occurred()) return nullptr;
   }
+  memcpy(b->fn, fn, sizeof fn);
   Py_RETURN_NONE;
 }
 
@@ -434,6 +441,7 @@ int plan_init(PyObject *self, PyObject *args, PyObject *)
     return -1;
   }
   if (!PyArg_ParseTuple(args, "O!IO!OO!", &BaseType, &nn, &pl->batch, &PyList_Type, &list, &input, &PyList_Type, &from)) return -1;
+  if (!bound((Base *)nn)) return -1;
   Py_INCREF(nn);
   pl->nn = nn;
   Py_INCREF(list);
@@ -521,6 +529,10 @@ PyObject *plan_run(PyObject *self, PyObject *x)
 {
   Plan *pl = (Plan *)self;
   Base *b = (Base *)pl->nn;
+  if (!b || !pl->calls) {
+    PyErr_SetString(PyExc_RuntimeError, "the plan has not been made");
+    return nullptr;
+  }
   for (const Whole &w : *pl->wholes)
     if (PyDict_Size(w.dict) != w.size) Py_RETURN_FALSE;
   for (const Guard &g : *pl->guards) {

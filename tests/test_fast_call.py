@@ -80,6 +80,14 @@ def test_plan_asks_for_addresses_at_each_run(nn):
             refused()
 
 
+def test_a_library_object_without_init_raises():
+    nn = api.PulpNN.__new__(api.PulpNN)
+    for call in (lambda: nn.set_batch(1), lambda: nn.pulp_nn_add(None, None, None, 1, 1, 1, 1, 1, 1), lambda: api._fast.Plan(nn, 1, [], None, []),
+                 lambda: api._fast.Plan.__new__(api._fast.Plan).run(None)):
+        with pytest.raises(RuntimeError):
+            call()
+
+
 POINTERS = dict({n: 7 for n in api.CONV_NAMES}, **{n: 8 for n in api.DW_NAMES}, pulp_nn_linear=6, pulp_nn_linear_out_32=4, pulp_nn_maxpool=2,
                 pulp_nn_avgpool=2, pulp_nn_add=3, pulp_nn_depthwise_3x3_s1=2, pulp_nn_hip_hwc_to_chw=2, pulp_nn_hip_depthwise_hwc=6,
                 pulp_nn_hip_dw_pw_hwc=2)
