@@ -10,7 +10,6 @@
 // not link against either library.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
-#include <structmember.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <stdint.h>
@@ -30,8 +29,8 @@ typedef signed char i8;
 
 enum Kind { CONV, DW, LINEAR, LINEAR32, MAXPOOL, AVGPOOL, ADD, DW3, HWC2CHW, DWHWC, DWPW, CHAIN, NKIND };
 
-// argument types in order: p = tensor / address / None, i = integer; names for keyword calls (null: positional only);
-// the last `optional` arguments default to zero / null
+// argument types in order: p = tensor / address / None, i = what int() takes, n = an integer; names for keyword calls
+// (null: positional only); the last `optional` arguments default to zero / null
 struct KindInfo {
   const char *spec;
   const char *names;
@@ -46,9 +45,9 @@ const KindInfo kinds[NKIND] = {
     {"ppiiiiiiiiiiiiiiiii", nullptr, 0},
     {"pppiiiiii", "in1 in2 out out_mult1 out_mult2 out_shift dim_h dim_w ch", 0},
     {"ppiiiiipiippiip", "In_Img Out_Img R C_ CH p_l p_r Kernel out_shift out_mult kappa lam flag_relu flag_batch_norm memory_chan", 1},
-    {"ppiiiii", "x out dim_x dim_y ch pad_top pad_bottom", 2},
-    {"ppppppiiiiiiiiii", "x bias out wt k lam out_mult out_shift dim_in_x dim_in_y ch dim_out_x dim_out_y stride flag_relu flag_batch_norm", 0},
-    {"ppiiiiiiippppiiiippppiiii",
+    {"ppnnnnn", "x out dim_x dim_y ch pad_top pad_bottom", 2},
+    {"ppppppnnnnnnnnnn", "x bias out wt k lam out_mult out_shift dim_in_x dim_in_y ch dim_out_x dim_out_y stride flag_relu flag_batch_norm", 0},
+    {"ppnnnnnnnppppnnnnppppnnnn",
      "x out dim_in_x dim_in_y ch dim_out_x dim_out_y ch_out stride dw_wt dw_bias dw_k dw_lam dw_mult dw_shift dw_relu dw_bn pw_w pw_bias pw_k "
      "pw_lam pw_mult pw_shift pw_relu pw_bn",
      0},
@@ -80,6 +79,29 @@ struct Args {
   int64_t s[20];
 };
 
+// an object with a tensor's methods -> device address
+bool other_ptr(PyObject *o, void **out)
+{
+  static const char *const asked[2] = {"is_cuda", "is_contiguous"};
+  static const char *const refusal[2] = {"PULP-NN HIP kernels take device tensors", "tensor must be contiguous"};
+  for (int i = 0; i < 2; i++) {
+    PyObject *v = i ? PyObject_CallMethod(o, asked[i], nullptr) : PyObject_GetAttrString(o, asked[i]);
+    if (!v) return false;
+    const int yes = PyObject_IsTrue(v);
+    Py_DECREF(v);
+    if (yes < 0) return false;
+    if (!yes) {
+      PyErr_SetString(PyExc_ValueError, refusal[i]);
+      return false;
+    }
+  }
+  PyObject *v = PyObject_CallMethod(o, "data_ptr", nullptr);
+  if (!v) return false;
+  *out = PyLong_AsVoidPtr(v);
+  Py_DECREF(v);
+  return *out || !PyErr_Occurred();
+}
+
 // tensor / address / None -> device address
 bool to_ptr(PyObject *o, void **out)
 try {
@@ -104,8 +126,7 @@ try {
     *out = PyLong_AsVoidPtr(o);
     return *out || !PyErr_Occurred();
   }
-  PyErr_Format(PyExc_TypeError, "expected a tensor, an address or None, not %.100s", Py_TYPE(o)->tp_name);
-  return false;
+  return other_ptr(o, out);
 } catch (const std::exception &e) {  // a tensor without storage (a fake or a functional one) has no address
   if (!PyErr_Occurred()) PyErr_SetString(PyExc_RuntimeError, e.what());
   return false;
@@ -124,12 +145,24 @@ bool to_int(PyObject *o, int64_t *out)
   return true;
 }
 
+bool to_integer(PyObject *o, int64_t *out)
+{
+  if (PyLong_CheckExact(o)) return to_int(o, out);
+  PyObject *n = PyNumber_Index(o);
+  if (!n) return false;
+  *out = (int64_t)PyLong_AsUnsignedLongLongMask(n);
+  Py_DECREF(n);
+  return true;
+}
+
 bool parse(Kind kind, PyObject *const *args, Py_ssize_t n, Args *a)
 {
   const char *spec = kinds[kind].spec;
   const Py_ssize_t want = (Py_ssize_t)strlen(spec);
   if (n > want || n < want - kinds[kind].optional) {
-    PyErr_Format(PyExc_AssertionError, "expected %zd arguments, got %zd", want, n);
+    // (the functions without names have as many scalars as the reference's, which is asserted)
+    const Py_ssize_t pointers = (Py_ssize_t)strspn(spec, "p");
+    PyErr_Format(kinds[kind].names || n < pointers ? PyExc_TypeError : PyExc_AssertionError, "expected %zd arguments, got %zd", want, n);
     return false;
   }
   int np = 0, ns = 0;
@@ -140,7 +173,7 @@ bool parse(Kind kind, PyObject *const *args, Py_ssize_t n, Args *a)
       np++;
     } else {
       a->s[ns] = 0;
-      if (i < n && !to_int(args[i], &a->s[ns])) return false;
+      if (i < n && !(spec[i] == 'i' ? to_int(args[i], &a->s[ns]) : to_integer(args[i], &a->s[ns]))) return false;
       ns++;
     }
   }
@@ -217,7 +250,7 @@ bool bound(const Base *b)
   return b->fn[F_LAST_ERROR] != nullptr;
 }
 
-// keyword arguments -> their places
+// keyword arguments -> their places (null: left out)
 bool place_keywords(Kind kind, PyObject *const *args, Py_ssize_t n, PyObject *kw, std::vector<PyObject *> *out)
 {
   const char *names = kinds[kind].names;
@@ -250,7 +283,6 @@ bool place_keywords(Kind kind, PyObject *const *args, Py_ssize_t n, PyObject *kw
         PyErr_Format(PyExc_TypeError, "missing argument '%s'", list[i].c_str());
         return false;
       }
-      (*out)[i] = Py_None;
     }
   return true;
 }
@@ -266,7 +298,7 @@ PyObject *method(PyObject *self, PyObject *const *args, Py_ssize_t n, PyObject *
     // (an omitted optional argument in the middle: zero)
     static PyObject *zero = PyLong_FromLong(0);
     for (size_t i = 0; i < placed.size(); i++)
-      if (placed[i] == Py_None && kinds[fn_kind[F]].spec[i] == 'i') placed[i] = zero;
+      if (!placed[i]) placed[i] = kinds[fn_kind[F]].spec[i] == 'p' ? Py_None : zero;
     args = placed.data();
     n = (Py_ssize_t)placed.size();
   }
@@ -329,8 +361,16 @@ PyMethodDef base_methods[] = {
     {"set_batch", set_batch, METH_O, nullptr},
     {"_bind", bind, METH_VARARGS, nullptr},
     {nullptr, nullptr, 0, nullptr}};
-PyMemberDef base_members[] = {{"check", T_BOOL, offsetof(Base, check), 0, "raise PulpNNError when the library rejects a call"},
-                              {nullptr, 0, 0, 0, nullptr}};
+PyObject *get_check(PyObject *self, void *) { return PyBool_FromLong(((Base *)self)->check); }
+int set_check(PyObject *self, PyObject *value, void *)
+{
+  const int yes = value ? PyObject_IsTrue(value) : 0;
+  if (yes < 0) return -1;
+  ((Base *)self)->check = (char)yes;
+  return 0;
+}
+PyGetSetDef base_getset[] = {{"check", get_check, set_check, "raise PulpNNError when the library rejects a call", nullptr},
+                             {nullptr, nullptr, nullptr, nullptr, nullptr}};
 PyTypeObject BaseType = {PyVarObject_HEAD_INIT(nullptr, 0)};
 
 // ---- Plan ---------------------------------------------------------------------------------------------------------------
@@ -634,7 +674,7 @@ PyMODINIT_FUNC PyInit__pulpnn_fast(void)
   BaseType.tp_flags = Py_TPFLAGS_DEFAULT | Py_TPFLAGS_BASETYPE;
   BaseType.tp_new = PyType_GenericNew;
   BaseType.tp_methods = base_methods;
-  BaseType.tp_members = base_members;
+  BaseType.tp_getset = base_getset;
   PlanType.tp_name = "_pulpnn_fast.Plan";
   PlanType.tp_basicsize = sizeof(Plan);
   PlanType.tp_flags = Py_TPFLAGS_DEFAULT;

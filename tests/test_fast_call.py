@@ -88,6 +88,50 @@ def test_a_library_object_without_init_raises():
             call()
 
 
+class TensorLike:
+    """Has what the binding asks a tensor for."""
+    is_cuda = True
+
+    def __init__(self, address, contiguous=True):
+        self.address, self.contiguous = address, contiguous
+
+    def is_contiguous(self):
+        return self.contiguous
+
+    def data_ptr(self):
+        return self.address
+
+
+def test_arguments_that_were_taken_or_refused_still_are(nn):
+    """What ctypes and the Python methods in front of it did: objects with a tensor's methods, error types, integers that
+    have to be integers, an omitted scalar that is given as None."""
+    lib = FakeLibrary()
+    fake = lib.bound()
+    fake.pulp_nn_add(TensorLike(0x1000), 0x2000, TensorLike(0x3000), 1, 1, 1, 1, 1, 1)
+    assert lib.seen == [("pulp_nn_add", 0x1000, 0x2000, 0x3000)]
+    host = TensorLike(0x1000)
+    host.is_cuda = False
+    for refused, error in ((TensorLike(0x1000, False), ValueError), (host, ValueError), ("text", AttributeError)):
+        with pytest.raises(error):
+            fake.pulp_nn_add(refused, None, None, 1, 1, 1, 1, 1, 1)
+    fake.pulp_nn_add(0, 0, 0, 1.0, "1", True, np.int64(1), 1, 1)      # the reference's scalars: whatever int() takes
+    for dim in (1.5, "1", None):                                     # the added entry points': integers
+        with pytest.raises(TypeError):
+            fake.hwc_to_chw(0, 0, dim, 1, 1)
+        with pytest.raises(TypeError):
+            fake.hwc_to_chw(0, 0, 1, 1, 1, pad_top=dim)
+    fake.hwc_to_chw(0, 0, np.int32(1), 1, 1, pad_bottom=2)
+    with pytest.raises(TypeError):                                   # counts: missing names, missing scalars
+        fake.pulp_nn_linear(0, 0, 0, 0, 0, 0, 1, 1, 1, 1, 1)
+    with pytest.raises(TypeError):
+        fake.pulp_nn_maxpool(0)
+    with pytest.raises(AssertionError):
+        fake.pulp_nn_maxpool(0, 0, 1, 2, 3)
+    for value in (1, "yes", 0, None):
+        nn.check = value
+        assert nn.check is bool(value)
+
+
 POINTERS = dict({n: 7 for n in api.CONV_NAMES}, **{n: 8 for n in api.DW_NAMES}, pulp_nn_linear=6, pulp_nn_linear_out_32=4, pulp_nn_maxpool=2,
                 pulp_nn_avgpool=2, pulp_nn_add=3, pulp_nn_depthwise_3x3_s1=2, pulp_nn_hip_hwc_to_chw=2, pulp_nn_hip_depthwise_hwc=6,
                 pulp_nn_hip_dw_pw_hwc=2)
