@@ -5,7 +5,7 @@ import importlib.machinery
 import importlib.util
 import os
 
-from .build import fast_path, lib_path
+from .build import fast_path, lib_path, tensor_path
 
 _U16, _I8, _INT, _PTR = C.c_uint16, C.c_int8, C.c_int, C.c_void_p
 
@@ -15,7 +15,6 @@ def _load_fast():
     path = fast_path()
     if not os.path.exists(path):
         return None
-    import torch  # noqa: F401  (the extension resolves its tensor type against the loaded torch)
     loader = importlib.machinery.ExtensionFileLoader("_pulpnn_fast", path)
     mod = importlib.util.module_from_spec(importlib.util.spec_from_loader("_pulpnn_fast", loader))
     loader.exec_module(mod)
@@ -23,6 +22,19 @@ def _load_fast():
 
 
 _fast = _load_fast()
+
+
+def _load_torch():
+    """Before a library is loaded: torch, where there is one, brings the HIP runtime that both then share, and its tensors
+    are told apart by _pulpnn_tensor.so.  Without torch the functions take addresses."""
+    try:
+        import torch  # noqa: F401
+    except ImportError:
+        return
+    if not os.path.exists(tensor_path()):
+        raise ImportError("%s is missing: build it with `python -m pulp_nn_amd.build`" % tensor_path())
+    lib = C.PyDLL(tensor_path())
+    _fast.set_tensor_function(C.cast(lib.pulpnn_tensor_address, _PTR).value)
 
 
 class HipBlock(C.Structure):
@@ -91,6 +103,7 @@ class PulpNN(_fast.Base if _fast else object):
             if not os.path.exists(need) or _fast is None:
                 raise ImportError("%s is missing: build it with `python -m pulp_nn_amd.build` "
                                   "(there is no CPU fallback)" % need)
+        _load_torch()
         self.bn_bits = bn_bits
         self.check = bool(check)
         self.path = path

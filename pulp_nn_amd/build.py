@@ -81,16 +81,21 @@ def fast_path():
     return os.path.join(LIBDIR, "_pulpnn_fast.so")
 
 
+def tensor_path():
+    return os.path.join(LIBDIR, "_pulpnn_tensor.so")
+
+
 def build_fast(verbose=False):
-    """The Python front end's call path (csrc/pybind_fast.cpp): a CPython extension module, host code only."""
+    """The Python front end's call path, host code only: csrc/pybind_fast.cpp, a CPython extension module, and
+    csrc/pybind_tensor.cpp, which knows torch's tensors."""
     import sysconfig
     from torch.utils import cpp_extension
     os.makedirs(LIBDIR, exist_ok=True)
+    gxx = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-I", sysconfig.get_paths()["include"]]
+    _run(gxx + [os.path.join(CSRC, "pybind_fast.cpp"), "-o", fast_path()], "g++", verbose)
     libs = cpp_extension.library_paths()
-    cmd = (["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-I", sysconfig.get_paths()["include"]] +
-           ["-I" + d for d in cpp_extension.include_paths()] + [os.path.join(CSRC, "pybind_fast.cpp"), "-o", fast_path()] +
-           ["-L" + d for d in libs] + ["-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10"] + ["-Wl,-rpath," + d for d in libs])
-    _run(cmd, "g++", verbose)
+    _run(gxx + ["-I" + d for d in cpp_extension.include_paths()] + [os.path.join(CSRC, "pybind_tensor.cpp"), "-o", tensor_path()] +
+         ["-L" + d for d in libs] + ["-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10"] + ["-Wl,-rpath," + d for d in libs], "g++", verbose)
     return fast_path()
 
 

@@ -7,10 +7,10 @@
 // is one Python call, and only the chain's input is converted per run.
 //
 // The entry points are looked up by ctypes (api.py loads the library) and handed over as addresses, so this module does
-// not link against either library.
+// not link against either library.  Nor against torch: what a tensor's address is says a function of _pulpnn_tensor.so
+// (pybind_tensor.cpp), handed over where torch can be imported.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
-#include <torch/csrc/autograd/python_variable.h>
 
 #include <stdint.h>
 #include <string.h>
@@ -102,34 +102,22 @@ bool other_ptr(PyObject *o, void **out)
   return *out || !PyErr_Occurred();
 }
 
+// 1 and the tensor's address, 0 if the object is no tensor, -1 with an exception set; null without torch
+int (*tensor_address)(PyObject *, void **) = nullptr;
+
 // tensor / address / None -> device address
 bool to_ptr(PyObject *o, void **out)
-try {
+{
   if (o == Py_None) {
     *out = nullptr;
     return true;
   }
-  if (THPVariable_Check(o)) {
-    const at::Tensor &t = THPVariable_Unpack(o);
-    if (!t.is_cuda()) {
-      PyErr_SetString(PyExc_ValueError, "PULP-NN HIP kernels take device tensors");
-      return false;
-    }
-    if (!t.is_contiguous()) {
-      PyErr_SetString(PyExc_ValueError, "tensor must be contiguous");
-      return false;
-    }
-    *out = t.data_ptr();
-    return true;
+  if (!PyLong_Check(o)) {
+    const int is = tensor_address ? tensor_address(o, out) : 0;
+    return is ? is > 0 : other_ptr(o, out);
   }
-  if (PyLong_Check(o)) {
-    *out = PyLong_AsVoidPtr(o);
-    return *out || !PyErr_Occurred();
-  }
-  return other_ptr(o, out);
-} catch (const std::exception &e) {  // a tensor without storage (a fake or a functional one) has no address
-  if (!PyErr_Occurred()) PyErr_SetString(PyExc_RuntimeError, e.what());
-  return false;
+  *out = PyLong_AsVoidPtr(o);
+  return *out || !PyErr_Occurred();
 }
 
 bool to_int(PyObject *o, int64_t *out)
@@ -464,7 +452,8 @@ bool add_guard(Plan *pl, PyObject *dict, PyObject *key, PyObject *value)
 bool is_scalar(PyObject *v)
 {
   if (v == Py_None || PyLong_Check(v) || PyFloat_Check(v) || PyUnicode_Check(v) || PyTuple_Check(v) || PyList_Check(v)) return true;
-  return PyNumber_Check(v) && Py_TYPE(v)->tp_hash != PyObject_HashNotImplemented && !THPVariable_Check(v);  // (numpy's scalars)
+  if (!PyNumber_Check(v) || Py_TYPE(v)->tp_hash == PyObject_HashNotImplemented) return false;
+  return !PyObject_HasAttrString(v, "data_ptr");  // (numpy's scalars, and no tensor)
 }
 
 // Plan(nn, batch, [(entry point, arguments), ...], input, [(dict, which), ...]): `input` is the object that stands
@@ -659,7 +648,17 @@ PyObject *plain(PyObject *, PyObject *const *args, Py_ssize_t n)
   Py_RETURN_TRUE;
 }
 
-PyMethodDef module_methods[] = {{"plain", (PyCFunction)(void (*)(void))plain, METH_FASTCALL, nullptr}, {nullptr, nullptr, 0, nullptr}};
+// set_tensor_function(address)
+PyObject *set_tensor_function(PyObject *, PyObject *address)
+{
+  void *p = PyLong_AsVoidPtr(address);
+  if (PyErr_Occurred()) return nullptr;
+  tensor_address = (int (*)(PyObject *, void **))p;
+  Py_RETURN_NONE;
+}
+
+PyMethodDef module_methods[] = {{"set_tensor_function", set_tensor_function, METH_O, nullptr},
+                                {"plain", (PyCFunction)(void (*)(void))plain, METH_FASTCALL, nullptr}, {nullptr, nullptr, 0, nullptr}};
 PyMethodDef plan_methods[] = {{"run", plan_run, METH_O, nullptr}, {nullptr, nullptr, 0, nullptr}};
 PyTypeObject PlanType = {PyVarObject_HEAD_INIT(nullptr, 0)};
 

@@ -1,6 +1,8 @@
 """The extension module behind the Python front end (csrc/pybind_fast.cpp), as far as it goes without a GPU: argument
 counts, keywords, rejected calls, and plans that notice what they were made from has changed."""
 import ctypes
+import os
+import subprocess
 import sys
 import types
 
@@ -391,3 +393,15 @@ def test_a_plan_does_not_keep_the_input():
     r.run(x)
     lib.seen.clear()
     assert sys.getrefcount(x) == before
+
+
+def test_addresses_need_no_torch():
+    """A caller that has raw addresses: torch is not needed where it cannot be imported."""
+    code = ("import sys; sys.modules['torch'] = None\n"
+            "from pulp_nn_amd import PulpNN, PulpNNError\n"
+            "nn = PulpNN(32)\n"
+            "try:\n    nn.pulp_nn_add(0, 0, 0, 1, 1, 1, 1, 1, 1)\n"
+            "except PulpNNError as e:\n    print('code', e.code)\n")
+    res = subprocess.run([sys.executable, "-c", code], stdout=subprocess.PIPE, stderr=subprocess.PIPE, text=True, timeout=100,
+                         cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
+    assert res.stdout == "code 1\n", res.stderr
