@@ -10,12 +10,15 @@ pointer arguments take torch tensors on the GPU (or raw device addresses).
 There is no CPU fallback: loading fails if the HIP libraries have not been built
 (python -m pulp_nn_amd.build).
 """
+import importlib
+
 _API = ("PulpNN", "PulpNNError", "lib_path")
 
 
 def __getattr__(name):
     # on first use, so that `from pulp_nn_amd import build` works before anything has been built
+    if name in ("api", "build"):
+        return importlib.import_module("." + name, __name__)
     if name in _API:
-        from . import api
-        return getattr(api, name)
+        return getattr(importlib.import_module(".api", __name__), name)
     raise AttributeError("module %r has no attribute %r" % (__name__, name))

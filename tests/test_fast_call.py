@@ -395,6 +395,13 @@ def test_a_plan_does_not_keep_the_input():
     assert sys.getrefcount(x) == before
 
 
+def in_a_new_process(code):
+    res = subprocess.run([sys.executable, "-c", code], stdout=subprocess.PIPE, stderr=subprocess.PIPE, text=True, timeout=100,
+                         cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
+    assert res.returncode == 0, res.stderr
+    return res.stdout
+
+
 def test_addresses_need_no_torch():
     """A caller that has raw addresses: torch is not needed where it cannot be imported."""
     code = ("import sys; sys.modules['torch'] = None\n"
@@ -402,6 +409,8 @@ def test_addresses_need_no_torch():
             "nn = PulpNN(32)\n"
             "try:\n    nn.pulp_nn_add(0, 0, 0, 1, 1, 1, 1, 1, 1)\n"
             "except PulpNNError as e:\n    print('code', e.code)\n")
-    res = subprocess.run([sys.executable, "-c", code], stdout=subprocess.PIPE, stderr=subprocess.PIPE, text=True, timeout=100,
-                         cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
-    assert res.stdout == "code 1\n", res.stderr
+    assert in_a_new_process(code) == "code 1\n"
+
+
+def test_submodules_are_attributes_of_the_package():
+    assert in_a_new_process("import pulp_nn_amd\nprint(pulp_nn_amd.build.__name__, pulp_nn_amd.api.__name__)") == "pulp_nn_amd.build pulp_nn_amd.api\n"
