@@ -11,7 +11,7 @@ _U16, _I8, _INT, _PTR = C.c_uint16, C.c_int8, C.c_int, C.c_void_p
 
 
 def _load_fast():
-    """The extension module, or None if it has not been built (PulpNN() then says so)."""
+    """The extension module, or None if it has not been built."""
     path = fast_path()
     if not os.path.exists(path):
         return None
@@ -21,6 +21,7 @@ def _load_fast():
     return mod
 
 
+_MISSING = "%s is missing: build it with `python -m pulp_nn_amd.build` (there is no CPU fallback)"
 _fast = _load_fast()
 
 
@@ -32,7 +33,7 @@ def _load_torch():
     except ImportError:
         return
     if not os.path.exists(tensor_path()):
-        raise ImportError("%s is missing: build it with `python -m pulp_nn_amd.build`" % tensor_path())
+        raise ImportError(_MISSING % tensor_path())
     lib = C.PyDLL(tensor_path())
     _fast.set_tensor_function(C.cast(lib.pulpnn_tensor_address, _PTR).value)
 
@@ -76,7 +77,7 @@ FAST_NAMES = CONV_NAMES + DW_NAMES + (
     "pulp_nn_hip_set_batch", "pulp_nn_hip_last_error")
 
 
-class PulpNN(_fast.Base if _fast else object):
+class _Methods:
     """One loaded library (32- or 64-bit batch-norm parameters).
 
     With check=True (default) every layer call raises PulpNNError if the library
@@ -99,10 +100,8 @@ class PulpNN(_fast.Base if _fast else object):
         if bn_bits not in (32, 64):
             raise ValueError("bn_bits must be 32 or 64")
         path = lib_path(bn_bits)
-        for need in (path, fast_path()):
-            if not os.path.exists(need) or _fast is None:
-                raise ImportError("%s is missing: build it with `python -m pulp_nn_amd.build` "
-                                  "(there is no CPU fallback)" % need)
+        if not os.path.exists(path):
+            raise ImportError(_MISSING % path)
         _load_torch()
         self.bn_bits = bn_bits
         self.check = bool(check)
@@ -218,16 +217,32 @@ class PulpNN(_fast.Base if _fast else object):
                           _ptr(pOut2), int(flag_relu), int(flag_batch_norm))
 
 
-def _methods():
-    """{name: attribute} of what a run over a table calls, as PulpNN has it."""
+def _define():
+    """PulpNN: the methods above on the extension module's base class."""
+    global PulpNN, _METHODS
+    PulpNN = type("PulpNN", (_Methods, _fast.Base), {"__doc__": _Methods.__doc__, "__module__": __name__})
+    # {name: attribute} of what a run over a table calls
     names = ("set_batch", "hwc_to_chw", "depthwise_hwc", "dw_pw_hwc", "dw_pw_chain_hwc", "_call", "__getattribute__",
              *(n for n in FAST_NAMES if "_hip_" not in n))
-    return {n: next(vars(c)[n] for c in PulpNN.__mro__ if n in vars(c)) for n in names}
-
-
-_METHODS = _methods() if _fast else None
+    _METHODS = {n: next(vars(c)[n] for c in PulpNN.__mro__ if n in vars(c)) for n in names}
 
 
 def plain(nn):
     """Whether nn's layer methods are PulpNN's own, so that a plan, which calls the library directly, does what they would do."""
     return _fast is not None and _fast.plain(nn, _METHODS)
+
+
+if _fast is not None:
+    _define()
+else:
+    class PulpNN:  # noqa: F811
+        """Stands in until the extension module has been built, which may happen in this process."""
+
+        def __new__(cls, *args, **kwargs):
+            global _fast
+            _fast = _fast or _load_fast()
+            if _fast is None:
+                raise ImportError(_MISSING % fast_path())
+            if PulpNN is cls:
+                _define()
+            return PulpNN(*args, **kwargs)

@@ -414,3 +414,21 @@ def test_addresses_need_no_torch():
 
 def test_submodules_are_attributes_of_the_package():
     assert in_a_new_process("import pulp_nn_amd\nprint(pulp_nn_amd.build.__name__, pulp_nn_amd.api.__name__)") == "pulp_nn_amd.build pulp_nn_amd.api\n"
+
+
+def test_binding_imported_before_the_build():
+    """The extension is built after the binding was imported: PulpNN works from then on; before, the error names the file."""
+    code = ("from pulp_nn_amd import api, build\n"
+            "import os\n"
+            "real = build.fast_path()\n"
+            "api._fast, api.fast_path = None, lambda: '/nonexistent/_pulpnn_fast.so'\n"
+            "source = open(api.__file__).read()\n"
+            "build.fast_path = api.fast_path\n"
+            "exec(compile(source, api.__file__, 'exec'), api.__dict__)\n"      # the binding as imported before the build
+            "from pulp_nn_amd.api import PulpNN as early\n"
+            "try:\n    early(32)\n"
+            "except ImportError as e:\n    print('_pulpnn_fast.so is missing' in str(e))\n"
+            "api.fast_path = build.fast_path = lambda: real\n"
+            "a, b = early(32), early(64)\n"
+            "print(a.bn_bits, b.bn_bits, type(a) is api.PulpNN, api.plain(a), early(32, check=False).check)\n")
+    assert in_a_new_process(code) == "True\n32 64 True True False\n"
