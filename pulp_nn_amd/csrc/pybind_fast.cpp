@@ -2,8 +2,8 @@
 //
 // A layer of a few MB takes the GPU 4 to 7 us.  Through ctypes a call costs 3.5 us of argument conversion (25 Python
 // objects, six of them tensors asked for their address) before hipLaunchKernel is reached; here it is a few tenths of a
-// microsecond.  `Base` is the base class of api.PulpNN: its methods take the reference's argument lists.  `Plan` is a
-// list of such calls with their arguments converted once, for a chain of layers on buffers that its owner keeps: a run
+// microsecond.  `Base` is the base class of api.PulpNN: its methods take the reference's argument lists.  `Recorder` makes
+// such calls and keeps them.  `Plan` is a list of such calls with their arguments converted once, for a chain of layers on buffers that its owner keeps: a run
 // is one Python call, and only the chain's input is converted per run.
 //
 // The entry points are looked up by ctypes (api.py loads the library) and handed over as addresses, so this module does
@@ -11,6 +11,7 @@
 // (pybind_tensor.cpp), handed over where torch can be imported.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
+#include <structmember.h>
 
 #include <stdint.h>
 #include <string.h>
@@ -361,6 +362,108 @@ PyGetSetDef base_getset[] = {{"check", get_check, set_check, "raise PulpNNError 
                              {nullptr, nullptr, nullptr, nullptr, nullptr}};
 PyTypeObject BaseType = {PyVarObject_HEAD_INIT(nullptr, 0)};
 
+// ---- Recorder -----------------------------------------------------------------------------------------------------------
+
+// Recorder(nn, x): stands in for nn during a walk over a table.  Makes the calls and keeps those that the library took, as Plan
+// takes them: `calls`, with `input` in the place of x (an address stands for itself), and in `calls_at` what `at` was.
+struct Recorder {
+  PyObject_HEAD
+  PyObject *nn, *x, *input, *calls, *calls_at, *at;
+};
+
+PyObject *note(Recorder *r, const char *name, const char *spec, PyObject *const *args, Py_ssize_t n)
+{
+  const Py_ssize_t want = (Py_ssize_t)strlen(spec);  // (what has been left out is zero or null)
+  PyObject *a = PyTuple_New(want > n ? want : n);
+  if (!a) return nullptr;
+  for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(a); i++) {
+    PyObject *o = i >= n ? (spec[i] == 'p' ? Py_None : nullptr) : (i < want && spec[i] == 'p' && args[i] == r->x) ? r->input : args[i];
+    if (o) Py_INCREF(o);
+    else if (!(o = PyLong_FromLong(0))) {
+      Py_DECREF(a);
+      return nullptr;
+    }
+    PyTuple_SET_ITEM(a, i, o);
+  }
+  PyObject *call = Py_BuildValue("(sN)", name, a);
+  const bool ok = call && !PyList_Append(r->calls, call) && !PyList_Append(r->calls_at, r->at);
+  Py_XDECREF(call);
+  if (!ok) return nullptr;
+  Py_RETURN_NONE;
+}
+
+template <int F>
+PyObject *recorded(PyObject *self, PyObject *const *args, Py_ssize_t n)
+{
+  Recorder *r = (Recorder *)self;
+  PyObject *done = method<F>(r->nn, args, n, nullptr);
+  if (!done) return nullptr;
+  Py_DECREF(done);
+  return note(r, fn_names[F], kinds[fn_kind[F]].spec, args, n);
+}
+
+// (the chain is a Python method of nn: it fills the block structs)
+PyObject *recorded_chain(PyObject *self, PyObject *const *args, Py_ssize_t n)
+{
+  Recorder *r = (Recorder *)self;
+  PyObject *m = PyObject_GetAttrString(r->nn, "dw_pw_chain_hwc");
+  PyObject *done = m ? PyObject_Vectorcall(m, args, (size_t)n, nullptr) : nullptr;
+  Py_XDECREF(m);
+  if (!done) return nullptr;
+  Py_DECREF(done);
+  return note(r, fn_names[F_CHAIN], "ppiii", args, n);
+}
+
+PyObject *recorder_set_batch(PyObject *self, PyObject *n) { return set_batch(((Recorder *)self)->nn, n); }
+
+PyObject *recorder_new(PyTypeObject *type, PyObject *args, PyObject *)
+{
+  PyObject *nn, *x;
+  if (!PyArg_ParseTuple(args, "O!O", &BaseType, &nn, &x)) return nullptr;
+  Recorder *r = (Recorder *)type->tp_alloc(type, 0);
+  if (!r) return nullptr;
+  Py_INCREF(r->nn = nn);
+  Py_INCREF(r->x = x);
+  r->calls = PyList_New(0);
+  r->calls_at = PyList_New(0);
+  Py_INCREF(r->at = Py_None);
+  if (PyLong_Check(x)) Py_INCREF(r->input = x);
+  else r->input = PyObject_CallNoArgs((PyObject *)&PyBaseObject_Type);
+  if (r->calls && r->calls_at && r->input) return (PyObject *)r;
+  Py_DECREF(r);
+  return nullptr;
+}
+
+void recorder_dealloc(PyObject *self)
+{
+  Recorder *r = (Recorder *)self;
+  for (PyObject *o : {r->nn, r->x, r->input, r->calls, r->calls_at, r->at}) Py_XDECREF(o);
+  Py_TYPE(self)->tp_free(self);
+}
+
+#define R(F, NAME) {NAME, (PyCFunction)(void (*)(void))recorded<F>, METH_FASTCALL, nullptr}
+PyMethodDef recorder_methods[] = {
+    R(F_CONV_HO, "pulp_nn_conv_Ho_parallel"),
+    R(F_PW_HOWO, "pulp_nn_pointwise_HoWo_parallel"),
+    R(F_DW_GENERIC, "pulp_nn_depthwise_generic"),
+    R(F_LINEAR, "pulp_nn_linear"),
+    R(F_LINEAR32, "pulp_nn_linear_out_32"),
+    R(F_MAXPOOL, "pulp_nn_maxpool"),
+    R(F_AVGPOOL, "pulp_nn_avgpool"),
+    R(F_ADD, "pulp_nn_add"),
+    R(F_HWC2CHW, "hwc_to_chw"),
+    R(F_DWHWC, "depthwise_hwc"),
+    R(F_DWPW, "dw_pw_hwc"),
+    {"dw_pw_chain_hwc", (PyCFunction)(void (*)(void))recorded_chain, METH_FASTCALL, nullptr},
+    {"set_batch", recorder_set_batch, METH_O, nullptr},
+    {nullptr, nullptr, 0, nullptr}};
+PyMemberDef recorder_members[] = {{"calls", T_OBJECT, offsetof(Recorder, calls), READONLY, nullptr},
+                                  {"calls_at", T_OBJECT, offsetof(Recorder, calls_at), READONLY, nullptr},
+                                  {"input", T_OBJECT, offsetof(Recorder, input), READONLY, nullptr},
+                                  {"at", T_OBJECT, offsetof(Recorder, at), 0, nullptr},
+                                  {nullptr, 0, 0, 0, nullptr}};
+PyTypeObject RecorderType = {PyVarObject_HEAD_INIT(nullptr, 0)};
+
 // ---- Plan ---------------------------------------------------------------------------------------------------------------
 
 // Addresses are asked for at each run, as a call by itself would: a tensor may have been given other storage since.
@@ -681,11 +784,20 @@ PyMODINIT_FUNC PyInit__pulpnn_fast(void)
   PlanType.tp_init = plan_init;
   PlanType.tp_dealloc = plan_dealloc;
   PlanType.tp_methods = plan_methods;
-  if (PyType_Ready(&BaseType) < 0 || PyType_Ready(&PlanType) < 0) return nullptr;
+  RecorderType.tp_name = "_pulpnn_fast.Recorder";
+  RecorderType.tp_basicsize = sizeof(Recorder);
+  RecorderType.tp_flags = Py_TPFLAGS_DEFAULT;
+  RecorderType.tp_new = recorder_new;
+  RecorderType.tp_dealloc = recorder_dealloc;
+  RecorderType.tp_methods = recorder_methods;
+  RecorderType.tp_members = recorder_members;
+  if (PyType_Ready(&BaseType) < 0 || PyType_Ready(&PlanType) < 0 || PyType_Ready(&RecorderType) < 0) return nullptr;
   PyObject *m = PyModule_Create(&module);
   if (!m) return nullptr;
   Py_INCREF(&BaseType);
   PyModule_AddObject(m, "Base", (PyObject *)&BaseType);
+  Py_INCREF(&RecorderType);
+  PyModule_AddObject(m, "Recorder", (PyObject *)&RecorderType);
   Py_INCREF(&PlanType);
   PyModule_AddObject(m, "Plan", (PyObject *)&PlanType);
   return m;

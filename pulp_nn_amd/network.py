@@ -80,31 +80,6 @@ def infer_shapes(layers, input_shape):
     return shapes
 
 
-class _Recorder:
-    """Stands in for a PulpNN during a walk over the table: makes the calls and keeps those that the library took, with
-    `input` in the place of the chain's input, and the layer each belongs to."""
-    _NAMES = {"hwc_to_chw": "pulp_nn_hip_hwc_to_chw", "depthwise_hwc": "pulp_nn_hip_depthwise_hwc",
-              "dw_pw_hwc": "pulp_nn_hip_dw_pw_hwc", "dw_pw_chain_hwc": "pulp_nn_hip_dw_pw_chain_hwc"}
-
-    def __init__(self, nn, x):
-        self.nn, self.x, self.input = nn, x, object()
-        self.calls, self.calls_at, self.at = [], [], None
-
-    def set_batch(self, n):
-        self.nn.set_batch(n)
-
-    def __getattr__(self, name):
-        method = getattr(self.nn, name)
-
-        def call(*args):
-            method(*args)
-            if name == "hwc_to_chw":
-                args += (0,) * (7 - len(args))   # pad_top, pad_bottom
-            self.calls.append((self._NAMES.get(name, name), tuple(self.input if a is self.x else a for a in args)))
-            self.calls_at.append(self.at)
-        return call
-
-
 class Runner:
     """Uploads the parameters once, owns the activation buffers and queues the chain.
 
@@ -241,7 +216,7 @@ class Runner:
             self._plan = None
         if not self._plannable or not self.layers or any(x is t for d in (self.act, self.chw) for t in d.values()):
             return self._walk(x, self.nn)
-        rec = _Recorder(self.nn, x)
+        rec = api._fast.Recorder(self.nn, x)
         out = self._walk(x, rec)
         self._lay_out_plan(rec, out)
         return out
@@ -268,18 +243,20 @@ class Runner:
         tensors = {"input": x, **{L["name"]: self.act[L["name"]] for L in self.layers[:first]}}
         out = x
         self.launches = launches
+        recorded, readers = nn is not self.nn, self._reader_counts()
         i = first
         while i < len(self.layers):
-            if isinstance(nn, _Recorder):
+            if recorded:
                 nn.at = (i, self.launches)
             L = self.layers[i]
-            n = self._chain_length(i) if self.chain_blocks else 0
+            block = L["op"] == "depthwise"
+            n = self._chain_length(i, readers) if block and self.chain_blocks else 0
             if n >= 2 and self._queue_chain(i, n, tensors, nn):
                 last = self.layers[i + 2 * n - 1]["name"]
                 out = tensors[last] = self.act[last]
                 i += 2 * n
                 continue
-            if self._block_fusable(i) and self._queue_block(i, tensors, nn):
+            if block and self._block_fusable(i, readers=readers) and self._queue_block(i, tensors, nn):
                 out = tensors[self.layers[i + 1]["name"]] = self.act[self.layers[i + 1]["name"]]
                 i += 2
                 continue
@@ -289,9 +266,9 @@ class Runner:
         return out
 
     # -- depthwise + pointwise as one launch ------------------------------------------------
-    def _block_fusable(self, i, policy=True):
+    def _block_fusable(self, i, policy=True, readers=None):
         """Layer i is a 3x3 / padding 1 depthwise layer whose only reader is the pointwise layer i + 1.
-        policy=False: only whether the block can be one launch, not whether it pays on its own."""
+        policy=False: only whether the block can be one launch, not whether it pays on its own.  readers: _reader_counts()."""
         if not (self.fused and self.fuse_blocks) or i in self.unfused_blocks or i + 1 >= len(self.layers):
             return False
         L, N = self.layers[i], self.layers[i + 1]
@@ -310,31 +287,34 @@ class Runner:
                     return False
             elif tuple(self.shapes[L["name"]][:2]) != (8, 8):
                 return False
-        if L["op"] != "depthwise" or N["op"] != "pointwise" or N["in"] != L["name"]:
-            return False
         sx, sy = L["strides"]
         if L["w"].shape[1:3] != (3, 3) or tuple(L["pads"]) != (1, 1, 1, 1) or sx != sy:
             return False
-        readers = [M for M in self.layers if (M["in"] == L["name"] or (M["op"] == "add" and L["name"] in M["in"]))]
-        return len(readers) == 1
+        return (readers or self._reader_counts())[L["name"]] == 1
 
-    def _readers(self, name):
-        return [M for M in self.layers if (M["in"] == name or (M["op"] == "add" and name in M["in"]))]
+    def _reader_counts(self):
+        """{tensor name: how many layers read it}"""
+        counts = {}
+        for M in self.layers:
+            for name in (set(M["in"]) if M["op"] == "add" else (M["in"],)):
+                counts[name] = counts.get(name, 0) + 1
+        return counts
 
-    def _chain_length(self, i):
+    def _chain_length(self, i, readers=None):
         """How many depthwise + pointwise blocks of one shape start at layer i (stride 1, as many channels out as in,
         every intermediate tensor read by the next layer only): such a run is one launch, with the activations kept
         in LDS from block to block."""
         if i in self.unchained:
             return 0
         n, shape = 0, None
-        while n < 8 and self._block_fusable(i + 2 * n, policy=False):
+        readers = readers or self._reader_counts()
+        while n < 8 and self._block_fusable(i + 2 * n, policy=False, readers=readers):
             L, N = self.layers[i + 2 * n], self.layers[i + 2 * n + 1]
             if L["strides"][0] != 1 or self.shapes[L["in"]] != self.shapes[N["name"]]:
                 break
             if shape is None:
                 shape = self.shapes[L["in"]]
-            if self.shapes[L["in"]] != shape or (n > 0 and len(self._readers(L["in"])) != 1):
+            if self.shapes[L["in"]] != shape or (n > 0 and readers[L["in"]] != 1):
                 break
             n += 1
         return n
