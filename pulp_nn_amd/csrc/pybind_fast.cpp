@@ -554,6 +554,7 @@ bool add_guard(Plan *pl, PyObject *dict, PyObject *key, PyObject *value)
 // a value that cannot change in place, or a list, whose items are kept
 bool is_scalar(PyObject *v)
 {
+  if (PyLong_CheckExact(v)) return true;
   if (v == Py_None || PyLong_Check(v) || PyFloat_Check(v) || PyUnicode_Check(v) || PyTuple_Check(v) || PyList_Check(v)) return true;
   if (!PyNumber_Check(v) || Py_TYPE(v)->tp_hash == PyObject_HashNotImplemented) return false;
   return !PyObject_HasAttrString(v, "data_ptr");  // (numpy's scalars, and no tensor)
@@ -581,17 +582,18 @@ int plan_init(PyObject *self, PyObject *args, PyObject *)
   pl->calls = new std::vector<Call>();
   pl->guards = new std::vector<Guard>();
   pl->wholes = new std::vector<Whole>();
+  pl->calls->reserve((size_t)PyList_GET_SIZE(list));
+  pl->guards->reserve(16 * (size_t)PyList_GET_SIZE(from));
   for (Py_ssize_t i = 0; i < PyList_GET_SIZE(from); i++) {
     PyObject *dict, *keys, *key, *value;
     if (!PyArg_ParseTuple(PyList_GET_ITEM(from, i), "O!O", &PyDict_Type, &dict, &keys)) return -1;
     if (keys == Py_None || PyAnySet_Check(keys)) {
       for (Py_ssize_t pos = 0; PyDict_Next(dict, &pos, &key, &value);) {
-        const int object = keys == Py_None ? 1 : PySet_Contains(keys, key);
-        if (object < 0 || !add_guard(pl, dict, key, value)) return -1;
-        if (!object && !is_scalar(value)) {
-          PyErr_Format(PyExc_TypeError, "%R is a %.100s, which may change in place", key, Py_TYPE(value)->tp_name);
-          return -1;
-        }
+        if (!add_guard(pl, dict, key, value)) return -1;
+        if (keys == Py_None || is_scalar(value)) continue;
+        const int object = PySet_Contains(keys, key);
+        if (!object) PyErr_Format(PyExc_TypeError, "%R is a %.100s, which may change in place", key, Py_TYPE(value)->tp_name);
+        if (object != 1) return -1;
       }
       Py_INCREF(dict);
       pl->wholes->push_back(Whole{dict, PyDict_Size(dict)});
