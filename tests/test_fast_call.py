@@ -44,12 +44,14 @@ def test_arguments_are_converted_like_ctypes_did(nn):
 
 
 def test_plan_notices_changed_entries(nn):
-    marker, table = object(), {"shift": 3}
+    marker, table = object(), {"shift": 100003}
     calls = [("pulp_nn_add", (marker, None, None, 1, 1, 1, 1, 1, 1))]
     plan = api._fast.Plan(nn, 1, calls, marker, [(table, ("shift", "mult"))])
     with pytest.raises(api.PulpNNError):            # it runs: the library sees the null pointers
         plan.run(0)
-    table["shift"] = int("3")
+    equal = int("100003")
+    assert equal is not table["shift"]              # an equal int that is another object: still what the plan was made from
+    table["shift"] = equal
     with pytest.raises(api.PulpNNError):
         plan.run(0)
     table["mult"] = 1                               # an entry that was absent
