@@ -46,12 +46,7 @@ struct DwGeom {
   // increments of (dword, row, channel) when the staging slot index grows by 256
   int inc_dw, inc_row, inc_c;
   int in_align4;  // input pointer and W are multiples of 4: aligned dword loads are safe
-  int out_vec4;   // output pointer and CH are multiples of 4: dword stores are safe
-  // Packing of layers with fewer than 64 channels (dw3x3_lin_kernel only): CH and B describe the
-  // input re-read as images of 64 planes (CHW images lie back to back, so that is the same memory);
-  // CHR is the real channel count, planes the real number of planes B_real * CHR.
-  int CHR;
-  long long planes;
+  long long planes;  // B * CH
 };
 
 #define DW_CG 64  // channels per workgroup (one per lane)
@@ -96,21 +91,9 @@ __device__ __forceinline__ void dw_stage(const DwGeom &g, unsigned *lds, const u
   }
 }
 
-// 4x4 byte transpose across the four lanes of a quad: in: byte j of lane q =
-// element (q, j); out: byte q' of lane j' = element (q', j').
-__device__ __forceinline__ unsigned quad_transpose4x4(unsigned v, int lane)
-{
-  // exchange 16-bit halves with lane ^ 2
-  unsigned t = (unsigned)__builtin_amdgcn_mov_dpp((int)v, 0x4E /* quad_perm [2,3,0,1] */, 0xF, 0xF, true);
-  v = (lane & 2) ? ((t >> 16) | (v & 0xFFFF0000u)) : ((v & 0x0000FFFFu) | (t << 16));
-  // exchange bytes with lane ^ 1
-  t = (unsigned)__builtin_amdgcn_mov_dpp((int)v, 0xB1 /* quad_perm [1,0,3,2] */, 0xF, 0xF, true);
-  v = (lane & 1) ? (((t >> 8) & 0x00FF00FFu) | (v & 0xFF00FF00u)) : ((v & 0x00FF00FFu) | ((t << 8) & 0xFF00FF00u));
-  return v;
-}
-
-// The same transpose with v_perm_b32: sel1 / sel2 are per-lane byte selectors
-// (quad_sel1 / quad_sel2 of the lane), so there is no per-lane branch or select.
+// 4x4 byte transpose across the four lanes of a quad: in: byte j of lane q = element (q, j); out: byte q' of lane j' =
+// element (q', j').  With v_perm_b32: sel1 / sel2 are per-lane byte selectors (quad_sel1 / quad_sel2 of the lane), so
+// there is no per-lane branch or select.
 // v_perm_b32 D, S0, S1, sel: selector values 0-3 pick bytes of S1, 4-7 bytes of S0.
 __device__ __forceinline__ unsigned quad_sel1(int lane) { return (lane & 2) ? 0x03020706u : 0x05040100u; }
 __device__ __forceinline__ unsigned quad_sel2(int lane) { return (lane & 1) ? 0x03070105u : 0x06020400u; }
@@ -161,12 +144,10 @@ struct DwColumn {
   int corr, mult, shift;
   bn_t k, lambda;
   unsigned wA[3], wB[3], sel1, sel2;
-  int store, nbytes;
 };
 
-// XR: LDS holds the raw input bytes and the ^ 0x80 is applied as a dword is read (the LDS-direct staging of
-// dw3x3_lin_kernel cannot apply it).
-template <int S, int PL, int MODE, bool FULL, bool EDGE, bool FASTQ, bool XR = false>
+// LDS holds the raw input bytes: the ^ 0x80 is applied as a dword is read (LDS-direct loads cannot apply it).
+template <int S, int PL, int MODE, bool EDGE, bool FASTQ>
 __device__ __forceinline__ void dw3x3_column(DwColumn c)
 {
   constexpr int O0 = 4 - PL;
@@ -178,12 +159,12 @@ __device__ __forceinline__ void dw3x3_column(DwColumn c)
   // step before it is used, so that the LDS latency is covered by the arithmetic of the row before
   auto fetch = [&](unsigned (&raw)[NS]) {
 #pragma unroll
-    for (int d = 0; d < NS; d++) raw[d] = in_row[d] ? c.p[d] : (XR ? 0u : 0x80808080u);
+    for (int d = 0; d < NS; d++) raw[d] = in_row[d] ? c.p[d] : 0u;
     c.p += c.LWD;
   };
   auto finish = [&](const unsigned (&raw)[NS], unsigned (&span)[NS]) {
 #pragma unroll
-    for (int d = 0; d < NS; d++) span[d] = XR ? raw[d] ^ 0x80808080u : raw[d];
+    for (int d = 0; d < NS; d++) span[d] = raw[d] ^ 0x80808080u;
   };
   auto read_row = [&](unsigned (&span)[NS]) {
     unsigned raw[NS];
@@ -206,15 +187,7 @@ __device__ __forceinline__ void dw3x3_column(DwColumn c)
   auto emit = [&](int (&acc)[4]) {
     unsigned packed = requant4_same<MODE, FASTQ>(acc[0], acc[1], acc[2], acc[3], c.k, c.lambda, c.mult, c.shift);
     packed = quad_transpose4x4_perm(packed, c.sel1, c.sel2);
-    if constexpr (FULL) {
-      *(unsigned *)c.o = packed;
-    } else {
-      if (c.store == 0) {
-        *(unsigned *)c.o = packed;
-      } else if (c.store == 1) {
-        for (int j = 0; j < c.nbytes; j++) c.o[j] = (uint8_t)(packed >> (8 * j));
-      }
-    }
+    *(unsigned *)c.o = packed;
     c.o += c.row_bytes;
   };
 
@@ -264,7 +237,8 @@ __device__ __forceinline__ void dw3x3_column(DwColumn c)
   }
 }
 
-// 3x3 depthwise, fast variant for W % 4 == 0 and a 16-byte aligned input.
+// 3x3 depthwise, fast variant for W % 4 == 0 and a 16-byte aligned input, whole groups of 64 channels and of 4 output
+// columns on a 4-byte aligned output: every lane stores one dword per output row without any bounds check.
 //
 // LDS holds the band exactly as it lies in memory (rows of W bytes back to back,
 // no column padding), so staging is a linear copy.  The columns left of 0 and right
@@ -275,19 +249,15 @@ __device__ __forceinline__ void dw3x3_column(DwColumn c)
 // also means every input dword is read from LDS once, not three times: the three
 // partial sums an input row contributes to are kept in registers.
 //
-// FULL: Wo % 4 == 0, CH % 64 == 0 and the output is 4-byte aligned, so every lane
-// stores one dword per output row without any bounds check.
+// The band is staged with buffer loads that write LDS directly, one instruction per channel, instead of through registers
+// (no staging registers, no LDS stores with their bank conflicts, no VALU work); the host checks that byte offsets fit 31
+// bits and that the channel stride leaves room for a band's last 16-byte piece.
 #ifndef DW_WAVES
 #define DW_WAVES 8  // waves per workgroup of dw3x3_lin_kernel
 #endif
-// DMA (FULL only; the host checks that byte offsets fit 31 bits and that the channel stride leaves room
-// for a band's last 16-byte piece): the band is staged with buffer loads that write LDS directly, one
-// instruction per channel, instead of through registers (no staging registers, no LDS stores with their
-// bank conflicts, no VALU work); LDS then holds raw bytes and the ^ 0x80 is applied as a dword is read.
-template <int S, int PL, int MODE, bool FULL, bool DMA = false>
+template <int S, int PL, int MODE>
 __global__ __launch_bounds__(64 * DW_WAVES) void dw3x3_lin_kernel(DwGeom g, EpiArgs e)
 {
-  static_assert(DMA && FULL, "whole 64-channel groups, staged by LDS-direct loads");
   constexpr int NWV = DW_WAVES, CPW = DW_CG / NWV;  // waves, channels staged per wave
   extern __shared__ unsigned dw_lds[];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -306,7 +276,7 @@ __global__ __launch_bounds__(64 * DW_WAVES) void dw3x3_lin_kernel(DwGeom g, EpiA
 
   // ---- stage -----------------------------------------------------------------
   const int r_lo = max(0, -iy_start), r_hi = min(g.NR, g.H - iy_start);  // rows of the band inside the image
-  if constexpr (DMA) {
+  {
     // Lane l fetches the 16-byte chunk l of a channel's band (dwords 4l .. 4l+3).  Dwords [lo_d, hi_d) lie inside
     // the image; a chunk wholly outside is requested out of range (zeros); a chunk that straddles the first or last
     // image row is left out and fetched dword by dword (runs of 64 dwords q1 / q2).
@@ -340,41 +310,34 @@ __global__ __launch_bounds__(64 * DW_WAVES) void dw3x3_lin_kernel(DwGeom g, EpiA
   }
 
   // ---- per-lane channel constants ------------------------------------------------
-  const bool ch_ok = c0 + lane < g.CH && (long long)b * g.CH + c0 + lane < g.planes;
-  const int ch = (c0 + lane) % g.CHR;  // real channel: index of the weights and constants
+  const int ch = c0 + lane;
   unsigned wA[3], wB[3];
-  int corr = 0;
+  int wsum = 0;
   bn_t kk = 0, ll = 0;
-  if (ch_ok) {
-    int wsum = 0;
 #pragma unroll
-    for (int i = 0; i < 3; i++) {
-      const int8_t *p = g.wt + (long long)ch * 9 + 3 * i;
-      const unsigned k0 = (uint8_t)p[0], k1 = (uint8_t)p[1], k2 = (uint8_t)p[2];
-      wA[i] = k0 | (k1 << 8) | (k2 << 16);
-      wB[i] = wA[i] << 8;
-      wsum += (int)p[0] + (int)p[1] + (int)p[2];
-    }
-    corr = 128 * wsum + (g.bias ? (int)g.bias[ch] : 0);
-    if (MODE == EPI_BN) {
-      kk = e.k[ch];
-      ll = e.lambda[ch];
-    }
-  } else {
-#pragma unroll
-    for (int i = 0; i < 3; i++) wA[i] = wB[i] = 0;
+  for (int i = 0; i < 3; i++) {
+    const int8_t *p = g.wt + (long long)ch * 9 + 3 * i;
+    const unsigned k0 = (uint8_t)p[0], k1 = (uint8_t)p[1], k2 = (uint8_t)p[2];
+    wA[i] = k0 | (k1 << 8) | (k2 << 16);
+    wB[i] = wA[i] << 8;
+    wsum += (int)p[0] + (int)p[1] + (int)p[2];
+  }
+  const int corr = 128 * wsum + (g.bias ? (int)g.bias[ch] : 0);
+  if (MODE == EPI_BN) {
+    kk = e.k[ch];
+    ll = e.lambda[ch];
   }
   const bool k_small = __all(bn_k_small(kk));
-  if constexpr (DMA) __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's LDS-direct loads have landed
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's LDS-direct loads have landed
   __syncthreads();
 
   // ---- compute -------------------------------------------------------------------------
-  const int xgroups = (g.Wo + 3) >> 2;
+  const int xgroups = g.Wo >> 2;
   const unsigned *lbase = dw_lds + lane * g.CSD - 1;
   DwColumn col;
   col.LWD = LWD;
   col.rows = rows;
-  col.row_bytes = (long long)g.Wo * g.CHR;
+  col.row_bytes = (long long)g.Wo * g.CH;
   col.corr = corr;
   col.k = kk;
   col.lambda = ll;
@@ -387,27 +350,21 @@ __global__ __launch_bounds__(64 * DW_WAVES) void dw3x3_lin_kernel(DwGeom g, EpiA
     col.wA[i] = wA[i];
     col.wB[i] = wB[i];
   }
-  const int cq = lane & ~3;
   const bool fastq = (MODE == EPI_BN) ? k_small : (e.shift >= 16);
   constexpr int NS = ((4 - PL) + 3 * S + 2) / 4 + 1;
 
   for (int xg = wave; xg < xgroups; xg += NWV) {
     col.dc0 = xg * S - 1;  // dword column of the first dword of the window
     col.p = lbase + xg * S;
-    // this lane stores 4 consecutive channels of one pixel: plane pq .. pq+3 -> image pq / CHR, channel pq % CHR
-    const long long pq = (long long)b * g.CH + c0 + cq;
-    col.o = g.out + (((pq / g.CHR) * g.Ho + oy0) * g.Wo + 4 * xg + (lane & 3)) * g.CHR + (int)(pq % g.CHR);
-    // 0: store a dword, 1: store the valid bytes one by one, 2: nothing to store
-    const long long left = min((long long)(g.CH - c0 - cq), g.planes - pq);  // planes this lane may write
-    col.store = (4 * xg + (lane & 3) >= g.Wo || left <= 0) ? 2 : ((g.out_vec4 && left >= 4) ? 0 : 1);
-    col.nbytes = (int)min(4ll, max(left, 0ll));
+    // this lane stores 4 consecutive channels of one pixel
+    col.o = g.out + (((long long)b * g.Ho + oy0) * g.Wo + 4 * xg + (lane & 3)) * g.CH + c0 + (lane & ~3);
     const bool edge = col.dc0 < 0 || col.dc0 + NS > LWD;
     if (fastq) {
-      if (edge) dw3x3_column<S, PL, MODE, FULL, true, true, DMA>(col);
-      else dw3x3_column<S, PL, MODE, FULL, false, true, DMA>(col);
+      if (edge) dw3x3_column<S, PL, MODE, true, true>(col);
+      else dw3x3_column<S, PL, MODE, false, true>(col);
     } else {
-      if (edge) dw3x3_column<S, PL, MODE, FULL, true, false, DMA>(col);
-      else dw3x3_column<S, PL, MODE, FULL, false, false, DMA>(col);
+      if (edge) dw3x3_column<S, PL, MODE, true, false>(col);
+      else dw3x3_column<S, PL, MODE, false, false>(col);
     }
   }
 }
@@ -543,22 +500,22 @@ __global__ __launch_bounds__(64 * DW_REG_WAVES) void dw3x3_rows_kernel(DwGeom g,
   const long long item = (long long)blockIdx.x * DW_REG_WAVES + (threadIdx.x >> 6);  // one per wave
   if (item >= g.planes / DW_CG * nseg) return;
   const int seg = (int)(item % nseg);
-  const long long P = item / nseg * DW_CG + lane;  // plane: image P / CHR, channel P % CHR
-  const int b = (int)(P / g.CHR), ch = (int)(P % g.CHR);
+  const long long P = item / nseg * DW_CG + lane;  // plane: image P / CH, channel P % CH
+  const int b = (int)(P / g.CH), ch = (int)(P % g.CH);
   const int oy0 = seg * R;
 
   const unsigned sel1 = quad_sel1(lane), sel2 = quad_sel2(lane);
   unsigned row[NIN][RD];
   if constexpr (HWC) {
-    const uint8_t *src = g.in + ((long long)b * g.H * WB + (lane & 3)) * g.CHR + (ch & ~3);
+    const uint8_t *src = g.in + ((long long)b * g.H * WB + (lane & 3)) * g.CH + (ch & ~3);
 #pragma unroll
     for (int r = 0; r < NIN; r++) {
       const int iy = oy0 * S - 1 + r;
       const bool ok = (unsigned)iy < (unsigned)g.H;
-      const uint8_t *rp = src + (long long)min(max(iy, 0), g.H - 1) * WB * g.CHR;
+      const uint8_t *rp = src + (long long)min(max(iy, 0), g.H - 1) * WB * g.CH;
 #pragma unroll
       for (int d = 0; d < RD; d++) {
-        const unsigned v = *(const unsigned *)(rp + (long long)(4 * d) * g.CHR);
+        const unsigned v = *(const unsigned *)(rp + (long long)(4 * d) * g.CH);
         row[r][d] = ok ? v : 0u;
       }
     }
@@ -599,7 +556,7 @@ __global__ __launch_bounds__(64 * DW_REG_WAVES) void dw3x3_rows_kernel(DwGeom g,
   }
   const bool fastq = (MODE == EPI_BN) ? __all(bn_k_small(kk)) : (e.shift >= 16);
   // after the quad transpose this lane holds the 4 channels of its quad for pixel column 4*xg + lane%4
-  uint8_t *obase = g.out + (((long long)b * g.Ho + oy0) * WO + (lane & 3)) * g.CHR + (ch & ~3);
+  uint8_t *obase = g.out + (((long long)b * g.Ho + oy0) * WO + (lane & 3)) * g.CH + (ch & ~3);
 
   auto body = [&](auto fq) {
     constexpr bool FASTQ = decltype(fq)::value;
@@ -624,7 +581,7 @@ __global__ __launch_bounds__(64 * DW_REG_WAVES) void dw3x3_rows_kernel(DwGeom g,
         }
         unsigned packed = requant4_same<MODE, FASTQ>(acc[0], acc[1], acc[2], acc[3], kk, ll, e.mult, e.shift);
         packed = quad_transpose4x4_perm(packed, sel1, sel2);
-        *(unsigned *)(obase + (long long)(ro * WO + 4 * xg) * g.CHR) = packed;
+        *(unsigned *)(obase + (long long)(ro * WO + 4 * xg) * g.CH) = packed;
       }
     }
   };

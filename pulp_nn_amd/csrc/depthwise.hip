@@ -38,10 +38,8 @@ void depthwise_common(const char *fn, const uint8_t *in, const int8_t *bias, uin
   g.pl = pl;
   g.sx = sx;
   g.sy = sy;
-  g.CHR = CH;
   g.planes = (long long)g.B * CH;
   g.cgroups = (CH + DW_CG - 1) / DW_CG;
-  g.out_vec4 = aligned(out, 4) && (CH % 4 == 0);
   const bool fast = kx == 3 && ky == 3 && sx == sy && (sx == 1 || sx == 2) && (pl == 0 || pl == 1);
   // small square planes, padding 1: one plane per lane, in registers
   const int ho_plane = (H - 1) / sx + 1;
@@ -149,9 +147,9 @@ void depthwise_common(const char *fn, const uint8_t *in, const int8_t *bias, uin
     const dim3 grid(g.total), block(64 * DW_WAVES);
 #define DW3L(S, PL)                                                                                                           \
   switch (mode) {                                                                                                             \
-    case EPI_BN: hipLaunchKernelGGL((dw3x3_lin_kernel<S, PL, EPI_BN, true, true>), grid, block, lin_lds, g_stream, g, e); break;     \
-    case EPI_MULT: hipLaunchKernelGGL((dw3x3_lin_kernel<S, PL, EPI_MULT, true, true>), grid, block, lin_lds, g_stream, g, e); break; \
-    default: hipLaunchKernelGGL((dw3x3_lin_kernel<S, PL, EPI_RAW, true, true>), grid, block, lin_lds, g_stream, g, e); break;        \
+    case EPI_BN: hipLaunchKernelGGL((dw3x3_lin_kernel<S, PL, EPI_BN>), grid, block, lin_lds, g_stream, g, e); break;     \
+    case EPI_MULT: hipLaunchKernelGGL((dw3x3_lin_kernel<S, PL, EPI_MULT>), grid, block, lin_lds, g_stream, g, e); break; \
+    default: hipLaunchKernelGGL((dw3x3_lin_kernel<S, PL, EPI_RAW>), grid, block, lin_lds, g_stream, g, e); break;        \
   }
     if (sx == 1 && pl == 1) { DW3L(1, 1) }
     else if (sx == 1) { DW3L(1, 0) }
