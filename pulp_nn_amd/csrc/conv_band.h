@@ -26,10 +26,6 @@
 #include "conv_band_geom.h"
 #include "igemm.h"
 
-typedef v4i v4i_b __attribute__((aligned(1)));
-typedef v2i v2i_b __attribute__((aligned(1)));
-typedef int i32_b __attribute__((aligned(1)));
-
 // the 16 bytes of v moved up by n bytes (0 < n < 16), zeros below
 __device__ __forceinline__ v4i bytes_up(v4i v, int n)
 {
@@ -37,13 +33,6 @@ __device__ __forceinline__ v4i bytes_up(v4i v, int n)
                         ((unsigned long long)(unsigned)v.x | ((unsigned long long)(unsigned)v.y << 32));
   t <<= 8 * n;
   return (v4i){(int)(unsigned)t, (int)(unsigned)(t >> 32), (int)(unsigned)(t >> 64), (int)(unsigned)(t >> 96)};
-}
-
-// bytes [0, n) of a dword, n clamped to [0, 4]
-__device__ __forceinline__ unsigned low_bytes(int n)
-{
-  const int m = min(n, 4);
-  return m <= 0 ? 0u : __builtin_amdgcn_alignbit(0u, 0xffffffffu, 32 - 8 * m);  // (4 bytes: a shift by 0)
 }
 
 // TN: 16-channel groups per wave; TM: 16-pixel groups per wave
@@ -97,7 +86,7 @@ __global__ __launch_bounds__(256) void conv_band_kernel(BandGeom g, EpiArgs e)
     const int n = n0 + tid;
     const bool ok = n < g.N;
     c_bias[tid] = (g.bias && ok) ? (int)g.bias[n] : 0;
-    c_k[tid] = g.mode == EPI_BN ? (ok ? e.k[n] : (bn_t)0) : g.mode == EPI_MULT ? (bn_t)e.mult : (bn_t)1;
+    c_k[tid] = (g.mode == EPI_BN && ok) ? e.k[n] : (bn_t)0;
     c_l[tid] = (g.mode == EPI_BN && ok) ? e.lambda[n] : (bn_t)0;
   }
   int *tab = (int *)(band_lds + g.tab_off);
@@ -128,7 +117,7 @@ __global__ __launch_bounds__(256) void conv_band_kernel(BandGeom g, EpiArgs e)
         const int iy = iy0 + row, ix = ix0 + col;
         const bool in = (unsigned)iy < (unsigned)g.H && (unsigned)ix < (unsigned)g.W && col < iw;
         const long long off = in ? ibase + ((long long)iy * g.W + ix) * g.Ci + min(16 * c16, g.Ci - 16) : 0;
-        v[u] = *(const v4i_b *)(g.in + max(off, 0ll));
+        v[u] = *(const v4i_u *)(g.in + max(off, 0ll));
         under[u] = off < 0 ? (int)-off : 0;
         ok[u] = in ? 0xffffffffu : 0u;
         last[u] = c16 == g.CG - 1;
@@ -240,9 +229,9 @@ __global__ __launch_bounds__(256) void conv_band_kernel(BandGeom g, EpiArgs e)
     if (p >= px) continue;
     uint8_t *o = ob + (long long)p * g.N;
     if (cb + 4 * TN <= g.N) {
-      if constexpr (TN == 4) *(v4i_b *)o = (v4i){(int)packed[s][0], (int)packed[s][1 % TN], (int)packed[s][2 % TN], (int)packed[s][3 % TN]};
-      else if constexpr (TN == 2) *(v2i_b *)o = (v2i){(int)packed[s][0], (int)packed[s][1 % TN]};
-      else *(i32_b *)o = (int)packed[s][0];
+      if constexpr (TN == 4) *(v4i_u *)o = (v4i){(int)packed[s][0], (int)packed[s][1 % TN], (int)packed[s][2 % TN], (int)packed[s][3 % TN]};
+      else if constexpr (TN == 2) *(v2i_u *)o = (v2i){(int)packed[s][0], (int)packed[s][1 % TN]};
+      else *(i32_u *)o = (int)packed[s][0];
     } else {
 #pragma unroll
       for (int c = 0; c < 4 * TN; c++)

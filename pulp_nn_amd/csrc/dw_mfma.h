@@ -33,16 +33,6 @@
 #include "memops.h"
 #include "requant.h"
 
-typedef v4i v4i_u __attribute__((aligned(1)));
-typedef int i32_u __attribute__((aligned(1)));
-
-// bytes [0, n) of a dword, n clamped to [0, 4]
-__device__ __forceinline__ unsigned dwm_low_bytes(int n)
-{
-  const int m = min(n, 4);
-  return m <= 0 ? 0u : __builtin_amdgcn_alignbit(0u, 0xffffffffu, 32 - 8 * m);  // (4 bytes: a shift by 0)
-}
-
 // MODE: requantisation branch; NM: MFMAs per (channel, 16 units) = ceil(ky * ND / 16); CB: channels per workgroup
 template <int CB, int NM, int MODE>
 __global__ __launch_bounds__(256) void dw_mfma_kernel(DwmGeom g, EpiArgs e)
@@ -76,7 +66,7 @@ __global__ __launch_bounds__(256) void dw_mfma_kernel(DwmGeom g, EpiArgs e)
         // bytes of the chunk inside the image
         unsigned mask[4];
 #pragma unroll
-        for (int d = 0; d < 4; d++) mask[d] = row_ok ? dwm_low_bytes(g.W - (x + 4 * d)) & ~dwm_low_bytes(-(x + 4 * d)) : 0u;
+        for (int d = 0; d < 4; d++) mask[d] = row_ok ? low_bytes(g.W - (x + 4 * d)) & ~low_bytes(-(x + 4 * d)) : 0u;
         for (int cb = cpi; cb < ncb; cb += UN * g.cpar) {
           v4i v[UN];
           int off[UN];
@@ -116,7 +106,7 @@ __global__ __launch_bounds__(256) void dw_mfma_kernel(DwmGeom g, EpiArgs e)
     if ((int)fastdiv((unsigned)t, g.d_ky) < ncb) {
       if (g.kx <= 4 && g.wt_bytes >= 4) {
         const int at = min(first, g.wt_bytes - 4);
-        w.x = (int)(((unsigned)*(const i32_u *)(g.wt + at) >> (8 * (first - at))) & dwm_low_bytes(g.kx));
+        w.x = (int)(((unsigned)*(const i32_u *)(g.wt + at) >> (8 * (first - at))) & low_bytes(g.kx));
       } else {
         for (int j = 0; j < g.kx; j++) {
           const unsigned v = (unsigned)(uint8_t)g.wt[first + j] << (8 * (j & 3));

@@ -155,7 +155,6 @@ __global__ __launch_bounds__(64 * NWV) void dwpw_fused_kernel(DwPwGeom g)
   int dw_w[3], dw_b;  // the nine filter bytes, bias
   bn_t dw_k, dw_l;
   auto load_dw = [&](const DwPwBlock &P, int ch) {
-    typedef int i32_u __attribute__((aligned(1)));
     const int8_t *p = P.dw_wt + (long long)ch * 9;
     dw_w[0] = *(const i32_u *)p;
     dw_w[1] = *(const i32_u *)(p + 4);

@@ -25,7 +25,6 @@ __global__ __launch_bounds__(256) void linear_skinny_any_kernel(SkinnyGeom g, Ep
   const bool active = mb < g.M;
 
   // weight rows past N and K chunks past K are read from a valid address and zeroed
-  typedef v4i v4i_r __attribute__((aligned(1)));
   const bool nok = n0 + l16 < g.N;
   const int8_t *wrow = g.w + (long long)min(n0 + l16, g.N - 1) * g.K;
   const uint8_t *arow[4];
@@ -51,9 +50,9 @@ __global__ __launch_bounds__(256) void linear_skinny_any_kernel(SkinnyGeom g, Ep
         const int kt = min(kb + u, kt1 - 1);
         const int p = 64 * kt + 16 * lgrp;
         const int ko = p >= g.K ? 0 : min(p, g.K - 16);
-        wf[u] = *(const v4i_r *)(wrow + ko);
+        wf[u] = *(const v4i_u *)(wrow + ko);
 #pragma unroll
-        for (int s = 0; s < 4; s++) af[u][s] = *(const v4i_r *)(arow[s] + ko);
+        for (int s = 0; s < 4; s++) af[u][s] = *(const v4i_u *)(arow[s] + ko);
       }
 #pragma unroll
       for (int u = 0; u < 4; u++) {

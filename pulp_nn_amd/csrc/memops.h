@@ -11,6 +11,10 @@
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v2i __attribute__((ext_vector_type(2)));
+// the same and a dword at any address
+typedef v4i v4i_u __attribute__((aligned(1)));
+typedef v2i v2i_u __attribute__((aligned(1)));
+typedef int i32_u __attribute__((aligned(1)));
 
 // Outputs at least this large are streamed past the caches.
 #define PULPNN_NT_BYTES (32ll << 20)
@@ -36,4 +40,11 @@ __device__ __forceinline__ void store4(void *p, int v)
 {
   if constexpr (NT) __builtin_nontemporal_store(v, (int *)p);
   else *(int *)p = v;
+}
+
+// bytes [0, n) of a dword, n clamped to [0, 4]
+__device__ __forceinline__ unsigned low_bytes(int n)
+{
+  const int m = min(n, 4);
+  return m <= 0 ? 0u : __builtin_amdgcn_alignbit(0u, 0xffffffffu, 32 - 8 * m);  // (4 bytes: a shift by 0)
 }

@@ -50,7 +50,7 @@ __global__ __launch_bounds__(64 * NW) void pw_any_kernel(PwAnyGeom g, EpiArgs e)
     const long long m = max(min(p0 + l16, px_end - 1), 0);
     const long long row = m * g.K;
 #pragma unroll
-    for (int ks = 0; ks < KS; ks++) a[ks] = *(const v4i_b *)(g.in + (KS == 1 ? max(row + koff[ks], 0ll) : row + koff[ks]));
+    for (int ks = 0; ks < KS; ks++) a[ks] = *(const v4i_u *)(g.in + (KS == 1 ? max(row + koff[ks], 0ll) : row + koff[ks]));
   };
   v4i b0[KS], b1[KS], b2[KS];
   load_a(b0, px);
@@ -70,7 +70,7 @@ __global__ __launch_bounds__(64 * NW) void pw_any_kernel(PwAnyGeom g, EpiArgs e)
         const int n = p * 64 + (i >> 2) * 16 + 4 * t + (i & 3), k = ks * 64 + 16 * c;
         const bool ok = n < nb && k < g.K;
         const long long off = ok ? (long long)(n0 + n) * g.K + min(k, g.K - 16) : 0;
-        v4i v = *(const v4i_b *)(g.w + max(off, 0ll));
+        v4i v = *(const v4i_u *)(g.w + max(off, 0ll));
         if (KS == 1 && __any(off < 0))
           if (off < 0) v = bytes_up(v, (int)-off);
         const int dup = k - (g.K - 16);  // > 0: the first bytes of the chunk are the chunk before's
@@ -183,8 +183,8 @@ __global__ __launch_bounds__(64 * NW) void pw_any_kernel(PwAnyGeom g, EpiArgs e)
     }
 #pragma unroll
     for (int r = 0; r < NP; r++) {
-      if constexpr (NT) __builtin_nontemporal_store(v[r], (v4i_b *)dst[r]);
-      else *(v4i_b *)dst[r] = v[r];
+      if constexpr (NT) __builtin_nontemporal_store(v[r], (v4i_u *)dst[r]);
+      else *(v4i_u *)dst[r] = v[r];
     }
   };
   auto stream = [&](auto nt) {
