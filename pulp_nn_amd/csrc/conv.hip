@@ -384,6 +384,11 @@ void conv_common(const char *fn, bool pointwise, const uint8_t *in, const int8_t
     // few output channels, which leave most of the tiled kernel's 128 x 64 tile empty and its many waves waiting for each
     // other (kernel times, tiled / band: 8x38x9 240 -> 32 s2 21.9 / 12.6 us; 2x8x13 48 -> 16 5x5 14.2 / 7.2; 31x19 80 -> 16
     // 10.6 / 6.8; 23x14 144 -> 35 12.0 / 8.8; but 133x16x28 176 -> 128 28.6 / 34.2, 252x12x29 64 -> 40 s2 7.3 / 8.4).
+    // 16 and 32 input channels stay with the tiled kernel, which takes two or four taps per K slice there.  It is the faster one
+    // from 40 output channels on (tiled / band, 32 -> 64 at batch 256 16x16 6.7 / 8.5, batch 133 28x28 10.8 / 14.5, batch 64 64x64
+    // 18.4 / 24.1; 8x57x43 32 -> 40 5.2 / 9.3) and the slower one below (256x16x16 32 -> 32 7.3 / 6.8, 32 -> 16 6.9 / 5.7; 256x8x8
+    // 32 -> 24 7.7 / 5.3; 64x32x32 16 -> 32 6.9 / 6.4; but 133x28x28 16 -> 32 7.7 / 8.3): a line at 32 channels that this rule
+    // does not draw.
     const bool whole16 = ch_in % 16 == 0 && aligned(in, 16) && aligned(w, 16);
     const bool few = ch_in == 16 || ch_in == 32 ? false : ch_in % 64 == 0 ? g.N <= 32 : g.N <= 64;
     if (!whole16 || few) {

@@ -16,9 +16,11 @@
 // one wave only: straight from global memory in MFMA operand layout, PF steps at a time, the next PF steps requested
 // before the current ones are multiplied.  128 * sum(w) comes from one more MFMA per weight fragment against ones.
 //
-// Bound: layers of up to a few MB, by the latency of load -> LDS -> multiply -> store; larger ones by LDS reads (one
-// fragment per TN MFMAs).  Measured, whole calls, against the 128 x 64 tile with a byte gather that these shapes took:
-// 57x43 24 -> 40 stride 2 batch 32 19.3 -> 9.0 us; 15x31 168 -> 16 batch 19 236 -> 11; 24x27 168 -> 176 5x5 stride 2 batch
+// Bound: layers of up to a few MB, by the latency of load -> LDS -> multiply -> store (57x43 24 -> 40: 15 MFMAs and 718 vector
+// instructions a wave, which waits half of its time; constants are waited for before the input is asked for); larger ones by
+// too few waves and the vector instructions around each MFMA (24x27 168 -> 176 5x5: 1.7 waves per SIMD, 6.6 vector instructions
+// per MFMA, matrix cores 20 % and LDS 10 % busy).  Measured, whole calls, against the 128 x 64 tile with a byte gather that these
+// shapes took: 57x43 24 -> 40 stride 2 batch 32 19.3 -> 9.4 us; 15x31 168 -> 16 batch 19 236 -> 11; 24x27 168 -> 176 5x5 stride 2 batch
 // 72 409 -> 46; 21x36 56 -> 32 stride 2 batch 25 82 -> 7.5; 14x14 24 -> 48 batch 31 19 -> 6.6 (the call's host time).
 #pragma once
 #include <type_traits>
@@ -86,7 +88,8 @@ __global__ __launch_bounds__(256) void conv_band_kernel(BandGeom g, EpiArgs e)
     const int n = n0 + tid;
     const bool ok = n < g.N;
     c_bias[tid] = (g.bias && ok) ? (int)g.bias[n] : 0;
-    c_k[tid] = (g.mode == EPI_BN && ok) ? e.k[n] : (bn_t)0;
+    // (only read for batch-norm; written in every mode, which is the shorter code: 57x43 24 -> 40 9.38 us, 9.46 with a branch)
+    c_k[tid] = g.mode == EPI_BN ? (ok ? e.k[n] : (bn_t)0) : g.mode == EPI_MULT ? (bn_t)e.mult : (bn_t)1;
     c_l[tid] = (g.mode == EPI_BN && ok) ? e.lambda[n] : (bn_t)0;
   }
   int *tab = (int *)(band_lds + g.tab_off);

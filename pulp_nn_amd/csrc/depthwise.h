@@ -252,6 +252,8 @@ __device__ __forceinline__ void dw3x3_column(DwColumn c)
 // The band is staged with buffer loads that write LDS directly, one instruction per channel, instead of through registers
 // (no staging registers, no LDS stores with their bank conflicts, no VALU work); the host checks that byte offsets fit 31
 // bits and that the channel stride leaves room for a band's last 16-byte piece.
+// Bound: the access pattern, and next to it vector-ALU issue (58x56x128 batch 256: 50.8 us; 53.2 with 64-bit divisions for
+// the output address of each column group).
 #ifndef DW_WAVES
 #define DW_WAVES 8  // waves per workgroup of dw3x3_lin_kernel
 #endif

@@ -20,10 +20,11 @@
 // (row, chunk) for all channels, so the masks are computed once.  The first and last bytes of the tensor are met by
 // clamping the address and shifting.
 //
-// Bound: short of bandwidth-sized layers, the set-up of a workgroup (some 400 vector instructions per wave: masks,
-// filter rows, lane tables) and the chain load -> LDS -> multiply -> LDS -> store.  Measured, whole calls, against the
+// Bound: small layers by the chain input -> LDS, filters -> LDS, constants -> LDS, multiply, LDS -> store (35x29x72: 520 vector
+// instructions a wave, most of them set-up, for 13 MFMAs, and 61 % of its time waiting), larger ones by the vector ALU (7x7x512
+// batch 256: 1038 instructions a wave are two thirds of the kernel's 23.7 us).  Measured, whole calls, against the
 // kernels it replaced (four outputs per lane with v_dot4 for 3x3, a byte loop for rows that are not whole dwords and for
-// other filters): 3x3 on 35x29x72 batch 32 36.7 -> 8.4 us; 17x17x408 batch 85 38.3 -> 18.3 (20 MB); 5x5 on 8x23x32 batch
+// other filters): 3x3 on 35x29x72 batch 32 36.7 -> 8.5 us; 17x17x408 batch 85 38.3 -> 18.3 (20 MB); 5x5 on 8x23x32 batch
 // 9 91 -> 7.0; 5x5 stride 2 on 60x11x416 batch 4 65 -> 7.7.
 #pragma once
 #include <type_traits>

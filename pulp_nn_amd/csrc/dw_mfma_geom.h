@@ -23,6 +23,8 @@ struct DwmGeom {
   int B, CH, H, W, Ho, Wo;
   int kx, ky, pt, pl, sx, sy;
   long long in_bytes;   // bytes of the whole input tensor
+  long long edge_bytes; // the same, or for planes of fewer than 16 bytes far below 0: there any tile may leave the tensor, as a row
+                        // outside the image loads from the start of its plane
   int wt_bytes;         // ... and of all filters
   int ND, rND;          // dwords of an input row behind 16 output columns; 65536 / ND + 1
   int RB, NR;           // output rows per tile, input rows behind them
@@ -32,9 +34,10 @@ struct DwmGeom {
   int w_off, c_off, o_off;  // LDS offsets: filter rows, per-channel constants, output tile
   int nper, cpar;       // staging: slots (row, chunk) a pass covers, channels side by side
   // tile index -> (channels, columns, rows, image); thread -> channel; slot -> row; unit -> row; pixel -> row (of a tile
-  // of full width, of the last one along a row); filter row -> channel
-  FastDiv d_cb, d_xt, d_band, d_nper, d_q, d_xg, d_wt, d_wt_last, d_ky;
-  int cblocks, xtiles, bands, total;
+  // of full width); filter row -> channel
+  FastDiv d_cb, d_xt, d_band, d_nper, d_q, d_xg, d_wt, d_ky;
+  int cblocks, xtiles, bands, total;  // (one aligned scalar load: what a workgroup asks for first)
+  FastDiv d_wt_last;  // pixel -> row of the last tile along a row
 };
 
 // One tile: CB channels from c0 on (ncb of them exist), output rows oy0 .. oy0 + rows - 1 of image b, output columns
@@ -65,10 +68,8 @@ PULPNN_HD bool dwm_edge(const DwmGeom &g, const DwmTile &t, long long before, in
 {
   const int plane = g.H * g.W, iy_last = iy0 + g.NR - 1 < g.H - 1 ? iy0 + g.NR - 1 : g.H - 1;
   const long long first = before + (long long)(iy0 > 0 ? iy0 : 0) * g.W + x0;
-  const long long last_plane = before + (long long)(t.ncb - 1) * plane;
-  const long long last = last_plane + (long long)iy_last * g.W + x0 + 16 * g.Q;
-  // (a row outside the image loads from the start of its plane, which in a plane of fewer than 16 bytes reaches past it)
-  return first < 0 || last > g.in_bytes || last_plane + 16 > g.in_bytes;
+  const long long last = before + (long long)(t.ncb - 1) * plane + (long long)iy_last * g.W + x0 + 16 * g.Q;
+  return first < 0 || last > g.edge_bytes;
 }
 
 // Bytes from the tile's first plane to the load of chunk column x in row iy of channel c (a row outside the image: the
@@ -108,6 +109,7 @@ bool dwm_shape(const DwLayer &L, int cus, int bn_bytes, DwmGeom *out, int *nm_ou
   g.sx = L.sx;
   g.sy = L.sy;
   g.in_bytes = (long long)L.B * L.CH * plane;
+  g.edge_bytes = plane < 16 ? -(1ll << 62) : g.in_bytes;
   g.wt_bytes = L.CH * L.kx * L.ky;
   g.ND = (15 * L.sx + L.kx + 3) / 4;
   g.rND = 65536 / g.ND + 1;

@@ -97,7 +97,11 @@ void dwpw_common(const char *fn, const unsigned char *Im_in, unsigned char *Im_o
   else if (g.KT == 2) hipLaunchKernelGGL((dwpw_fused_kernel<WB, RR, 1, NW, TM, 2, true, NT>), grid, block, lds, g_stream, g); \
   else hipLaunchKernelGGL((dwpw_fused_kernel<WB, RR, 1, NW, TM, 4, true, NT>), grid, block, lds, g_stream, g);
   // Stage-2 blocks of 64 pixels x 32 channels instead of 32 x 64: each weight fragment then goes to one wave of the tile,
-  // not to two.
+  // not to two.  Chains of width 8 take it (part of what brought five blocks of 8x8x256 from 48 to 36 us, see
+  // dwpw_fused.h).  Width 4 makes no difference (five blocks of 4x4x256 28.3 / 28.3 us, two of
+  // 4x4x64 8.6 / 8.6).  Single blocks, which do not take it, would gain at widths 8 and 16 where a tile is 64 pixels (32 x 64 /
+  // 64 x 32, batch 256: 16x16x256 33.3 / 23.2 us, 16x16x128 14.3 / 12.6, 8x8x256 11.0 / 9.3, 16x16x128 -> 256 stride 2 8.8 / 8.0)
+  // and lose nowhere measured.
   const bool wide_px = g.BM % 64 == 0 && C >= 64;
   if (n_blocks > 1) {
     // (stride 1 only; the widest planes never fit the LDS of a chained launch)

@@ -186,7 +186,7 @@ void igemm_kernel(ConvGeom g, EpiArgs e)
   __shared__ __attribute__((aligned(16))) uint8_t As[NBUF][BM * IGEMM_BK];
   __shared__ __attribute__((aligned(16))) int8_t Ws[NBUF][BN * IGEMM_BK];
   __shared__ int wsum[BN];
-  // per-channel constants of the tile, fetched while the first K slice is on its way
+  // per-channel constants of the tile, fetched by the first wave ahead of its first K slice
   __shared__ int cbias[BN];
   __shared__ bn_t ck_[MODE == EPI_BN ? BN : 1], cl_[MODE == EPI_BN ? BN : 1];
 

@@ -12,7 +12,9 @@
 // activation fragments (64 rows x 64 bytes, shared by all workgroups and therefore
 // cache resident) of four K slices at a time straight from global memory in the
 // MFMA operand layout - twenty loads in flight, no staging - and the partial sums
-// of the K parts meet in LDS at the end.
+// of the K parts meet in LDS at the end.  What bounds 1024 -> 4096 at 64 rows (4.5 MB in 6 us, 0.7 us at a copy's rate) is
+// two dependent round trips to memory, operands and then bias, k and lambda in the epilogue, and an epilogue of all 64 rows
+// by one wave of the four.
 //
 // Arithmetic as in igemm.h: activations as a ^ 0x80 with bias + 128 * sum_k w
 // added back.

@@ -8,7 +8,9 @@
 // shifted into place).  Channels: blocks of up to 256, zero weights past the last one; a step's bytes are gathered in a
 // per-wave LDS tile and written in 16-byte pieces, the last piece of a pixel being its last 16 bytes.
 //
-// Bound: HBM (K + N bytes per pixel).  Measured, whole calls, against the tiled kernel whose operands were gathered byte
+// Bound: not HBM alone.  The three layers below move their bytes (K + N per pixel) at 2.4, 3.7 and 2.7 TB/s where a copy reaches
+// 6.2; LDS is busy half of the time (weight fragments, the output tile; a fifth of that bank conflicts) and waves wait 38 to
+// 52 % of theirs.  Measured, whole calls, against the tiled kernel whose operands were gathered byte
 // by byte: 19x28 120 -> 424 batch 234 267 -> 26 us (68 MB); 56x23 304 -> 100 batch 234 100 -> 35 (122 MB); 63x26 9 -> 256
 // batch 92 55 -> 14; 24x28 367 -> 176 batch 14 30 -> 13; 25x11 64 -> 136 batch 152 21 -> 7.0.
 #pragma once
