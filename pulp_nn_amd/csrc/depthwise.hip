@@ -73,9 +73,11 @@ void depthwise_common(const char *fn, const uint8_t *in, const int8_t *bias, uin
   }
   // Layers that fill the machine with one workgroup per image and 64 channels (two per compute unit): the plane
   // streamed through LDS, 8 rows of it per request.  Up to 14 groups of 4 output columns, 64 KiB of LDS.  A chunk
-  // costs a barrier and a round trip to memory however few rows it holds, so at stride 1 (where the band kernel is
-  // within 3 %) only planes of whole chunks take this kernel: 56 rows do, the 58 pre-padded rows of
-  // pulp_nn_depthwise_3x3_s1 run 7 % faster in bands.
+  // costs a barrier and a round trip to memory however few rows it holds, so at stride 1 only planes of whole chunks
+  // take this kernel: 56 rows do, the 58 pre-padded rows of pulp_nn_depthwise_3x3_s1 run faster in bands (57 / 51 us).
+  // Kernel times streamed / in bands, stride 1: 56x56x128 batch 256 52.1 / 54.2 us, 48x48x256 batch 128 36.2 / 40.1, 40x52x64
+  // batch 512 34.4 / 36.1; but 64 images of 56x56x512 54.6 / 54.3, and 24x40x128 batch 256 (three chunks) 21.0 / 16.2: a line
+  // at more chunks that this rule does not draw.
   const int stream_csd = (2 * DWS_ROWS * (W / 4)) | 1;
   const size_t stream_lds = 4 * ((size_t)DW_CG * stream_csd + 8 * (size_t)(Wo / 4));
   const bool stream = lin && Wo / 4 <= 16 - DWS_LOADERS && stream_lds <= 64 * 1024 && DWS_ROWS * W <= 1024 &&
