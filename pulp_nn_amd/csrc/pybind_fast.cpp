@@ -560,7 +560,31 @@ bool is_scalar(PyObject *v)
   return !PyObject_HasAttrString(v, "data_ptr");  // (numpy's scalars, and no tensor)
 }
 
-// Plan(nn, batch, [(entry point, arguments), ...], input, [(dict, which), ...]): `input` is the object that stands
+bool guard_dict(Plan *pl, PyObject *dict, PyObject *which)
+{
+  PyObject *key, *value;
+  if (!PyDict_Check(dict) || (which != Py_None && !PyAnySet_Check(which) && !PyTuple_Check(which))) {
+    PyErr_SetString(PyExc_TypeError, "a plan is made from dictionaries, and keys in a tuple, a set or None");
+    return false;
+  }
+  if (PyTuple_Check(which)) {
+    for (Py_ssize_t j = 0; j < PyTuple_GET_SIZE(which); j++)
+      if (!add_guard(pl, dict, PyTuple_GET_ITEM(which, j), PyDict_GetItem(dict, PyTuple_GET_ITEM(which, j)))) return false;
+    return true;
+  }
+  for (Py_ssize_t pos = 0; PyDict_Next(dict, &pos, &key, &value);) {
+    if (!add_guard(pl, dict, key, value)) return false;
+    if (which == Py_None || is_scalar(value)) continue;
+    const int object = PySet_Contains(which, key);
+    if (!object) PyErr_Format(PyExc_TypeError, "%R is a %.100s, which may change in place", key, Py_TYPE(value)->tp_name);
+    if (object != 1) return false;
+  }
+  Py_INCREF(dict);
+  pl->wholes->push_back(Whole{dict, PyDict_Size(dict)});
+  return true;
+}
+
+// Plan(nn, batch, [(entry point, arguments), ...], input, [(dict or list of them, which), ...]): `input` is the object that stands
 // for the chain's input in the arguments.  The chain entry point's arguments are (x, out, dim_x, dim_y, ch, [block, ...]).  The
 // pairs name the entries the calls were made from, as a tuple of keys, None (all of the dictionary's, and that there are no
 // others) or a set (the same; the values of other keys than these have to be numbers, texts, tuples or lists, not arrays, which
@@ -583,28 +607,16 @@ int plan_init(PyObject *self, PyObject *args, PyObject *)
   pl->guards = new std::vector<Guard>();
   pl->wholes = new std::vector<Whole>();
   pl->calls->reserve((size_t)PyList_GET_SIZE(list));
-  pl->guards->reserve(16 * (size_t)PyList_GET_SIZE(from));
+  pl->guards->reserve(32 * (size_t)PyList_GET_SIZE(list));
   for (Py_ssize_t i = 0; i < PyList_GET_SIZE(from); i++) {
-    PyObject *dict, *keys, *key, *value;
-    if (!PyArg_ParseTuple(PyList_GET_ITEM(from, i), "O!O", &PyDict_Type, &dict, &keys)) return -1;
-    if (keys == Py_None || PyAnySet_Check(keys)) {
-      for (Py_ssize_t pos = 0; PyDict_Next(dict, &pos, &key, &value);) {
-        if (!add_guard(pl, dict, key, value)) return -1;
-        if (keys == Py_None || is_scalar(value)) continue;
-        const int object = PySet_Contains(keys, key);
-        if (!object) PyErr_Format(PyExc_TypeError, "%R is a %.100s, which may change in place", key, Py_TYPE(value)->tp_name);
-        if (object != 1) return -1;
-      }
-      Py_INCREF(dict);
-      pl->wholes->push_back(Whole{dict, PyDict_Size(dict)});
+    PyObject *of, *which;
+    if (!PyArg_ParseTuple(PyList_GET_ITEM(from, i), "OO", &of, &which)) return -1;
+    if (!PyList_Check(of)) {
+      if (!guard_dict(pl, of, which)) return -1;
       continue;
     }
-    if (!PyTuple_Check(keys)) {
-      PyErr_SetString(PyExc_TypeError, "the keys are a tuple, a set or None");
-      return -1;
-    }
-    for (Py_ssize_t j = 0; j < PyTuple_GET_SIZE(keys); j++)
-      if (!add_guard(pl, dict, PyTuple_GET_ITEM(keys, j), PyDict_GetItem(dict, PyTuple_GET_ITEM(keys, j)))) return -1;
+    for (Py_ssize_t j = 0; j < PyList_GET_SIZE(of); j++)
+      if (!guard_dict(pl, PyList_GET_ITEM(of, j), which)) return -1;
   }
   for (Py_ssize_t i = 0; i < PyList_GET_SIZE(list); i++) {
     const char *name;

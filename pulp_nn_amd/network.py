@@ -230,9 +230,9 @@ class Runner:
 
     def _lay_out_plan(self, rec, out):
         """The calls of a walk and the entries they were made from."""
-        made_from = [(L, _ARRAYS) for L in self.layers] + [(d, None) for d in (*self.params, self.act, self.chw, self.shapes)]
         try:
-            plan = api._fast.Plan(self.nn, self.batch, rec.calls, rec.input, made_from)
+            plan = api._fast.Plan(self.nn, self.batch, rec.calls, rec.input,
+                                  [(self.layers, _ARRAYS), (self.params, None), ([self.act, self.chw, self.shapes], None)])
         except Exception:   # (an entry that may change in place without a trace, for one: no plan, the calls are made)
             return self._forget(plannable=False)
         self._plan = (self._choices(), self._objects(), plan, out, self.launches, rec.calls_at)
@@ -243,13 +243,15 @@ class Runner:
         tensors = {"input": x, **{L["name"]: self.act[L["name"]] for L in self.layers[:first]}}
         out = x
         self.launches = launches
-        recorded, readers = nn is not self.nn, self._reader_counts()
+        recorded, readers = nn is not self.nn, None
         i = first
         while i < len(self.layers):
             if recorded:
                 nn.at = (i, self.launches)
             L = self.layers[i]
             block = L["op"] == "depthwise"
+            if block and readers is None:
+                readers = self._reader_counts()
             n = self._chain_length(i, readers) if block and self.chain_blocks else 0
             if n >= 2 and self._queue_chain(i, n, tensors, nn):
                 last = self.layers[i + 2 * n - 1]["name"]
