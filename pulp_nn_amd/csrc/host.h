@@ -13,6 +13,7 @@
 #include <mutex>
 
 #include "conv_band_geom.h"
+#include "dw_hwc_geom.h"
 #include "dw_mfma_geom.h"
 #include "requant.h"
 
@@ -79,6 +80,7 @@ void linear_common(const char *fn, int mode, const uint8_t *in, const int8_t *bi
 bool launch_conv_band(int mode, const ConvLayer &L, const EpiArgs &e, int cus, hipStream_t s);
 bool launch_pw_any(int mode, const uint8_t *in, const int8_t *w, const int8_t *bias, uint8_t *out, long long M, int N, int K,
                    const EpiArgs &e, int cus, hipStream_t s);
+bool launch_dw_hwc(int mode, const DwLayer &L, const EpiArgs &e, int cus, hipStream_t s);
 bool launch_dw_mfma(int mode, const DwLayer &L, const EpiArgs &e, int cus, hipStream_t s);
 
 #pragma GCC visibility pop
