@@ -25,12 +25,74 @@
 #include "memops.h"
 #include "requant.h"
 
+// The forms of kk * acc + ll, shift, saturation: with the 24-bit multiplier (|acc| < 2^23 and kk of 24 bits, no narrowing), with the
+// 32-bit one, the same with the reference's narrowing to int16_t behind the shift (multiplier branch, shifts below 16), and in
+// the 64-bit build batch-norm with kk of 32 bits and with any kk.
+enum { DWH_FAST = 0, DWH_MUL32 = 1, DWH_NARROW = 2, DWH_BN64_SMALL = 3, DWH_BN64 = 4 };
+// k_small: all kk fit 24 (64-bit build: 32) bits; acc24: |acc| < 2^23
+__device__ __forceinline__ int dwh_form(int mode, int shift, bool k_small, bool acc24)
+{
+#if PULPNN_BN_BITS == 64
+  if (mode == EPI_BN) return k_small ? DWH_BN64_SMALL : DWH_BN64;
+#else
+  if (mode == EPI_BN) return k_small && acc24 ? DWH_FAST : DWH_MUL32;
+#endif
+  if (mode == EPI_MULT && shift < 16) return DWH_NARROW;
+  return acc24 ? DWH_FAST : DWH_MUL32;
+}
+// f(std::integral_constant<int, form>)
+template <class F>
+__device__ __forceinline__ void dwh_with_form(int form, F f)
+{
+  if (form == DWH_FAST) f(std::integral_constant<int, DWH_FAST>{});
+#if PULPNN_BN_BITS == 64
+  else if (form == DWH_BN64_SMALL) f(std::integral_constant<int, DWH_BN64_SMALL>{});
+  else if (form == DWH_BN64) f(std::integral_constant<int, DWH_BN64>{});
+#endif
+  else if (form == DWH_MUL32) f(std::integral_constant<int, DWH_MUL32>{});
+  else f(std::integral_constant<int, DWH_NARROW>{});
+}
+
+// four requantised bytes (four consecutive channels of one pixel)
+template <int FORM>
+__device__ __forceinline__ unsigned dwh_requant(const v4i &acc, const bn_t (&kk)[4], const bn_t (&ll)[4], int shift)
+{
+  int v[4], sh = shift;
+#pragma unroll
+  for (int r = 0; r < 4; r++) {
+    if constexpr (FORM == DWH_FAST) {
+      v[r] = __mul24(acc[r], (int)kk[r]) + (int)ll[r];
+    } else if constexpr (FORM == DWH_MUL32 || FORM == DWH_NARROW) {
+      v[r] = (int)((unsigned)acc[r] * (unsigned)kk[r] + (unsigned)ll[r]);
+      if (FORM == DWH_NARROW) v[r] = (int)(short)(v[r] >> shift);
+    } else if constexpr (FORM == DWH_BN64_SMALL) {
+      const long long x = (long long)(int)kk[r] * (long long)acc[r] + (long long)ll[r];
+      v[r] = shift >= 32 ? (int)(x >> 32) : (int)__builtin_amdgcn_alignbit((unsigned)(x >> 32), (unsigned)x, shift);
+    } else {
+      const unsigned long long x = (unsigned long long)kk[r] * (unsigned long long)(long long)acc[r] + (unsigned long long)ll[r];
+      v[r] = (int)(unsigned)(unsigned long long)((long long)x >> shift);
+    }
+  }
+  if (FORM == DWH_NARROW || FORM == DWH_BN64) sh = 0;
+  if (FORM == DWH_BN64_SMALL) sh = shift >= 32 ? shift - 32 : 0;
+  return ashr_sat_pack4(v[0], v[1], v[2], v[3], sh);
+}
+
+// v[s] of lane (l16, lgrp): four bytes, channels 4 * lgrp .., of pixel 16 * s + l16.  Afterwards v[q] of lane (l16, lgrp) is channels 4 * q ..
+// of pixel 16 * lgrp + l16: sixteen contiguous bytes of pixel `lane`.
+__device__ __forceinline__ v4i dwh_pixels(const unsigned (&v)[4])
+{
+  const auto a = __builtin_amdgcn_permlane32_swap(v[0], v[2], false, false), b = __builtin_amdgcn_permlane32_swap(v[1], v[3], false, false);
+  const auto c = __builtin_amdgcn_permlane16_swap(a[0], b[0], false, false), d = __builtin_amdgcn_permlane16_swap(a[1], b[1], false, false);
+  return (v4i){(int)c[0], (int)c[1], (int)d[0], (int)d[1]};
+}
+
 // What a wave keeps per 16 * NT channels.
 template <int NT>
 struct DwhChannels {
   v4i A[NT][3];                 // weight operands, per filter row
   bn_t kk[NT][4], ll[NT][4];    // requantisation of channel 4 * NT * (lane / 16) + 4 * t + r: kk * acc + ll, then the shift
-  bool fast;                    // the 24-bit (64-bit build: 32 x 32) multiplier is exact and nothing is narrowed
+  int form;
 };
 
 // The raw parameters of the channels: requested early, turned into DwhChannels behind the first input.
@@ -102,43 +164,42 @@ __device__ __forceinline__ void dwh_channels(DwhChannels<NT> &c, const DwhParams
         c.ll[t][r] = (bn_t)(int)((unsigned)k * (unsigned)corr + (unsigned)p.l[t][r]);
     }
   }
-  c.fast = mode == EPI_BN ? (bool)__all(ks) : mode == EPI_MULT ? shift >= 16 : true;
+  c.form = dwh_form(mode, shift, (bool)__all(ks), true);  // |acc| <= 9 * 128 * 128
 }
 
-// four requantised bytes (four consecutive channels of one pixel); |acc| <= 9 * 128 * 128
-template <bool FAST>
-__device__ __forceinline__ unsigned dwh_requant(const v4i &acc, const bn_t (&kk)[4], const bn_t (&ll)[4], int mode, int shift)
+// Walks a strip of one tile of 16 channels down `rows` output rows: next() is the operand of the next input row (one more than needed
+// is asked for), put(bytes) takes four requantised channels of the next output row.
+template <int S, int FORM, class Next, class Put>
+__device__ __forceinline__ void dwh_walk(const DwhChannels<1> &c, int shift, int rows, Next next, Put put)
 {
-  int v[4], sh = shift;
-#if PULPNN_BN_BITS == 64
-  if (mode == EPI_BN) {
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-      if constexpr (FAST) {
-        const long long x = (long long)(int)kk[r] * (long long)acc[r] + (long long)ll[r];
-        v[r] = shift >= 32 ? (int)(x >> 32) : (int)__builtin_amdgcn_alignbit((unsigned)(x >> 32), (unsigned)x, shift);
-      } else {
-        const unsigned long long x = (unsigned long long)kk[r] * (unsigned long long)(long long)acc[r] + (unsigned long long)ll[r];
-        v[r] = (int)(unsigned)(unsigned long long)((long long)x >> shift);
+  const v4i zero = {0, 0, 0, 0};
+  // N: the output row that the last input row started; M (stride 1): the one before it
+  v4i M = zero, N, F, cur = next(), nxt = next();
+  N = __builtin_amdgcn_mfma_i32_16x16x64_i8(c.A[0][0], cur, zero, 0, 0, 0);
+  if constexpr (S == 1) {
+    cur = next();
+    M = __builtin_amdgcn_mfma_i32_16x16x64_i8(c.A[0][1], nxt, N, 0, 0, 0);
+    N = __builtin_amdgcn_mfma_i32_16x16x64_i8(c.A[0][0], nxt, zero, 0, 0, 0);
+  } else {
+    cur = next();
+  }
+  for (int r = 0; r < rows; r++) {
+    if constexpr (S == 1) {
+      F = __builtin_amdgcn_mfma_i32_16x16x64_i8(c.A[0][2], cur, M, 0, 0, 0);
+      M = __builtin_amdgcn_mfma_i32_16x16x64_i8(c.A[0][1], cur, N, 0, 0, 0);
+      N = __builtin_amdgcn_mfma_i32_16x16x64_i8(c.A[0][0], cur, zero, 0, 0, 0);
+      cur = next();
+    } else {
+      N = __builtin_amdgcn_mfma_i32_16x16x64_i8(c.A[0][1], nxt, N, 0, 0, 0);
+      F = __builtin_amdgcn_mfma_i32_16x16x64_i8(c.A[0][2], cur, N, 0, 0, 0);
+      N = __builtin_amdgcn_mfma_i32_16x16x64_i8(c.A[0][0], cur, zero, 0, 0, 0);
+      if (r + 1 < rows) {
+        nxt = next();
+        cur = next();
       }
     }
-    sh = FAST && shift >= 32 ? shift - 32 : 0;
-    return ashr_sat_pack4(v[0], v[1], v[2], v[3], sh);
+    put(dwh_requant<FORM>(F, c.kk[0], c.ll[0], shift));
   }
-#endif
-  if (FAST) {
-#pragma unroll
-    for (int r = 0; r < 4; r++) v[r] = __mul24(acc[r], (int)kk[r]) + (int)ll[r];
-  } else {
-#pragma unroll
-    for (int r = 0; r < 4; r++) v[r] = (int)((unsigned)acc[r] * (unsigned)kk[r] + (unsigned)ll[r]);
-    if (mode == EPI_MULT) {  // the reference's narrowing to int16_t
-#pragma unroll
-      for (int r = 0; r < 4; r++) v[r] = (int)(short)(v[r] >> shift);
-      sh = 0;
-    }
-  }
-  return ashr_sat_pack4(v[0], v[1], v[2], v[3], sh);
 }
 
 template <int W, int S>
@@ -147,8 +208,7 @@ __global__ __launch_bounds__(256, 2) void dw_hwc_kernel(DwhGeom g, EpiArgs e, in
   constexpr int NT = 64 / W, WO = W / S, XS = WO / 16;  // tiles of 16 channels, strips of 16 columns
   constexpr int PD = 4;                                 // input rows in flight
   constexpr int ROW = dwh_row_bytes<W>();
-  constexpr bool OUT_L = NT == 1;                       // output rows are put together in LDS
-  __shared__ __attribute__((aligned(16))) unsigned char rows_l[4][2 * ROW + (OUT_L ? 1024 : 0)];  // per wave: two input rows, 64 chunks of output
+  __shared__ __attribute__((aligned(16))) unsigned char rows_l[4][2 * ROW];  // per wave: two input rows
   const int lane = threadIdx.x & 63, l16 = lane & 15, lgrp = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int q8 = (int)gridDim.x >> 3, rem = (int)gridDim.x & 7, x8 = blockIdx.x & 7;  // a contiguous range per XCD
@@ -184,9 +244,7 @@ __global__ __launch_bounds__(256, 2) void dw_hwc_kernel(DwhGeom g, EpiArgs e, in
   for (int x = 0; x < XS; x++)
 #pragma unroll
     for (int j = 0; j < NT; j++) from[x][j] = lds + dwh_lds<W>((16 * x + l16) * S + min(lgrp, 2), j);
-  unsigned char *out_l = lds + 2 * ROW;
   const unsigned ooff = dwh_out_offset<W, S>(g, it, lane);
-  unsigned char *oput = out_l + 16 * l16 + 4 * lgrp;
   DwhChannels<NT> c;
   dwh_channels<NT>(c, p, mode, e.shift, lane);
 
@@ -202,8 +260,8 @@ __global__ __launch_bounds__(256, 2) void dw_hwc_kernel(DwhGeom g, EpiArgs e, in
   const v4i zero = {0, 0, 0, 0};
   // N: the output row that the last input row started; M (stride 1): the one before it
   v4i M[XS][NT], N[XS][NT], F[XS][NT];
-  auto walk = [&](auto fast) {
-    constexpr bool FAST = decltype(fast)::value;
+  auto walk = [&](auto form) {
+    constexpr int FORM = decltype(form)::value;
     auto row = [&](int slot, auto role_tag) {
       constexpr int ROLE = decltype(role_tag)::value;  // bits: the filter rows that this input row takes part in
 #pragma unroll
@@ -224,6 +282,9 @@ __global__ __launch_bounds__(256, 2) void dw_hwc_kernel(DwhGeom g, EpiArgs e, in
         }
       }
     };
+    // one tile: the 64 pixels of a row, or with stride 2 of two rows, change places between lanes so that one store writes their
+    // 1 KB in memory order, instead of four of 256 bytes in 4-byte pieces
+    unsigned v1[4];
     // u: which of the rows that are put together this is
     auto emit = [&](int r, int u) {
       typedef unsigned v4u __attribute__((ext_vector_type(4)));
@@ -232,9 +293,9 @@ __global__ __launch_bounds__(256, 2) void dw_hwc_kernel(DwhGeom g, EpiArgs e, in
       for (int x = 0; x < XS; x++) {
         vnt v;
 #pragma unroll
-        for (int t = 0; t < NT; t++) v[t] = dwh_requant<FAST>(F[x][t], c.kk[t], c.ll[t], mode, e.shift);
-        if constexpr (OUT_L) {
-          *(unsigned *)(oput + 512 * u + 256 * x) = v[0];
+        for (int t = 0; t < NT; t++) v[t] = dwh_requant<FORM>(F[x][t], c.kk[t], c.ll[t], e.shift);
+        if constexpr (NT == 1) {
+          v1[2 * u + x] = v[0];
         } else {
           const bool ok = dwh_out_ok<W, S>(it, r, lane);
           const int soff = ok ? (r * WO + 16 * x) * g.C : 0;
@@ -242,17 +303,12 @@ __global__ __launch_bounds__(256, 2) void dw_hwc_kernel(DwhGeom g, EpiArgs e, in
           else __builtin_amdgcn_raw_buffer_store_b128(v, rsrc_o, ok ? ooff : DWH_OOB, soff, 0);
         }
       }
-      // (the dwords a lane has of a pixel are 16 bytes apart from lane to lane: in LDS they become whole chunks in memory order,
-      // one store of 1 KB instead of four of 256 bytes in 4-byte pieces; two or four dwords a lane gain nothing by it)
-      if constexpr (OUT_L) {
+      if constexpr (NT == 1) {
         if (u == S - 1) {
-          __builtin_amdgcn_wave_barrier();
-          asm volatile("" ::: "memory");
-          const v4u v = *(const v4u *)(out_l + 16 * lane);
+          const v4i p = dwh_pixels(v1);
           const int r0 = r - u;
-          __builtin_amdgcn_raw_buffer_store_b128(v, rsrc_o, dwh_out_ok<W, S>(it, r0, lane) ? ooff : DWH_OOB, r0 < it.rows ? r0 * WO * g.C : 0, 0);
-          __builtin_amdgcn_wave_barrier();
-          asm volatile("" ::: "memory");
+          __builtin_amdgcn_raw_buffer_store_b128((v4u){(unsigned)p.x, (unsigned)p.y, (unsigned)p.z, (unsigned)p.w}, rsrc_o, dwh_out_ok<W, S>(it, r0, lane) ? ooff : DWH_OOB,
+                                                 r0 < it.rows ? r0 * WO * g.C : 0, 0);
         }
       }
     };
@@ -288,6 +344,5 @@ __global__ __launch_bounds__(256, 2) void dw_hwc_kernel(DwhGeom g, EpiArgs e, in
       }
     }
   };
-  if (c.fast) walk(std::true_type{});
-  else walk(std::false_type{});
+  dwh_with_form(c.form, walk);
 }

@@ -51,8 +51,7 @@ PULPNN_HD unsigned dwh_in_offset(const DwhGeom &g, const DwhItem &it, int lane)
   constexpr int NT = 64 / W;
   return ((it.b * (unsigned)g.H + (unsigned)(it.oy0 * S)) * W + (unsigned)(lane / NT)) * (unsigned)g.C + (unsigned)(it.c0 + 16 * (lane % NT));
 }
-// Output rows.  With one tile of 16 channels (W = 64) a row's bytes meet in LDS and a lane writes one of its 16-byte chunks, with
-// stride 2 one of the two rows'; otherwise a lane writes the 4 * NT channels of pixel l16 of strip x.  Offset in the output of
+// Output rows.  With one tile of 16 channels (W = 64) a lane writes one pixel of a row, with stride 2 of the two rows from r on; otherwise a lane writes the 4 * NT channels of pixel l16 of strip x.  Offset in the output of
 // what a lane writes of output row 0 (strip 0); row r is r * Wo * C further, strip x is 16 * x * C.
 template <int W, int S>
 PULPNN_HD unsigned dwh_out_offset(const DwhGeom &g, const DwhItem &it, int lane)

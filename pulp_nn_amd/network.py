@@ -18,7 +18,8 @@ produces the tensor called like the layer.  Activations are HWC uint8, batch out
                 as one launch (pulp_nn_hip_dw_pw_hwc) and the depthwise result is not
                 materialised: Runner(..., fuse_blocks=True) for every such pair, False for none,
                 "auto" (the default) where it is not slower: as Runner.tune() measured it on the
-                batch at hand, else for blocks whose output plane is 8 x 8 pixels
+                batch at hand, else for blocks whose output plane is 8 x 8 pixels, small blocks, and
+                blocks whose depthwise layer alone would need a layout change
   maxpool       kernel (kx,ky), strides, pads, out_hw      -> pulp_nn_maxpool
   avgpool       kernel, strides, pads, out_hw, lam, shift, add, requant -> pulp_nn_avgpool
   add           in = (a, b), m1, m2, shift                 -> pulp_nn_add
@@ -276,19 +277,28 @@ class Runner:
         L, N = self.layers[i], self.layers[i + 1]
         if L["op"] != "depthwise" or N["op"] != "pointwise" or N["in"] != L["name"]:
             return False
-        # "auto": only where the single launch is not slower than the two.  Runner.tune() times both forms of every
-        # such block on the batch at hand and records the faster one in block_choice.  Without that measurement the
-        # rule is the shape of the fused kernel's work: it pays where an image's output plane is 8 x 8 pixels, so
-        # that one workgroup takes whole images and each of its eight waves one item of the depthwise stage (on
-        # MI355X at batch 256: 11.2 us against 5.9 + 6.4 for 16-pixel planes at stride 2, 11.8 against 5.4 + 7.1
-        # for 8-pixel planes at stride 1); larger output planes split an image over workgroups that each run the
-        # whole load -> depthwise -> MFMA -> store chain, smaller ones leave waves without an item.
+        # "auto": where the single launch is not slower than the two.  Runner.tune() times both forms of every such block on
+        # the batch at hand and records the faster one in block_choice.  Without that measurement the rule is
+        #   * output planes of 8 x 8 pixels, a whole image per workgroup (two launches / one at batch 256: 16x16x128 -> 256 at
+        #     stride 2 10.2 / 8.1 us, 8x8x256 11.6 / 8.8);
+        #   * blocks whose depthwise result is small, so that launches and round trips to memory are most of the time: less than
+        #     1 MB (16x16x128 at batch 16 9.1 / 5.7 us, 4x4x512 at batch 64 9.5 / 9.3), at most 4 MB for planes of 32 x 32
+        #     pixels and more (64x64x16 at batch 64 11.5 / 9.7, at batch 256 20.2 / 24.3; 32x32x64 at batch 64 10.3 / 7.8, at
+        #     batch 256 16.9 / 19.1).  Smaller planes would gain up to some 4 MB too (16x16x128 at batch 128 13.0 / 8.1); the line
+        #     is lower there because a fused pair's depthwise result is not materialised, and tables are read at such batches;
+        #   * blocks whose depthwise layer alone has no kernel for HWC input and would be two launches itself (64x64x16 at batch
+        #     255 39.0 / 24.5 us, three launches / one).
         if policy and self.fuse_blocks == "auto":
             if i in self.block_choice:
                 if not self.block_choice[i]:
                     return False
-            elif tuple(self.shapes[L["name"]][:2]) != (8, 8):
-                return False
+            else:
+                Ho, Wo, Cc = self.shapes[L["name"]]
+                size = self.batch * Ho * Wo * Cc
+                small = size < 2 ** 20 or (Ho * Wo >= 1024 and size <= 2 ** 22)
+                relaid = Cc % 64 != 0 and (self.shapes[L["in"]][1] <= 8 or (self.batch * Cc) % 64 != 0)
+                if (Ho, Wo) != (8, 8) and not small and not relaid:
+                    return False
         sx, sy = L["strides"]
         if L["w"].shape[1:3] != (3, 3) or tuple(L["pads"]) != (1, 1, 1, 1) or sx != sy:
             return False

@@ -1,0 +1,102 @@
+// Walks the tiles of dwpw_kernel and dwpw_chain_kernel on the host, with the kernels' own arithmetic (csrc/dwpw_geom.h): shapes that the
+// entry points take but no tile fits, loads of another byte than the one meant, LDS places outside their range, activations that are
+// left out or written twice, output pixels left out.
+// Blocks on stdin, one a line: B C H W Co S chained bn_bytes cus.  One line out per block: "ok WAVES", "no" (refused) or what is wrong.
+#include <stdio.h>
+#include <stdlib.h>
+
+#include <string>
+#include <vector>
+
+#include "../../pulp_nn_amd/csrc/dwpw_geom.h"
+
+template <int W, int S>
+static std::string check(int B, int C, int H, int Co, int chained, int bn_bytes, int cus)
+{
+  constexpr int WO = W / S;
+  const int Ho = (H - 1) / S + 1;
+  if (dwpw_refusal(B, C, W, Ho, WO, Co, S, chained ? 2 : 1, cus, bn_bytes)) return "no";
+  DwPwTile g;
+  if (!dwpw_shape(B, C, H, W, Ho, Co, S, chained, cus, bn_bytes, &g)) return "taken, but no tile fits";
+  const int act_bytes = (64 << g.lpxb) * C, x_bytes = g.par_off - g.x_off, BM = 64 << g.lpxb;
+  if (g.lds > 160 * 1024 || g.x_off < act_bytes || g.CS * g.slabs != C || (g.CS % 64 && C >= 64) || g.TR * WO > BM || g.TR % g.R || (g.whole && Ho % g.R) ||
+      (g.waves != 4 && g.waves != 8 && g.waves != 16) || (g.kp == 1) != (C <= 64) || g.w_off + dwpw_par(C, bn_bytes, true).bytes > g.lds + dwpw_par(C, bn_bytes, true).bytes ||
+      (g.cf_per << g.lsplit) * 16 < Co || (chained && (g.lsplit || g.slabs != 1)))
+    return "shape";
+  const int cgs = g.CS / 16, ids[] = {0, g.tiles / 2, g.tiles - 1};
+  long long outputs = 0;
+  for (int t = 0; t < g.tiles; t++) outputs += dwpw_place<WO>(g, (unsigned)t).live;
+  if (outputs != (long long)B * Ho * WO) return "output pixels: " + std::to_string(outputs);
+  for (const int id : ids) {
+    const DwPwPlace at = dwpw_place<WO>(g, (unsigned)id);
+    // input: every place of a pixel once, from the right byte
+    std::vector<int> src(x_bytes / 16, -2);  // image pixel behind a 16-byte place: -1 padding
+    const int chunks = dwpw_chunks<W>(g);
+    for (int c = 0; c < chunks + 4096; c++) {
+      const DwPwChunk k = dwpw_chunk<W, S>(g, at, c);
+      if (c >= chunks) {
+        if (k.off >= 0) return "load past the last chunk";
+        continue;
+      }
+      if (k.lds < 0 || k.lds + 16 > x_bytes || k.lds % 16) return "input place";
+      if (src[k.lds / 16] != -2) return "input place twice";
+      src[k.lds / 16] = -1;
+      if (k.off >= 0) {
+        if (k.off + 16 > dwpw_rows_in(g) * W * C) return "input offset";
+        const long long row = dwpw_first_row<S>(g, at) + k.off / C / W;
+        if (row < 0 || row >= (long long)B * H) return "row outside the input";
+        if (k.off % C != 16 * ((k.lds / 16) % (g.pitch / 16))) return "channel";
+        src[k.lds / 16] = (int)(row * W + k.off / C % W);
+      }
+    }
+    // depthwise stage: every activation of a real pixel once, from the rows and columns around it
+    std::vector<unsigned char> act(act_bytes / 16);
+    for (int it = 0; it < cgs * g.nst; it++) {
+      const int st = (int)fastdiv((unsigned)it, g.d_n), cg = it - st * cgs;
+      for (int l16 = 0; l16 < 16; l16++)
+        for (int kx = 0; kx < 3; kx++) {
+          const DwPwLane n = dwpw_lane<W, S>(g, st, l16, kx);
+          if (n.x < 0 || n.x + ((g.R - 1) * S + 3) * (W + 2) * g.pitch + 16 * cg + 16 > x_bytes) return "a strip's rows";  // (one row past the last)
+          for (int r = 0; r < g.R; r++) {
+            const int px = n.px + r * WO;
+            if (px < 0 || px >= BM) return "pixel";
+            const int p = dwpw_act(g, px, 16 * cg);
+            if (p < 0 || p + 16 > act_bytes || p % 16) return "activation place";
+            if (n.live && kx == 0 && act[p / 16]++) return "activation twice";
+            if (!n.live || px >= at.live) continue;
+            const int row = px / WO, y = g.whole ? row % Ho : at.oy0 + row, b = at.b0 + (g.whole ? row / Ho : 0), x = px % WO;
+            for (int fy = 0; fy < 3; fy++) {
+              const int iy = y * S - 1 + fy, ix = x * S - 1 + kx;
+              const int want = iy >= 0 && iy < H && ix >= 0 && ix < W ? (b * H + iy) * W + ix : -1;
+              if (src[(n.x + (r * S + fy) * (W + 2) * g.pitch + 16 * cg) / 16] != want) return "operand of another pixel";
+            }
+          }
+        }
+    }
+    for (int px = 0; px < g.TR * WO; px++)
+      for (int cg = 0; cg < cgs; cg++)
+        if (!act[dwpw_act(g, px, 16 * cg) / 16]) return "activation left out";
+    if (chained)
+      for (int px = 0; px < at.live; px++) {
+        const int p = dwpw_next_x<W>(g, px);
+        if (p < 0 || p + C > x_bytes || src[p / 16] != (at.b0 * H) * W + px) return "next block's input";
+      }
+  }
+  return "ok " + std::to_string(g.waves);
+}
+
+int main()
+{
+  char line[256];
+  while (fgets(line, sizeof line, stdin)) {
+    int B, C, H, W, Co, S, chained, bn, cus;
+    if (sscanf(line, "%d %d %d %d %d %d %d %d %d", &B, &C, &H, &W, &Co, &S, &chained, &bn, &cus) != 9) return 1;
+    std::string said = "no";
+#define AT(w)                                                                 \
+  if (W == w && S == 1) said = check<w, 1>(B, C, H, Co, chained, bn, cus);    \
+  if (W == w && S == 2 && w > 4) said = check<w, w == 4 ? 1 : 2>(B, C, H, Co, chained, bn, cus);
+    AT(64) AT(32) AT(16) AT(8) AT(4)
+    puts(said.c_str());
+    fflush(stdout);
+  }
+}

@@ -1,0 +1,30 @@
+"""The tiles of the depthwise + pointwise kernels walked on the host (tests/host/dwpw_walk.cpp) for shapes of the whole range that the entry
+points take: a tile for each of them, every operand the right pixel's, every activation written once."""
+import os
+import random
+import subprocess
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+
+def test_tiles_on_the_host(tmp_path):
+    exe = str(tmp_path / "dwpw_walk")
+    subprocess.run(["g++", "-O2", "-std=c++17", "-fsanitize=undefined", "-fno-sanitize-recover=all",
+                    os.path.join(HERE, "host", "dwpw_walk.cpp"), "-o", exe], check=True)
+    r, blocks = random.Random(11), []
+    for W in (64, 32, 16, 8, 4):
+        for S in (1, 2):
+            for C in [16, 32] + [64 * n for n in (1, 2, 3, 4, 5, 6, 8, 11, 16)]:
+                for chained in ((0, 1, 1) if S == 1 else (0,)):
+                    for _ in range(3):
+                        H = r.choice([4, 8, 8, 16, 16, 24, 32, 40, 64]) - (r.randint(0, 1) if S == 2 else 0)
+                        Co = C if chained else 16 * r.choice([1, 2, 3, 5, 8, 16, 32, 64, 100])
+                        blocks.append((r.choice([1, 2, 4, 7, 60, 64, 256]), C, H, W, Co, S, chained, r.choice([4, 8]), r.choice([64, 256])))
+    res = subprocess.run([exe], input="\n".join(" ".join(map(str, b)) for b in blocks), stdout=subprocess.PIPE, stderr=subprocess.PIPE, text=True,
+                         timeout=110)
+    said = res.stdout.split("\n")[:-1]
+    for b, s in zip(blocks, said):
+        assert s.startswith("ok") or s == "no", "block %s: %s" % (b, s)
+    assert res.returncode == 0, res.stderr
+    taken = [b for b, s in zip(blocks, said) if s != "no"]
+    assert len(said) == len(blocks) and len(taken) > 200 and sum(b[6] for b in taken) > 30
