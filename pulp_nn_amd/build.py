@@ -24,7 +24,7 @@ def lib_path(bn_bits):
 
 
 # translation units of the library: the host layer with most kernels, and kernel families compiled beside it
-UNITS = ("conv", "conv_band", "pw_any", "dwpw", "depthwise", "dw_hwc", "dw_mfma", "pulp_nn_hip")
+UNITS = ("conv", "conv_band", "conv_rows", "pw_any", "dwpw", "depthwise", "dw_hwc", "dw_mfma", "pulp_nn_hip")
 
 
 def _run(cmd, what, verbose):

@@ -186,36 +186,19 @@ void launch_igemm(int mode, ConvGeom &g, const EpiArgs &e, hipStream_t s)
   else launch_igemm_tile<GATHER_BYTES>(mode, g, e, s);
 }
 
-// Direct (vector ALU) convolution for small filters and at most 32 channels.  rows: the filter
-// has at most 3 rows of at most 12 bytes and is gathered a row at a time (smallk_rows_kernel);
-// otherwise it is at most 32 bytes long and gathered byte by byte (smallk_conv_kernel).
+// Direct (vector ALU) convolution for filters of at most 32 bytes and at most 32 channels, gathered byte by byte.
 template <int NCH>
-void launch_smallk(int mode, bool rows, ConvGeom &g, const EpiArgs &e, hipStream_t s)
+void launch_smallk(int mode, ConvGeom &g, const EpiArgs &e, hipStream_t s)
 {
   g.vec_store = (g.N == NCH) && aligned(g.out, 16);
   g.nt = (long long)g.M * g.N >= PULPNN_NT_BYTES;
   dim3 grid((unsigned)((g.M + 255) / 256)), block(256);
-  if (rows) {
-    // runs of 256 pixels per workgroup: as many as leave every compute unit its eight workgroups
-    const long long runs = (g.M + 255) / 256;
-    g.tiles_n = (int)std::max<long long>(1, std::min<long long>(8, runs / (8ll * num_cus())));
-    g.d_howo = fastdiv_make((unsigned)g.HoWo);
-    g.d_wo = fastdiv_make((unsigned)g.Wo);
-    grid = dim3((unsigned)((runs + g.tiles_n - 1) / g.tiles_n));
-    switch (mode) {
-      case EPI_BN: hipLaunchKernelGGL((smallk_rows_kernel<NCH, EPI_BN>), grid, block, 0, s, g, e); break;
-      case EPI_MULT: hipLaunchKernelGGL((smallk_rows_kernel<NCH, EPI_MULT>), grid, block, 0, s, g, e); break;
-      default: hipLaunchKernelGGL((smallk_rows_kernel<NCH, EPI_RAW>), grid, block, 0, s, g, e); break;
-    }
-    return;
-  }
   switch (mode) {
     case EPI_BN: hipLaunchKernelGGL((smallk_conv_kernel<NCH, EPI_BN>), grid, block, 0, s, g, e); break;
     case EPI_MULT: hipLaunchKernelGGL((smallk_conv_kernel<NCH, EPI_MULT>), grid, block, 0, s, g, e); break;
     default: hipLaunchKernelGGL((smallk_conv_kernel<NCH, EPI_RAW>), grid, block, 0, s, g, e); break;
   }
 }
-
 
 template <bool ANY>
 void launch_skinny(int mode, const SkinnyGeom &g, const EpiArgs &e, dim3 grid, hipStream_t s)
@@ -370,15 +353,15 @@ void conv_common(const char *fn, bool pointwise, const uint8_t *in, const int8_t
   g.sx = sx;
   g.sy = sy;
   g.in_img = (long long)dim_in_x * dim_in_y * ch_in;
-  // a filter row is kx * ch_in contiguous input bytes: three aligned dwords cover it if it is at
-  // most 9 bytes long, or 12 with rows that start on a dword
-  const int row_bytes = (int)kx * ch_in;
-  const long long batch = (g.M + g.HoWo - 1) / g.HoWo;
-  const bool rows = ky <= 3 && (row_bytes <= 9 || (row_bytes <= 12 && ch_in % 4 == 0)) && aligned(g.in, 4) &&
-                    batch * g.in_img < 0x7ffffff0LL;
-  if ((rows || g.K <= 4 * SMALLK_KD) && g.N <= 32) {
-    if (g.N <= 16) launch_smallk<16>(mode, rows, g, e, g_stream);
-    else launch_smallk<32>(mode, rows, g, e, g_stream);
+  // Filters of up to four rows of up to 16 bytes: a row is one 16-byte slot of K on the matrix cores, whatever the geometry.  Small pointwise
+  // layers of 16 channels leave three slots of four empty; up to 32 output channels that is still the faster one (64x64 16 -> 32 batch 1
+  // 6.9 us a pixel per lane, 3.6 here), beyond them the tiled kernel is (20x20 16 -> 256 batch 3 3.9 us, 4.4 here; batch 20 4.1 / 5.0).
+  const ConvLayer L = {in, w, bias, out, (int)g_batch, dim_in_y, dim_in_x, ch_in, dim_out_y, dim_out_x, ch_out, kx, ky, pt, pl, sx, sy};
+  const bool tiled16 = kx == 1 && ky == 1 && ch_in == 16 && ch_out > 32 && aligned(in, 16) && aligned(w, 16);
+  if (!tiled16 && launch_conv_rows(mode, L, e, num_cus(), g_stream)) return check_launch(fn);
+  if (g.K <= 4 * SMALLK_KD && g.N <= 32) {
+    if (g.N <= 16) launch_smallk<16>(mode, g, e, g_stream);
+    else launch_smallk<32>(mode, g, e, g_stream);
   } else {
     // Channel counts that are not whole 16-byte chunks: from a band of the input in LDS (conv_band.h).  So are layers of
     // few output channels, which leave most of the tiled kernel's 128 x 64 tile empty and its many waves waiting for each
@@ -392,7 +375,6 @@ void conv_common(const char *fn, bool pointwise, const uint8_t *in, const int8_t
     const bool whole16 = ch_in % 16 == 0 && aligned(in, 16) && aligned(w, 16);
     const bool few = ch_in == 16 || ch_in == 32 ? false : ch_in % 64 == 0 ? g.N <= 32 : g.N <= 64;
     if (!whole16 || few) {
-      const ConvLayer L = {in, w, bias, out, (int)g_batch, dim_in_y, dim_in_x, ch_in, dim_out_y, dim_out_x, ch_out, kx, ky, pt, pl, sx, sy};
       if (launch_conv_band(mode, L, e, num_cus(), g_stream)) return check_launch(fn);
     }
     launch_igemm(mode, g, e, g_stream);

@@ -77,6 +77,7 @@ void linear_common(const char *fn, int mode, const uint8_t *in, const int8_t *bi
 
 // ---- kernels with a launcher of their own: false, with nothing queued, for a geometry the kernel does not take ---
 
+bool launch_conv_rows(int mode, const ConvLayer &L, const EpiArgs &e, int cus, hipStream_t s);
 bool launch_conv_band(int mode, const ConvLayer &L, const EpiArgs &e, int cus, hipStream_t s);
 bool launch_pw_any(int mode, const uint8_t *in, const int8_t *w, const int8_t *bias, uint8_t *out, long long M, int N, int K,
                    const EpiArgs &e, int cus, hipStream_t s);
