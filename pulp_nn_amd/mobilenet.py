@@ -103,7 +103,8 @@ class Runner(network.Runner):
     kernel for it; otherwise, and with fused=False, the chain is the reference's:
     pulp_nn_hip_hwc_to_chw + pulp_nn_depthwise_generic.  fuse_blocks: a depthwise layer and the
     pointwise layer behind it run as one launch (pulp_nn_hip_dw_pw_hwc); the depthwise results are
-    then not materialised (self.activations holds stale buffers for them).  chain_blocks: the run of
+    then not materialised (self.activations holds stale buffers for them, except for pairs that the
+    default fuses because they are small).  chain_blocks: the run of
     five identical blocks on 8 x 8 x 256 is one launch (pulp_nn_hip_dw_pw_chain_hwc); only its last
     output is materialised."""
 
@@ -112,7 +113,11 @@ class Runner(network.Runner):
         super().__init__(nn, descriptor(net), (128, 128, 3), net["batch"], fused=fused, fuse_blocks=fuse_blocks,
                          chain_blocks=chain_blocks)
         self.logits = self.act["fc"].view(net["batch"], 1000)
-        self.activations = [self.act[L["name"]] for L in net["layers"]]
+
+    @property
+    def activations(self):
+        """The buffers of the layers in front of the classifier, in order (read through self.act)."""
+        return [self.act[L["name"]] for L in self.net["layers"]]
 
     def run(self, x):
         """x: device tensor B,128,128,3 uint8.  Returns the int32 logits tensor (B,1000)."""

@@ -19,7 +19,9 @@ produces the tensor called like the layer.  Activations are HWC uint8, batch out
                 materialised: Runner(..., fuse_blocks=True) for every such pair, False for none,
                 "auto" (the default) where it is not slower: as Runner.tune() measured it on the
                 batch at hand, else for blocks whose output plane is 8 x 8 pixels, small blocks, and
-                blocks whose depthwise layer alone would need a layout change
+                blocks whose depthwise layer alone would need a layout change.  The depthwise
+                results of the latter two can be had all the same: reading Runner.act computes them
+                for the run before, and the runs after it make the two launches
   maxpool       kernel (kx,ky), strides, pads, out_hw      -> pulp_nn_maxpool
   avgpool       kernel, strides, pads, out_hw, lam, shift, add, requant -> pulp_nn_avgpool
   add           in = (a, b), m1, m2, shift                 -> pulp_nn_add
@@ -32,6 +34,9 @@ shift (out_shift).  shift = None on a bn layer means "to be calibrated": Runner.
 sets it to floor(log2(max |acc * k|)) - 7 over the batch it is given, computed on the GPU
 (pulp_nn_hip_calib_conv / pulp_nn_hip_calib_depthwise), layer by layer along the chain.
 """
+import collections.abc
+import weakref
+
 import numpy as np
 
 from . import api
@@ -81,6 +86,61 @@ def infer_shapes(layers, input_shape):
     return shapes
 
 
+class _Activations(dict):
+    """Runner.act, {tensor name: buffer}: a tensor is handed out with the last run's values in it, also one that the run left
+    out by the rule for small blocks; a buffer that the caller puts in its place is written by the next run."""
+
+    def __init__(self, runner, buffers):
+        super().__init__(buffers)
+        self._runner = weakref.ref(runner)
+
+    def __getitem__(self, name):
+        runner = self._runner()
+        if runner is not None and name in self:
+            runner._hand_out(name)
+        return super().__getitem__(name)
+
+    def __setitem__(self, name, buffer):
+        runner = self._runner()
+        if runner is not None:
+            runner._ask(name)
+        super().__setitem__(name, buffer)
+
+    def update(self, *args, **kwargs):
+        for name, buffer in dict(*args, **kwargs).items():
+            self[name] = buffer
+
+    def __ior__(self, other):
+        self.update(other)
+        return self
+
+    def get(self, name, default=None):
+        return self[name] if name in self else default
+
+    def values(self):
+        return collections.abc.ValuesView(self)
+
+    def items(self):
+        return collections.abc.ItemsView(self)
+
+    def pop(self, name, *default):
+        if name in self:
+            self[name]
+        return super().pop(name, *default)
+
+    def setdefault(self, name, default=None):
+        return self[name] if name in self else super().setdefault(name, default)
+
+    def __iter__(self):   # (its own, so that dict(act) and {**act} read the entries through __getitem__ too)
+        return super().__iter__()
+
+    def copy(self):
+        return dict(self)
+
+    def __reduce__(self):
+        return dict, (dict(self),)
+
+
 class Runner:
     """Uploads the parameters once, owns the activation buffers and queues the chain.
 
@@ -114,11 +174,12 @@ class Runner:
             if L.get("k") is not None:
                 P["k"], P["lam"] = dev(L["k"], bn_np), dev(L["lam"], bn_np)
             self.params.append(P)
-        self.act = {}
+        act = {}
         for L in layers:
             H, W, Cc = self.shapes[L["name"]]
             dt = torch.int32 if L["op"] == "linear_out_32" else torch.uint8
-            self.act[L["name"]] = torch.empty((batch, H, W, Cc), dtype=dt, device="cuda")
+            act[L["name"]] = torch.empty((batch, H, W, Cc), dtype=dt, device="cuda")
+        self.act = _Activations(self, act)
         self.chw = {}
         for L in layers:
             if L["op"] == "depthwise":
@@ -131,6 +192,31 @@ class Runner:
         self._plan = None        # (choices, objects, plan, result tensor, launches, [(layer, launches) before a call])
         self._plannable = plannable
 
+    # -- buffers ----------------------------------------------------------------------------
+    _asked = frozenset()     # depthwise layers (indices) whose results the caller has asked for
+    _left_out = frozenset()  # ... whose results the last run left out because their blocks are small
+
+    def _buffer(self, name):
+        return dict.__getitem__(self.act, name)
+
+    def _ask(self, name):
+        """Runs to come write tensor `name`; its layer's index, for a depthwise layer."""
+        i = next((i for i, L in enumerate(self.layers) if L["name"] == name and L["op"] == "depthwise"), None)
+        if i is not None:
+            self._asked |= {i}
+        return i
+
+    def _hand_out(self, name):
+        """The caller is given the buffer of tensor `name`: what the last run did not write into it is computed now."""
+        i = self._ask(name)
+        if i in self._left_out:
+            src, batch = self.layers[i]["in"], self.nn.get_batch()
+            self.nn.set_batch(self.batch)
+            try:
+                self._queue(i, {src: self._buffer(src)})
+            finally:
+                self.nn.set_batch(batch)
+
     # -- one layer ------------------------------------------------------------------------
     def _requant_args(self, L, P):
         relu, bn = L.get("relu", 0), L.get("bn", 0)
@@ -140,7 +226,7 @@ class Runner:
 
     def _queue(self, i, tensors, nn=None):
         L, P, nn = self.layers[i], self.params[i], nn or self.nn
-        op, out = L["op"], self.act[L["name"]]
+        op, out = L["op"], self._buffer(L["name"])
         if op == "add":
             a, b = tensors[L["in"][0]], tensors[L["in"][1]]
             H, W, Cc = self.shapes[L["name"]]
@@ -215,7 +301,7 @@ class Runner:
                     self._plan = None
                     return self._walk(x, self.nn, *calls_at[done])
             self._plan = None
-        if not self._plannable or not self.layers or any(x is t for d in (self.act, self.chw) for t in d.values()):
+        if not self._plannable or not self.layers or any(x is t for d in (self.act, self.chw) for t in dict.values(d)):
             return self._walk(x, self.nn)
         rec = api._fast.Recorder(self.nn, x)
         out = self._walk(x, rec)
@@ -224,7 +310,7 @@ class Runner:
 
     def _choices(self):
         return (len(self.layers), len(self.params), self.batch, self.fused, self.fuse_blocks, self.chain_blocks, tuple(self.unfused),
-                tuple(self.unfused_blocks), tuple(self.unchained), tuple(self.block_choice.items()))
+                tuple(self.unfused_blocks), tuple(self.unchained), tuple(self.block_choice.items()), self._asked)
 
     def _objects(self):
         return (self.nn, self.layers, self.params, self.act, self.chw, self.shapes, *self.layers, *self.params)
@@ -241,9 +327,10 @@ class Runner:
     def _walk(self, x, nn, first=0, launches=0):
         """Queues the layers from `first` on, the ones before it being queued in `launches` launches."""
         nn.set_batch(self.batch)
-        tensors = {"input": x, **{L["name"]: self.act[L["name"]] for L in self.layers[:first]}}
+        tensors = {"input": x, **{L["name"]: self._buffer(L["name"]) for L in self.layers[:first]}}
         out = x
         self.launches = launches
+        self._left_out = frozenset(i for i in self._left_out if i < first)
         recorded, readers = nn is not self.nn, None
         i = first
         while i < len(self.layers):
@@ -256,11 +343,13 @@ class Runner:
             n = self._chain_length(i, readers) if block and self.chain_blocks else 0
             if n >= 2 and self._queue_chain(i, n, tensors, nn):
                 last = self.layers[i + 2 * n - 1]["name"]
-                out = tensors[last] = self.act[last]
+                out = tensors[last] = self._buffer(last)
                 i += 2 * n
                 continue
             if block and self._block_fusable(i, readers=readers) and self._queue_block(i, tensors, nn):
-                out = tensors[self.layers[i + 1]["name"]] = self.act[self.layers[i + 1]["name"]]
+                out = tensors[self.layers[i + 1]["name"]] = self._buffer(self.layers[i + 1]["name"])
+                if self._small(i):
+                    self._left_out |= {i}
                 i += 2
                 continue
             out = tensors[L["name"]] = self._queue(i, tensors, nn)
@@ -278,31 +367,36 @@ class Runner:
         if L["op"] != "depthwise" or N["op"] != "pointwise" or N["in"] != L["name"]:
             return False
         # "auto": where the single launch is not slower than the two.  Runner.tune() times both forms of every such block on
-        # the batch at hand and records the faster one in block_choice.  Without that measurement the rule is
-        #   * output planes of 8 x 8 pixels, a whole image per workgroup (two launches / one at batch 256: 16x16x128 -> 256 at
-        #     stride 2 10.2 / 8.1 us, 8x8x256 11.6 / 8.8);
-        #   * blocks whose depthwise result is small, so that launches and round trips to memory are most of the time: less than
-        #     1 MB (16x16x128 at batch 16 9.1 / 5.7 us, 4x4x512 at batch 64 9.5 / 9.3), at most 4 MB for planes of 32 x 32
-        #     pixels and more (64x64x16 at batch 64 11.5 / 9.7, at batch 256 20.2 / 24.3; 32x32x64 at batch 64 10.3 / 7.8, at
-        #     batch 256 16.9 / 19.1).  Smaller planes would gain up to some 4 MB too (16x16x128 at batch 128 13.0 / 8.1); the line
-        #     is lower there because a fused pair's depthwise result is not materialised, and tables are read at such batches;
-        #   * blocks whose depthwise layer alone has no kernel for HWC input and would be two launches itself (64x64x16 at batch
-        #     255 39.0 / 24.5 us, three launches / one).
+        # the batch at hand and records the faster one in block_choice.  Without that measurement: output planes of 8 x 8
+        # pixels, a whole image per workgroup (two launches / one at batch 256: 16x16x128 -> 256 at stride 2 10.2 / 8.1 us,
+        # 8x8x256 11.6 / 8.8), and small blocks
         if policy and self.fuse_blocks == "auto":
-            if i in self.block_choice:
-                if not self.block_choice[i]:
-                    return False
-            else:
-                Ho, Wo, Cc = self.shapes[L["name"]]
-                size = self.batch * Ho * Wo * Cc
-                small = size < 2 ** 20 or (Ho * Wo >= 1024 and size <= 2 ** 22)
-                relaid = Cc % 64 != 0 and (self.shapes[L["in"]][1] <= 8 or (self.batch * Cc) % 64 != 0)
-                if (Ho, Wo) != (8, 8) and not small and not relaid:
-                    return False
+            if not (self.block_choice[i] if i in self.block_choice else self.shapes[L["name"]][:2] == (8, 8) or self._small(i)):
+                return False
         sx, sy = L["strides"]
         if L["w"].shape[1:3] != (3, 3) or tuple(L["pads"]) != (1, 1, 1, 1) or sx != sy:
             return False
         return (readers or self._reader_counts())[L["name"]] == 1
+
+    def _small(self, i):
+        """Whether fuse_blocks="auto" makes one launch of depthwise layer i and the next because the block is small, or because
+        the depthwise layer alone would be two launches itself.  Not where its result is asked for, or could not be computed
+        again for a caller who asks after the run, from an input that may be gone by then."""
+        L = self.layers[i]
+        if self.fuse_blocks != "auto" or i in self.block_choice or i in self._asked or L["in"] == "input" or not isinstance(self.act, _Activations):
+            return False
+        # Small: launches and round trips to memory are most of the time.  Two launches / one: 16x16x128 at batch 16 9.1 / 5.7 us,
+        # 4x4x512 at batch 64 9.5 / 9.3; 64x64x16 at batch 64 11.5 / 9.7, at batch 256 20.2 / 24.3; 32x32x64 at batch 64 10.3 / 7.8, at
+        # batch 256 16.9 / 19.1; so at most 4 MB for planes of 32 x 32 pixels and more.  Smaller planes would gain up to some 4 MB
+        # too (16x16x128 at batch 128 13.0 / 8.1), but tables of 1 MB and more keep the launches per layer that callers count on.
+        Ho, Wo, Cc = self.shapes[L["name"]]
+        size = self.batch * Ho * Wo * Cc
+        if (Ho, Wo) == (8, 8):
+            return False
+        if size < 2 ** 20 or (Ho * Wo >= 1024 and size <= 2 ** 22):
+            return True
+        # No kernel for HWC input: 64x64x16 at batch 255 39.0 / 24.5 us, three launches / one
+        return Cc % 64 != 0 and (self.shapes[L["in"]][1] <= 8 or (self.batch * Cc) % 64 != 0)
 
     def _reader_counts(self):
         """{tensor name: how many layers read it}"""
@@ -341,7 +435,7 @@ class Runner:
             k2, l2, m2, s2, r2, b2 = self._requant_args(N, Q)
             blocks.append((P["w"], P.get("bias"), k1, l1, m1, s1, r1, b1, Q["w"], Q.get("bias"), k2, l2, m2, s2, r2, b2))
         try:
-            nn.dw_pw_chain_hwc(tensors[self.layers[i]["in"]], self.act[self.layers[i + 2 * n - 1]["name"]], W, H, Cc, blocks)
+            nn.dw_pw_chain_hwc(tensors[self.layers[i]["in"]], self._buffer(self.layers[i + 2 * n - 1]["name"]), W, H, Cc, blocks)
         except PulpNNError as err:
             if err.code != 2:
                 raise
@@ -357,7 +451,7 @@ class Runner:
         k1, l1, m1, s1, r1, b1 = self._requant_args(L, P)
         k2, l2, m2, s2, r2, b2 = self._requant_args(N, Q)
         try:
-            nn.dw_pw_hwc(tensors[L["in"]], self.act[N["name"]], W, H, Cc, Wo, Ho, Co, L["strides"][0], P["w"], P.get("bias"),
+            nn.dw_pw_hwc(tensors[L["in"]], self._buffer(N["name"]), W, H, Cc, Wo, Ho, Co, L["strides"][0], P["w"], P.get("bias"),
                          k1, l1, m1, s1, r1, b1, Q["w"], Q.get("bias"), k2, l2, m2, s2, r2, b2)
         except PulpNNError as err:
             if err.code != 2:
@@ -416,7 +510,7 @@ class Runner:
         tensors = {"input": x}
         self.run(x)
         for L in self.layers:
-            tensors[L["name"]] = self.act[L["name"]]
+            tensors[L["name"]] = self._buffer(L["name"])
         self.nn.sync()
 
         def timed(fn):

@@ -1,5 +1,6 @@
 """The extension module behind the Python front end (csrc/pybind_fast.cpp), as far as it goes without a GPU: argument
 counts, keywords, rejected calls, and plans that notice what they were made from has changed."""
+import copy
 import ctypes
 import os
 import subprocess
@@ -384,6 +385,67 @@ def test_the_first_run_lays_the_plan_out():
     lib.seen.clear()
     r.run(0x300)
     assert lib.seen[0] == ("pulp_nn_hip_dw_pw_chain_hwc", 0x300, r.act["p2"], r.params[0]["w"], r.params[2]["w"])
+
+
+def small_blocks():
+    """Blocks on 16 x 16 planes: one that reads the input, one behind it."""
+    def bn(n):
+        return dict(bias=np.zeros(n, np.int8), k=np.ones(n), lam=np.zeros(n), relu=1, bn=1, mult=0, shift=5)
+
+    def dw(name, src):
+        return dict(bn(64), op="depthwise", name=name, **{"in": src}, w=np.zeros((64, 3, 3), np.int8), pads=[1, 1, 1, 1], strides=[1, 1])
+
+    def pw(name, src, co):
+        return dict(bn(co), op="pointwise", name=name, **{"in": src}, w=np.zeros((co, 1, 1, 64), np.int8))
+
+    return [dw("d1", "input"), pw("p1", "d1", 64), dw("d2", "p1"), pw("p2", "d2", 32)]
+
+
+def test_depthwise_results_of_small_blocks_can_be_read():
+    """The rule that makes one launch of a small block: whoever reads the depthwise result, before or after the run, gets it as
+    from the two launches."""
+    def runner():
+        lib = FakeLibrary()
+        nn = lib.bound()
+        nn._lib.pulp_nn_hip_get_batch = lambda: lib.batch
+        r = bare_runner(nn, small_blocks(), (16, 16, 64), batch=4)
+        r.act = network._Activations(r, r.act)
+        return lib, r
+
+    def calls(lib, r, x):
+        lib.seen.clear()
+        r.run(x)
+        return [c[0].replace("pulp_nn_", "").replace("hip_", "") for c in lib.seen]
+
+    two, one = ["depthwise_hwc", "pointwise_HoWo_parallel"], ["dw_pw_hwc"]
+    readers = [lambda r: r.act["d2"], lambda r: r.act.get("d2"), lambda r: dict(r.act)["d2"], lambda r: {**r.act}["d2"],
+               lambda r: list(r.act.values())[2], lambda r: dict(r.act.items())["d2"], lambda r: r.act.copy()["d2"],
+               lambda r: r.act.setdefault("d2"), lambda r: copy.deepcopy(r.act)["d2"]]
+    for read in readers:
+        lib, r = runner()
+        for x in (0x100, 0x200, 0x300):
+            assert calls(lib, r, x) == two + one and r.launches == 3   # the input may be gone when d1 is read: two launches
+        lib.seen.clear()
+        lib.batch = 7                                     # (the caller's)
+        buffer = read(r)
+        assert buffer == dict.__getitem__(r.act, "d2") and lib.batch == 7
+        assert [(c[0], c[1], c[3]) for c in lib.seen] == [("pulp_nn_hip_depthwise_hwc", dict.__getitem__(r.act, "p1"), buffer)]
+        for x in (0x100, 0x200):
+            assert calls(lib, r, x) == two + two and r.launches == 4
+        lib.seen.clear()
+        read(r)
+        assert not lib.seen
+    lib, r = runner()
+    r.act["d2"]                                           # held from before the first run on
+    assert calls(lib, r, 0x100) == two + two
+    for put in (lambda r: r.act.__setitem__("d2", 0x990000), lambda r: r.act.update(d2=0x990000)):
+        lib, r = runner()
+        assert calls(lib, r, 0x100) == two + one
+        put(r)                                            # a buffer of the caller's
+        assert calls(lib, r, 0x100) == two + two and lib.seen[2][3] == 0x990000
+    lib, r = runner()
+    r.act = dict(r.act)                                   # and a dictionary that does not tell who reads it
+    assert calls(lib, r, 0x100) == two + two
 
 
 def test_a_plan_does_not_keep_the_input():

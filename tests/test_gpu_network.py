@@ -266,3 +266,36 @@ def test_plan_falls_back_and_takes_new_inputs():
     for x in xs[:2]:
         check(x, torch.from_numpy(x).cuda(), "changed shift")
     L.set_batch(1)
+
+
+def test_every_tensor_of_small_blocks_can_be_read():
+    """Batches so small that depthwise and pointwise layers run as one launch: the depthwise results read after a run are the
+    oracle's, in buffers read for the first time and in buffers held from an earlier run."""
+    r = rng_for(22800)
+    B, C = 3, 64
+
+    def bn(n, shift):
+        return dict(bias=rand_s8(r, (n,)), k=r.integers(256, 1025, n), lam=r.integers(-2 ** 16, 2 ** 16 + 1, n), relu=1, bn=1, shift=shift)
+
+    layers = [dict(op="conv", name="stem", **{"in": "input"}, w=rand_s8(r, (C, 3, 3, 3)), pads=(1, 1, 1, 1), strides=(1, 1), **bn(C, 15))]
+    for i, stride in enumerate((1, 2, 1)):
+        layers += [dict(op="depthwise", name="d%d" % i, **{"in": layers[-1]["name"]}, w=rand_s8(r, (C, 3, 3)), pads=(1, 1, 1, 1),
+                        strides=(stride, stride), **bn(C, 14)),
+                   dict(op="pointwise", name="p%d" % i, **{"in": "d%d" % i}, w=rand_s8(r, (C, 1, 1, C)), **bn(C, 15))]
+    L = nn(32)
+    L.use_torch_stream()
+    runner = network.Runner(L, layers, (32, 32, 3), B)
+    held = None
+    for n in range(3):
+        x = rand_u8(r, (B, 32, 32, 3))
+        want = net_oracle.forward(layers, runner.shapes, x, 32, keep=True)
+        out = runner.run(torch.from_numpy(x).cuda())
+        assert runner.launches == (7 if held else 4)
+        L.set_batch(1)
+        got = held or {name: runner.act[name] for name in ("d0", "p0", "d1", "p1", "d2", "p2")}
+        torch.cuda.synchronize()
+        assert L.get_batch() == 1
+        for name, t in got.items():
+            assert_same(t.cpu().numpy(), want[name], "run %d, %s" % (n, name))
+        assert_same(out.cpu().numpy(), want["p2"], "run %d" % n)
+        held = got
