@@ -168,8 +168,9 @@ inline const char *dwpw_refusal(long long B, int C, int W, int Ho, int Wo, int C
 // 9.9 / 9.0; batch 8, tiles of 64 pixels, 16x16x128 6.8 / 5.7 / 6.3.
 inline int dwpw_waves(int C, bool whole, int px) { return C == 16 ? 4 : C <= 64 || (!whole && px * C <= 8192) ? 8 : 16; }
 
-// Tile of NI whole images (whole) or of px output pixels, at most `waves` waves per workgroup.  False if it does not fit.
-inline bool dwpw_tile(DwPwTile &g, int W, int S, bool chain, int cus, int bn_bytes, int NI, int px, int waves)
+// Tile of NI whole images (whole) or of px output pixels, at most `waves` waves per workgroup, at least `least` slabs of input.  False if it
+// does not fit.
+inline bool dwpw_tile(DwPwTile &g, int W, int S, bool chain, int cus, int bn_bytes, int NI, int px, int waves, int least)
 {
   const int WO = W / S, CF = g.Co / 16, C = g.C;
   g.NI = NI;
@@ -180,7 +181,8 @@ inline bool dwpw_tile(DwPwTile &g, int W, int S, bool chain, int cus, int bn_byt
   // all channels' input at once if that is no more than 56 KB, else equal slabs of them
   long long x = 0;
   for (int parts = 1; parts <= std::max(1, C / 64); parts++) {
-    if (parts > 1 && (chain || C / 64 % parts)) continue;
+    if (parts > 1 && (chain || C / 64 % parts || (parts < least && parts < C / 64))) continue;
+    if (least > 1 && parts == 1) continue;
     g.CS = C / parts;
     g.slabs = parts;
     g.pitch = 16 * ((g.CS / 16) | 1);
@@ -226,16 +228,18 @@ inline bool dwpw_shape(int B, int C, int H, int W, int Ho, int Co, int S, bool c
   const int WO = W / S;
   g.whole = chain || Ho * WO <= 64;
   bool ok = false;
+  // (more slabs than the input alone asks for only where nothing fits beside it: two output rows of 1024 channels)
+  for (int least = 1; least <= std::max(1, chain ? 1 : C / 64) && !ok; least *= 2)
   for (int waves = 16; waves >= 4 && !ok; waves /= 2) {
     if (g.whole) {
       // images until the tile has 64 pixels, as long as their input fits without being cut into slabs
       for (int ni = std::min(B, std::max(1, 64 / (Ho * WO))); ni >= 1 && !ok; ni /= 2)
-        ok = dwpw_tile(g, W, S, chain, cus, bn_bytes, ni, 0, waves) && (g.slabs == 1 || ni == 1);
+        ok = dwpw_tile(g, W, S, chain, cus, bn_bytes, ni, 0, waves, least) && (g.slabs == 1 || ni == 1);
     } else {
       // 256, 128 or 64 pixels: the most that leave every compute unit sixteen waves
       int px = 256;
       while (px > 64 && (px < WO || (long long)B * ((Ho + px / WO - 1) / (px / WO)) * dwpw_waves(C, false, px) < 16ll * cus)) px /= 2;
-      for (; px >= 64 && !ok; px /= 2) ok = dwpw_tile(g, W, S, chain, cus, bn_bytes, 1, px, waves);
+      for (; px >= 64 && !ok; px /= 2) ok = dwpw_tile(g, W, S, chain, cus, bn_bytes, 1, px, waves, least);
     }
   }
   if (!ok) return false;

@@ -2,8 +2,10 @@
 // entry points take but no tile fits, loads of another byte than the one meant, LDS places outside their range, activations that are
 // left out or written twice, output pixels left out.
 // Blocks on stdin, one a line: B C H W Co S chained bn_bytes cus.  One line out per block: "ok WAVES", "no" (refused) or what is wrong.
+// A line "every": a tile for every shape that the entry points take, up to heights that only add tiles: the number of them.
 #include <stdio.h>
 #include <stdlib.h>
+#include <string.h>
 
 #include <string>
 #include <vector>
@@ -85,10 +87,39 @@ static std::string check(int B, int C, int H, int Co, int chained, int bn_bytes,
   return "ok " + std::to_string(g.waves);
 }
 
+// every W, S, C and bn, heights up to three tiles of 256 pixels, and channels out and batches on both sides of every line
+static std::string every()
+{
+  long long taken = 0;
+  for (const int W : {64, 32, 16, 8, 4})
+    for (int S = 1; S <= 2; S++)
+      for (int C = 16; C <= 1024; C += C < 32 ? 16 : C < 64 ? 32 : 64)
+        for (int H = 1; H <= 3 * 256 * S * S / W + 2; H++)
+          for (const int Co : {16, 32, 48, 64, 96, 128, 192, 256, 320, 512, 1008, 1024, 2048, 4096})
+            for (const int B : {1, 2, 3, 4, 15, 16, 60, 64, 128, 255, 256, 257, 512, 1000, 1024, 5000})
+              for (int chained = 0; chained < (S == 1 && Co == 16 ? 2 : 1); chained++)
+                for (const int bn : {4, 8})
+                  for (const int cus : {64, 256}) {
+                    const int Ho = (H - 1) / S + 1, co = chained ? C : Co;
+                    if (dwpw_refusal(B, C, W, Ho, W / S, co, S, chained ? 2 : 1, cus, bn)) continue;
+                    DwPwTile g;
+                    taken++;
+                    if (dwpw_shape(B, C, H, W, Ho, co, S, chained, cus, bn, &g) && g.lds <= 160 * 1024) continue;
+                    char what[256];
+                    snprintf(what, sizeof what, "taken, but no tile fits: %d %d %d %d %d %d %d %d %d", B, C, H, W, co, S, chained, bn, cus);
+                    return what;
+                  }
+  return std::to_string(taken);
+}
+
 int main()
 {
   char line[256];
   while (fgets(line, sizeof line, stdin)) {
+    if (!strncmp(line, "every", 5)) {
+      puts(every().c_str());
+      continue;
+    }
     int B, C, H, W, Co, S, chained, bn, cus;
     if (sscanf(line, "%d %d %d %d %d %d %d %d %d", &B, &C, &H, &W, &Co, &S, &chained, &bn, &cus) != 9) return 1;
     std::string said = "no";

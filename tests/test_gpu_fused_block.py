@@ -27,6 +27,7 @@ GEOMS = [
     (300, 8, 8, 64, 16, 1),      # many small images, a single 16-channel output group
     (9, 8, 16, 320, 96, 2),      # H = 8, W = 16, five K slices (two passes over the weights)
     (4, 8, 8, 64, 2048, 1),      # 2048 output channels: legal because so few images are split over workgroups by channels
+    (5, 3, 16, 1024, 256, 2),    # two output rows of 1024 channels
 ]
 FLAGS = [((1, 1), (1, 1)), ((1, 0), (1, 1)), ((1, 1), (1, 0)), ((0, 0), (0, 0)), ((2, 0), (0, 1))]
 
