@@ -122,13 +122,12 @@ __global__ __launch_bounds__(1024) void dwpw_kernel(DwPwGeom g)
   int w_cf = -1;                                                // channels whose first slices are there, or on their way
   auto load_w = [&](DwPwBlockArg P, int cf, int kt0) {
     const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)P->pw_w, 0, (unsigned)T.Co * (unsigned)T.C, 0x00020000);
-    // (four lanes fetch the 64 bytes of a row's slice, which costs the address unit a quarter of four rows' 16 bytes; which of them
-    // fetches which 16 depends on the row, as in the activation operand)
-    const int row = lane >> 2, chunk = (lane & 3) ^ ((row >> 1) & 3);
-    const unsigned off = KP > 1 || 16 * chunk < T.C ? (unsigned)((16 * cf + row) * T.C + 16 * chunk) : 0x80000000u;
+    const unsigned off = dwpw_w_lane(T.C, cf, lane, KP == 1);
 #pragma unroll
-    for (int kk = 0; kk < KP; kk++)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr_t)(wl + 1024 * kk), 16, off, KP == 1 || kt0 + kk < KT ? 64 * (kt0 + kk) : 0x40000000, 0, 0);
+    for (int kk = 0; kk < KP; kk++) {
+      const DwPwWeight at = KP == 1 ? DwPwWeight{off, 64 * kt0} : dwpw_w_slice(T.C, off, kt0 + kk);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr_t)(wl + 1024 * kk), 16, at.off, at.add, 0, 0);
+    }
   };
   const int cgs = T.CS / 16, nitems = cgs * T.nst;  // items of the depthwise stage: 16 channels of a strip
 

@@ -21,11 +21,10 @@ __device__ __forceinline__ void dwpw_par_load(unsigned char *par, const int8_t *
   typedef __attribute__((address_space(3))) void *lds_ptr_t;
   const DwPwPar at = dwpw_par(C, (int)sizeof(bn_t), filter != nullptr);
   for (int to = 1024 * wave; to < at.bytes; to += 16 * 1024) {
-    const char *src = to < at.k ? (const char *)bias : to < at.l ? (const char *)k : to < at.f ? (const char *)lambda : (const char *)filter;
-    const int first = to - (to < at.k ? 0 : to < at.l ? at.k : to < at.f ? at.l : at.f);
-    const int bytes = to < at.k ? (bias ? C : 0) : to < at.f ? (bn ? C * (int)sizeof(bn_t) : 0) : 9 * C;
-    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)src, 0, bytes, 0x00020000);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr_t)(par + to), 16, 16 * lane, first, 0, 0);
+    const DwPwParPiece p = dwpw_par_piece(at, C, (int)sizeof(bn_t), bias != nullptr, bn, to);
+    const char *src = (p.array == 0 ? (const char *)bias : p.array == 1 ? (const char *)k : p.array == 2 ? (const char *)lambda : (const char *)filter) + p.first;
+    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)src, 0, p.bytes, 0x00020000);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr_t)(par + to), 16, 16 * lane, 0, 0, 0);
   }
 }
 // LDS of the launch: the tile's, the pointwise layer's parameters, and a row that pixels past the last one are written to.
@@ -57,13 +56,12 @@ __global__ __launch_bounds__(1024) void dwpw_chain_kernel(DwPwGeom g)
     int ln = lane;  // (opaque: the address is computed when the loads are issued, not kept from block to block)
     asm volatile("" : "+v"(ln));
     const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)P->pw_w, 0, C * C, 0x00020000);
-    // (four lanes fetch the 64 bytes of a row's slice, which costs the address unit a quarter of four rows' 16 bytes; which of them
-    // fetches which 16 depends on the row, as in the activation operand)
-    const int row = ln >> 2, chunk = (ln & 3) ^ ((row >> 1) & 3);
-    const unsigned off = KP > 1 || 16 * chunk < C ? (unsigned)(((pw_on ? 16 * cf : 0) + row) * C + 16 * chunk) : 0x80000000u;
+    const unsigned off = dwpw_w_lane(C, pw_on ? cf : 0, ln, KP == 1);
 #pragma unroll
-    for (int kk = 0; kk < KP; kk++)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr_t)(wl + 1024 * kk), 16, off, KP == 1 || 64 * kk < C ? 64 * kk : 0x40000000, 0, 0);
+    for (int kk = 0; kk < KP; kk++) {
+      const DwPwWeight at = KP == 1 ? DwPwWeight{off, 0} : dwpw_w_slice(C, off, kk);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr_t)(wl + 1024 * kk), 16, at.off, at.add, 0, 0);
+    }
   };
   auto load_dw = [&](DwPwBlockArg P) {
     dwpw_par_load(par_dw, P->dw_wt, P->dw_bias, P->e_dw.k, P->e_dw.lambda, P->mode_dw == EPI_BN, C, wave, lane);

@@ -115,6 +115,42 @@ PULPNN_HD DwPwPar dwpw_par(int C, int bn_bytes, bool filter)
   return p;
 }
 
+// What one instruction of 16 bytes a lane fetches of them, to place `to` (a multiple of 1 KB): array (0 bias, 1 k, 2 lambda, 3 filter), first byte in
+// it, and bytes from there on that exist: lanes past them are out of range and get zeros.  (By the lane's own offset: what the scalar offset of a
+// load adds does not count where the range is checked.)
+struct DwPwParPiece {
+  int array, first, bytes;
+};
+PULPNN_HD DwPwParPiece dwpw_par_piece(const DwPwPar &at, int C, int bn_bytes, bool bias, bool bn, int to)
+{
+  DwPwParPiece p;
+  p.array = to < at.k ? 0 : to < at.l ? 1 : to < at.f ? 2 : 3;
+  p.first = to - (p.array == 0 ? 0 : p.array == 1 ? at.k : p.array == 2 ? at.l : at.f);
+  const int all = p.array == 0 ? (bias ? C : 0) : p.array == 3 ? 9 * C : bn ? C * bn_bytes : 0;
+  p.bytes = all > p.first ? all - p.first : 0;
+  return p;
+}
+
+// The pointwise layer's weights on their way to LDS: 16 rows (channels out) of 64 bytes, slice kt of K; four lanes fetch the 64 contiguous bytes of a
+// row.  Offset of the lane's 16 bytes and what the scalar offset adds; bytes and slices that do not exist are out of range by the lane's own offset.
+#define DWPW_OOB 0x80000000u
+struct DwPwWeight {
+  unsigned off;
+  int add;
+};
+// (narrow: C may be less than 64)
+PULPNN_HD unsigned dwpw_w_lane(int C, int cf, int lane, bool narrow)
+{
+  // (which of the four fetches which 16 bytes depends on the row, as in the activation operand)
+  const int row = lane >> 2, chunk = (lane & 3) ^ ((row >> 1) & 3);
+  return !narrow || 16 * chunk < C ? (unsigned)((16 * cf + row) * C + 16 * chunk) : DWPW_OOB;
+}
+PULPNN_HD DwPwWeight dwpw_w_slice(int C, unsigned lane_off, int kt)
+{
+  const bool ok = 64 * kt < C;
+  return DwPwWeight{ok ? lane_off : DWPW_OOB, ok ? 64 * kt : 0};
+}
+
 // The shapes that pulp_nn_hip_dw_pw_hwc and pulp_nn_hip_dw_pw_chain_hwc (n_blocks > 1) take, by the limits that their declarations state:
 // the rows a wave takes at once, 1024 output channels per workgroup, whole images and 64 KB of LDS for a chain.  (dwpw_kernel alone could
 // do more; what a caller may rely on is what the declarations say.)  The reason of a refusal, or null.

@@ -1,5 +1,5 @@
 // Walks the tiles of dwpw_kernel and dwpw_chain_kernel on the host, with the kernels' own arithmetic (csrc/dwpw_geom.h): shapes that the
-// entry points take but no tile fits, loads of another byte than the one meant, LDS places outside their range, activations that are
+// entry points take but no tile fits, loads of another byte than the one meant or past an array, LDS places outside their range, activations that are
 // left out or written twice, output pixels left out.
 // Blocks on stdin, one a line: B C H W Co S chained bn_bytes cus.  One line out per block: "ok WAVES", "no" (refused) or what is wrong.
 // A line "every": a tile for every shape that the entry points take, up to heights that only add tiles: the number of them.
@@ -11,6 +11,36 @@
 #include <vector>
 
 #include "../../pulp_nn_amd/csrc/dwpw_geom.h"
+
+// Loads whose range is checked by the lane's own offset: none may reach past its array, whatever the scalar offset adds.
+static const char *loads(int C, int Co, int kp, int bn_bytes)
+{
+  for (int cf = 0; cf < Co / 16; cf++)
+    for (int kt = 0; kt < (C + 63) / 64 + kp; kt++)
+      for (int lane = 0; lane < 64; lane++) {
+        const unsigned off = dwpw_w_lane(C, cf, lane, C <= 64);
+        const DwPwWeight at = dwpw_w_slice(C, off, kt);
+        const int row = lane >> 2, byte = 16 * ((lane & 3) ^ ((row >> 1) & 3)) + 64 * kt;
+        if (at.off < (unsigned)(Co * C) ? byte >= C || (int)at.off + at.add != (16 * cf + row) * C + byte : byte < C || at.add) return "weights";
+      }
+  for (int form = 0; form < 8; form++) {
+    const bool filter = form & 1, bias = form & 2, bn = form & 4;
+    const DwPwPar at = dwpw_par(C, bn_bytes, filter);
+    std::vector<int> seen[4] = {std::vector<int>(C), std::vector<int>(C * bn_bytes), std::vector<int>(C * bn_bytes), std::vector<int>(9 * C)};
+    for (int to = 0; to < at.bytes; to += 1024) {
+      const DwPwParPiece p = dwpw_par_piece(at, C, bn_bytes, bias, bn, to);
+      for (int lane = 0; lane < 64; lane++) {
+        if (16 * lane >= p.bytes) continue;
+        for (int b = p.first + 16 * lane; b < p.first + 16 * lane + 16; b++)
+          if (b >= (int)seen[p.array].size() || seen[p.array][b]++) return "parameters past their array";
+      }
+    }
+    for (int array = 0; array < 4; array++)
+      for (const int n : seen[array])
+        if (n != (array == 0 ? bias : array == 3 ? filter : bn)) return "parameters left out";
+  }
+  return nullptr;
+}
 
 template <int W, int S>
 static std::string check(int B, int C, int H, int Co, int chained, int bn_bytes, int cus)
@@ -25,6 +55,7 @@ static std::string check(int B, int C, int H, int Co, int chained, int bn_bytes,
       (g.waves != 4 && g.waves != 8 && g.waves != 16) || (g.kp == 1) != (C <= 64) || g.w_off + dwpw_par(C, bn_bytes, true).bytes > g.lds + dwpw_par(C, bn_bytes, true).bytes ||
       (g.cf_per << g.lsplit) * 16 < Co || (chained && (g.lsplit || g.slabs != 1)))
     return "shape";
+  if (const char *wrong = loads(C, Co < 128 ? Co : 128, g.kp, bn_bytes)) return wrong;
   const int cgs = g.CS / 16, ids[] = {0, g.tiles / 2, g.tiles - 1};
   long long outputs = 0;
   for (int t = 0; t < g.tiles; t++) outputs += dwpw_place<WO>(g, (unsigned)t).live;
