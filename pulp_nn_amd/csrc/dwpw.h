@@ -95,6 +95,14 @@ __device__ __forceinline__ DwPwBlockArg dwpw_block(int j)
   asm volatile("" : "+s"(p));
   return (DwPwBlockArg)(p + offsetof(DwPwGeom, blk)) + j;
 }
+// ... and bytes per 64-byte slice of K of the activation operand.
+__device__ __forceinline__ int dwpw_act_step()
+{
+  typedef const __attribute__((address_space(4))) char *bytes_t;
+  bytes_t p = (bytes_t)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return 64 * *(const __attribute__((address_space(4))) int *)(p + offsetof(DwPwGeom, t) + offsetof(DwPwTile, act_px));
+}
 
 // W, S: input width, stride.  KP: slices of K whose weights are in LDS at once.  CHAIN: g.nblocks blocks back to back; otherwise the
 // one block g.blk[0].
@@ -163,7 +171,7 @@ __global__ __launch_bounds__(1024) void dwpw_kernel(DwPwGeom g)
       if (first) {
         if (slab) dwpw_barrier();  // everybody is done with the slab before
         const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)(g.in + (dwpw_first_row<S>(T, at) * W) * T.C + slab * T.CS), 0,
-                                                                              (dwpw_rows_in(T) * W) * T.C, 0x00020000);
+                                                                              (dwpw_rows_in(T) * W) * T.C - slab * T.CS, 0x00020000);
         const int chunks = dwpw_chunks<W>(T);
         constexpr int UN = 4;
 #pragma unroll 1
@@ -187,11 +195,13 @@ __global__ __launch_bounds__(1024) void dwpw_kernel(DwPwGeom g)
       const DwPwBlockArg P = dwpw_block(j);
       const int mode = P->mode_dw, shift = P->e_dw.shift;
       const unsigned char *filter = par + dwpw_par(T.C, (int)sizeof(bn_t), true).f + l16 * 9 + min(lgrp, 2);
+      const int act_step = CHAIN ? 4096 << T.lpxb : dwpw_act_step();
       DwhChannels<1> c;
       int set = -1;  // channel group that c holds
 #pragma unroll 1
       for (int it = wave; it < nitems; it += NWV) {
         const int st = (int)fastdiv((unsigned)it, T.d_n), cg = it - st * cgs, ch = slab * T.CS + 16 * cg;
+        if (!CHAIN && ch >= T.C) continue;  // (the last slab may have fewer channels)
         if (set != cg) {
           const v4i ones = {0x01010101, 0x01010101, 0x01010101, 0x01010101};
           v4i s = {0, 0, 0, 0};
@@ -216,7 +226,7 @@ __global__ __launch_bounds__(1024) void dwpw_kernel(DwPwGeom g)
           return v;
         };
         auto put = [&](unsigned v) {
-          if (n.live) *(unsigned *)(dwpw_lds + (narrow ? px * T.C + ch : (((ch >> 6) << T.lpxb) << 12) + px * 64 + ((((ch >> 4) & 3) ^ ((px >> 1) & 3)) << 4)) + 4 * lgrp) = v ^ 0x80808080u;
+          if (n.live) *(unsigned *)(dwpw_lds + (narrow ? px * T.C + ch : (ch >> 6) * act_step + px * 64 + ((((ch >> 4) & 3) ^ ((px >> 1) & 3)) << 4)) + 4 * lgrp) = v ^ 0x80808080u;
           px += WO;
         };
         dwh_with_form(c.form, [&](auto form) { dwh_walk<S, decltype(form)::value>(c, shift, T.R, next, put); });
@@ -224,7 +234,7 @@ __global__ __launch_bounds__(1024) void dwpw_kernel(DwPwGeom g)
     }
     // ---- pointwise stage ---------------------------------------------------------------------------------------------------
     const DwPwBlockArg P = dwpw_block(j);
-    const int mode = P->mode_pw, shift = P->e_pw.shift;
+    const int mode = P->mode_pw, shift = P->e_pw.shift, act_step = CHAIN ? 4096 << T.lpxb : dwpw_act_step();
     __builtin_amdgcn_s_waitcnt(DWPW_WAIT_VM(0));  // this wave's weights
     dwpw_barrier();
 #pragma unroll 1
@@ -260,7 +270,7 @@ __global__ __launch_bounds__(1024) void dwpw_kernel(DwPwGeom g)
             v4i af[4];
 #pragma unroll
             for (int s = 0; s < 4; s++) af[s] = *(const v4i *)(a0 + s * sstep);
-            a0 += 4096 << T.lpxb;
+            a0 += act_step;
             wacc = __builtin_amdgcn_mfma_i32_16x16x64_i8(wf, ones, wacc, 0, 0, 0);
 #pragma unroll
             for (int s = 0; s < 4; s++) acc[s] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wf, af[s], acc[s], 0, 0, 0);

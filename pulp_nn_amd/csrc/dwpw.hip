@@ -1,6 +1,7 @@
 // Depthwise + pointwise blocks as one launch: which shapes, and the launch (the tile's shape: dwpw_geom.h).
 #include "host.h"
 
+#include "dwpw16.h"
 #include "dwpw_chain.h"
 
 namespace {
@@ -45,6 +46,17 @@ bool launch_s2(int W, const DwPwGeom &g)
   return W == 64 ? launch<64, 2, false>(g) : W == 32 ? launch<32, 2, false>(g) : W == 16 ? launch<16, 2, false>(g) : launch<8, 2, false>(g);
 }
 
+// Few planes 16 pixels wide at stride 2 (the rule, and what it measured: dwpw_small16)
+void launch16(const DwPwGeom &g, int B, int C, int H, int Ho, int Co, int cus)
+{
+  const int M = B * Ho * 8, tiles = (M + DWPW16_PX - 1) / DWPW16_PX, split = dwpw16_split(tiles, Co, cus);
+  const DwPw16Geom t = {g.in, g.out, M, C, H, Ho, Co, split, fastdiv_make((unsigned)Ho), g.blk[0]};
+  const size_t lds = (size_t)dwpw16_lds(C, Co, split, (int)sizeof(bn_t));
+  const dim3 grid((unsigned)(tiles * split)), block(64 * DWPW16_WAVES);
+  if (C == 128) hipLaunchKernelGGL(dwpw16_kernel<2>, grid, block, lds, g_stream, t);
+  else hipLaunchKernelGGL(dwpw16_kernel<4>, grid, block, lds, g_stream, t);
+}
+
 }  // namespace
 
 // Common part of pulp_nn_hip_dw_pw_hwc (one block) and pulp_nn_hip_dw_pw_chain_hwc (several).
@@ -80,7 +92,8 @@ void dwpw_common(const char *fn, const unsigned char *Im_in, unsigned char *Im_o
   if (refusal) return set_error(PULP_NN_HIP_ERR_UNSUPPORTED, fn, refusal);
   g.in = Im_in;
   g.out = Im_out;
-  if (!dwpw_shape((int)g_batch, C, H, W, Ho, Co, S, n_blocks > 1, num_cus(), (int)sizeof(bn_t), &g.t) ||
+  if (n_blocks == 1 && dwpw_small16(g_batch, C, W, Ho, Co, S, num_cus())) launch16(g, (int)g_batch, C, H, Ho, Co, num_cus());
+  else if (!dwpw_shape((int)g_batch, C, H, W, Ho, Co, S, n_blocks > 1, num_cus(), (int)sizeof(bn_t), &g.t) ||
       !(n_blocks > 1 ? launch_s1<true>(W, g) : S == 1 ? launch_s1<false>(W, g) : launch_s2(W, g)))
     return set_error(PULP_NN_HIP_ERR_UNSUPPORTED, fn, "no fused kernel for this geometry: call the depthwise and the pointwise layer separately");
   check_launch(fn);

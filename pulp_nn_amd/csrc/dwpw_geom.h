@@ -14,8 +14,9 @@ struct DwPwTile {
   int B, C, H, Ho, Co;
   int whole, NI, TR;     // whole images, how many; output rows of a tile
   int lpxb;              // log2 of the tile's blocks of 64 pixels
+  int act_px;            // pixels of the activation operand (a multiple of 16; of 64 in chains and with more than one block)
   int R, nrb, nst;       // depthwise stage: rows of a strip, row blocks of a tile, strips (16 columns, or fewer of several row blocks)
-  int CS, slabs;         // channels whose input is in LDS at a time
+  int CS, slabs;         // channels whose input is in LDS at a time (the last slab may have fewer)
   int XR, pitch;         // rows of input in LDS, bytes per pixel (an odd number of 16-byte chunks)
   int x_off, lds;        // LDS: where the input starts, bytes in all
   int waves, tiles, lsplit, cf_per;  // 2^lsplit workgroups share a tile, with cf_per 16-channel groups of output each
@@ -89,7 +90,7 @@ PULPNN_HD DwPwLane dwpw_lane(const DwPwTile &g, int st, int l16, int kx)
 // Activation operand: 16 channels from c on (a multiple of 16) of pixel px.
 PULPNN_HD int dwpw_act(const DwPwTile &g, int px, int c)
 {
-  return g.C < 64 ? px * g.C + c : (((c >> 6) << g.lpxb) << 12) + px * 64 + ((((c >> 4) & 3) ^ ((px >> 1) & 3)) << 4);
+  return g.C < 64 ? px * g.C + c : (c >> 6) * (64 * g.act_px) + px * 64 + ((((c >> 4) & 3) ^ ((px >> 1) & 3)) << 4);
 }
 
 // Chains: pixel px's place as an input pixel of the next block (whole images, stride 1).
@@ -199,55 +200,88 @@ inline const char *dwpw_refusal(long long B, int C, int W, int Ho, int Wo, int C
   return nullptr;
 }
 
+// Planes 16 pixels wide at stride 2 with 128 channels or more go to dwpw16_kernel while there is no more than one tile of 64 output pixels for every
+// four compute units, with up to 512 channels out for every two.  dwpw_kernel / dwpw16_kernel: 16x16x256 batch 1 7.9 / 7.2 us, batch 32 8.7 / 8.4, batch 128
+// 9.7 / 9.1; 16x16x512 batch 64 17.1 / 15.2, batch 128 18.7 / 16.6; 16x16x128 batch 1 6.1 / 5.8, batch 128 7.2 / 6.2.  Past the lines: 16x16x512 -> 1024 batch
+// 96 20.9 / 24.4; 16x16x128 batch 160 7.4 / 8.0, batch 256 7.6 / 8.5.
+inline bool dwpw_small16(long long B, int C, int W, int Ho, int Co, int S, int cus)
+{
+  return W == 16 && S == 2 && C >= 128 && B * Ho * 8 <= (Co <= 512 ? 32ll : 16ll) * cus;
+}
+
+#define DWPW16_PX 32  // output pixels of a tile of it: four rows, two of them one item of the depthwise stage
+// Workgroups that share such a tile, each with a part of the output channels: as many as leave every compute unit one, and no workgroup
+// more than 1024 channels.  LDS of one of them: the activation operand, and bias, k and lambda of its channels.
+inline int dwpw16_split(int tiles, int Co, int cus)
+{
+  int split = 1;
+  for (const int blocks = (Co + 63) / 64; split * 2 <= blocks && (2ll * tiles * split <= cus || blocks > 16 * split);) split *= 2;
+  return split;
+}
+inline int dwpw16_lds(int C, int Co, int split, int bn_bytes) { return DWPW16_PX * C + ((Co + 63) / 64 + split - 1) / split * 64 * (4 + 2 * bn_bytes); }
+
 // Waves of a workgroup for a tile of px pixels: a wave's item is 16 channels of 16 or more pixels.  Measured, call by call at batch 256 with 4 /
 // 8 / 16 waves: 64x64x16 in tiles of 256 pixels 31.2 / 39.3 / 68.1 us, 32x32x64 27.4 / 21.9 / 27.9, 16x16x128 22.0 / 14.8 / 12.8, 8x8x256 whole 13.6 /
-// 9.9 / 9.0; batch 8, tiles of 64 pixels, 16x16x128 6.8 / 5.7 / 6.3.
-inline int dwpw_waves(int C, bool whole, int px) { return C == 16 ? 4 : C <= 64 || (!whole && px * C <= 8192) ? 8 : 16; }
+// 9.9 / 9.0; batch 8, tiles of 64 pixels, 16x16x128 6.8 / 5.7 / 6.3.  8 / 16 waves at batch 64: 8x8x128 5.8 / 6.7, two images of 4x4x128 5.6 / 5.8,
+// but one 5.7 / 5.4.
+inline int dwpw_waves(int C, int px) { return C == 16 ? 4 : C <= 64 || (C <= 128 && px >= 32 && px <= 64) ? 8 : 16; }
 
-// Tile of NI whole images (whole) or of px output pixels, at most `waves` waves per workgroup, at least `least` slabs of input.  False if it
-// does not fit.
-inline bool dwpw_tile(DwPwTile &g, int W, int S, bool chain, int cus, int bn_bytes, int NI, int px, int waves, int least)
+// Tile of NI whole images (whole) or of px output pixels.  0 if it does not fit, 1 with fewer waves than it should have, else 2.
+inline int dwpw_tile(DwPwTile &g, int W, int S, bool chain, int cus, int bn_bytes, int NI, int px)
 {
-  const int WO = W / S, CF = g.Co / 16, C = g.C;
+  const int WO = W / S, CF = g.Co / 16, C = g.C, units = C < 64 ? 1 : C / 64;
   g.NI = NI;
   g.TR = g.whole ? NI * g.Ho : std::min(std::max(1, px / WO), g.Ho);
   g.bands = g.whole ? 1 : (g.Ho + g.TR - 1) / g.TR;
   for (g.lpxb = 0; (64 << g.lpxb) < g.TR * WO;) g.lpxb++;
-  g.x_off = (64 << g.lpxb) * C;
-  // all channels' input at once if that is no more than 56 KB, else equal slabs of them
-  long long x = 0;
-  for (int parts = 1; parts <= std::max(1, C / 64); parts++) {
-    if (parts > 1 && (chain || C / 64 % parts || (parts < least && parts < C / 64))) continue;
-    if (least > 1 && parts == 1) continue;
-    g.CS = C / parts;
-    g.slabs = parts;
-    g.pitch = 16 * ((g.CS / 16) | 1);
-    g.XR = g.whole ? g.NI * (g.H + 2) : (g.TR - 1) * S + 3;
-    x = (long long)(g.XR + 1) * (W + 2) * g.pitch;  // (a walk reads one row past the last one it needs)
-    if (x <= 56 * 1024) break;
-  }
+  g.act_px = g.lpxb || chain ? 64 << g.lpxb : (g.TR * WO + 15) & ~15;
+  g.x_off = g.act_px * C;
+  g.XR = g.whole ? g.NI * (g.H + 2) : (g.TR - 1) * S + 3;
   const long long tiles = (long long)((g.B + g.NI - 1) / g.NI) * g.bands;
-  if (g.x_off + x > 160 * 1024 || tiles > 0x7fffffff / 64) return false;
+  if (g.x_off > 160 * 1024 || tiles > 0x7fffffff / 64) return 0;
   g.tiles = (int)tiles;
   // (a tile is shared only as long as that gives no compute unit a second workgroup: each of them computes the depthwise stage)
   for (g.lsplit = 0; !chain && ((long long)g.tiles << (g.lsplit + 1)) <= cus && (2 << g.lsplit) <= CF / 4;) g.lsplit++;
   g.cf_per = (CF + (1 << g.lsplit) - 1) >> g.lsplit;
-  // depthwise stage: rows per strip, as many as leave every wave a strip
-  const int cgs = g.CS / 16;
-  auto strips = [&](int r) { return WO >= 16 ? g.TR / r * (WO / 16) : (g.TR / r + 16 / WO - 1) / (16 / WO); };
-  const int want = std::min(waves, dwpw_waves(C, g.whole, g.TR * WO));
-  for (g.R = 4; g.R > 1 && (g.TR % g.R || g.Ho % g.R || strips(g.R) * cgs < want);) g.R /= 2;
-  g.nrb = g.TR / g.R;
-  g.nst = strips(g.R);
-  const int most = std::max(g.nst * cgs, g.cf_per << g.lpxb);
-  for (g.waves = 4; g.waves < most && g.waves < want;) g.waves *= 2;
-  // LDS: activation operand, input, depthwise parameters, weights (all of K at once for up to eight slices, if that fits)
-  g.par_off = (int)((g.x_off + x + 1023) & ~1023);
-  g.w_off = g.par_off + dwpw_par(C, bn_bytes, true).bytes;
-  const int busy = chain ? g.waves : std::min(g.waves, g.cf_per << g.lpxb);
-  g.kp = C <= 64 ? 1 : C <= 256 || g.w_off + busy * 8 * 1024 > 150 * 1024 ? 4 : 8;
-  g.lds = g.w_off + busy * g.kp * 1024;
-  return g.lds <= 160 * 1024;
+  const int want = C > 64 && (chain || (g.whole && W == 16 && S == 2)) ? 16 : dwpw_waves(C, g.TR * WO), par = dwpw_par(C, bn_bytes, true).bytes;
+  // LDS: activation operand, input, depthwise parameters, weights.  A slab of the input costs a round trip to memory and two barriers, so
+  // there are as few as fit (16x16x256 stride 2, batch 16, two slabs / one: 9.5 / 8.3 us; 8x8x512 10.9 / 9.5).  The weights of a wave are all of
+  // K at once for up to eight slices, if that fits, else four.  More than five slabs of 64 channels only if half as many waves, with room for
+  // fewer weights, do not get along with fewer of them (16x16x640 stride 2, batch 128, 16 waves and ten slabs / 8 and four: 36.8 / 28.9; but
+  // 64x64x320, five slabs / two: 61.4 / 76.2), and 4 waves (16x16x768 stride 2 26.2 us, 8 waves 18.7) only where nothing else fits.
+  DwPwTile best = {};
+  int with = 0;
+  for (int waves = want; waves >= 4 && !(waves == 4 && best.lds); waves /= 2) {
+    for (int parts = 1; parts <= (chain ? 1 : units); parts++) {
+      DwPwTile t = g;
+      t.CS = C < 64 ? C : 64 * ((units + parts - 1) / parts);
+      t.slabs = (C + t.CS - 1) / t.CS;
+      if (t.slabs != parts) continue;
+      t.pitch = 16 * ((t.CS / 16) | 1);
+      const long long x = (long long)(t.XR + 1) * (W + 2) * t.pitch;  // (a walk reads one row past the last one it needs)
+      if (t.x_off + x > 160 * 1024) continue;
+      // depthwise stage: rows per strip, as many as leave every wave a strip; in a chain no wave a second one (dwpw_chain_kernel)
+      const int cgs = t.CS / 16;
+      auto strips = [&](int r) { return WO >= 16 ? t.TR / r * (WO / 16) : (t.TR / r + 16 / WO - 1) / (16 / WO); };
+      for (t.R = 4; t.R > 1 && (t.TR % t.R || t.Ho % t.R || (strips(t.R) * cgs < waves && !(chain && strips(t.R / 2) * cgs > 16)));) t.R /= 2;
+      t.nrb = t.TR / t.R;
+      t.nst = strips(t.R);
+      const int most = std::max(t.nst * cgs, t.cf_per << t.lpxb);
+      for (t.waves = 4; t.waves < most && t.waves < waves;) t.waves *= 2;
+      t.par_off = (int)((t.x_off + x + 1023) & ~1023);
+      t.w_off = t.par_off + par;
+      const int busy = chain ? t.waves : std::min(t.waves, t.cf_per << t.lpxb);
+      t.kp = C <= 64 ? 1 : C <= 256 || t.w_off + busy * 8 * 1024 > 150 * 1024 ? 4 : 8;
+      t.lds = t.w_off + busy * t.kp * 1024;
+      if (t.lds > 160 * 1024) continue;
+      if (!best.lds || t.slabs < best.slabs) best = t, with = waves;
+      break;
+    }
+    if (best.lds && (best.slabs <= 5 || best.CS >= 128)) break;
+  }
+  if (!best.lds) return 0;
+  g = best;
+  return with < want ? 1 : 2;
 }
 
 // W = 4 .. 64, a power of two; C = 16, 32 or a multiple of 64; Co a multiple of 16.  chain: whole images and all channels per workgroup.
@@ -261,21 +295,47 @@ inline bool dwpw_shape(int B, int C, int H, int W, int Ho, int Co, int S, bool c
   g.H = H;
   g.Ho = Ho;
   g.Co = Co;
-  const int WO = W / S;
-  g.whole = chain || Ho * WO <= 64;
+  const int WO = W / S, img = Ho * WO;
+  g.whole = chain || img <= 64;
   bool ok = false;
-  // (more slabs than the input alone asks for only where nothing fits beside it: two output rows of 1024 channels)
-  for (int least = 1; least <= std::max(1, chain ? 1 : C / 64) && !ok; least *= 2)
-  for (int waves = 16; waves >= 4 && !ok; waves /= 2) {
-    if (g.whole) {
-      // images until the tile has 64 pixels, as long as their input fits without being cut into slabs
-      for (int ni = std::min(B, std::max(1, 64 / (Ho * WO))); ni >= 1 && !ok; ni /= 2)
-        ok = dwpw_tile(g, W, S, chain, cus, bn_bytes, ni, 0, waves, least) && (g.slabs == 1 || ni == 1);
-    } else {
-      // 256, 128 or 64 pixels: the most that leave every compute unit sixteen waves
-      int px = 256;
-      while (px > 64 && (px < WO || (long long)B * ((Ho + px / WO - 1) / (px / WO)) * dwpw_waves(C, false, px) < 16ll * cus)) px /= 2;
-      for (; px >= 64 && !ok; px /= 2) ok = dwpw_tile(g, W, S, chain, cus, bn_bytes, 1, px, waves, least);
+  // whether a tile half as large than g makes a second workgroup per compute unit, where there are that many tiles (64x64x64 -> 64 stride
+  // 2 batch 256, 256 / 128 pixels 41.4 / 34.7 us; 16x16x64 stride 2 batch 1024 four / two images 11.7 / 10.1)
+  auto two = [&](int px, int ni, int half) {
+    DwPwTile t = g;
+    return px > 64 && g.lds > 80 * 1024 && 2ll * g.tiles > cus && dwpw_tile(t, W, S, chain, cus, bn_bytes, ni, half) == 2 && t.lds <= 80 * 1024;
+  };
+  if (chain) {
+    // images until the tile has 64 pixels, as long as they fit with all waves
+    for (int ni = std::min(B, std::max(1, 64 / img)); ni >= 1 && !ok; ni /= 2) ok = dwpw_tile(g, W, S, chain, cus, bn_bytes, ni, 0) >= (ni == 1 ? 1 : 2);
+  } else if (g.whole) {
+    // One image, or as many as leave every compute unit one workgroup (two of 8 waves), up to 128 pixels: its set-up is paid once for all of
+    // them.  One / two / four images: 4x4x128 batch 256 5.6 / 6.0 / 6.6 us, batch 1024 11.9 / 10.7 / 7.5; 8x8x64 batch 1024 11.1 / 8.6 / 9.2.  Up to 64
+    // pixels with fewer workgroups where one small image leaves most of a block of 64 pixels empty, and reads all weights for that: 4x4x384
+    // batch 256 11.3 / 9.7 / 9.3, 4x4x512 -> 1024 batch 128 13.1 / 11.1 / 10.6.  Not where that takes more than 64 KB of input or cuts it in slabs,
+    // unless there is more than one round of workgroups (8x8x512 stride 2, two images in two slabs / one in one: batch 128 12.4 / 11.3, batch 512
+    // 16.4 / 26.4; four in eight 28.0).
+    const int one = img > 16 && C <= 128 ? 2 * cus : cus, few = img > 16 || C < 256 ? one : C < 320 ? cus / 4 : cus / 16;
+    auto groups = [&](int ni) { return (B + ni - 1) / ni; };
+    int ni = 1;
+    while (groups(ni) > (ni * img < 64 ? few : one) && 2 * ni * img <= 128) ni *= 2;
+    for (; ni >= 1 && !ok; ni /= 2) {
+      const int fits = dwpw_tile(g, W, S, chain, cus, bn_bytes, ni, 0);
+      if (ni == 1) ok = fits != 0;
+      else if (fits != 2 || two(ni * img, ni / 2, 0)) ok = false;
+      else if (ni * img <= 32 ? groups(ni / 2) >= cus : groups(ni / 2) > cus) ok = g.slabs <= (ni * img <= 32 ? 6 : 2);
+      else ok = g.slabs == 1 && g.par_off - g.x_off <= 64 * 1024;
+    }
+  } else {
+    // 64 pixels, 128 where that leaves every compute unit a workgroup, 256 where it leaves it sixteen waves
+    auto tiles = [&](int px) { return (long long)B * ((Ho + px / WO - 1) / (px / WO)); };
+    int px = 256;
+    while (px > 64 && (px < WO || tiles(px) < cus || (px == 256 && tiles(px) * dwpw_waves(C, px) < 16ll * cus))) px /= 2;
+    // ... but not 256 where the waves would then fetch weights again more than twice (64x64x128 -> 256 batch 64, 256 / 128 pixels 87.3 / 72.6 us)
+    if (px == 256 && C > 64 && 4 * (Co / 16) > 3 * dwpw_waves(C, px)) px = 128;
+    for (; px >= 64 && !ok; px /= 2) {
+      const int fits = dwpw_tile(g, W, S, chain, cus, bn_bytes, 1, px);
+      // (with all its waves, and few slabs, while half a tile has four rows: of three rows of input one belongs to a row of output alone)
+      ok = px / 2 < std::max(64, WO) ? fits != 0 : (px / 2 < 4 * WO ? fits != 0 : fits == 2 && g.slabs <= 2) && !two(px, 1, px / 2);
     }
   }
   if (!ok) return false;

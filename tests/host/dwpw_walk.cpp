@@ -50,17 +50,22 @@ static std::string check(int B, int C, int H, int Co, int chained, int bn_bytes,
   if (dwpw_refusal(B, C, W, Ho, WO, Co, S, chained ? 2 : 1, cus, bn_bytes)) return "no";
   DwPwTile g;
   if (!dwpw_shape(B, C, H, W, Ho, Co, S, chained, cus, bn_bytes, &g)) return "taken, but no tile fits";
-  const int act_bytes = (64 << g.lpxb) * C, x_bytes = g.par_off - g.x_off, BM = 64 << g.lpxb;
-  if (g.lds > 160 * 1024 || g.x_off < act_bytes || g.CS * g.slabs != C || (g.CS % 64 && C >= 64) || g.TR * WO > BM || g.TR % g.R || (g.whole && Ho % g.R) ||
-      (g.waves != 4 && g.waves != 8 && g.waves != 16) || (g.kp == 1) != (C <= 64) || g.w_off + dwpw_par(C, bn_bytes, true).bytes > g.lds + dwpw_par(C, bn_bytes, true).bytes ||
-      (g.cf_per << g.lsplit) * 16 < Co || (chained && (g.lsplit || g.slabs != 1)))
+  const int act_bytes = g.act_px * C, x_bytes = g.par_off - g.x_off, BM = g.act_px, KT = (C + 63) / 64;
+  const int nblk = g.cf_per << g.lpxb, loading = chained ? g.waves : nblk < g.waves ? nblk : g.waves;  // blocks, waves with weights of their own
+  if (g.lds > 160 * 1024 || g.x_off < act_bytes || (g.slabs - 1) * g.CS >= C || g.CS * g.slabs < C || (g.CS % 64 && C >= 64) || g.TR * WO > BM || BM > 64 << g.lpxb || BM % 16 ||
+      g.TR % g.R || (g.whole && Ho % g.R) || (g.waves != 4 && g.waves != 8 && g.waves != 16) || (g.kp == 1 && C > 64) || (C < 64 && g.kp != 1) ||
+      g.par_off + dwpw_par(C, bn_bytes, true).bytes > g.w_off || g.w_off + loading * g.kp * 1024 > g.lds || (g.cf_per << g.lsplit) * 16 < Co ||
+      (chained && (g.lsplit || g.slabs != 1)))
     return "shape";
+  // the multiply reads blocks of 64 pixels, also where there are fewer
+  if ((C < 64 ? ((64 << g.lpxb) - 1) * C + C : (KT - 1) * 64 * g.act_px + ((64 << g.lpxb) - 1) * 64 + 64) > g.lds) return "operand past the LDS";
   if (const char *wrong = loads(C, Co < 128 ? Co : 128, g.kp, bn_bytes)) return wrong;
   const int cgs = g.CS / 16, ids[] = {0, g.tiles / 2, g.tiles - 1};
   long long outputs = 0;
   for (int t = 0; t < g.tiles; t++) outputs += dwpw_place<WO>(g, (unsigned)t).live;
   if (outputs != (long long)B * Ho * WO) return "output pixels: " + std::to_string(outputs);
-  for (const int id : ids) {
+  for (const int id : ids)
+   for (int slab = 0; slab < g.slabs; slab += g.slabs > 1 ? g.slabs - 1 : 1) {
     const DwPwPlace at = dwpw_place<WO>(g, (unsigned)id);
     // input: every place of a pixel once, from the right byte
     std::vector<int> src(x_bytes / 16, -2);  // image pixel behind a 16-byte place: -1 padding
@@ -75,7 +80,8 @@ static std::string check(int B, int C, int H, int Co, int chained, int bn_bytes,
       if (src[k.lds / 16] != -2) return "input place twice";
       src[k.lds / 16] = -1;
       if (k.off >= 0) {
-        if (k.off + 16 > dwpw_rows_in(g) * W * C) return "input offset";
+        if (slab * g.CS + k.off % C >= C) continue;  // (past the last channel: nobody reads it)
+        if (k.off + 16 > dwpw_rows_in(g) * W * C - slab * g.CS) return "input offset";
         const long long row = dwpw_first_row<S>(g, at) + k.off / C / W;
         if (row < 0 || row >= (long long)B * H) return "row outside the input";
         if (k.off % C != 16 * ((k.lds / 16) % (g.pitch / 16))) return "channel";
@@ -85,7 +91,8 @@ static std::string check(int B, int C, int H, int Co, int chained, int bn_bytes,
     // depthwise stage: every activation of a real pixel once, from the rows and columns around it
     std::vector<unsigned char> act(act_bytes / 16);
     for (int it = 0; it < cgs * g.nst; it++) {
-      const int st = (int)fastdiv((unsigned)it, g.d_n), cg = it - st * cgs;
+      const int st = (int)fastdiv((unsigned)it, g.d_n), cg = it - st * cgs, ch = slab * g.CS + 16 * cg;
+      if (ch >= C) continue;
       for (int l16 = 0; l16 < 16; l16++)
         for (int kx = 0; kx < 3; kx++) {
           const DwPwLane n = dwpw_lane<W, S>(g, st, l16, kx);
@@ -93,7 +100,7 @@ static std::string check(int B, int C, int H, int Co, int chained, int bn_bytes,
           for (int r = 0; r < g.R; r++) {
             const int px = n.px + r * WO;
             if (px < 0 || px >= BM) return "pixel";
-            const int p = dwpw_act(g, px, 16 * cg);
+            const int p = dwpw_act(g, px, ch);
             if (p < 0 || p + 16 > act_bytes || p % 16) return "activation place";
             if (n.live && kx == 0 && act[p / 16]++) return "activation twice";
             if (!n.live || px >= at.live) continue;
@@ -107,8 +114,8 @@ static std::string check(int B, int C, int H, int Co, int chained, int bn_bytes,
         }
     }
     for (int px = 0; px < g.TR * WO; px++)
-      for (int cg = 0; cg < cgs; cg++)
-        if (!act[dwpw_act(g, px, 16 * cg) / 16]) return "activation left out";
+      for (int ch = slab * g.CS; ch < C && ch < (slab + 1) * g.CS; ch += 16)
+        if (!act[dwpw_act(g, px, ch) / 16]) return "activation left out";
     if (chained)
       for (int px = 0; px < at.live; px++) {
         const int p = dwpw_next_x<W>(g, px);
@@ -135,7 +142,11 @@ static std::string every()
                     if (dwpw_refusal(B, C, W, Ho, W / S, co, S, chained ? 2 : 1, cus, bn)) continue;
                     DwPwTile g;
                     taken++;
-                    if (dwpw_shape(B, C, H, W, Ho, co, S, chained, cus, bn, &g) && g.lds <= 160 * 1024) continue;
+                    if (!chained && dwpw_small16(B, C, W, Ho, co, S, cus)) {  // dwpw16_kernel: items of two rows, constants of 1024 channels, 64 KB
+                      const int split = dwpw16_split((B * Ho * 8 + DWPW16_PX - 1) / DWPW16_PX, co, cus);
+                      if (Ho % 2 == 0 && C % 64 == 0 && ((co + 63) / 64 + split - 1) / split <= 16 && dwpw16_lds(C, co, split, bn) <= 65536) continue;
+                    }
+                    else if (dwpw_shape(B, C, H, W, Ho, co, S, chained, cus, bn, &g) && g.lds <= 160 * 1024) continue;
                     char what[256];
                     snprintf(what, sizeof what, "taken, but no tile fits: %d %d %d %d %d %d %d %d %d", B, C, H, W, co, S, chained, bn, cus);
                     return what;

@@ -22,6 +22,9 @@ def test_tiles_on_the_host(tmp_path):
                         blocks.append((r.choice([1, 2, 4, 7, 60, 64, 256]), C, H, W, Co, S, chained, r.choice([4, 8]), r.choice([64, 256])))
     every = subprocess.run([exe], input="every", stdout=subprocess.PIPE, text=True, timeout=110).stdout.strip()
     assert every.isdigit() and int(every) > 5000000, every
+    # (more images and channels than a tile has room for at once, and slabs of different widths)
+    blocks += [(b, C, H, W, Co, S, 0, bn, 256) for W, H, S in ((4, 4, 1), (8, 8, 1), (8, 8, 2), (16, 16, 2), (16, 3, 2), (64, 20, 1)) for C in (64, 192, 448, 704, 1024)
+               for b in (40, 300, 513, 1025) for Co in (48, 512) for bn in (4, 8) if b * H * W * C < 4e7]
     res = subprocess.run([exe], input="\n".join(" ".join(map(str, b)) for b in blocks), stdout=subprocess.PIPE, stderr=subprocess.PIPE, text=True,
                          timeout=110)
     said = res.stdout.split("\n")[:-1]

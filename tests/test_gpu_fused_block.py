@@ -27,7 +27,16 @@ GEOMS = [
     (300, 8, 8, 64, 16, 1),      # many small images, a single 16-channel output group
     (9, 8, 16, 320, 96, 2),      # H = 8, W = 16, five K slices (two passes over the weights)
     (4, 8, 8, 64, 2048, 1),      # 2048 output channels: legal because so few images are split over workgroups by channels
+    (70, 16, 16, 448, 64, 2),    # input in two slabs of different widths, more planes than dwpw16_kernel takes
+    (65, 16, 16, 128, 80, 2),
     (5, 3, 16, 1024, 256, 2),    # two output rows of 1024 channels
+    (3, 4, 16, 192, 48, 2),      # tiles over two images, the last one half full
+    (1, 16, 16, 640, 1024, 2),   # a tile shared by many workgroups
+    (3, 12, 64, 320, 48, 1),     # one row a tile
+    (40, 20, 64, 64, 32, 1),     # a last tile of fewer rows
+    (600, 8, 8, 64, 16, 1),      # several images a tile, the last tile not full
+    (601, 4, 4, 512, 64, 1),
+    (300, 8, 8, 512, 64, 2),
 ]
 FLAGS = [((1, 1), (1, 1)), ((1, 0), (1, 1)), ((1, 1), (1, 0)), ((0, 0), (0, 0)), ((2, 0), (0, 1))]
 
@@ -95,6 +104,57 @@ def test_fused_block(geom, flags, bn_bits):
     assert mid.max() > 0 and (mid < 255).any() and want.max() > 0 and (want < 255).any(), "degenerate case"
 
 
+@pytest.mark.parametrize("bn_bits", [32, 64])
+@pytest.mark.parametrize("geom", [(3, 8, 8, 128, 48, 1, 1), (3, 16, 16, 192, 32, 2, 1), (70, 16, 16, 128, 32, 2, 1), (2, 32, 32, 32, 16, 2, 1), (2, 8, 8, 256, 256, 1, 3),
+                                  (2, 16, 16, 64, 64, 1, 2)], ids=lambda g: "x".join(map(str, g)))
+def test_requantisation_forms_and_unaligned_parameters(geom, bn_bits):
+    """Blocks and chains with multipliers past the fast forms, shifts below 16, and filters, biases and constants that start anywhere."""
+    B, H, W, C, Co, stride, nb = geom
+    r = rng_for(9700 + C + Co)
+
+    def anywhere(a, step):                      # a copy on the GPU, `step` bytes behind an aligned address
+        if a is None:
+            return None
+        t = torch.zeros(a.nbytes + 16, dtype=torch.uint8, device="cuda")
+        t[step:step + a.nbytes] = torch.from_numpy(np.ascontiguousarray(a).view(np.uint8).reshape(-1).copy()).cuda()
+        return t.data_ptr() + step, t
+
+    L = nn(bn_bits)
+    for form in ("large", "mult 14", "mult 16", "raw"):
+        relu, bn, shift, mult = {"large": (1, 1, 17, 0), "mult 14": (1, 0, 14, 700), "mult 16": (1, 0, 16, 700), "raw": (0, 0, 7, 0)}[form]
+        x = cur = rand_u8(r, (B, H, W, C))
+        blocks, keep = [], []
+        for j in range(nb):
+            args = []
+            for n, ch in ((0, C), (1, Co)):
+                w, b = rand_s8(r, (ch, 3, 3) if n == 0 else (Co, 1, 1, C)), rand_s8(r, (ch,))
+                k, lam = r.integers(256, 1025, ch), r.integers(-2 ** 16, 2 ** 16 + 1, ch)
+                k[ch // 2] = 2 ** 25 if bn_bits == 32 else 2 ** 33       # past the fast multiplier: 24 or 32 bits
+                if n == 0:
+                    mid = oracle.depthwise_generic(np.ascontiguousarray(cur.transpose(0, 3, 1, 2)), w, b, k, lam, mult, shift, (1, 1, 1, 1),
+                                                   (stride, stride), relu, bn, bn_bits)
+                else:
+                    cur = oracle.pointwise(mid, w, b, k, lam, mult, shift, relu, bn, bn_bits)
+                t = np.int64 if bn_bits == 64 else np.int32
+                step = t().nbytes
+                dev_args = [anywhere(w, 16 if n else 1 + j), anywhere(b, 3), anywhere(k.astype(t), step), anywhere(lam.astype(t), step)]
+                keep.append(dev_args)
+                args += [a[0] for a in dev_args] + [mult, shift, relu, bn]
+            blocks.append(tuple(args))
+        out = torch.full(cur.shape, 0xA5, dtype=torch.uint8, device="cuda")
+        L.set_batch(B)
+        try:
+            if nb > 1:
+                L.dw_pw_chain_hwc(dev(x), out, W, H, C, blocks)
+            else:
+                L.dw_pw_hwc(dev(x), out, W, H, C, cur.shape[2], cur.shape[1], Co, stride, *blocks[0])
+            L.sync()
+        finally:
+            L.set_batch(1)
+        assert np.array_equal(out.cpu().numpy(), cur), form
+        assert mid.max() > 0 and cur.max() > 0, "degenerate case"
+
+
 def test_fused_block_rejects_what_it_cannot_do():
     L = nn(32)
     x = torch.zeros((1, 12, 12, 64), dtype=torch.uint8, device="cuda")      # width 12: no kernel
@@ -132,6 +192,9 @@ CHAINS = [
     (3, 8, 8, 384, 2),       # 64-pixel x 32-channel blocks of the pointwise stage: two passes over K
     (2, 8, 8, 192, 3),       # ... three K slices
     (3, 4, 8, 128, 2),       # tiles of 32 pixels: blocks of 32 pixels x 64 channels
+    (2, 16, 16, 32, 3),      # rows of 32 and of 16 bytes of activations
+    (4, 16, 4, 16, 2),
+    (4, 4, 4, 192, 2),       # strips of four rows, so that no wave takes two
 ]
 
 
