@@ -47,6 +47,8 @@ void depthwise_common(const char *fn, const uint8_t *in, const int8_t *bias, uin
                      Wo == ho_plane && CH % DW_CG == 0 && aligned(in, hwc_in ? 4 : 16) && aligned(out, 4) &&
                      (long long)g.B * g.cgroups <= 0x7fffffffLL;
   // rows of 16, 32 or 64 bytes, padding 1, any height: a few rows of a plane per lane, in registers
+  // (Batch x channels of whole groups of 64: dw3x3_rows_kernel needs it.  The HWC kernel on the matrix cores does not, but HWC layers
+  // have no other kernel, and which calls are refused does not depend on how a buffer is aligned.)
   const bool rowsk = !plane && fast && pt == 1 && pl == 1 && (W == 16 || W == 32 || W == 64) && Wo == (W - 1) / sx + 1 &&
                      Ho <= (H - 1) / sy + 1 && CH % 4 == 0 && ((long long)g_batch * CH) % DW_CG == 0 && aligned(in, hwc_in ? 4 : 16) &&
                      aligned(out, 4) && (long long)g_batch * CH / DW_CG * Ho < 0x7fffffffLL;
@@ -85,8 +87,9 @@ void depthwise_common(const char *fn, const uint8_t *in, const int8_t *bias, uin
                       (long long)g_batch * (CH / DW_CG) >= 2ll * num_cus();
   if (hwc_in && !plane && !rowsk)
     return set_error(PULP_NN_HIP_ERR_UNSUPPORTED, fn, "no fused kernel for this geometry: use pulp_nn_hip_hwc_to_chw and the CHW entry point");
-  // HWC rows of 16, 32 or 64 pixels: on the matrix cores where the channels are whole tiles and the maps 16-byte aligned.  (16-pixel
-  // rows at stride 2 and 8 x 8 and 4 x 4 planes stay in registers: 4.4 and 3.1-3.9 us at batch 256, of which 3 are the launch.)
+  // HWC rows of 16, 32 or 64 pixels: on the matrix cores where the channels are whole tiles, the maps 16-byte aligned and the layer not one
+  // of the large ones that dwh_wide names.  (16-pixel rows at stride 2 and 8 x 8 and 4 x 4 planes stay in registers: 4.4 and 3.1-3.9 us
+  // at batch 256, of which 3 are the launch.)
   if (hwc_in && rowsk) {
     const DwLayer L = {in, wt, bias, out, (int)g_batch, CH, H, W, Ho, Wo, kx, ky, pt, pl, sx, sy};
     if (launch_dw_hwc(mode, L, e, num_cus(), g_stream)) return check_launch(fn);

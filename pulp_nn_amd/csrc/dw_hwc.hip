@@ -18,7 +18,7 @@ bool launch(int mode, const DwLayer &L, const EpiArgs &e, int cus, hipStream_t s
 
 bool launch_dw_hwc(int mode, const DwLayer &L, const EpiArgs &e, int cus, hipStream_t s)
 {
-  if (!aligned(L.in, 16) || !aligned(L.out, 16)) return false;
+  if (!aligned(L.in, 16) || !aligned(L.out, 16) || dwh_wide(L)) return false;
   if (L.sx == 1) return launch<64, 1>(mode, L, e, cus, s) || launch<32, 1>(mode, L, e, cus, s) || launch<16, 1>(mode, L, e, cus, s);
   return launch<64, 2>(mode, L, e, cus, s) || launch<32, 2>(mode, L, e, cus, s);
 }

@@ -76,6 +76,14 @@ PULPNN_HD int dwh_lds(int col, int chunk)
 template <int W>
 PULPNN_HD constexpr int dwh_row_bytes() { return (W + 2) * (64 / W) * 16; }
 
+#define DWH_LARGE (64ll << 20)  // input and output, bytes
+inline long long dwh_bytes(const DwLayer &L) { return (long long)L.B * L.CH * ((long long)L.H * L.W + (long long)L.Ho * L.Wo); }
+// Large layers of rows of 64 pixels and 128 channels or more, where dw3x3_rows_kernel, which reads 64 channels of a pixel at a time, is
+// the faster one; here / there: stride 1 64x64x128 batch 45 (47 MB in and out) 16.8 / 16.1 us, 91 37.1 / 33.4, 64x64x512 batch 22 36.9 / 33.6, 45 67.8 /
+// 60.8, 35x64x128 batch 167 36.7 / 35.9, but 7x64x256 batch 418 36.3 / 38.8; stride 2 64x64x192 batch 61 (59 MB) 17.0 / 18.8, 122 42.7 / 35.7, 35x64x512
+// batch 83 43.6 / 39.2, 7x64x256 batch 837 43.4 / 35.8.
+inline bool dwh_wide(const DwLayer &L) { return L.W == 64 && L.CH >= 128 && (L.sx == 2 || L.Ho >= 16) && dwh_bytes(L) > DWH_LARGE; }
+
 // False for a layer the kernel does not take.
 template <int W, int S>
 bool dwh_shape(const DwLayer &L, int cus, DwhGeom *out)
@@ -94,12 +102,25 @@ bool dwh_shape(const DwLayer &L, int cus, DwhGeom *out)
   g.H = L.H;
   g.Ho = L.Ho;
   g.cblocks = L.CH / (16 * NT);
-  // As many rows per wave as leave every SIMD one wave, at most 16: a wave reads two (stride 2: one) rows more than it needs by
-  // itself, and sets up its channels' operands, some 100 instructions, for all of its rows.  Call by call, rows per wave 2 / 4 / 8 /
-  // 16 at batch 256: 64x64x16 12.9 / 9.4 / 9.3 / 9.1 us, 32x32x64 14.0 / 10.0 / 9.5 / 8.7; batch 64 4.8 / 4.3 / 5.0 / 6.7 and 5.3 / 4.5 / 5.4 / 7.0.
-  g.R = 16;
-  while (g.R > 1 && (long long)L.B * ((L.Ho + g.R - 1) / g.R) * g.cblocks < 4ll * cus) g.R /= 2;
-  g.bands = (L.Ho + g.R - 1) / g.R;
+  // Rows per wave, 16 or a fraction of it: a wave walks down its rows one after the other and reads up to two more than it needs by
+  // itself, and a SIMD whose waves are all resident takes about as long as that for each of them.  So the least product of rows and
+  // rounds, in bands of one height (35 rows are 12 + 12 + 11, not 16 + 16 + 3), and the more rows where two are equal.  Rows per wave 2 / 4 /
+  // 8 / 16 at batch 64 (1024 waves at 4 rows) 64x64x16 4.8 / 4.3 / 5.0 / 6.7 us, at batch 256 12.9 / 9.4 / 9.3 / 9.1; 16x16x128 batch 244 (976 waves at 8 rows)
+  // 4 / 8 rows 7.8 / 6.9, 35x32x128 batch 55 (1980, 1100) 7.2 / 9.0; 35x64x32 batch 334 16 + 16 + 3 rows 11.3, 12 + 12 + 11 10.3.
+  // At most 8 in large layers where a wave's 16 or 32 bytes of a pixel are a small part of it: the waves that read the rest of its lines
+  // run apart from each other, the further the more rows they walk, and the lines are gone when they come.  8 / 16 rows: 64x64x64 batch 256
+  // 40.9 / 43.4 us, 32x32x1024 batch 45 35.7 / 40.2, stride 2 64x64x512 batch 22 19.5 / 23.7, but 64x64x64 batch 256 24.8 / 21.8.
+  const int least = S == 1 ? 4 : 2;  // rows that the kernel's loop does at a time
+  long long cost = 0;
+  for (int R = dwh_bytes(L) > DWH_LARGE && NT < 4 && g.cblocks > 2 * S ? 8 : 16; R >= 1; R /= 2) {
+    const int even = (L.Ho + (L.Ho + R - 1) / R - 1) / ((L.Ho + R - 1) / R), rows = even > least ? (even + least - 1) / least * least : even;
+    const int bands = (L.Ho + rows - 1) / rows;
+    const long long waves = (long long)L.B * bands * g.cblocks, c = (waves + 4 * cus - 1) / (4 * cus) * (S * even + 2);
+    if (cost && c >= cost) continue;
+    cost = c;
+    g.R = rows;
+    g.bands = bands;
+  }
   const long long total = (long long)L.B * g.bands * g.cblocks;
   if (total > 0x7fffffffLL - 4) return false;
   g.total = (int)total;

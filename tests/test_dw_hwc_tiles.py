@@ -28,3 +28,16 @@ def test_rows_on_the_host(tmp_path):
     for l, s in zip(layers, said):
         assert s.startswith("ok") or (s == "no" and l[0] * l[1] * l[2] * l[3] + l[3] * l[1] >= 2 ** 31 - 1), "layer %s: %s" % (l, s)
     assert sum(s == "no" for s in said) == 5
+
+
+def test_bands_are_even(tmp_path):
+    """Bands of nearly one height; the rows that a wave takes are few where that leaves no SIMD a second wave, and where many waves share the
+    lines of a pixel in a large layer."""
+    exe = str(tmp_path / "dw_hwc_walk")
+    subprocess.run(["g++", "-O1", "-std=c++17", os.path.join(HERE, "host", "dw_hwc_walk.cpp"), "-o", exe], check=True)
+    cases = [((334, 32, 35, 64, 35, 1, 256), 12), ((334, 32, 19, 64, 19, 1, 256), 8), ((244, 128, 16, 16, 16, 1, 256), 8),
+             ((55, 128, 35, 32, 35, 1, 256), 4), ((64, 128, 11, 16, 11, 1, 256), 2), ((64, 16, 64, 64, 64, 1, 256), 4), ((256, 16, 64, 64, 64, 1, 256), 16),
+             ((45, 1024, 32, 32, 32, 1, 256), 8), ((22, 512, 64, 64, 32, 2, 256), 8), ((256, 64, 64, 64, 32, 2, 256), 16), ((1, 16, 3, 64, 3, 1, 256), 1)]
+    res = subprocess.run([exe], input="\n".join(" ".join(map(str, c[0])) for c in cases), stdout=subprocess.PIPE, text=True, timeout=100)
+    for (c, rows), s in zip(cases, res.stdout.split("\n")):
+        assert s == "ok %d" % rows, (c, s)
