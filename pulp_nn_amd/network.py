@@ -194,7 +194,7 @@ class Runner:
 
     # -- buffers ----------------------------------------------------------------------------
     _asked = frozenset()     # depthwise layers (indices) whose results the caller has asked for
-    _left_out = frozenset()  # ... whose results the last run left out because their blocks are small
+    _left_out = ()           # ... whose results the last run left out because their blocks are small
 
     def _buffer(self, name):
         return dict.__getitem__(self.act, name)
@@ -330,7 +330,7 @@ class Runner:
         tensors = {"input": x, **{L["name"]: self._buffer(L["name"]) for L in self.layers[:first]}}
         out = x
         self.launches = launches
-        self._left_out = frozenset(i for i in self._left_out if i < first)
+        left_out = self._left_out = [i for i in self._left_out if i < first]
         recorded, readers = nn is not self.nn, None
         i = first
         while i < len(self.layers):
@@ -346,10 +346,11 @@ class Runner:
                 out = tensors[last] = self._buffer(last)
                 i += 2 * n
                 continue
-            if block and self._block_fusable(i, readers=readers) and self._queue_block(i, tensors, nn):
+            small = block and self._small(i)
+            if block and self._block_fusable(i, readers=readers, small=small) and self._queue_block(i, tensors, nn):
                 out = tensors[self.layers[i + 1]["name"]] = self._buffer(self.layers[i + 1]["name"])
-                if self._small(i):
-                    self._left_out |= {i}
+                if small:
+                    left_out.append(i)
                 i += 2
                 continue
             out = tensors[L["name"]] = self._queue(i, tensors, nn)
@@ -358,9 +359,10 @@ class Runner:
         return out
 
     # -- depthwise + pointwise as one launch ------------------------------------------------
-    def _block_fusable(self, i, policy=True, readers=None):
+    def _block_fusable(self, i, policy=True, readers=None, small=None):
         """Layer i is a 3x3 / padding 1 depthwise layer whose only reader is the pointwise layer i + 1.
-        policy=False: only whether the block can be one launch, not whether it pays on its own.  readers: _reader_counts()."""
+        policy=False: only whether the block can be one launch, not whether it pays on its own.
+        readers, small: _reader_counts() and _small(i), where the caller has them."""
         if not (self.fused and self.fuse_blocks) or i in self.unfused_blocks or i + 1 >= len(self.layers):
             return False
         L, N = self.layers[i], self.layers[i + 1]
@@ -371,7 +373,8 @@ class Runner:
         # pixels, a whole image per workgroup (two launches / one at batch 256: 16x16x128 -> 256 at stride 2 10.2 / 8.1 us,
         # 8x8x256 11.6 / 8.8), and small blocks
         if policy and self.fuse_blocks == "auto":
-            if not (self.block_choice[i] if i in self.block_choice else self.shapes[L["name"]][:2] == (8, 8) or self._small(i)):
+            if not (self.block_choice[i] if i in self.block_choice else self.shapes[L["name"]][:2] == (8, 8) or
+                    (self._small(i) if small is None else small)):
                 return False
         sx, sy = L["strides"]
         if L["w"].shape[1:3] != (3, 3) or tuple(L["pads"]) != (1, 1, 1, 1) or sx != sy:
