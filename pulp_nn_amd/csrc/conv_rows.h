@@ -4,16 +4,18 @@
 // A filter row of a pixel is kx * Ci contiguous bytes of the HWC input, so the four 16-byte slots of K of one v_mfma_i32_16x16x64_i8
 // are the filter's rows: a lane fetches 16 bytes from the dword below a row's first byte and shifts them into place, and 16 pixels x 16 channels are one instruction, whatever the geometry.
 // Bytes behind a row's end meet zero weights; columns outside the image are cleared, and rows outside it, where a wave has any; the
-// first and the last bytes of the tensor are met by clamping the address and shifting.  The filters are fetched the same way.  No LDS, no
-// barrier: a wave is an independent item.
+// first and the last bytes of the tensor are met by clamping the address and shifting.  The filters are fetched the same way.  No barrier:
+// a wave is an independent item.  LDS is used in two places, a part of it per wave, and relies on a wave's accesses being served in order: for
+// the input of rows of 64 output pixels (ROWS_ROW64 below), and for results of 33 to 63 channels.
 //
 // Rows of the MFMA are dealt so that a lane ends up with 4 * NT consecutive channels of its pixel (dw_hwc.h); with NT == 1 and 16
 // channels in all, the four pixels of a lane's four units change places between lanes and a store is 16 bytes a lane, 1 KB in memory order.
 //
 // Replaces v_dot4 with one pixel per lane, which took 370 vector instructions per 64 pixels and 16 channels, and the band in LDS
-// (conv_band.h) for such filters of more than 32 channels.  Bound: memory latency, at two to four groups of 64 pixels per wave.  Call by
-// call, before / now: 128x128x3 -> 16 stride 2 batch 256 15.2 / 13.3 us, batch 1 4.2 / 4.0; 32x32x3 -> 64 batch 64 8.9 / 6.5, batch 1 5.7 / 4.7;
-// 57x43x3 -> 40 batch 64 21.8 / 11.0; 64x64x4 -> 256 batch 32 37.5 / 18.7; 64x64x5 -> 16 stride 2 batch 64 6.5 / 4.1; 64x64x16 -> 32 1x1 6.9 / 3.6.
+// (conv_band.h) for such filters of more than 32 channels.  Bound: memory latency, at one to eight groups of 64 pixels per wave (rows_shape).
+// Call by call, before / now: 128x128x3 -> 16 stride 2 batch 256 15.8 / 13.1 us, batch 1 4.2 / 4.0; 32x32x3 -> 64 batch 64 8.9 / 5.8, batch 1 5.7 / 4.7;
+// 57x43x3 -> 40 batch 64 21.8 / 11.0; 64x64x4 -> 256 batch 32 37.5 / 18.7; 64x64x5 -> 16 stride 2 batch 64 6.5 / 4.1; 64x64x16 -> 32 1x1 6.9 / 3.6.  A few
+// small filters of few channels are slower: 64x64x1 -> 6 batch 256 13.8 / 15.3, 191x16x3 -> 16 3x1 batch 286 14.1 / 15.8, 5x20x1 -> 16 2x2 3.6 / 4.0.
 // Reference semantics:
 // 32bit/src/pulp_nn_conv_Ho_parallel.c:76-183 (im2col order ky, kx, ci) and pulp_nn_matmul.c:144-216 (requantisation).
 #pragma once
@@ -51,13 +53,22 @@ __global__ __launch_bounds__(256, NT == 4 ? 2 : 4) void conv_rows_kernel(RowsGeo
 
   // ---- the first pixels ------------------------------------------------------------------------------------------------------
   constexpr bool ROW16 = PLACE != ROWS_ANY, STAGED = PLACE == ROWS_ROW64;
-  __shared__ __attribute__((aligned(16))) unsigned char rows_l[4][STAGED ? 4 * ROWS_PITCH : 16];
+  // Whether results can be put together in LDS: with four tiles.  (With fewer tiles the way there is longer than their few odd stores, 13x30x2 -> 7
+  // 3x2 batch 13 4.6 / 5.2 us, 102x128x5 -> 26 3x3 batch 18 8.6 / 9.4; in the 64-bit build it takes the registers of a third wave per SIMD, 20x16x4 ->
+  // 261 4x3 batch 45 10.5 / 11.5.)
+  constexpr bool GATHER = NT == 4 && sizeof(bn_t) == 4;
+  __shared__ __attribute__((aligned(16))) unsigned char rows_l[4][GATHER ? 1024 * NT : STAGED ? 4 * ROWS_PITCH : 16];
   unsigned char *mine = rows_l[wave];
   int grp = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 * g.npass + wave);
   RowsWindow win[4];
   v4i v[4];
   int more[4] = {0, 0, 0, 0};
-  const int loff = rows_lane(g, ROW16 ? l16 : 0, lgrp);
+  // The slots of rows that the filter does not have meet zero weights: they repeat its last row, and ask neither for memory of their own nor
+  // for a look at the image's edges; 158x198x2 -> 7 4x1 batch 253 111 us with rows of their own, 80 so.  (Leaving them out of the load is worse: a
+  // load that not all lanes take part in is waited for as a whole, 5x20x1 -> 16 2x2 4.0 / 4.5.)
+  const bool has_row = lgrp < g.ky;
+  const int slot = min(lgrp, g.ky - 1);
+  const int loff = rows_lane(g, ROW16 ? l16 : 0, slot);
   typedef v4i v4i_4 __attribute__((aligned(4)));
   auto request = [&]() {
     if constexpr (STAGED) {
@@ -66,7 +77,7 @@ __global__ __launch_bounds__(256, NT == 4 ? 2 : 4) void conv_rows_kernel(RowsGeo
       for (int u = 0; u < 4; u++) win[u] = RowsWindow{w.at + 16 * u * g.sx * g.Ci, w.iy, w.ix + 16 * u * g.sx};
 #pragma unroll
       for (int i = 0; i < 2; i++) {
-        const int fy = 2 * i + (lane >> 5);
+        const int fy = min(2 * i + (lane >> 5), g.ky - 1);
         v[i] = *(const v4i_4 *)(g.in + (unsigned)rows_chunk_at(g, w.at + fy * g.W * g.Ci, min(lane & 31, rows_chunks(g) - 1)));
       }
       return;
@@ -83,69 +94,102 @@ __global__ __launch_bounds__(256, NT == 4 ? 2 : 4) void conv_rows_kernel(RowsGeo
   };
   request();
 
-  // ---- filters and constants ---------------------------------------------------------------------------------------------------
+  // ---- filters and constants, all of them requested before the first is used ---------------------------------------------------------
   // Row i of tile t is channel 4 * NT * (i / 4) + 4 * t + i % 4; slot lgrp of it the channel's filter row lgrp.
   v4i A[NT];
-  {
-    const int wbytes = g.N * g.K;
-    int off[NT];
+  const int wbytes = g.N * g.K;
+  int off[NT];
 #pragma unroll
-    for (int t = 0; t < NT; t++) {
-      off[t] = (n0 + 4 * NT * (l16 >> 2) + 4 * t + (l16 & 3)) * g.K + lgrp * g.L;
-      A[t] = *(const v4i_u *)(g.w + (unsigned)max(min(off[t], wbytes - 16), 0));
-    }
-    const bool row = lgrp < g.ky;
-#pragma unroll
-    for (int t = 0; t < NT; t++) {
-      const bool ok = row && off[t] < wbytes;
-      const int late = ok ? off[t] - max(min(off[t], wbytes - 16), 0) : 0;
-      if (__any(late > 0)) A[t] = bytes_shift(A[t], late);
-#pragma unroll
-      for (int d = 0; d < 4; d++) A[t][d] = ok ? (int)((unsigned)A[t][d] & below(g.L - 4 * d)) : 0;
-    }
+  for (int t = 0; t < NT; t++) {
+    off[t] = (n0 + 4 * NT * (l16 >> 2) + 4 * t + (l16 & 3)) * g.K + lgrp * g.L;
+    A[t] = *(const v4i_u *)(g.w + (unsigned)max(min(off[t], wbytes - 16), 0));
   }
   const int cb = n0 + 4 * NT * lgrp;  // the lane's channels
+  typedef bn_t bn4 __attribute__((ext_vector_type(4), aligned(sizeof(bn_t))));
+  const bn_t same = mode == EPI_MULT ? (bn_t)e.mult : (bn_t)1;
   bn_t kk[NT][4], ll[NT][4];
+  int bias[NT];  // four bytes
+#pragma unroll
+  for (int t = 0; t < NT; t++) {
+    bias[t] = 0;
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      kk[t][r] = same;
+      ll[t][r] = 0;
+    }
+  }
+  if (g.N >= 4) {
+    // (past the last channel the last four, turned into place further down)
+#pragma unroll
+    for (int t = 0; t < NT; t++) {
+      const int c = min(cb + 4 * t, g.N - 4);
+      if (g.bias) bias[t] = *(const i32_u *)(g.bias + c);
+      if (mode == EPI_BN) {
+        const bn4 k = *(const bn4 *)(e.k + c), l = *(const bn4 *)(e.lambda + c);
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          kk[t][r] = k[r];
+          ll[t][r] = l[r];
+        }
+      }
+    }
+  } else {
+    for (int c = 0; c < g.N; c++) {
+      if (g.bias) bias[0] |= (int)(uint8_t)g.bias[c] << (8 * c);
+      if (mode == EPI_BN) {
+#pragma unroll
+        for (int r = 0; r < 3; r++) {
+          if (r != c) continue;
+          kk[0][r] = e.k[c];
+          ll[0][r] = e.lambda[c];
+        }
+      }
+    }
+  }
+  if (g.N >= 4 && n0 + 16 * NT > g.N && (g.N & 3)) {
+#pragma unroll
+    for (int t = 0; t < NT; t++) {
+      const int by = cb + 4 * t - min(cb + 4 * t, g.N - 4);  // (channels from by = 4 on do not exist)
+      bias[t] = (int)((unsigned)bias[t] >> (8 * (by & 3)));
+#pragma unroll
+      for (int turn = 1; turn < 4; turn *= 2) {
+        bn_t k[4], l[4];
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          k[r] = by & turn ? kk[t][(r + turn) & 3] : kk[t][r];
+          l[r] = by & turn ? ll[t][(r + turn) & 3] : ll[t][r];
+        }
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          kk[t][r] = k[r];
+          ll[t][r] = l[r];
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < NT; t++) {
+    const bool ok = has_row && off[t] < wbytes;
+    const int late = ok ? off[t] - max(min(off[t], wbytes - 16), 0) : 0, keep = ok ? -1 : 0;
+    if (__any(late > 0)) A[t] = bytes_shift(A[t], max(late, 0));
+#pragma unroll
+    for (int d = 0; d < 4; d++) A[t][d] &= (int)below(g.L - 4 * d) & keep;
+  }
   bool ks = true;
 #pragma unroll
   for (int t = 0; t < NT; t++) {
     const v4i ones = {0x01010101, 0x01010101, 0x01010101, 0x01010101}, zero = {0, 0, 0, 0};
     const v4i s = __builtin_amdgcn_mfma_i32_16x16x64_i8(A[t], ones, zero, 0, 0, 0);
-    typedef bn_t bn4 __attribute__((ext_vector_type(4), aligned(sizeof(bn_t))));
-    bn4 k, l = {0, 0, 0, 0};
-    int b[4] = {0, 0, 0, 0};
-    const bn_t same = mode == EPI_MULT ? (bn_t)e.mult : (bn_t)1;
-    k = (bn4){same, same, same, same};
-    const int c = cb + 4 * t;
-    if (n0 + 16 * NT <= g.N) {
-      const int bytes = g.bias ? *(const i32_u *)(g.bias + c) : 0;
-#pragma unroll
-      for (int r = 0; r < 4; r++) b[r] = (int)(int8_t)((unsigned)bytes >> (8 * r));
-      if (mode == EPI_BN) {
-        k = *(const bn4 *)(e.k + c);
-        l = *(const bn4 *)(e.lambda + c);
-      }
-    } else {
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const int cr = min(c + r, g.N - 1);
-        b[r] = g.bias ? (int)g.bias[cr] : 0;
-        if (mode == EPI_BN) {
-          k[r] = e.k[cr];
-          l[r] = e.lambda[cr];
-        }
-      }
-    }
 #pragma unroll
     for (int r = 0; r < 4; r++) {
-      const int corr = 128 * s[r] + b[r];
-      kk[t][r] = k[r];
-      ks = ks && bn_k_small(k[r]);
+      const int corr = 128 * s[r] + (int)(int8_t)((unsigned)bias[t] >> (8 * r));
+      const bn_t k = kk[t][r];
+      ks = ks && bn_k_small(k);
 #if PULPNN_BN_BITS == 64
-      if (mode == EPI_BN) ll[t][r] = (bn_t)((unsigned long long)k[r] * (unsigned long long)(long long)corr + (unsigned long long)l[r]);
+      if (mode == EPI_BN) ll[t][r] = (bn_t)((unsigned long long)k * (unsigned long long)(long long)corr + (unsigned long long)ll[t][r]);
       else
 #endif
-        ll[t][r] = (bn_t)(int)((unsigned)k[r] * (unsigned)corr + (unsigned)l[r]);
+        ll[t][r] = (bn_t)(int)((unsigned)k * (unsigned)corr + (unsigned)ll[t][r]);
     }
   }
   const int form = dwh_form(mode, e.shift, (bool)__all(ks), true);  // |acc| <= 64 * 128 * 128
@@ -160,7 +204,7 @@ __global__ __launch_bounds__(256, NT == 4 ? 2 : 4) void conv_rows_kernel(RowsGeo
       asm volatile("" ::: "memory");
 #pragma unroll
       for (int u = 0; u < 4; u++) {
-        const int *p = (const int *)(mine + ROWS_PITCH * lgrp + (((win[0].at + lgrp * g.W * g.Ci) & 3) + (16 * u + l16) * g.sx * g.Ci & ~3));
+        const int *p = (const int *)(mine + ROWS_PITCH * slot + (((win[0].at + slot * g.W * g.Ci) & 3) + (16 * u + l16) * g.sx * g.Ci & ~3));
         v[u] = (v4i){p[0], p[1], p[2], p[3]};
         if (rows_long(g)) more[u] = p[4];
       }
@@ -173,9 +217,9 @@ __global__ __launch_bounds__(256, NT == 4 ? 2 : 4) void conv_rows_kernel(RowsGeo
       if (ROW16 ? rows_edge(g, win[u]) : true) {
         RowsWindow w = win[u];
         if (ROW16) w.ix += l16 * g.sx;
-        const RowsKeep n = rows_keep(g, w, lgrp);
-        const bool end = n.row && rows_near_end(g, at);
-        if (ROW16 || __any(!n.row || end || n.lo > 0 || n.hi < g.L)) {
+        const RowsKeep n = rows_keep(g, w, slot);
+        const bool end = has_row && n.row && rows_near_end(g, at);
+        if (ROW16 || __any(has_row && (!n.row || end || n.lo > 0 || n.hi < g.L))) {
           if (__any(end)) {  // (first and last rows of the whole tensor)
             const int from = rows_exact(g, at);
             const v4i exact = bytes_shift(*(const v4i_u *)(g.in + (unsigned)from), min(max(at - from, -16), 16));
@@ -211,20 +255,55 @@ __global__ __launch_bounds__(256, NT == 4 ? 2 : 4) void conv_rows_kernel(RowsGeo
       const unsigned p[4] = {q[0][0], q[1][0], q[2][0], q[3][0]};
       const v4i o = dwh_pixels(p);
       if (m0 + lane < g.M) *(v4i_u *)(g.out + (long long)(m0 + lane) * 16) = o;
+    } else if (GATHER && g.gather) {
+      // the results of the 64 pixels are 64 * N contiguous bytes: put together in the wave's part of LDS
+      // (the channels left as a value that the compiler does not know: it would keep all comparisons with it in scalar registers)
+      int left = g.N - cb;
+      asm volatile("" : "+v"(left));
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        unsigned char *o = mine + (16 * u + l16) * g.N + cb;
+#pragma unroll
+        for (int t = 0; t < NT; t++) {
+          if (4 * t + 4 <= left) *(i32_u *)(o + 4 * t) = (int)q[u][t];
+          else
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+              if (4 * t + r < left) o[4 * t + r] = (unsigned char)(q[u][t] >> (8 * r));
+        }
+      }
+      __builtin_amdgcn_wave_barrier();
+      asm volatile("" ::: "memory");
+      const int bytes = min(64, g.M - m0) * g.N;
+      uint8_t *o = g.out + (long long)m0 * g.N;
+      for (int i = 16 * lane; i < bytes; i += 1024) {
+        if (i + 16 <= bytes) *(v4i_u *)(o + i) = *(const v4i *)(mine + i);
+        else
+          for (int j = i; j < bytes; j++) o[j] = mine[j];
+      }
+      __builtin_amdgcn_wave_barrier();
+      asm volatile("" ::: "memory");
     } else {
+      int left = g.N - cb;
+      asm volatile("" : "+v"(left));
 #pragma unroll
       for (int u = 0; u < 4; u++) {
         const int m = m0 + 16 * u + l16;
         uint8_t *o = g.out + (long long)m * g.N + cb;
         if (m >= g.M) continue;
-        if (cb + 4 * NT <= g.N) {
+        if (4 * NT <= left) {
           if constexpr (NT == 4) *(v4i_u *)o = (v4i){(int)q[u][0], (int)q[u][1 % NT], (int)q[u][2 % NT], (int)q[u][3 % NT]};
           else if constexpr (NT == 2) *(v2i_u *)o = (v2i){(int)q[u][0], (int)q[u][1 % NT]};
           else *(i32_u *)o = (int)q[u][0];
         } else {
 #pragma unroll
-          for (int c = 0; c < 4 * NT; c++)
-            if (cb + c < g.N) o[c] = (uint8_t)(q[u][c >> 2] >> (8 * (c & 3)));
+          for (int t = 0; t < NT; t++) {
+            if (4 * t + 4 <= left) *(i32_u *)(o + 4 * t) = (int)q[u][t];
+            else
+#pragma unroll
+              for (int r = 0; r < 4; r++)
+                if (4 * t + r < left) o[4 * t + r] = (uint8_t)(q[u][t] >> (8 * r));
+          }
         }
       }
     }

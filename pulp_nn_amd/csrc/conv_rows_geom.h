@@ -15,6 +15,7 @@ struct RowsGeom {
   int M, N, K, L;       // output pixels, channels, bytes of a filter and of one of its rows
   int H, W, Ci, Ho, Wo, kx, ky, pt, pl, sx, sy;
   int total;            // bytes of input
+  bool gather;          // a wave has whole pixels, not in whole pieces: worth putting together in LDS before they are stored
   int groups, npass;    // groups of 64 pixels; how many a wave takes, 4 apart
   FastDiv d_wo, d_ho;
 };
@@ -114,6 +115,7 @@ inline bool rows_shape(const uint8_t *in, const int8_t *w, const int8_t *bias, u
   g.sx = sx;
   g.sy = sy;
   g.total = (int)total;
+  g.gather = N <= 16 * nt && N % (4 * nt) != 0;
   g.groups = (int)((M + 63) / 64);
   // groups per wave: as many as leave every SIMD eight waves, at most 8 (the filters are set up once for all of them)
   const long long blocks = (N + 16 * nt - 1) / (16 * nt);

@@ -22,10 +22,25 @@ GEOMS = [  # B, H, W, Ci, Co, (kx, ky), (sx, sy), (t, b, l, r)
     (40, 20, 40, 3, 100, (3, 3), (1, 1), (1, 1, 1, 1)),      # four 16-channel groups a wave, several groups of pixels
     (300, 16, 64, 3, 32, (5, 2), (1, 1), (0, 1, 4, 0)),
 ]
+STORES = [  # channel counts whose pixels are put together before they are stored, batches that end within a group of 64 pixels
+    (253, 15, 19, 2, 7, (4, 1), (1, 1), (0, 0, 1, 1)),
+    (3, 5, 16, 13, 14, (1, 1), (1, 1), (0, 0, 0, 0)),
+    (1, 3, 23, 4, 1, (3, 3), (1, 1), (1, 1, 1, 1)),
+    (2, 5, 64, 3, 3, (3, 3), (1, 1), (1, 1, 1, 1)),
+    (70, 33, 16, 4, 47, (3, 3), (1, 1), (1, 1, 1, 1)),
+    (64, 17, 64, 3, 63, (3, 2), (1, 1), (1, 0, 1, 1)),
+    (20, 37, 49, 3, 30, (3, 3), (1, 1), (1, 1, 1, 1)),
+    (1, 2, 17, 16, 29, (1, 2), (1, 1), (1, 0, 0, 0)),
+    (9, 48, 54, 2, 7, (1, 1), (1, 1), (0, 0, 0, 0)),         # filters of fewer than 16 bytes in all
+    (5, 12, 16, 1, 15, (1, 1), (1, 1), (0, 0, 0, 0)),
+    (3, 9, 64, 1, 1, (3, 3), (1, 1), (1, 1, 1, 1)),
+    (2, 30, 33, 2, 2, (2, 1), (1, 1), (0, 0, 1, 0)),
+    (40, 24, 48, 3, 131, (3, 3), (1, 1), (1, 1, 1, 1)),      # more than one block of channels: the last one's tail by dwords
+]
 
 
 @pytest.mark.parametrize("bn_bits", [32, 64])
-@pytest.mark.parametrize("geom", GEOMS, ids=lambda g: "x".join(map(str, g[:5])) + "_%dx%d" % g[5])
+@pytest.mark.parametrize("geom", GEOMS + STORES, ids=lambda g: "x".join(map(str, g[:5])) + "_%dx%d" % g[5])
 def test_rows(geom, bn_bits):
     B, H, W, Ci, Co, (kx, ky), strides, pads = geom
     r = rng_for(8800 + Ci + Co)
