@@ -226,7 +226,7 @@ __global__ __launch_bounds__(1024) void dwpw_kernel(DwPwGeom g)
           return v;
         };
         auto put = [&](unsigned v) {
-          if (n.live) *(unsigned *)(dwpw_lds + (narrow ? px * T.C + ch : (ch >> 6) * act_step + px * 64 + ((((ch >> 4) & 3) ^ ((px >> 1) & 3)) << 4)) + 4 * lgrp) = v ^ 0x80808080u;
+          if (n.live) *(unsigned *)(dwpw_lds + DWPW_ACT_AT(narrow, T.C, act_step, px, ch) + 4 * lgrp) = v ^ 0x80808080u;
           px += WO;
         };
         dwh_with_form(c.form, [&](auto form) { dwh_walk<S, decltype(form)::value>(c, shift, T.R, next, put); });

@@ -13,24 +13,24 @@ bool launch_kp(const DwPwGeom &g)
   hipLaunchKernelGGL((dwpw_kernel<W, S, KP, CHAIN>), dim3((unsigned)g.t.tiles << g.t.lsplit), dim3(64 * g.t.waves), (size_t)g.t.lds, g_stream, g);
   return true;
 }
-template <int W, int KP>
+template <int W>
 bool launch_chain(const DwPwGeom &g)
 {
   const int lds = dwpw_chain_lds(g.t.lds, g.t.C);
   if (lds > 160 * 1024) return false;
   for (int j = 0; j < g.nblocks; j++)
     if (!aligned(g.blk[j].dw_wt, 4) || !aligned(g.blk[j].dw_bias, 4) || !aligned(g.blk[j].pw_bias, 4)) return false;
-  if (!raise_lds_limit<dwpw_chain_kernel<W, KP>>((size_t)lds)) return false;
-  hipLaunchKernelGGL((dwpw_chain_kernel<W, KP>), dim3((unsigned)g.t.tiles), dim3(1024), (size_t)lds, g_stream, g);
+  if (!raise_lds_limit<dwpw_chain_kernel<W>>((size_t)lds)) return false;
+  hipLaunchKernelGGL((dwpw_chain_kernel<W>), dim3((unsigned)g.t.tiles), dim3(1024), (size_t)lds, g_stream, g);
   return true;
 }
 template <int W, int S, bool CHAIN>
 bool launch(const DwPwGeom &g)
 {
   if constexpr (CHAIN && W <= 16) {
-    // every wave of sixteen at most one item of either stage
-    if (g.t.waves == 16 && g.t.C / 16 * g.t.nst <= 16 && g.t.C / 16 << g.t.lpxb <= 16)
-      if (g.t.C <= 64 ? launch_chain<W, 1>(g) : launch_chain<W, 4>(g)) return true;
+    // every wave of sixteen at most one item of either stage (up to 256 channels, so the four slices of K that the kernel has in LDS; tiles of 64
+    // channels or fewer have fewer waves)
+    if (g.t.waves == 16 && g.t.kp == DWPW_CHAIN_KP && g.t.C / 16 * g.t.nst <= 16 && g.t.C / 16 << g.t.lpxb <= 16 && launch_chain<W>(g)) return true;
   }
   return g.t.kp == 1 ? launch_kp<W, S, 1, CHAIN>(g) : g.t.kp == 4 ? launch_kp<W, S, 4, CHAIN>(g) : launch_kp<W, S, 8, CHAIN>(g);
 }

@@ -1,5 +1,5 @@
-// A run of depthwise + pointwise blocks whose stages give every wave of a workgroup at most one item: 16 channels of a strip, 64 pixels x
-// 16 channels (8 x 8 and 4 x 4 planes of up to 256 channels, 16 x 16 of 64).  The arithmetic and the tile of dwpw_kernel; what differs is that
+// A run of depthwise + pointwise blocks whose stages give every one of sixteen waves at most one item: 16 channels of a strip, 64 pixels x
+// 16 channels (tiles of up to 64 pixels and of 128, 192 or 256 channels, of up to 128 pixels and 128 channels).  The arithmetic and the tile of dwpw_kernel; what differs is that
 // a block is straight-line code with the next block's loads in flight: the next depthwise layer's parameters are asked for behind the
 // barrier in the middle of a block, the weights behind the multiply, the next pointwise layer's parameters behind the barrier at its end,
 // all of them to LDS, and each is waited for half a block later.
@@ -31,7 +31,8 @@ __device__ __forceinline__ void dwpw_par_load(unsigned char *par, const int8_t *
 PULPNN_HD int dwpw_chain_spare(int tile_lds, int C) { return tile_lds + dwpw_par(C, (int)sizeof(bn_t), false).bytes; }
 PULPNN_HD int dwpw_chain_lds(int tile_lds, int C) { return dwpw_chain_spare(tile_lds, C) + 1024; }
 
-template <int W, int KP>
+#define DWPW_CHAIN_KP 4  // slices of K whose weights are in LDS: all of them
+template <int W>
 __global__ __launch_bounds__(1024) void dwpw_chain_kernel(DwPwGeom g)
 {
   extern __shared__ __attribute__((aligned(16))) unsigned char dwpw_lds[];
@@ -42,24 +43,22 @@ __global__ __launch_bounds__(1024) void dwpw_chain_kernel(DwPwGeom g)
   const DwPwPlace at = dwpw_place<W>(T, blockIdx.x);
   unsigned char *xin = dwpw_lds + T.x_off;
   const int C = T.C, cgs = C / 16, nitems = cgs * T.nst, nblk = cgs << T.lpxb;
-  const bool narrow = KP == 1 && C < 64;
 
   // the wave's item of the depthwise stage and its block of the pointwise stage
   const int st = (int)fastdiv((unsigned)wave, T.d_n), ch = 16 * (wave - st * cgs), cf = wave >> T.lpxb, px0 = 64 * (wave & ((1 << T.lpxb) - 1));
   const bool dw_on = wave < nitems, pw_on = wave < nblk;
-  const int kb = 16 * lgrp;
 
-  unsigned char *wl = dwpw_lds + T.w_off + wave * (1024 * KP);  // the wave's own weights: KP slices of 16 rows of 64 bytes
+  unsigned char *wl = dwpw_lds + T.w_off + wave * (1024 * DWPW_CHAIN_KP);  // the wave's own weights: four slices of 16 rows of 64 bytes
   unsigned char *par_dw = dwpw_lds + T.par_off, *par_pw = dwpw_lds + T.lds;
   auto load_w = [&](DwPwBlockArg P) {
     typedef __attribute__((address_space(3))) void *lds_ptr_t;
     int ln = lane;  // (opaque: the address is computed when the loads are issued, not kept from block to block)
     asm volatile("" : "+v"(ln));
     const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)P->pw_w, 0, C * C, 0x00020000);
-    const unsigned off = dwpw_w_lane(C, pw_on ? cf : 0, ln, KP == 1);
+    const unsigned off = dwpw_w_lane(C, pw_on ? cf : 0, ln, false);
 #pragma unroll
-    for (int kk = 0; kk < KP; kk++) {
-      const DwPwWeight at = KP == 1 ? DwPwWeight{off, 0} : dwpw_w_slice(C, off, kk);
+    for (int kk = 0; kk < DWPW_CHAIN_KP; kk++) {
+      const DwPwWeight at = dwpw_w_slice(C, off, kk);
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr_t)(wl + 1024 * kk), 16, at.off, at.add, 0, 0);
     }
   };
@@ -97,8 +96,7 @@ __global__ __launch_bounds__(1024) void dwpw_chain_kernel(DwPwGeom g)
   // places that stay the same from block to block
   const DwPwLane n = dwpw_lane<W, 1>(T, dw_on ? st : 0, l16, min(lgrp, 2));
   const int src0 = T.x_off + n.x + ch, rowb = (W + 2) * T.pitch;
-  const int act0 = (narrow ? ch : ((ch >> 6) << T.lpxb) << 12) + 4 * lgrp;
-  const int a0 = narrow ? (px0 + l16) * C + (kb < C ? kb : 0) : (px0 + l16) * 64 + ((lgrp ^ ((l16 >> 1) & 3)) << 4);
+  const int step = 4096 << T.lpxb, a0 = DWPW_ACT_AT(false, C, step, px0 + l16, 16 * lgrp);
   // (pixels past the last one are written to a spare row)
   const int x0 = pw_on && px0 + lane < at.live ? T.x_off + dwpw_next_x<W>(T, px0 + lane) + 16 * cf : dwpw_chain_spare(T.lds, C) + 16 * lane;
   const int blocks = g.nblocks;
@@ -146,7 +144,7 @@ __global__ __launch_bounds__(1024) void dwpw_chain_kernel(DwPwGeom g)
           return v;
         };
         auto put = [&](unsigned v) {
-          if (n.live) *(unsigned *)(dwpw_lds + act0 + (narrow ? px * C : px * 64 + ((((ch >> 4) & 3) ^ ((px >> 1) & 3)) << 4))) = v ^ 0x80808080u;
+          if (n.live) *(unsigned *)(dwpw_lds + DWPW_ACT_AT(false, C, step, px, ch) + 4 * lgrp) = v ^ 0x80808080u;
           px += W;
         };
         dwh_with_form(form, [&](auto f) { dwh_walk<1, decltype(f)::value>(c, shift, T.R, next, put); });
@@ -164,15 +162,14 @@ __global__ __launch_bounds__(1024) void dwpw_chain_kernel(DwPwGeom g)
     for (int s = 0; s < 4; s++) acc[s] = (v4i){0, 0, 0, 0};
     {
       const unsigned char *a = dwpw_lds + a0, *w = wl + l16 * 64 + ((lgrp ^ ((l16 >> 1) & 3)) << 4);
-      const int sstep = narrow ? 16 * C : 1024;
 #pragma unroll
-      for (int kk = 0; kk < KP; kk++) {
-        if (KP == 1 || 64 * kk < C) {
+      for (int kk = 0; kk < DWPW_CHAIN_KP; kk++) {
+        if (64 * kk < C) {
           v4i af[4];
           const v4i wf = *(const v4i *)(w + 1024 * kk);
 #pragma unroll
-          for (int s = 0; s < 4; s++) af[s] = *(const v4i *)(a + s * sstep);
-          a += 4096 << T.lpxb;
+          for (int s = 0; s < 4; s++) af[s] = *(const v4i *)(a + s * 1024);
+          a += step;
           wacc = __builtin_amdgcn_mfma_i32_16x16x64_i8(wf, ones, wacc, 0, 0, 0);
 #pragma unroll
           for (int s = 0; s < 4; s++) acc[s] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wf, af[s], acc[s], 0, 0, 0);
@@ -193,7 +190,7 @@ __global__ __launch_bounds__(1024) void dwpw_chain_kernel(DwPwGeom g)
         for (int s = 0; s < 4; s++) v[s] = dwh_requant<decltype(f)::value>(acc[s], kk, ll, shift);
         *(v4i *)(dwpw_lds + x0) = dwh_pixels(v) ^ (int)0x80808080;
       });
-    __builtin_amdgcn_s_waitcnt(DWPW_WAIT_VM(KP));  // the next depthwise stage's parameters: all but the weights
+    __builtin_amdgcn_s_waitcnt(DWPW_WAIT_VM(DWPW_CHAIN_KP));  // the next depthwise stage's parameters: all but the weights
     dwpw_barrier();
     load_pw(dwpw_block(j + 1));  // (everybody has read this block's)
   }
