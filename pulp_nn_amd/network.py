@@ -327,7 +327,8 @@ class Runner:
     def _walk(self, x, nn, first=0, launches=0):
         """Queues the layers from `first` on, the ones before it being queued in `launches` launches."""
         nn.set_batch(self.batch)
-        tensors = {"input": x, **{L["name"]: self._buffer(L["name"]) for L in self.layers[:first]}}
+        act, held = self.act, dict.__getitem__
+        tensors = {"input": x, **{L["name"]: held(act, L["name"]) for L in self.layers[:first]}}
         out = x
         self.launches = launches
         left_out = self._left_out = [i for i in self._left_out if i < first]
@@ -343,16 +344,19 @@ class Runner:
             n = self._chain_length(i, readers) if block and self.chain_blocks else 0
             if n >= 2 and self._queue_chain(i, n, tensors, nn):
                 last = self.layers[i + 2 * n - 1]["name"]
-                out = tensors[last] = self._buffer(last)
+                out = tensors[last] = held(act, last)
                 i += 2 * n
                 continue
-            small = block and self._small(i)
-            if block and self._block_fusable(i, readers=readers, small=small) and self._queue_block(i, tensors, nn):
-                out = tensors[self.layers[i + 1]["name"]] = self._buffer(self.layers[i + 1]["name"])
-                if small:
-                    left_out.append(i)
-                i += 2
-                continue
+            if block:
+                small = self._small(i)
+                # (a run of one block is one that can be one launch)
+                if (self._pays(i, small) if n else self._block_fusable(i, readers=readers, small=small)) and self._queue_block(i, tensors, nn):
+                    name = self.layers[i + 1]["name"]
+                    out = tensors[name] = held(act, name)
+                    if small:
+                        left_out.append(i)
+                    i += 2
+                    continue
             out = tensors[L["name"]] = self._queue(i, tensors, nn)
             self.launches += 2 if (L["op"] == "depthwise" and (not self.fused or i in self.unfused)) else 1
             i += 1
@@ -368,38 +372,42 @@ class Runner:
         L, N = self.layers[i], self.layers[i + 1]
         if L["op"] != "depthwise" or N["op"] != "pointwise" or N["in"] != L["name"]:
             return False
-        # "auto": where the single launch is not slower than the two.  Runner.tune() times both forms of every such block on
-        # the batch at hand and records the faster one in block_choice.  Without that measurement: output planes of 8 x 8
-        # pixels, a whole image per workgroup (two launches / one at batch 256: 16x16x128 -> 256 at stride 2 10.2 / 8.1 us,
-        # 8x8x256 11.6 / 8.8), and small blocks
-        if policy and self.fuse_blocks == "auto":
-            if not (self.block_choice[i] if i in self.block_choice else self.shapes[L["name"]][:2] == (8, 8) or
-                    (self._small(i) if small is None else small)):
-                return False
+        if policy and not self._pays(i, small):
+            return False
         sx, sy = L["strides"]
         if L["w"].shape[1:3] != (3, 3) or tuple(L["pads"]) != (1, 1, 1, 1) or sx != sy:
             return False
         return (readers or self._reader_counts())[L["name"]] == 1
 
+    def _pays(self, i, small=None):
+        """Whether a block that can be one launch is to be one.  small: _small(i), where the caller has it."""
+        # "auto": where the single launch is not slower than the two.  Runner.tune() times both forms of every such block on
+        # the batch at hand and records the faster one in block_choice.  Without that measurement: output planes of 8 x 8
+        # pixels, a whole image per workgroup (two launches / one at batch 256: 16x16x128 -> 256 at stride 2 10.2 / 8.1 us,
+        # 8x8x256 11.6 / 8.8), and small blocks
+        if self.fuse_blocks != "auto":
+            return True
+        if i in self.block_choice:
+            return self.block_choice[i]
+        return (self._small(i) if small is None else small) or self.shapes[self.layers[i]["name"]][:2] == (8, 8)
+
     def _small(self, i):
         """Whether fuse_blocks="auto" makes one launch of depthwise layer i and the next because the block is small, or because
         the depthwise layer alone would be two launches itself.  Not where its result is asked for, or could not be computed
         again for a caller who asks after the run, from an input that may be gone by then."""
-        L = self.layers[i]
-        if self.fuse_blocks != "auto" or i in self.block_choice or i in self._asked or L["in"] == "input" or not isinstance(self.act, _Activations):
-            return False
         # Small: launches and round trips to memory are most of the time.  Two launches / one: 16x16x128 at batch 16 9.1 / 5.7 us,
         # 4x4x512 at batch 64 9.5 / 9.3; 64x64x16 at batch 64 11.5 / 9.7, at batch 256 20.2 / 24.3; 32x32x64 at batch 64 10.3 / 7.8, at
         # batch 256 16.9 / 19.1; so at most 4 MB for planes of 32 x 32 pixels and more.  Smaller planes would gain up to some 4 MB
         # too (16x16x128 at batch 128 13.0 / 8.1), but tables of 1 MB and more keep the launches per layer that callers count on.
+        # No kernel for HWC input: 64x64x16 at batch 255 39.0 / 24.5 us, three launches / one.
+        L = self.layers[i]
         Ho, Wo, Cc = self.shapes[L["name"]]
         size = self.batch * Ho * Wo * Cc
-        if (Ho, Wo) == (8, 8):
+        if not (size < 2 ** 20 or (size <= 2 ** 22 and Ho * Wo >= 1024) or
+                (Cc % 64 != 0 and (self.shapes[L["in"]][1] <= 8 or (self.batch * Cc) % 64 != 0))):
             return False
-        if size < 2 ** 20 or (Ho * Wo >= 1024 and size <= 2 ** 22):
-            return True
-        # No kernel for HWC input: 64x64x16 at batch 255 39.0 / 24.5 us, three launches / one
-        return Cc % 64 != 0 and (self.shapes[L["in"]][1] <= 8 or (self.batch * Cc) % 64 != 0)
+        return not (Ho == Wo == 8 or self.fuse_blocks != "auto" or i in self.block_choice or i in self._asked or L["in"] == "input" or
+                    not isinstance(self.act, _Activations))
 
     def _reader_counts(self):
         """{tensor name: how many layers read it}"""
@@ -415,15 +423,15 @@ class Runner:
         in LDS from block to block."""
         if i in self.unchained:
             return 0
-        n, shape = 0, None
+        n, layers, shapes, shape = 0, self.layers, self.shapes, None
         readers = readers or self._reader_counts()
-        while n < 8 and self._block_fusable(i + 2 * n, policy=False, readers=readers):
-            L, N = self.layers[i + 2 * n], self.layers[i + 2 * n + 1]
-            if L["strides"][0] != 1 or self.shapes[L["in"]] != self.shapes[N["name"]]:
+        while n < 8 and i + 2 * n + 1 < len(layers):
+            L = layers[i + 2 * n]
+            if L["op"] != "depthwise" or L["strides"][0] != 1 or (n > 0 and readers[L["in"]] != 1):
                 break
-            if shape is None:
-                shape = self.shapes[L["in"]]
-            if self.shapes[L["in"]] != shape or (n > 0 and readers[L["in"]] != 1):
+            shape = shape or shapes[L["in"]]
+            if shapes[L["in"]] != shape or shapes[layers[i + 2 * n + 1]["name"]] != shape or \
+                    not self._block_fusable(i + 2 * n, policy=False, readers=readers):
                 break
             n += 1
         return n
