@@ -427,7 +427,7 @@ class Runner:
         readers = readers or self._reader_counts()
         while n < 8 and i + 2 * n + 1 < len(layers):
             L = layers[i + 2 * n]
-            if L["op"] != "depthwise" or L["strides"][0] != 1 or (n > 0 and readers[L["in"]] != 1):
+            if L["op"] != "depthwise" or L["strides"][0] != 1 or (n > 0 and (L["in"] != layers[i + 2 * n - 1]["name"] or readers[L["in"]] != 1)):
                 break
             shape = shape or shapes[L["in"]]
             if shapes[L["in"]] != shape or shapes[layers[i + 2 * n + 1]["name"]] != shape or \

@@ -448,6 +448,21 @@ def test_depthwise_results_of_small_blocks_can_be_read():
     assert calls(lib, r, 0x100) == two + two
 
 
+def test_blocks_of_two_branches_are_no_chain():
+    """Two blocks of one shape, one after the other in the table, that read different tensors: each is called on its own input."""
+    dw1, pw1, dw2, pw2 = small_table()[:4]
+    pool = dict(op="maxpool", **{"in": "input"}, kernel=[2, 2], strides=[2, 2], out_hw=[8, 8])
+    table = [dict(pool, name="a"), dict(pool, name="b"), dict(dw1, **{"in": "a"}), pw1, dict(dw2, **{"in": "b"}), pw2,
+             dict(op="add", name="sum", **{"in": ("p1", "p2")}, m1=1, m2=1, shift=1)]
+    lib = FakeLibrary()
+    r = bare_runner(lib.bound(), table, (16, 16, 64))
+    for x in (0x100, 0x200):
+        lib.seen.clear()
+        r.run(x)
+        assert [c[0] for c in lib.seen][2:4] == ["pulp_nn_hip_dw_pw_hwc"] * 2 and len(lib.seen) == r.launches == 5
+        assert [c[1] for c in lib.seen][2:4] == [r.act["a"], r.act["b"]] and [c[2] for c in lib.seen][2:4] == [r.act["p1"], r.act["p2"]]
+
+
 def test_a_plan_does_not_keep_the_input():
     lib = FakeLibrary()
     r = bare_runner(lib.bound(), small_table(), (8, 8, 64))
