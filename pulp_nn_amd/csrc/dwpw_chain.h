@@ -7,7 +7,7 @@
 // Bound: one workgroup per image and compute unit, four waves per SIMD.  Of the 8000 cycles a block of 64 pixels x 256 channels takes, the
 // set-up of operands and constants is 900, the depthwise rows 1500, the multiply 1300, requantisation 900, requests for the next
 // block 700, the rest waiting at the two barriers for the waves that share a SIMD with three others: instructions issued, some 450 a
-// wave.  Five blocks of 8x8x256: 32.8 -> 19.2 us at batch 256, 31.9 -> 17.8 at batch 1 (with the depthwise stage on the vector ALU 6000 cycles of
+// wave.  Five blocks of 8x8x256: 32.8 -> 19.9 us at batch 256, 31.9 -> 17.6 at batch 1 (with the depthwise stage on the vector ALU 6000 cycles of
 // 14000, weights in operand layout and constants per wave 2500 to 4500 of requests).
 #pragma once
 #include "dwpw.h"
