@@ -22,7 +22,7 @@ bool launch_cb(int mode, const DwLayer &L, const EpiArgs &e, int cus, hipStream_
   DwmGeom g;
   int nm;
   size_t lds;
-  if (!dwm_shape<CB>(L, cus, (int)sizeof(bn_t), &g, &nm, &lds)) return false;
+  if (!dwm_shape<CB>(L, cus, &g, &nm, &lds)) return false;
   if (nm == 1) launch_mode<CB, 1>(mode, g, e, lds, s);
   else if (nm == 2) launch_mode<CB, 2>(mode, g, e, lds, s);
   else if (nm == 3) launch_mode<CB, 3>(mode, g, e, lds, s);

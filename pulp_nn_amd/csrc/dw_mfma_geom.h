@@ -7,6 +7,10 @@
 
 #include "fastdiv.h"
 
+// LDS bytes of a filter row: 8 zeros and its up to 8 bytes; of one wave's filter rows: those of a quarter of the channels, and 8 zeros.
+enum { DWM_WROW = 16 };
+PULPNN_HD int dwm_wpart(int channels, int ky) { return channels / 4 * ky * DWM_WROW + 16; }
+
 struct DwLayer {
   const uint8_t *in;
   const int8_t *wt;
@@ -23,19 +27,18 @@ struct DwmGeom {
   int B, CH, H, W, Ho, Wo;
   int kx, ky, pt, pl, sx, sy;
   long long in_bytes;   // bytes of the whole input tensor
-  long long edge_bytes; // the same, or for planes of fewer than 16 bytes far below 0: there any tile may leave the tensor, as a row
-                        // outside the image loads from the start of its plane
-  int wt_bytes;         // ... and of all filters
+  long long edge_bytes; // a tile whose last plane ends behind this byte may load behind the tensor
+  int wt_bytes;         // bytes of all filters
   int ND, rND;          // dwords of an input row behind 16 output columns; 65536 / ND + 1
   int RB, NR;           // output rows per tile, input rows behind them
   int XT;               // groups of 16 output columns per tile
   int pitch, CS;        // LDS bytes per staged row and per channel
   int Q;                // 16-byte chunks staged per row
-  int w_off, c_off, o_off;  // LDS offsets: filter rows, per-channel constants, output tile
+  int w_off, o_off;     // LDS offsets: filter rows (DWM_WROW bytes each), output tile
   int nper, cpar;       // staging: slots (row, chunk) a pass covers, channels side by side
   // tile index -> (channels, columns, rows, image); thread -> channel; slot -> row; unit -> row; pixel -> row (of a tile
-  // of full width); filter row -> channel
-  FastDiv d_cb, d_xt, d_band, d_nper, d_q, d_xg, d_wt, d_ky;
+  // of full width)
+  FastDiv d_cb, d_xt, d_band, d_nper, d_q, d_xg, d_wt;
   int cblocks, xtiles, bands, total;  // (one aligned scalar load: what a workgroup asks for first)
   FastDiv d_wt_last;  // pixel -> row of the last tile along a row
 };
@@ -64,12 +67,9 @@ PULPNN_HD DwmTile dwm_tile(const DwmGeom &g, unsigned id)
 }
 
 // Whether a 16-byte load of the tile may leave the tensor (before: bytes of the tensor in front of the tile's first plane).
-PULPNN_HD bool dwm_edge(const DwmGeom &g, const DwmTile &t, long long before, int iy0, int x0)
+PULPNN_HD bool dwm_edge(const DwmGeom &g, const DwmTile &t, long long before)
 {
-  const int plane = g.H * g.W, iy_last = iy0 + g.NR - 1 < g.H - 1 ? iy0 + g.NR - 1 : g.H - 1;
-  const long long first = before + (long long)(iy0 > 0 ? iy0 : 0) * g.W + x0;
-  const long long last = before + (long long)(t.ncb - 1) * plane + (long long)iy_last * g.W + x0 + 16 * g.Q;
-  return first < 0 || last > g.edge_bytes;
+  return before < g.pl || before + t.ncb * (g.H * g.W) > g.edge_bytes;
 }
 
 // Bytes from the tile's first plane to the load of chunk column x in row iy of channel c (a row outside the image: the
@@ -83,10 +83,10 @@ PULPNN_HD int dwm_out_row(const DwmGeom &g, const DwmTile &t, int p)
   return (int)fastdiv((unsigned)p, t.xt + 1 == g.xtiles ? g.d_wt_last : g.d_wt);
 }
 
-// Tile shape for CB channels per workgroup; bn_bytes: bytes of a batch-norm parameter.  nm: MFMAs per (channel, 16 units);
+// Tile shape for CB channels per workgroup.  nm: MFMAs per (channel, 16 units);
 // lds: dynamic LDS of the launch.  False for a layer the kernel does not take.
 template <int CB>
-bool dwm_shape(const DwLayer &L, int cus, int bn_bytes, DwmGeom *out, int *nm_out, size_t *lds_out)
+bool dwm_shape(const DwLayer &L, int cus, DwmGeom *out, int *nm_out, size_t *lds_out)
 {
   const long long plane = (long long)L.H * L.W;
   if (L.kx > 8 || L.kx * L.ky > 256 || L.sx > 4 || L.pl > 64 || plane * CB > (1 << 29) || (long long)L.B * L.CH * plane < 16) return false;
@@ -109,7 +109,6 @@ bool dwm_shape(const DwLayer &L, int cus, int bn_bytes, DwmGeom *out, int *nm_ou
   g.sx = L.sx;
   g.sy = L.sy;
   g.in_bytes = (long long)L.B * L.CH * plane;
-  g.edge_bytes = plane < 16 ? -(1ll << 62) : g.in_bytes;
   g.wt_bytes = L.CH * L.kx * L.ky;
   g.ND = (15 * L.sx + L.kx + 3) / 4;
   g.rND = 65536 / g.ND + 1;
@@ -117,7 +116,7 @@ bool dwm_shape(const DwLayer &L, int cus, int bn_bytes, DwmGeom *out, int *nm_ou
   if (nm > 5) return false;
   g.cblocks = (L.CH + CB - 1) / CB;
   const int xg = (L.Wo + 15) / 16;
-  const int fixed = CB * L.ky * 8 + CB * (4 + 2 * bn_bytes);
+  const int fixed = 4 * dwm_wpart(CB, L.ky);
   // LDS of a tile, in 64 bits: a tall output at a large row stride would reach over more input rows than an int counts
   // (the fields are what they should be for tiles that fit)
   auto shape = [&](int xt, int rb) -> long long {
@@ -148,15 +147,18 @@ bool dwm_shape(const DwLayer &L, int cus, int bn_bytes, DwmGeom *out, int *nm_ou
   if (total > 0x7fffffffLL) return false;
   g.total = (int)total;
   g.w_off = CB * g.CS;
-  g.c_off = g.w_off + CB * L.ky * 8;
-  g.o_off = (g.c_off + CB * (4 + 2 * bn_bytes) + 15) & ~15;
+  g.o_off = g.w_off + fixed;
+  // The last chunk of a row may reach over the end of its plane, by less than `over`.  Where a row outside the image, which loads
+  // from the start of its plane, may do so too (planes of fewer than 16 bytes), and where the channels of a pass are too far apart
+  // for 32-bit offsets, every tile counts as one that may leave the tensor: each of its loads is held inside.
+  const long long over = std::max(0ll, 16ll * g.XT * g.sx * (g.xtiles - 1) - g.pl + 16ll * g.Q - g.W);
+  g.edge_bytes = plane < 16 || plane * CB > (1 << 27) ? -(1ll << 62) : g.in_bytes - over;
   g.d_cb = fastdiv_make((unsigned)g.cblocks);
   g.d_xt = fastdiv_make((unsigned)g.xtiles);
   g.d_band = fastdiv_make((unsigned)g.bands);
   g.nper = std::min(g.NR * g.Q, 256);
-  g.cpar = 256 / g.nper;
+  g.cpar = std::min(256 / g.nper, CB);
   g.d_nper = fastdiv_make((unsigned)g.nper);
-  g.d_ky = fastdiv_make((unsigned)L.ky);
   g.d_q = fastdiv_make((unsigned)g.Q);
   g.d_xg = fastdiv_make((unsigned)g.XT);
   g.d_wt = fastdiv_make((unsigned)std::min(16 * xt, L.Wo));

@@ -48,3 +48,6 @@ __device__ __forceinline__ unsigned low_bytes(int n)
   const int m = min(n, 4);
   return m <= 0 ? 0u : __builtin_amdgcn_alignbit(0u, 0xffffffffu, 32 - 8 * m);  // (4 bytes: a shift by 0)
 }
+// bits [0, n) of a dword, n clamped to [0, 32], and all but them: three instructions each
+__device__ __forceinline__ unsigned low_bits(int n) { return (unsigned)((0xffffffffull << min(max(n, 0), 32)) >> 32); }
+__device__ __forceinline__ unsigned high_bits(int n) { return (unsigned)(0xffffffffull << min(max(n, 0), 32)); }

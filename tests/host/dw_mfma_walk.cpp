@@ -1,6 +1,6 @@
 // Walks the tiles of dw_mfma_kernel on the host, with the kernel's own tile arithmetic (csrc/dw_mfma_geom.h), and reports
 // loads that leave the input, LDS ranges that overlap, and output pixels that are written to a wrong place or not at all.
-// Layers on stdin, one a line: B CH H W Ho Wo kx ky pt pl sx sy bn_bytes cus.  One line out per layer: "ok TILES", "no" (not
+// Layers on stdin, one a line: B CH H W Ho Wo kx ky pt pl sx sy (bytes of a batch-norm parameter) cus.  One line out per layer: "ok TILES", "no" (not
 // taken by the kernel) or what is wrong.
 #include <stdio.h>
 #include <stdlib.h>
@@ -18,12 +18,12 @@ static std::string wrong(const char *what, const DwmTile &t, long long a, long l
 }
 
 template <int CB>
-static std::string check(const DwLayer &L, int bn_bytes, int cus)
+static std::string check(const DwLayer &L, int cus)
 {
   DwmGeom g;
   int nm;
   size_t lds;
-  if (!dwm_shape<CB>(L, cus, bn_bytes, &g, &nm, &lds)) return "no";
+  if (!dwm_shape<CB>(L, cus, &g, &nm, &lds)) return "no";
   const long long plane = (long long)L.H * L.W, bytes = (long long)L.B * L.CH * plane;
   if (lds > 65536) return "more LDS than a launch may ask for";
   if (g.in_bytes != bytes) return "size of the input: " + std::to_string(g.in_bytes) + " for " + std::to_string(bytes);
@@ -37,7 +37,7 @@ static std::string check(const DwLayer &L, int bn_bytes, int cus)
     if ((int)t.b >= L.B || t.c0 >= L.CH || t.rows <= 0 || t.wt <= 0 || t.ncb <= 0) return wrong("empty tile", t, t.rows, t.wt);
     const long long before = ((long long)t.b * L.CH + t.c0) * plane;
     const int iy0 = t.oy0 * g.sy - g.pt, x0 = 16 * t.xg0 * g.sx - g.pl;
-    const bool edge = dwm_edge(g, t, before, iy0, x0);
+    const bool edge = dwm_edge(g, t, before);
     const long long behind = g.in_bytes - before - 16;
     const int lo = (int)std::max(-before, -(1ll << 30)), hi = (int)std::min(behind, 0x7fffffffll);
     for (int row = 0; row < g.NR; row++)
@@ -50,8 +50,8 @@ static std::string check(const DwLayer &L, int bn_bytes, int cus)
             if (iy >= 0 && iy < L.H && x + j >= 0 && x + j < L.W && (j + off - at < 0 || j + off - at > 15))
               return wrong("byte of the image not loaded", t, iy, x + j);
         }
-    if (g.NR * g.pitch > g.CS || 16 * g.Q > g.pitch || CB * g.CS > g.w_off || g.w_off + CB * L.ky * 8 > g.c_off ||
-        g.c_off + CB * (4 + 2 * bn_bytes) > g.o_off || g.o_off + (size_t)t.rows * t.wt * (CB + 4) > lds)
+    if (g.NR * g.pitch > g.CS || 16 * g.Q > g.pitch || CB * g.CS > g.w_off || g.w_off + 4 * dwm_wpart(CB, L.ky) > g.o_off ||
+        g.o_off + (size_t)t.rows * t.wt * (CB + 4) > lds)
       return wrong("LDS ranges", t, g.o_off, (long long)lds);
     for (int p = 0; p < t.rows * t.wt; p++)
       if (dwm_out_row(g, t, p) * (L.Wo - t.wt) != (p / t.wt) * (L.Wo - t.wt)) return wrong("output pixel misplaced", t, p, dwm_out_row(g, t, p));
@@ -67,9 +67,9 @@ int main()
   int bn_bytes, cus;
   while (scanf("%d %d %d %d %d %d %d %d %d %d %d %d %d %d", &L.B, &L.CH, &L.H, &L.W, &L.Ho, &L.Wo, &L.kx, &L.ky, &L.pt, &L.pl, &L.sx, &L.sy,
                &bn_bytes, &cus) == 14) {
-    std::string s = check<16>(L, bn_bytes, cus);
+    std::string s = check<16>(L, cus);
     if (s.compare(0, 2, "ok") == 0 || s == "no") {
-      const std::string s64 = (long long)L.Ho * L.Wo <= 64 ? check<64>(L, bn_bytes, cus) : "no";
+      const std::string s64 = (long long)L.Ho * L.Wo <= 64 ? check<64>(L, cus) : "no";
       if (s64.compare(0, 2, "ok") != 0 && s64 != "no") s = "64 channels: " + s64;
     }
     puts(s.c_str());

@@ -34,9 +34,23 @@ GEOMS = [
 ]
 
 
+# where the loads of filters, constants and input rows change form
+SETUP_GEOMS = [
+    (1, 3, 1, 9, 1, 2, (0, 0, 0, 0), (1, 1)),        # 6 bytes of filters: fewer than one load
+    (1, 4, 5, 6, 1, 2, (0, 0, 0, 1), (1, 1)),        # 8 bytes: one load
+    (2, 3, 6, 7, 3, 1, (1, 1, 0, 0), (1, 1)),        # 9: the last rows are loaded too early
+    (1, 21, 40, 8, 17, 1, (8, 8, 0, 0), (1, 1)),     # 68 filter rows in a wave
+    (1, 2, 3, 20, 1, 8, (0, 0, 64, 3), (1, 1)),      # rows that begin 64 bytes before the tensor
+    (3, 40, 2, 7, 2, 3, (1, 1, 5, 5), (1, 1)),       # 14 bytes a plane, several blocks of channels
+    (2, 33, 3, 6, 3, 3, (1, 1, 1, 1), (1, 1)),       # 18 bytes a plane: a chunk reaches over the next one
+    (300, 80, 8, 8, 3, 3, (1, 1, 1, 1), (2, 2)),     # 64 channels per workgroup, 16 in the last: one quad for each wave
+    (350, 100, 6, 6, 5, 5, (2, 2, 2, 2), (1, 1)),    # ... 36: three quads for each of three waves
+]
+
+
 @pytest.mark.parametrize("bn_bits", [32, 64])
 @pytest.mark.parametrize("flags", [(1, 1), (1, 0), (0, 0)])
-@pytest.mark.parametrize("geom", GEOMS, ids=lambda g: "x".join(map(str, g[:6])) + "s%d%d" % g[7])
+@pytest.mark.parametrize("geom", GEOMS + SETUP_GEOMS, ids=lambda g: "x".join(map(str, g[:6])) + "s%d%d" % g[7])
 def test_depthwise_shapes(geom, flags, bn_bits):
     B, CH, H, W, ky, kx, pads, strides = geom
     relu, bn = flags
