@@ -20,9 +20,14 @@
 // stages give each wave one item).
 //
 // Bound: the chain parameters and input -> LDS -> multiply -> LDS -> multiply -> store, and the instructions of a wave in it, some 900
-// with 128 channels; large batches by that chain too, two to four workgroups per compute unit covering each other.  Call by call, against
-// the vector-ALU depthwise stage that this replaced: 64x64x16 -> 32 batch 1 13.6 -> 5.1 us, batch 256 42.4 -> 25.1; 16x16x128 7.4 -> 5.5 and
-// 14.6 -> 11.1; 16x16x128 -> 256 stride 2 6.2 -> 6.2 and 9.2 -> 7.8; 8x8x256 7.3 -> 6.5 and 11.2 -> 8.6; 4x4x512 8.5 -> 8.5 and 12.4 -> 10.3.
+// with 128 channels, 8 clocks for one that needs the one before; large batches by that chain too, two to four workgroups per compute unit
+// covering each other.  What a block reads from memory is asked for in one trip, the input first (some 2000 clocks from another XCD's
+// writes), then the parameters straight to LDS, the weights, and the constants of the pointwise stage; two 16-byte loads of input a lane at a
+// time (four cost 14 registers, one wave of five per SIMD and on 64x64x16 -> 32 batch 256 2.5 us).  With the parameters through
+// registers, array by array, and each number of the launch read where it is used, a wave took 10800 clocks from end to end on 64x64x16 ->
+// 32, now 8200.  Call by call, before that / now: 64x64x16 -> 32 batch 1 5.0 / 4.15 us, batch 256 24.7 / 23.0; 64x64x32 -> 64 stride 2
+// batch 256 21.0 / 17.8; 32x32x64 batch 1 5.3 / 4.5; 16x16x128 batch 64 6.4 / 5.9; 16x16x64 -> 128 6.1 / 5.2.  (With the vector-ALU
+// depthwise stage 64x64x16 -> 32 was 13.6 and 42.4.)
 #pragma once
 #include <stddef.h>
 
@@ -104,6 +109,22 @@ __device__ __forceinline__ int dwpw_act_step()
   return 64 * *(const __attribute__((address_space(4))) int *)(p + offsetof(DwPwGeom, t) + offsetof(DwPwTile, act_px));
 }
 
+// One layer's parameters to LDS (DwPwPar) by the workgroup as a whole, 1 KB an instruction: sixteen waves that each fetch their own 16
+// channels' into registers keep the address units busy for 2500 cycles a block.
+// Every one of the waves asks for its share (loads without a source are out of range: zeros).  Filter and bias 4-byte aligned.
+__device__ __forceinline__ void dwpw_par_load(unsigned char *par, const int8_t *filter, const int8_t *bias, const bn_t *k, const bn_t *lambda, bool bn, int C, int wave,
+                                              int waves, int lane)
+{
+  typedef __attribute__((address_space(3))) void *lds_ptr_t;
+  const DwPwPar at = dwpw_par(C, (int)sizeof(bn_t), filter != nullptr);
+  for (int to = 1024 * wave; to < at.bytes; to += waves * 1024) {
+    const DwPwParPiece p = dwpw_par_piece(at, C, (int)sizeof(bn_t), bias != nullptr, bn, to);
+    const char *src = (p.array == 0 ? (const char *)bias : p.array == 1 ? (const char *)k : p.array == 2 ? (const char *)lambda : (const char *)filter) + p.first;
+    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)src, 0, p.bytes, 0x00020000);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr_t)(par + to), 16, 16 * lane, 0, 0, 0);
+  }
+}
+
 // W, S: input width, stride.  KP: slices of K whose weights are in LDS at once.  CHAIN: g.nblocks blocks back to back; otherwise the
 // one block g.blk[0].
 template <int W, int S, int KP, bool CHAIN>
@@ -114,7 +135,20 @@ __global__ __launch_bounds__(1024) void dwpw_kernel(DwPwGeom g)
   typedef bn_t bn4 __attribute__((ext_vector_type(4), aligned(sizeof(bn_t))));
   typedef __attribute__((address_space(3))) void *lds_ptr_t;
   constexpr int WO = W / S;
-  const DwPwTile &T = g.t;
+  DwPwTile &T = g.t;
+  // The launch's numbers at once and opaque (as in dw_mfma_kernel), the block's pointers with them.
+  asm volatile("" : "+s"(T.C), "+s"(T.H), "+s"(T.Ho), "+s"(T.Co), "+s"(T.whole), "+s"(T.NI), "+s"(T.TR), "+s"(T.lpxb), "+s"(T.R), "+s"(T.nst),
+               "+s"(T.CS), "+s"(T.XR), "+s"(T.pitch), "+s"(T.x_off), "+s"(T.waves));
+  asm volatile("" : "+s"(T.lsplit), "+s"(T.cf_per), "+s"(T.par_off), "+s"(T.w_off), "+s"(T.bands), "+s"(T.slabs), "+s"(T.act_px), "+s"(g.in),
+               "+s"(T.nrb), "+s"(T.B));
+  DwPwBlock only = g.blk[0];
+  if constexpr (!CHAIN)
+    asm volatile("" : "+s"(only.dw_wt), "+s"(only.dw_bias), "+s"(only.pw_w), "+s"(only.pw_bias), "+s"(only.e_dw.k), "+s"(only.e_dw.lambda),
+                 "+s"(only.e_pw.k), "+s"(only.e_pw.lambda), "+s"(only.e_dw.shift), "+s"(only.e_pw.shift), "+s"(only.mode_dw), "+s"(only.mode_pw));
+  auto block = [&](int j) {
+    if constexpr (CHAIN) return dwpw_block(j);
+    else return (const DwPwBlock *)&only;
+  };
   const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, lgrp = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), NWV = T.waves, NTH = 64 * NWV;
   const int part = blockIdx.x & ((1 << T.lsplit) - 1);
@@ -128,7 +162,7 @@ __global__ __launch_bounds__(1024) void dwpw_kernel(DwPwGeom g)
   const int cf_lo = part * T.cf_per, nblk = max(min(T.cf_per, T.Co / 16 - cf_lo), 0) << T.lpxb;
   unsigned char *wl = dwpw_lds + T.w_off + wave * (1024 * KP);  // the wave's own weights: KP slices of 16 rows of 64 bytes
   int w_cf = -1;                                                // channels whose first slices are there, or on their way
-  auto load_w = [&](DwPwBlockArg P, int cf, int kt0) {
+  auto load_w = [&](auto P, int cf, int kt0) {
     const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)P->pw_w, 0, (unsigned)T.Co * (unsigned)T.C, 0x00020000);
     const unsigned off = dwpw_w_lane(T.C, cf, lane, KP == 1);
 #pragma unroll
@@ -142,22 +176,36 @@ __global__ __launch_bounds__(1024) void dwpw_kernel(DwPwGeom g)
 #pragma unroll 1
   for (int j = 0; j < nblocks; j++) {
     const bool first = !CHAIN || j == 0, last = !CHAIN || j == nblocks - 1;
-    // ---- weights on their way to LDS, depthwise parameters to LDS -----------------------------------------------------------
-    {
-      const DwPwBlockArg P = dwpw_block(j);
-      if (wave < nblk) {
-        w_cf = cf_lo + (wave >> T.lpxb);
-        load_w(P, w_cf, 0);
+    // ---- one trip to memory: the input's first part, weights and depthwise parameters on their way to LDS, the constants of the wave's
+    // first block of the pointwise stage ------------------------------------------------------------------------------------------
+    const auto P = block(j);
+    const int cf_first = cf_lo + (wave >> T.lpxb);
+    constexpr int UN = 2;  // 16-byte loads in flight per lane
+    v4u v[UN];
+    int to[UN];
+    const int chunks = dwpw_chunks<W>(T);
+    // (t0: the wave's first chunk; what none of its lanes needs is left out)
+    auto load_x = [&](int slab, int t0) {
+      const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)(g.in + (dwpw_first_row<S>(T, at) * W) * T.C + slab * T.CS), 0,
+                                                                            (dwpw_rows_in(T) * W) * T.C - slab * T.CS, 0x00020000);
+#pragma unroll
+      for (int u = 0; u < UN; u++) {
+        if (t0 + NTH * u >= chunks) break;
+        const DwPwChunk c = dwpw_chunk<W, S>(T, at, t0 + lane + NTH * u);
+        to[u] = c.lds;
+        v[u] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, c.off >= 0 ? (unsigned)c.off : 0x80000000u, 0, 0);
       }
+    };
+    if (first) load_x(0, 64 * wave);
+    // (many slices of weights behind the input: in front of it they would hold it up)
+    if (KP == 1 && wave < nblk) load_w(P, w_cf = cf_first, 0);
+    if ((((unsigned)(unsigned long long)P->dw_wt | (unsigned)(unsigned long long)P->dw_bias) & 3) == 0) {
+      dwpw_par_load(par, P->dw_wt, P->dw_bias, P->e_dw.k, P->e_dw.lambda, P->mode_dw == EPI_BN, T.C, wave, NWV, lane);
+    } else {
       const DwPwPar off = dwpw_par(T.C, (int)sizeof(bn_t), true);
       const int8_t *wt = P->dw_wt, *bias = P->dw_bias;
-      if ((((unsigned)(unsigned long long)wt | (unsigned)(unsigned long long)bias) & 3) == 0) {
-        for (int i = tid; i < 9 * T.C / 4; i += NTH) *(int *)(par + off.f + 4 * i) = ((const int *)wt)[i];
-        for (int i = tid; i < T.C / 4; i += NTH) *(int *)(par + 4 * i) = bias ? ((const int *)bias)[i] : 0;
-      } else {
-        for (int i = tid; i < 9 * T.C; i += NTH) par[off.f + i] = (unsigned char)wt[i];
-        for (int i = tid; i < T.C; i += NTH) par[i] = bias ? (unsigned char)bias[i] : 0;
-      }
+      for (int i = tid; i < 9 * T.C; i += NTH) par[off.f + i] = (unsigned char)wt[i];
+      for (int i = tid; i < T.C; i += NTH) par[i] = bias ? (unsigned char)bias[i] : 0;
       const bool bn = P->mode_dw == EPI_BN;
       const bn_t *k = P->e_dw.k, *l = P->e_dw.lambda;
       for (int i = tid; i < T.C; i += NTH) {
@@ -165,34 +213,40 @@ __global__ __launch_bounds__(1024) void dwpw_kernel(DwPwGeom g)
         *(bn_t *)(par + off.l + i * (int)sizeof(bn_t)) = bn ? l[i] : (bn_t)0;
       }
     }
+    // the constants of the lane's four channels of output
+    int bias = 0;
+    bn4 k = {0, 0, 0, 0}, l = {0, 0, 0, 0};
+    auto load_pw = [&](int cf) {
+      const int n = 16 * cf + 4 * lgrp;
+      if (P->pw_bias) bias = *(const i32_u *)(P->pw_bias + n);
+      if (P->mode_pw == EPI_BN) {
+        k = *(const bn4 *)(P->e_pw.k + n);
+        l = *(const bn4 *)(P->e_pw.lambda + n);
+      }
+    };
+    if (wave < nblk) load_pw(cf_first);
 #pragma unroll 1
     for (int slab = 0; slab < (CHAIN ? 1 : T.slabs); slab++) {
       // ---- input -> LDS ------------------------------------------------------------------------------------------------
       if (first) {
         if (slab) dwpw_barrier();  // everybody is done with the slab before
-        const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)(g.in + (dwpw_first_row<S>(T, at) * W) * T.C + slab * T.CS), 0,
-                                                                              (dwpw_rows_in(T) * W) * T.C - slab * T.CS, 0x00020000);
-        const int chunks = dwpw_chunks<W>(T);
-        constexpr int UN = 4;
 #pragma unroll 1
-        for (int t0 = tid; t0 < chunks; t0 += NTH * UN) {
-          v4u v[UN];
-          int to[UN];
+        for (int t0 = 64 * wave; t0 < chunks; t0 += NTH * UN) {
+          if (slab || t0 != 64 * wave) load_x(slab, t0);
 #pragma unroll
           for (int u = 0; u < UN; u++) {
-            const DwPwChunk c = dwpw_chunk<W, S>(T, at, t0 + NTH * u);
-            to[u] = c.lds;
-            v[u] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, c.off >= 0 ? (unsigned)c.off : 0x80000000u, 0, 0);
+            if (t0 + NTH * u >= chunks) break;
+            if (t0 + lane + NTH * u < chunks) *(v4i *)(xin + to[u]) = (v4i){(int)v[u].x, (int)v[u].y, (int)v[u].z, (int)v[u].w} ^ (int)0x80808080;
           }
-#pragma unroll
-          for (int u = 0; u < UN; u++)
-            if (t0 + NTH * u < chunks) *(v4i *)(xin + to[u]) = (v4i){(int)v[u].x, (int)v[u].y, (int)v[u].z, (int)v[u].w} ^ (int)0x80808080;
         }
+      }
+      if (slab == 0) {
+        __builtin_amdgcn_s_waitcnt(DWPW_WAIT_VM(0));  // (a wave without input has parameters on their way to LDS)
+        if (KP > 1 && wave < nblk) load_w(P, w_cf = cf_first, 0);
       }
       dwpw_barrier();
 
       // ---- depthwise stage ---------------------------------------------------------------------------------------------
-      const DwPwBlockArg P = dwpw_block(j);
       const int mode = P->mode_dw, shift = P->e_dw.shift;
       const unsigned char *filter = par + dwpw_par(T.C, (int)sizeof(bn_t), true).f + l16 * 9 + min(lgrp, 2);
       const int act_step = CHAIN ? 4096 << T.lpxb : dwpw_act_step();
@@ -233,21 +287,13 @@ __global__ __launch_bounds__(1024) void dwpw_kernel(DwPwGeom g)
       }
     }
     // ---- pointwise stage ---------------------------------------------------------------------------------------------------
-    const DwPwBlockArg P = dwpw_block(j);
     const int mode = P->mode_pw, shift = P->e_pw.shift, act_step = CHAIN ? 4096 << T.lpxb : dwpw_act_step();
     __builtin_amdgcn_s_waitcnt(DWPW_WAIT_VM(0));  // this wave's weights
     dwpw_barrier();
 #pragma unroll 1
     for (int blk = wave; blk < nblk; blk += NWV) {
       const int cf = cf_lo + (blk >> T.lpxb), px0 = 64 * (blk & ((1 << T.lpxb) - 1));
-      // the constants of the lane's four channels
-      const int n = 16 * cf + 4 * lgrp;
-      const int bias = P->pw_bias ? *(const i32_u *)(P->pw_bias + n) : 0;
-      bn4 k = {0, 0, 0, 0}, l = {0, 0, 0, 0};
-      if (mode == EPI_BN) {
-        k = *(const bn4 *)(P->e_pw.k + n);
-        l = *(const bn4 *)(P->e_pw.lambda + n);
-      }
+      if (blk != wave) load_pw(cf);
       const v4i ones = {0x01010101, 0x01010101, 0x01010101, 0x01010101};
       v4i acc[4], wacc = {0, 0, 0, 0};
 #pragma unroll

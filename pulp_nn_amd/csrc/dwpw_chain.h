@@ -12,21 +12,6 @@
 #pragma once
 #include "dwpw.h"
 
-// One layer's parameters to LDS (DwPwPar) by the workgroup as a whole, 1 KB an instruction: sixteen waves that each fetch their own 16
-// channels' into registers keep the address units busy for 2500 cycles a block.
-// Every wave of sixteen asks for its share (loads without a source are out of range: zeros).  Filter and bias 4-byte aligned.
-__device__ __forceinline__ void dwpw_par_load(unsigned char *par, const int8_t *filter, const int8_t *bias, const bn_t *k, const bn_t *lambda, bool bn, int C, int wave,
-                                              int lane)
-{
-  typedef __attribute__((address_space(3))) void *lds_ptr_t;
-  const DwPwPar at = dwpw_par(C, (int)sizeof(bn_t), filter != nullptr);
-  for (int to = 1024 * wave; to < at.bytes; to += 16 * 1024) {
-    const DwPwParPiece p = dwpw_par_piece(at, C, (int)sizeof(bn_t), bias != nullptr, bn, to);
-    const char *src = (p.array == 0 ? (const char *)bias : p.array == 1 ? (const char *)k : p.array == 2 ? (const char *)lambda : (const char *)filter) + p.first;
-    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)src, 0, p.bytes, 0x00020000);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr_t)(par + to), 16, 16 * lane, 0, 0, 0);
-  }
-}
 // LDS of the launch: the tile's, the pointwise layer's parameters, and a row that pixels past the last one are written to.
 PULPNN_HD int dwpw_chain_spare(int tile_lds, int C) { return tile_lds + dwpw_par(C, (int)sizeof(bn_t), false).bytes; }
 PULPNN_HD int dwpw_chain_lds(int tile_lds, int C) { return dwpw_chain_spare(tile_lds, C) + 1024; }
@@ -63,10 +48,10 @@ __global__ __launch_bounds__(1024) void dwpw_chain_kernel(DwPwGeom g)
     }
   };
   auto load_dw = [&](DwPwBlockArg P) {
-    dwpw_par_load(par_dw, P->dw_wt, P->dw_bias, P->e_dw.k, P->e_dw.lambda, P->mode_dw == EPI_BN, C, wave, lane);
+    dwpw_par_load(par_dw, P->dw_wt, P->dw_bias, P->e_dw.k, P->e_dw.lambda, P->mode_dw == EPI_BN, C, wave, 16, lane);
   };
   auto load_pw = [&](DwPwBlockArg P) {
-    dwpw_par_load(par_pw, nullptr, P->pw_bias, P->e_pw.k, P->e_pw.lambda, P->mode_pw == EPI_BN, C, wave, lane);
+    dwpw_par_load(par_pw, nullptr, P->pw_bias, P->e_pw.k, P->e_pw.lambda, P->mode_pw == EPI_BN, C, wave, 16, lane);
   };
   load_dw(dwpw_block(0));
   load_w(dwpw_block(0));
