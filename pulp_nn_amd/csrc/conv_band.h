@@ -13,15 +13,21 @@
 // pixel (and weight row) would start in front of its tensor: that one is shifted into place.
 //
 // The waves of a workgroup split the channels (WN of them; the others split the pixels), so a weight byte is fetched by
-// one wave only: straight from global memory in MFMA operand layout, PF steps at a time, the next PF steps requested
-// before the current ones are multiplied.  128 * sum(w) comes from one more MFMA per weight fragment against ones.
+// one wave only, straight to the wave's own part of LDS, a group of PF K steps ahead of the one it multiplies.  Four lanes fetch the 64
+// bytes of a row's step: in MFMA operand layout, sixteen rows side by side, a load keeps the address unit 56 to 64 clocks
+// instead of 16, and the layers of many channels were bound by that.  128 * sum(w) comes from one more MFMA per weight fragment against ones.
 //
-// Bound: layers of up to a few MB, by the latency of load -> LDS -> multiply -> store (57x43 24 -> 40: 15 MFMAs and 718 vector
-// instructions a wave, which waits half of its time; constants are waited for before the input is asked for); larger ones by
-// too few waves and the vector instructions around each MFMA (24x27 168 -> 176 5x5: 1.7 waves per SIMD, 6.6 vector instructions
-// per MFMA, matrix cores 20 % and LDS 10 % busy).  Measured, whole calls, against the 128 x 64 tile with a byte gather that these
-// shapes took: 57x43 24 -> 40 stride 2 batch 32 19.3 -> 9.4 us; 15x31 168 -> 16 batch 19 236 -> 11; 24x27 168 -> 176 5x5 stride 2 batch
-// 72 409 -> 46; 21x36 56 -> 32 stride 2 batch 25 82 -> 7.5; 14x14 24 -> 48 batch 31 19 -> 6.6 (the call's host time).
+// Everything is asked for in one trip to memory, the input first; a thread walks over the pixels of the band with its chunk of a
+// pixel, so a load's place costs it some fifteen instructions.  (Weights first, constants waited for before the input is asked for, each
+// place from divisions: 2200 clocks until the constants were asked for, 1600 until the input was, of 11500 in all on 57x43 24 -> 40.)
+//
+// Bound: layers of up to a few MB, by the chain load -> LDS -> multiply -> store and the instructions of a wave in it; larger ones by
+// the vector instructions around each MFMA and by LDS, which holds input, weights and with them the workgroups that share a compute
+// unit.  Whole calls, weights in registers in operand layout and tiles for two workgroups a compute unit / now: 57x43 24 -> 40 stride 2 batch 32
+// 9.8 / 6.7 us; 15x31 168 -> 16 batch 19 11.3 / 9.7; 56x56 100 -> 100 batch 16 25.9 / 16.7; 40x30 250 -> 250 stride 2 batch 60 115 / 47;
+// 13x19 90 -> 192 5x5 batch 70 125 / 36; 24x27 168 -> 176 5x5 stride 2 batch 72 47.4 / 44.6; over 380 layers the mean is 0.90; slower by
+// more than 2 %: 23x14 144 -> 35 batch 23 8.3 / 8.6 and 37x19 48 -> 20 batch 22 5.7 / 5.9.  (The 128 x 64 tile with a byte gather,
+// which these shapes took before: 19.3, 236 and 409 us for the first, the second and the last.)
 #pragma once
 #include <type_traits>
 
@@ -37,16 +43,26 @@ __device__ __forceinline__ v4i bytes_up(v4i v, int n)
   return (v4i){(int)(unsigned)t, (int)(unsigned)(t >> 32), (int)(unsigned)(t >> 64), (int)(unsigned)(t >> 96)};
 }
 
-// TN: 16-channel groups per wave; TM: 16-pixel groups per wave
-template <int TN, int TM>
-__global__ __launch_bounds__(256) void conv_band_kernel(BandGeom g, EpiArgs e)
+// s_waitcnt vmcnt(n), n < 16; lgkmcnt(0)
+#define BAND_WAIT_VM(n) (0x0F70 | (n))
+#define BAND_WAIT_LDS 0xC07F
+
+// TN: 16-channel groups per wave; TM: 16-pixel groups per wave; PF: K steps of a group of weights
+template <int TN, int TM, int PF>
+__global__ __launch_bounds__(256, TN * TM <= 4 ? 4 : TN * TM == 8 ? 3 : TN * TM == 16 ? 2 : 1) void conv_band_kernel(BandGeom g, EpiArgs e)
 {
-  constexpr int PF = TN == 4 ? 2 : TN == 2 ? 4 : 8;  // K steps whose weights are in flight
   extern __shared__ __attribute__((aligned(16))) unsigned char band_lds[];
+  typedef unsigned v4u __attribute__((ext_vector_type(4)));
+  typedef __attribute__((address_space(3))) void *lds_ptr_t;
+  // the launch's numbers at once and opaque (as in dw_mfma_kernel)
+  asm volatile("" : "+s"(g.total), "+s"(g.nblocks), "+s"(g.xtiles), "+s"(g.bands), "+s"(g.in), "+s"(g.w), "+s"(g.bias), "+s"(g.N), "+s"(g.K),
+               "+s"(g.H), "+s"(g.W), "+s"(g.Ci), "+s"(g.Ho), "+s"(g.Wo), "+s"(g.CG));
+  asm volatile("" : "+s"(g.CP), "+s"(g.NK), "+s"(g.R), "+s"(g.PC), "+s"(g.IW), "+s"(g.WN), "+s"(g.cpp), "+s"(g.ppp), "+s"(g.in_bytes),
+               "+s"(g.w_off), "+s"(g.sx), "+s"(g.sy), "+s"(e.k), "+s"(e.lambda), "+s"(g.mode));
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l16 = lane & 15, lgrp = lane >> 4;
-  const int wave_n = wave & (g.WN - 1), wave_m = wave / g.WN;
+  const int wave_n = wave & (g.WN - 1), wave_m = g.WN == 4 ? 0 : g.WN == 2 ? wave >> 1 : wave;
 
   const unsigned id = (unsigned)xcd_remap(blockIdx.x, g.total);
   const unsigned t1 = fastdiv(id, g.d_nb), t2 = fastdiv(t1, g.d_xt), b = fastdiv(t2, g.d_band);
@@ -56,142 +72,213 @@ __global__ __launch_bounds__(256) void conv_band_kernel(BandGeom g, EpiArgs e)
   const int pc = min(g.PC, g.Wo - ox0), rows = min(g.R, g.Ho - oy0);
   const int px = rows * pc;
 
-  // ---- weight fragments: row i of fragment t is channel wn0 + (i/4)*4*TN + 4*t + i%4 -----------------------------
-  const int wn0 = n0 + wave_n * 16 * TN;
-  const __amdgpu_buffer_rsrc_t rsrc_w = __builtin_amdgcn_make_buffer_rsrc((void *)g.w, 0, (unsigned)g.N * (unsigned)g.K, 0x00020000);
-  const int nslots = g.kx * g.ky * g.CG;
-  const int wrow = wn0 + (l16 >> 2) * (4 * TN) + (l16 & 3);
-  v4i wf[2][PF][TN];
-  auto load_w = [&](v4i (&wb)[PF][TN], int kk0) {
-    typedef unsigned v4u __attribute__((ext_vector_type(4)));
+  // ---- ask for the input's first part --------------------------------------------------------------------------------
+  // A thread keeps its chunk of a pixel and walks over the pixels of the band, ppp a pass.  Offsets count from 16 bytes before the band's
+  // first pixel, which may lie in the padding; what is outside the image is out of the buffer's range and reads as zeros.
+  const int iy0 = oy0 * g.sy - g.pt, ix0 = ox0 * g.sx - g.pl;
+  const int nr = (rows - 1) * g.sy + g.ky;
+  const long long first = (long long)b * g.H * g.W * g.Ci + ((long long)iy0 * g.W + ix0) * g.Ci - 16;
+  const __amdgpu_buffer_rsrc_t rsrc_x =
+      __builtin_amdgcn_make_buffer_rsrc((void *)(g.in + first), 0, (int)min(g.in_bytes - first, 0x7fffffffll), 0x00020000);
+  const bool near = g.Ci < 16 && first < 0;                   // chunks may begin in front of the tensor: loaded too late
+  const int lo = (int)min(max(-first, 0ll), 0x7fffffffll);
+  const int p0 = (int)fastdiv((unsigned)tid, g.d_cpp), c_thr = tid - p0 * g.cpp;
+  const int passes = (int)fastdiv((unsigned)(nr * g.IW - 1), g.d_ppp) + 1;
+  const int dup = 16 * g.CG - g.Ci;  // bytes of a pixel's last chunk that the one before it has too
+  constexpr int UN = 4;
+  v4u v[UN];
+  int dst[UN], voff[UN];
+  int row, col, c16;
+  auto start = [&](int cb) {  // chunks cb .. cb + cpp - 1 of all pixels
+    row = (int)fastdiv((unsigned)p0, g.d_iw);
+    col = p0 - row * g.IW;
+    c16 = cb + c_thr;
+    if (p0 >= g.ppp || c16 >= g.CG) row = 1 << 20;
+  };
+  auto load = [&](int pass) {
 #pragma unroll
-    for (int p = 0; p < PF; p++) {
-      const int q = 4 * (kk0 + p) + lgrp;
-      const int tap = (int)fastdiv((unsigned)q, g.d_cg), c16 = q - tap * g.CG;
-      const int ko = tap * g.Ci + min(16 * c16, g.Ci - 16);
-#pragma unroll
-      for (int t = 0; t < TN; t++) {
-        const int n = wrow + 4 * t, off = n * g.K + ko;
-        const v4u v = __builtin_amdgcn_raw_buffer_load_b128(rsrc_w, (q < nslots && n < g.N) ? (unsigned)max(off, 0) : 0xffffffffu, 0, 0);
-        wb[p][t] = (v4i){(int)v.x, (int)v.y, (int)v.z, (int)v.w};
-        if (g.Ci < 16 && __any(off < 0))
-          if (off < 0) wb[p][t] = bytes_up(wb[p][t], -off);
-      }
+    for (int u = 0; u < UN; u++) {
+      if (pass + u >= passes) break;
+      const bool in = row < nr && (unsigned)(iy0 + row) < (unsigned)g.H && (unsigned)(ix0 + col) < (unsigned)g.W;
+      voff[u] = (row * g.W + col) * g.Ci + min(16 * c16, g.Ci - 16) + 16;
+      dst[u] = row < nr ? (row * g.IW + col) * g.CP + 16 * c16 : -1;
+      v[u] = __builtin_amdgcn_raw_buffer_load_b128(rsrc_x, in ? (unsigned)(near ? max(voff[u], lo) : voff[u]) : 0xffffffffu, 0, 0);
+      if (near && !in) voff[u] = lo;
+      col += g.scol;
+      row += g.srow;
+      if (col >= g.IW) col -= g.IW, row++;
     }
   };
-  load_w(wf[0], 0);
+  start(0);
+  load(0);
 
-  // ---- per-channel constants and the tap table -> LDS ---------------------------------------------------------------
+  // ---- ... the constants of the thread's channel -----------------------------------------------------------------------
+  int p_bias = 0;
+  bn_t p_k = g.mode == EPI_MULT ? (bn_t)e.mult : (bn_t)1, p_l = 0;
+  if (tid < nch && n0 + tid < g.N) {
+    if (g.bias) p_bias = (int)g.bias[n0 + tid];
+    if (g.mode == EPI_BN) {
+      p_k = e.k[n0 + tid];
+      p_l = e.lambda[n0 + tid];
+    }
+  }
+
+  // ---- ... and the first two groups of weights, on their way to the wave's part of LDS --------------------------------------
+  // Row i of fragment t is channel wn0 + (i/4)*4*TN + 4*t + i%4.  Four lanes fetch the four chunks of a row's step, 64 bytes side by side.
+  const int wn0 = n0 + wave_n * 16 * TN;
+  constexpr unsigned OOB = 0x90000000u;  // (out of range whatever a row's offset adds or takes away)
+  const int ntaps = g.kx * g.ky, ngroups = (g.NK + PF - 1) / PF;
+  unsigned char *wl = band_lds + g.w_off + wave * band_wbytes(TN, PF);
+  const int wr = lane >> 2, wj = (lane & 3) ^ ((wr >> 1) & 3);
+  unsigned nrow[TN];
+#pragma unroll
+  for (int t = 0; t < TN; t++) {
+    const int n = wn0 + (wr >> 2) * (4 * TN) + 4 * t + (wr & 3);
+    nrow[t] = n < g.N ? (unsigned)(n * g.K) : OOB;
+  }
+  int wtap = (int)fastdiv((unsigned)wj, g.d_cg), wc = wj - wtap * g.CG;  // the lane's tap and chunk in the next step that is asked for
+  auto load_w = [&](int half) {
+    const __amdgpu_buffer_rsrc_t rsrc_w = __builtin_amdgcn_make_buffer_rsrc((void *)g.w, 0, (unsigned)g.N * (unsigned)g.K, 0x00020000);
+#pragma unroll
+    for (int p = 0; p < PF; p++) {
+      const int ko = wtap * g.Ci + min(16 * wc, g.Ci - 16);
+#pragma unroll
+      for (int t = 0; t < TN; t++)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_w, (lds_ptr_t)(wl + 1024 * ((half * PF + p) * TN + t)), 16,
+                                                 (int)(wtap < ntaps ? nrow[t] + (unsigned)ko : OOB), 0, 0, 0);
+      wc += g.wc;
+      wtap += g.wtap;
+      if (wc >= g.CG) wc -= g.CG, wtap++;
+    }
+  };
+  load_w(0);
+  if (ngroups > 1) load_w(1);
+  // fewer than 16 channels: the first chunks of channel 0 begin in front of the tensor, and are made from its first 16 bytes
+  const bool w_near = g.Ci < 16 && wn0 == 0;
+  v4i w_head = {0, 0, 0, 0};
+  if (w_near) w_head = *(const v4i_u *)g.w;
+
+  // ---- the tap table: LDS offset of chunk q of the filter; its lowest bit: a pixel's last chunk --------------------------------
+  int *tab = (int *)(band_lds + g.tab_off);
+  for (int q = tid; q < 4 * PF * ngroups; q += 256) {
+    const int tap = (int)fastdiv((unsigned)q, g.d_cg), c = q - tap * g.CG;
+    const int fy = (int)fastdiv((unsigned)tap, g.d_kx), fx = tap - fy * g.kx;
+    tab[q] = tap < ntaps ? (fy * g.IW + fx) * g.CP + 16 * c + (c == g.CG - 1 ? 1 : 0) : 0;  // (chunks past the filter: zero weights)
+  }
+  // the lanes' pixels
+  int base[TM];
+#pragma unroll
+  for (int s = 0; s < TM; s++) {
+    const int p = min((wave_m * TM + s) * 16 + l16, px - 1);
+    const int y = (int)fastdiv((unsigned)p, g.d_pc), x = g.R > 1 ? p - y * pc : p;
+    base[s] = ((g.R > 1 ? y : 0) * g.sy * g.IW + x * g.sx) * g.CP;
+  }
+  // ones where a chunk holds a byte that counts: all of it, or the end of a pixel's last chunk
+  v4i ones_last;
+#pragma unroll
+  for (int d = 0; d < 4; d++) ones_last[d] = (int)(0x01010101u & ~low_bytes(dup - 4 * d));
+  __builtin_amdgcn_sched_barrier(0);
+
+  // ---- constants and input -> LDS --------------------------------------------------------------------------------------------
   int *c_bias = (int *)(band_lds + g.c_off);
   bn_t *c_k = (bn_t *)(c_bias + nch), *c_l = c_k + nch;
   if (tid < nch) {
-    const int n = n0 + tid;
-    const bool ok = n < g.N;
-    c_bias[tid] = (g.bias && ok) ? (int)g.bias[n] : 0;
-    // (only read for batch-norm; written in every mode, which is the shorter code: 57x43 24 -> 40 9.38 us, 9.46 with a branch)
-    c_k[tid] = g.mode == EPI_BN ? (ok ? e.k[n] : (bn_t)0) : g.mode == EPI_MULT ? (bn_t)e.mult : (bn_t)1;
-    c_l[tid] = (g.mode == EPI_BN && ok) ? e.lambda[n] : (bn_t)0;
+    c_bias[tid] = p_bias;
+    c_k[tid] = p_k;
+    c_l[tid] = p_l;
   }
-  int *tab = (int *)(band_lds + g.tab_off);
-  for (int q = tid; q < 4 * g.NK; q += 256) {
-    const int tap = (int)fastdiv((unsigned)q, g.d_cg), c16 = q - tap * g.CG;
-    const int fy = (int)fastdiv((unsigned)tap, g.d_kx), fx = tap - fy * g.kx;
-    tab[q] = q < nslots ? (fy * g.IW + fx) * g.CP + 16 * c16 : 0;  // (slots past the filter: zero weights)
-  }
-
-  // ---- stage the input ------------------------------------------------------------------------------------------------
-  {
-    const int iy0 = oy0 * g.sy - g.pt, ix0 = ox0 * g.sx - g.pl;
-    const int iw = (pc - 1) * g.sx + g.kx, nr = (rows - 1) * g.sy + g.ky;
-    const int chunks = nr * g.IW * g.CG;
-    const long long ibase = (long long)b * g.H * g.W * g.Ci;
-    const int dup = 16 * g.CG - g.Ci;  // bytes of a pixel's last chunk that the one before it has too
-    constexpr int UN = 4;
-    for (int t0 = tid; t0 < chunks; t0 += 256 * UN) {
-      v4i v[UN];
-      int dst[UN], under[UN];
-      unsigned ok[UN];
-      bool last[UN];
+  for (int cb = 0;;) {
+    v4u keep;  // a pixel's last chunk: not the bytes that the chunk before it has
+#pragma unroll
+    for (int d = 0; d < 4; d++) keep[d] = c16 == g.CG - 1 ? ~low_bytes(dup - 4 * d) : 0xffffffffu;
+    for (int pass = 0;;) {
 #pragma unroll
       for (int u = 0; u < UN; u++) {
-        const int t = min(t0 + 256 * u, chunks - 1);
-        const int p = (int)fastdiv((unsigned)t, g.d_cg), c16 = t - p * g.CG;
-        const int row = (int)fastdiv((unsigned)p, g.d_iw), col = p - row * g.IW;
-        const int iy = iy0 + row, ix = ix0 + col;
-        const bool in = (unsigned)iy < (unsigned)g.H && (unsigned)ix < (unsigned)g.W && col < iw;
-        const long long off = in ? ibase + ((long long)iy * g.W + ix) * g.Ci + min(16 * c16, g.Ci - 16) : 0;
-        v[u] = *(const v4i_u *)(g.in + max(off, 0ll));
-        under[u] = off < 0 ? (int)-off : 0;
-        ok[u] = in ? 0xffffffffu : 0u;
-        last[u] = c16 == g.CG - 1;
-        dst[u] = p * g.CP + 16 * c16;
+        if (pass + u >= passes) break;
+        if (near && __any(voff[u] < lo))
+          if (voff[u] < lo) {
+            const v4i w = bytes_up((v4i){(int)v[u].x, (int)v[u].y, (int)v[u].z, (int)v[u].w}, lo - voff[u]);
+            v[u] = (v4u){(unsigned)w.x, (unsigned)w.y, (unsigned)w.z, (unsigned)w.w};
+          }
+        if (dst[u] >= 0) *(v4u *)(band_lds + dst[u]) = (v[u] ^ 0x80808080u) & keep;
       }
-#pragma unroll
-      for (int u = 0; u < UN; u++) {
-        if (g.Ci < 16 && __any(under[u]))
-          if (under[u]) v[u] = bytes_up(v[u], under[u]);
-        v4i w;
-#pragma unroll
-        for (int d = 0; d < 4; d++) w[d] = (int)(((unsigned)v[u][d] & ok[u]) ^ 0x80808080u);
-        if (dup) {
-#pragma unroll
-          for (int d = 0; d < 4; d++) w[d] &= last[u] ? (int)~low_bytes(dup - 4 * d) : -1;
-        }
-        if (t0 + 256 * u < chunks) *(v4i *)(band_lds + dst[u]) = w;
-      }
+      pass += UN;
+      if (pass >= passes) break;
+      load(pass);
     }
+    cb += g.cpp;
+    if (cb >= g.CG) break;
+    start(cb);
+    load(0);
   }
-  __syncthreads();
+  // (not __syncthreads(), which would also wait for the weights, which only their wave reads)
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(BAND_WAIT_LDS);
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
 
   // ---- multiply -----------------------------------------------------------------------------------------------------------
   v4i acc[TN][TM], wacc[TN];
-  int base[TM];
 #pragma unroll
   for (int t = 0; t < TN; t++) {
     wacc[t] = (v4i){0, 0, 0, 0};
 #pragma unroll
     for (int s = 0; s < TM; s++) acc[t][s] = (v4i){0, 0, 0, 0};
   }
-#pragma unroll
-  for (int s = 0; s < TM; s++) {
-    const int p = min((wave_m * TM + s) * 16 + l16, px - 1);
-    const int y = (int)fastdiv((unsigned)p, g.d_pc), x = p - y * pc;
-    base[s] = (y * g.sy * g.IW + x * g.sx) * g.CP;
-  }
-  // ones where a chunk holds a byte that counts: all of it, or the end of a pixel's last chunk
-  const int dup = 16 * g.CG - g.Ci;
-  v4i ones_last;
-#pragma unroll
-  for (int d = 0; d < 4; d++) ones_last[d] = (int)(0x01010101u & ~low_bytes(dup - 4 * d));
   const v4i ones_all = {0x01010101, 0x01010101, 0x01010101, 0x01010101};
-  auto steps = [&](v4i (&wb)[PF][TN], int kk0) {
+  const unsigned char *wfrag = wl + l16 * 64 + ((lgrp ^ ((l16 >> 1) & 3)) << 4);
+  auto steps = [&](int half, int kk0) {
+    int toff[PF];
+#pragma unroll
+    for (int p = 0; p < PF; p++) toff[p] = tab[4 * (kk0 + p) + lgrp];
+    if (w_near && kk0 < 4) {
+#pragma unroll
+      for (int p = 0; p < PF; p++) {
+        const int q = 4 * (kk0 + p) + wj, off = q * g.Ci + g.Ci - 16;
+        if (wr == 0 && off < 0 && q < ntaps) *(v4i *)(wl + (half * PF + p) * TN * 1024 + 16 * lane) = bytes_up(w_head, -off);
+      }
+      asm volatile("" ::: "memory");
+    }
 #pragma unroll
     for (int p = 0; p < PF; p++) {
-      if (kk0 + p < g.NK) {
-        const int q = 4 * (kk0 + p) + lgrp;
-        const int toff = tab[q];
-        v4i ones = ones_all;
-        if (dup) {
-          const int c16 = q - (int)fastdiv((unsigned)q, g.d_cg) * g.CG;
-          if (c16 == g.CG - 1) ones = ones_last;
-        }
-        v4i af[TM];
+      v4i ones = ones_all;
+      if (dup) {
 #pragma unroll
-        for (int s = 0; s < TM; s++) af[s] = *(const v4i *)(band_lds + base[s] + toff);
-#pragma unroll
-        for (int t = 0; t < TN; t++) wacc[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wb[p][t], ones, wacc[t], 0, 0, 0);
-#pragma unroll
-        for (int s = 0; s < TM; s++)
-#pragma unroll
-          for (int t = 0; t < TN; t++) acc[t][s] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wb[p][t], af[s], acc[t][s], 0, 0, 0);
+        for (int d = 0; d < 4; d++) ones[d] = toff[p] & 1 ? ones_last[d] : ones_all[d];
       }
+      v4i af[TM], wf[TN];
+#pragma unroll
+      for (int t = 0; t < TN; t++) wf[t] = *(const v4i *)(wfrag + ((half * PF + p) * TN + t) * 1024);
+#pragma unroll
+      for (int s = 0; s < TM; s++) af[s] = *(const v4i *)(band_lds + base[s] + (toff[p] & ~1));
+#pragma unroll
+      for (int t = 0; t < TN; t++) wacc[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wf[t], ones, wacc[t], 0, 0, 0);
+#pragma unroll
+      for (int s = 0; s < TM; s++)
+#pragma unroll
+        for (int t = 0; t < TN; t++) acc[t][s] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wf[t], af[s], acc[t][s], 0, 0, 0);
     }
   };
-  for (int kk = 0; kk < g.NK; kk += 2 * PF) {
-    if (kk + PF < g.NK) load_w(wf[1], kk + PF);
-    steps(wf[0], kk);
-    if (kk + 2 * PF < g.NK) load_w(wf[0], kk + 2 * PF);
-    if (kk + PF < g.NK) steps(wf[1], kk + PF);
+  // a group is waited for behind the one that was asked for after it
+  auto ready = [&](bool another) {
+    if (another) __builtin_amdgcn_s_waitcnt(BAND_WAIT_VM(PF * TN));
+    else __builtin_amdgcn_s_waitcnt(BAND_WAIT_VM(0));
+    asm volatile("" ::: "memory");
+  };
+  auto again = [&](int half) {  // (the group that lies there has been read)
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(BAND_WAIT_LDS);
+    load_w(half);
+  };
+#pragma unroll 1
+  for (int i = 0; i < ngroups; i += 2) {
+    ready(i + 1 < ngroups);
+    steps(0, i * PF);
+    if (i + 1 >= ngroups) break;
+    if (i + 2 < ngroups) again(0);
+    ready(i + 2 < ngroups);
+    steps(1, (i + 1) * PF);
+    if (i + 3 < ngroups) again(1);
   }
 
   // ---- epilogue: acc[t][s][r] = channel cb + 4*t + r of pixel 16*s + l16 -----------------------------------------------

@@ -5,21 +5,20 @@
 
 namespace {
 
-template <int TN>
-bool launch_tm(int tm, const BandGeom &g, const EpiArgs &e, size_t lds, hipStream_t s)
+template <int TN, int TM, int PF>
+bool launch(const BandGeom &g, const EpiArgs &e, size_t lds, hipStream_t s)
 {
-  const dim3 grid((unsigned)g.total), block(256);
-  if (tm == 2) {
-    if (!raise_lds_limit<conv_band_kernel<TN, 2>>(lds)) return false;
-    hipLaunchKernelGGL((conv_band_kernel<TN, 2>), grid, block, lds, s, g, e);
-  } else if (tm == 4) {
-    if (!raise_lds_limit<conv_band_kernel<TN, 4>>(lds)) return false;
-    hipLaunchKernelGGL((conv_band_kernel<TN, 4>), grid, block, lds, s, g, e);
-  } else {
-    if (!raise_lds_limit<conv_band_kernel<TN, 8>>(lds)) return false;
-    hipLaunchKernelGGL((conv_band_kernel<TN, 8>), grid, block, lds, s, g, e);
-  }
+  if (!raise_lds_limit<conv_band_kernel<TN, TM, PF>>(lds)) return false;
+  hipLaunchKernelGGL((conv_band_kernel<TN, TM, PF>), dim3((unsigned)g.total), dim3(256), lds, s, g, e);
   return true;
+}
+template <int TN>
+bool launch_tm(int tm, int pf, const BandGeom &g, const EpiArgs &e, size_t lds, hipStream_t s)
+{
+  if constexpr (TN == 1)
+    if (tm == 2 && pf != 2) return pf == 4 ? launch<1, 2, 4>(g, e, lds, s) : launch<1, 2, 1>(g, e, lds, s);
+  return tm == 2 ? launch<TN, 2, band_pf(TN, 2)>(g, e, lds, s) : tm == 4 ? launch<TN, 4, band_pf(TN, 4)>(g, e, lds, s)
+                                                                               : launch<TN, 8, band_pf(TN, 8)>(g, e, lds, s);
 }
 
 }  // namespace
@@ -27,11 +26,11 @@ bool launch_tm(int tm, const BandGeom &g, const EpiArgs &e, size_t lds, hipStrea
 bool launch_conv_band(int mode, const ConvLayer &L, const EpiArgs &e, int cus, hipStream_t s)
 {
   BandGeom g;
-  int tn, tm;
+  int tn, tm, pf;
   size_t lds;
-  if (mode == EPI_OUT32 || !band_shape(L, cus, (int)sizeof(bn_t), &g, &tn, &tm, &lds)) return false;
+  if (mode == EPI_OUT32 || !band_shape(L, cus, (int)sizeof(bn_t), &g, &tn, &tm, &lds, &pf)) return false;
   g.mode = mode;
-  if (tn == 1) return launch_tm<1>(tm, g, e, lds, s);
-  if (tn == 2) return launch_tm<2>(tm, g, e, lds, s);
-  return launch_tm<4>(tm, g, e, lds, s);
+  if (tn == 1) return launch_tm<1>(tm, pf, g, e, lds, s);
+  if (tn == 2) return launch_tm<2>(tm, pf, g, e, lds, s);
+  return launch_tm<4>(tm, pf, g, e, lds, s);
 }

@@ -27,14 +27,22 @@ struct BandGeom {
   int IW, NR;          // input columns and rows behind them
   int WN;              // waves along the channels (1, 2 or 4 of four)
   int mode;
-  int tab_off, c_off;  // LDS offsets: tap table, per-channel constants
+  int tab_off, c_off, w_off;  // LDS offsets: tap table, per-channel constants, weights of the four waves
   int nblocks, xtiles, bands, total;
-  FastDiv d_nb, d_xt, d_band, d_cg, d_iw, d_pc, d_kx;
+  int cpp, ppp, srow, scol;   // staging: chunks of a pixel side by side, pixels of a pass, and those as rows and columns of the band
+  int wtap, wc;               // four chunks further: taps and chunks
+  long long in_bytes;
+  FastDiv d_nb, d_xt, d_band, d_cg, d_iw, d_pc, d_kx, d_cpp, d_ppp;
 };
+
+// K steps whose weights a wave asks for together (two such groups are in LDS), by its 16-channel and 16-pixel groups.  With one 16-channel
+// group and two of pixels: four or one, see there.
+PULPNN_HD constexpr int band_pf(int tn, int tm) { return tn == 1 ? 2 : tn == 2 ? (tm == 8 ? 1 : 2) : 1; }
+PULPNN_HD constexpr int band_wbytes(int tn, int pf) { return 2 * pf * tn * 1024; }
 
 // Tile shape; bn_bytes: bytes of a batch-norm parameter.  tn, tm: 16-channel and 16-pixel groups per wave; lds: dynamic LDS
 // of the launch.  False for a layer the kernel does not take.
-inline bool band_shape(const ConvLayer &L, int cus, int bn_bytes, BandGeom *out, int *tn_out, int *tm_out, size_t *lds_out)
+inline bool band_shape(const ConvLayer &L, int cus, int bn_bytes, BandGeom *out, int *tn_out, int *tm_out, size_t *lds_out, int *pf_out = nullptr)
 {
   if ((long long)L.N * L.kx * L.ky * L.Ci >= 0x7fffffffLL || (long long)L.kx * L.ky * L.Ci < 16) return false;
   if ((long long)L.B * L.H * L.W * L.Ci < 16 || (long long)L.H * L.W * L.Ci >= (1ll << 40)) return false;
@@ -74,38 +82,49 @@ inline bool band_shape(const ConvLayer &L, int cus, int bn_bytes, BandGeom *out,
   const int wm = 4 / g.WN;
   // LDS of a tile, in 64 bits: strides and filters far larger than the image give more bytes than an int counts (the fields
   // are what they should be for tiles that fit)
-  auto lds_for = [&](int r, int pc) -> long long {
+  auto lds_for = [&](int r, int pc, int t) -> long long {
     const long long iw = (pc - 1) * (long long)L.sx + L.kx, nr = (r - 1) * (long long)L.sy + L.ky;
-    const long long tab = nr * iw * g.CP, c = tab + 16ll * g.NK;
+    const long long tab = nr * iw * g.CP, c = tab + 16ll * ((g.NK + 3) & ~3);  // (whole groups of steps)
+    const long long w = (c + 16ll * tn * g.WN * (4 + 2 * bn_bytes) + 1023) & ~1023ll;
     g.R = r;
     g.PC = pc;
     g.IW = (int)iw;
     g.NR = (int)nr;
     g.tab_off = (int)tab;
     g.c_off = (int)c;
-    return c + 16ll * tn * g.WN * (4 + 2 * bn_bytes);
+    g.w_off = (int)w;
+    // (offsets inside a tile's input have to fit an int as well)
+    return (nr - 1) * L.W * L.Ci + iw * L.Ci < 0x7ffffff0ll ? w + 4ll * band_wbytes(tn, band_pf(tn, t)) : 1ll << 40;
   };
-  // the largest run of pixels whose input fits; fewer while that leaves compute units idle
+  constexpr int MOST = 160 * 1024 - 512;
+  // The run of pixels of a workgroup: the one with which the busiest compute unit has least to do, a workgroup's set-up counting as
+  // three 16-pixel groups of 16 channels a wave, two of 32, one of 64.  (64 channels a wave take 500 registers with eight groups: one wave per SIMD, so up to four there.)
   int tm = 0, r = 1, pc = 1;
-  const int tries[] = {8, 4, 2};
-  for (const int t : tries) {
+  long long least = 0;
+  for (int t = tn == 4 ? 4 : 8; t >= 2; t /= 2) {
     const int px = 16 * t * wm;
-    pc = std::min(px, g.Wo);
-    r = std::max(1, std::min(px / pc, g.Ho));
-    if (pc < g.Wo) r = 1;
-    while (r > 1 && lds_for(r, pc) > 64 * 1024) r--;
-    const long long lds = lds_for(r, pc);
-    const long long wgs = (long long)B * ((g.Ho + r - 1) / r) * ((g.Wo + pc - 1) / pc) * ((g.N + 16 * tn * g.WN - 1) / (16 * tn * g.WN));
+    int tpc = std::min(px, g.Wo), tr = tpc < g.Wo ? 1 : std::max(1, std::min(px / tpc, g.Ho));
+    while (tr > 1 && lds_for(tr, tpc, t) > 80 * 1024) tr--;
+    while (t == 2 && tpc > 1 && lds_for(tr, tpc, t) > MOST) tpc = (tpc + 1) / 2;
+    if (t > 2 && lds_for(tr, tpc, t) > 80 * 1024) continue;
+    const long long wgs = (long long)B * ((g.Ho + tr - 1) / tr) * ((g.Wo + tpc - 1) / tpc) * ((g.N + 16 * tn * g.WN - 1) / (16 * tn * g.WN));
+    if (t > 2 && wgs < cus) continue;
+    const long long work = (wgs + cus - 1) / cus * ((tn == 4 ? 1 : 4 - tn) + (tr * tpc + 16 * wm - 1) / (16 * wm));
+    if (tm && work >= least) continue;
+    least = work;
     tm = t;
-    if (lds <= (t == 2 ? 150 : 64) * 1024 && (wgs >= 2ll * cus || t == 2)) break;
+    r = tr;
+    pc = tpc;
   }
   g.xtiles = (g.Wo + pc - 1) / pc;
   // a row split evenly, rows spread evenly over the bands
   if (g.xtiles > 1) pc = (int)(((long long)g.Wo + g.xtiles - 1) / g.xtiles);
   g.bands = (g.Ho + r - 1) / r;
   r = (g.Ho + g.bands - 1) / g.bands;
-  const long long lds = lds_for(r, pc);
-  if (lds > 150 * 1024) return false;
+  // (no more pixels a wave than the tile has: all waves take part where LDS holds few rows)
+  while (tm > 2 && r * pc <= 16 * (tm / 2) * wm && lds_for(r, pc, tm / 2) <= MOST) tm /= 2;
+  long long lds = lds_for(r, pc, tm);
+  if (lds > MOST) return false;
   g.nblocks = (g.N + 16 * tn * g.WN - 1) / (16 * tn * g.WN);
   const long long total = (long long)B * g.bands * g.xtiles * g.nblocks;
   if (total > 0x7fffffffLL) return false;
@@ -117,8 +136,30 @@ inline bool band_shape(const ConvLayer &L, int cus, int bn_bytes, BandGeom *out,
   g.d_iw = fastdiv_make((unsigned)g.IW);
   g.d_pc = fastdiv_make((unsigned)g.PC);
   g.d_kx = fastdiv_make((unsigned)g.kx);
+  g.cpp = std::min(g.CG, 256);
+  g.ppp = 256 / g.cpp;
+  g.srow = g.ppp / g.IW;
+  g.scol = g.ppp % g.IW;
+  g.wtap = 4 / g.CG;
+  g.wc = 4 % g.CG;
+  g.in_bytes = (long long)L.B * L.H * L.W * L.Ci;
+  g.d_cpp = fastdiv_make((unsigned)g.cpp);
+  g.d_ppp = fastdiv_make((unsigned)g.ppp);
   *tn_out = tn;
   *tm_out = tm;
+  // Groups of weights: four steps for long filters in launches of few workgroups, which wait for their weights; one where that lets another
+  // workgroup share a compute unit (call times, two / four steps: 8x38x9 240 -> 32 stride 2 11.4 / 11.0; 57x43 24 -> 40 stride 2 batch 32
+  // 8.0 / 8.5, 19x33 85 -> 8 batch 123 11.1 / 13.7; two / one: 27x39 pointwise 320 -> 8 batch 215 25.7 / 20.7).
+  int pf = band_pf(tn, tm);
+  if (tn == 1 && tm == 2) {
+    const auto with = [&](int n) { return lds + 4 * (band_wbytes(1, n) - band_wbytes(1, pf)); };
+    const int to = g.NK > 8 && total <= 2ll * cus && with(4) <= (total <= cus ? MOST : 80 * 1024) ? 4
+                   : total > 2ll * cus && MOST / with(1) > MOST / with(2) && MOST / with(2) < 3    ? 1
+                                                                                                   : 2;
+    lds = with(to);
+    pf = to;
+  }
+  if (pf_out) *pf_out = pf;
   *lds_out = (size_t)lds;
   return true;
 }

@@ -21,11 +21,23 @@ CONV = [
     (2, 7, 9, 250, 20, 5, 5, (2, 2, 2, 2), (1, 1)),    # K = 6250: several rounds of weight prefetch
     (1, 20, 17, 144, 35, 3, 3, (1, 1, 1, 1), (1, 1)),  # whole chunks, few output channels
 ]
+# where the band kernel's groups of weights, its passes over the input and its tiles change form
+BAND = [
+    (2, 10, 19, 112, 32, 3, 3, (1, 1, 1, 1), (1, 1)),   # few workgroups, 16 K steps: groups of four
+    (1, 12, 20, 250, 16, 3, 3, (1, 1, 1, 1), (2, 2)),   # ... an odd number of groups, one wave along the channels
+    (1, 3, 4, 4100, 5, 2, 2, (0, 0, 0, 0), (1, 1)),     # 257 chunks a pixel: two rounds of 256
+    (3, 9, 6, 3, 70, 7, 7, (3, 3, 3, 3), (1, 1)),       # three channels, 13 K steps: the first 16 chunks of channel 0 in several groups
+    (1, 6, 8, 1, 140, 4, 5, (2, 1, 2, 2), (1, 1)),      # ... and one channel with four groups of 16 a wave
+    (260, 6, 7, 24, 100, 3, 3, (1, 1, 1, 1), (1, 1)),   # two groups a wave, eight of pixels
+    (40, 21, 26, 8, 150, 3, 3, (1, 1, 1, 1), (1, 1)),   # four and four
+    (1, 5, 150, 256, 20, 5, 5, (2, 2, 2, 2), (2, 1)),   # a tile that LDS holds part of a row for
+]
 POINTWISE = [
     # B, H, W, Ci, Co
     (40, 33, 31, 8, 16), (40, 33, 31, 15, 17), (40, 33, 31, 17, 31), (30, 32, 33, 63, 66), (30, 32, 33, 65, 130),
     (30, 32, 33, 130, 255), (24, 33, 33, 257, 64), (24, 33, 33, 500, 100), (24, 33, 33, 512, 260), (40, 32, 32, 48, 424),
     (9, 29, 31, 72, 20), (3, 9, 7, 9, 5), (1, 1, 1, 20, 24), (2, 5, 5, 600, 30),
+    (75, 30, 31, 320, 8),  # (band kernel: weights a step at a time)
 ]
 
 
@@ -42,7 +54,7 @@ def _requant(r, n, bn_bits, relu, bn, K):
 
 @pytest.mark.parametrize("bn_bits", [32, 64])
 @pytest.mark.parametrize("flags", [(1, 1), (1, 0), (0, 0)])
-@pytest.mark.parametrize("geom", CONV, ids=lambda g: "x".join(map(str, g[:7])))
+@pytest.mark.parametrize("geom", CONV + BAND, ids=lambda g: "x".join(map(str, g[:7])))
 def test_conv_any_channels(geom, flags, bn_bits):
     B, H, W, Ci, Co, ky, kx, pads, strides = geom
     relu, bn = flags
