@@ -135,11 +135,15 @@ bool launch_igemm_patch(int mode, ConvGeom &g, const EpiArgs &e, hipStream_t s)
 // 128 px x 64 ch tiles, for layers too small to fill the machine with larger ones.  With at most five
 // K slices (K <= 320) a tile's whole K extent fits in LDS and is fetched in one go.  Eight waves of 32 x 32 per tile
 // rather than four of 64 x 32: these layers are a chain of latencies (gather, stage, multiply, store), and with twice
-// the waves every link is issued in half the time (config 0: 7.0 -> 6.6 us).
+// the waves every link is issued in half the time (config 0: 7.0 -> 6.6 us).  Longer ones nine slices at a time in 110 KB where
+// every tile has a compute unit to itself (16x16 64 -> 64 batch 64 6.4 -> 5.6 us, 14x14 128 -> 128 batch 60 9.9 -> 8.8, 12x12 256 -> 200 batch 5
+// 14.4 -> 13.3; but 316 tiles, 10x10 256 -> 256 batch 100, 19.5 -> 26.5).
 template <int GATHER>
 void launch_igemm_small(int mode, ConvGeom &g, const EpiArgs &e, hipStream_t s)
 {
   if (GATHER != GATHER_BYTES && g.K <= 5 * IGEMM_BK) launch_igemm_mode<2, 4, 2, GATHER, 2, 5>(mode, g, e, s);
+  else if (GATHER == GATHER_UNIFORM && (long long)((g.M + 127) / 128) * ((g.N + 63) / 64) <= num_cus())
+    launch_igemm_mode<2, 4, 2, GATHER, 2, GATHER == GATHER_UNIFORM ? 9 : 0>(mode, g, e, s);
   else launch_igemm_mode<2, 4, 2, GATHER, 2>(mode, g, e, s);
 }
 
@@ -377,8 +381,8 @@ void conv_common(const char *fn, bool pointwise, const uint8_t *in, const int8_t
     // chunk by chunk, on images of up to some 60000 pixels in all (tiled / band: 12x12 112 -> 71 batch 146 16.5 / 10.3 us, 41x11 160 -> 100 batch 2
     // 12.9 / 9.1, 59x17 96 -> 128 batch 7 8.7 / 8.2; but 42x31 48 -> 96 batch 54 14.4 / 18.3, 34x53 176 -> 128 batch 36 29.1 / 34.9; the mean over 52
     // layers is 0.88, over the 44 on this side of the line 0.85, two of them slower: 63x21 96 -> 96 stride 2 batch 39 9.3 / 11.0), as long as a tile's
-    // input leaves LDS to a second workgroup (5x5 on 208 channels 66 / 124).
-    const bool odd64 = ch_in % 64 && g.N <= 128 && g.M <= 60000 && (kx * ky <= 9 || ch_in <= 96);
+    // input leaves LDS to a second workgroup (5x5 on 208 channels 66 / 124), and not for pointwise layers (12x11 48 -> 112 batch 5 4.0 / 5.0).
+    const bool odd64 = ch_in % 64 && g.N <= 128 && g.M <= 60000 && kx * ky > 1 && (kx * ky <= 9 || ch_in <= 96);
     const bool few = ch_in == 16 || ch_in == 32 ? false : ch_in % 64 == 0 ? g.N <= 32 : g.N <= 64 || odd64;
     if (!whole16 || few) {
       if (launch_conv_band(mode, L, e, num_cus(), g_stream)) return check_launch(fn);

@@ -163,10 +163,9 @@ __device__ __forceinline__ void igemm_epilogue(v4i (&acc)[TN][TM], const ConvGeo
   }
 }
 
-// ONEPASS > 0: the layer has at most ONEPASS K slices and the whole K extent of a tile is staged at
-// once: all global loads of the tile are issued back to back (one memory round trip instead of one
-// per slice), then staged, and after a single barrier the slices are multiplied one after the other.
-// Layers this short are bound by those round trips, not by bytes or multiplies.
+// ONEPASS > 0: up to ONEPASS K slices of a tile are staged at once: their global loads are issued back to back (one
+// memory round trip instead of one per slice), then staged, and after a single barrier the slices are multiplied one after
+// the other.  Layers this small are bound by those round trips, not by bytes or multiplies.
 template <int TN, int WAVES_M, int WAVES_N, int GATHER, int MODE, int TM = 4, int ONEPASS = 0>
 __global__ __launch_bounds__(64 * WAVES_M * WAVES_N,
                             (WAVES_M * WAVES_N > 8 || TM > 4) ? 1 : (WAVES_M * WAVES_N > 4 || GATHER == GATHER_BYTES || ONEPASS ? 2 : IGEMM_MINB))
@@ -190,6 +189,13 @@ void igemm_kernel(ConvGeom g, EpiArgs e)
   __shared__ int cbias[BN];
   __shared__ bn_t ck_[MODE == EPI_BN ? BN : 1], cl_[MODE == EPI_BN ? BN : 1];
 
+  // the launch's numbers at once and opaque (as in dw_mfma_kernel; the chunk gather, which is bound by its arithmetic, is 2-5 % slower with it)
+  if constexpr (UNI) {
+    asm volatile("" : "+s"(g.tiles_total), "+s"(g.tiles_n), "+s"(g.in), "+s"(g.w), "+s"(g.bias), "+s"(g.out), "+s"(g.M), "+s"(g.N), "+s"(g.K),
+                 "+s"(g.H), "+s"(g.W), "+s"(g.Ci), "+s"(g.HoWo), "+s"(g.Wo), "+s"(g.in_img));
+    asm volatile("" : "+s"(g.kx), "+s"(g.ky), "+s"(g.pt), "+s"(g.pl), "+s"(g.sx), "+s"(g.sy), "+s"(g.batch), "+s"(g.ci_shift), "+s"(g.rkx),
+                 "+s"(g.vec_store), "+s"(g.nt), "+s"(e.k), "+s"(e.lambda), "+s"(e.mult), "+s"(e.shift));
+  }
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
   const int wave_m = wave % WAVES_M, wave_n = wave / WAVES_M;
@@ -441,40 +447,71 @@ void igemm_kernel(ConvGeom g, EpiArgs e)
       for (int s = 0; s < TM; s++)
         acc[t][s] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wf[t], af[s], acc[t][s], 0, 0, 0);
   };
-  // Slices past the end are loaded and staged but never multiplied: no branches needed.
-  // (The loop is kept rolled: unrolled by two it costs 60 more registers and a workgroup per CU.)
-  for (int c = tid; c < BN; c += NTH) {
-    const int n = n0 + c;
-    int b = 0;
-    bn_t kv = 0, lv = 0;
-    if (n < g.N) {
-      if (g.bias) b = (MODE == EPI_OUT32) ? ((const int *)g.bias)[n] : (int)g.bias[n];
-      if (MODE == EPI_BN) {
-        kv = e.k[n];
-        lv = e.lambda[n];
+  // The constants of the tile's channels are asked for with the first slices and written to LDS behind them.
+  constexpr int NC = (BN + NTH - 1) / NTH;
+  int p_b[NC];
+  bn_t p_k[NC], p_l[NC];
+  auto load_constants = [&]() {
+#pragma unroll
+    for (int i = 0; i < NC; i++) {
+      const int n = n0 + tid + NTH * i;
+      p_b[i] = 0;
+      p_k[i] = p_l[i] = 0;
+      if (tid + NTH * i < BN && n < g.N) {
+        if (g.bias) p_b[i] = (MODE == EPI_OUT32) ? ((const int *)g.bias)[n] : (int)g.bias[n];
+        if (MODE == EPI_BN) {
+          p_k[i] = e.k[n];
+          p_l[i] = e.lambda[n];
+        }
       }
     }
-    cbias[c] = b;
-    if (MODE == EPI_BN) {
-      ck_[c] = kv;
-      cl_[c] = lv;
+  };
+  auto store_constants = [&]() {
+#pragma unroll
+    for (int i = 0; i < NC; i++) {
+      const int c = tid + NTH * i;
+      if (c >= BN) break;
+      cbias[c] = p_b[i];
+      if (MODE == EPI_BN) {
+        ck_[c] = p_k[i];
+        cl_[c] = p_l[i];
+      }
     }
+  };
+  // (the chunk gather keeps the loads' arithmetic busy for so long that its constants are there before: first, and stored at once)
+  if constexpr (!UNI) {
+    load_constants();
+    store_constants();
   }
   if constexpr (ONEPASS > 0) {
-    Staged R[ONEPASS];
+    // up to ONEPASS slices at a time
+    for (int k0 = 0;;) {
+      Staged R[ONEPASS];
 #pragma unroll
-    for (int kt = 0; kt < ONEPASS; kt++)
-      if (kt < KT) gload(R[kt]);
+      for (int kt = 0; kt < ONEPASS; kt++)
+        if (k0 + kt < KT) gload(R[kt]);
+      if (k0 == 0 && UNI) load_constants();
+      if (k0) __syncthreads();  // (the slices before have been multiplied)
 #pragma unroll
-    for (int kt = 0; kt < ONEPASS; kt++)
-      if (kt < KT) sts(R[kt], kt, true);
-    __syncthreads();
+      for (int kt = 0; kt < ONEPASS; kt++)
+        if (k0 + kt < KT) sts(R[kt], kt, true);
+      if (k0 == 0 && UNI) store_constants();
+      __syncthreads();
 #pragma unroll
-    for (int kt = 0; kt < ONEPASS; kt++)
-      if (kt < KT) compute(kt);
+      for (int kt = 0; kt < ONEPASS; kt++)
+        if (k0 + kt < KT) compute(kt);
+      k0 += ONEPASS;
+      // (Layers of more than five slices come here with nine.  As a loop the constants' loads stay behind those of the operands also with
+      // five: 16x16 32 -> 64 batch 1 4.18 us, 4.35 without; the chunk gather, straight-line, is 2-8 % faster without.)
+      if (!UNI || k0 >= KT) break;
+    }
   } else {
+    // Slices past the end are loaded and staged but never multiplied: no branches needed.
+    // (The loop is kept rolled: unrolled by two it costs 60 more registers and a workgroup per CU.)
     gload(R0);
+    if constexpr (UNI) load_constants();
     sts(R0, 0, true);
+    if constexpr (UNI) store_constants();
     __syncthreads();
 #pragma unroll 1
     for (int kt = 0; kt < KT; kt++) {

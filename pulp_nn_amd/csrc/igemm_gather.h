@@ -3,6 +3,8 @@
 #pragma once
 #include "fastdiv.h"
 
+PULPNN_HD int igemm_clamp(int n, int most) { return n < 0 ? 0 : n > most ? most : n; }
+
 // What a lane keeps for one pixel row of the tile: the byte offset of its chunk at tap (0, 0), from a buffer that starts
 // (pt * W + pl) * Ci bytes in front of the input, and one bit per tap that lies outside the image.  SUB: several taps per K
 // slice (16 or 32 input channels); ck: the lane's 16-byte chunk of the slice.  G: ConvGeom.
@@ -18,12 +20,17 @@ PULPNN_HD void igemm_row_gather(const G &g, int m, int ck, unsigned *poff, unsig
     const int oy = (int)fastdiv((unsigned)rem, g.d_wo), ox = rem - oy * g.Wo;
     *poff = (unsigned)b * (unsigned)g.in_img + (unsigned)((oy * g.sy * g.W + ox * g.sx) * g.Ci) +
             (SUB ? (16u * ck) & (unsigned)(g.Ci - 1) : 16u * ck);
-    if (SUB) *pinv = ~0u << (g.kx * g.ky);  // taps past the filter (the tail of the last K slice)
-    for (int fy_ = 0, t = 0; fy_ < g.ky; fy_++)
-      for (int fx_ = 0; fx_ < g.kx; fx_++, t++) {
-        const int iy = oy * g.sy - g.pt + fy_, ix = ox * g.sx - g.pl + fx_;
-        if ((unsigned)iy >= (unsigned)g.H || (unsigned)ix >= (unsigned)g.W) *pinv |= 1u << t;
-      }
+    // taps inside the image: columns fx_lo .. fx_hi - 1 of rows fy_lo .. fy_hi - 1, a bit pattern of columns times one bit per row
+    const int iy = oy * g.sy - g.pt, ix = ox * g.sx - g.pl;
+    if (g.kx * g.ky == 1) {
+      *pinv = (unsigned)iy < (unsigned)g.H && (unsigned)ix < (unsigned)g.W ? ~1u : ~0u;
+      return;
+    }
+    const int fy_hi = igemm_clamp(g.H - iy, g.ky), fy_lo = igemm_clamp(-iy, fy_hi), fx_hi = igemm_clamp(g.W - ix, g.kx), fx_lo = igemm_clamp(-ix, fx_hi);
+    unsigned rows = 0;
+    for (int fy_ = 0; fy_ < g.ky; fy_++) rows |= 1u << (fy_ * g.kx);
+    const unsigned in_rows = rows & (unsigned)((1ull << (fy_hi * g.kx)) - (1ull << (fy_lo * g.kx)));
+    *pinv = ~((unsigned)((1ull << fx_hi) - (1ull << fx_lo)) * in_rows);  // (SUB: the tail of the last K slice past the filter too)
   }
 }
 

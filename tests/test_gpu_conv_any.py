@@ -32,6 +32,17 @@ BAND = [
     (40, 21, 26, 8, 150, 3, 3, (1, 1, 1, 1), (1, 1)),   # four and four
     (1, 5, 150, 256, 20, 5, 5, (2, 2, 2, 2), (2, 1)),   # a tile that LDS holds part of a row for
 ]
+# small layers of the tiled kernel: nine K slices at a time, taps outside the image on every side
+TILED = [
+    (1, 9, 11, 64, 40, 3, 3, (1, 1, 1, 1), (1, 1)),     # nine slices
+    (1, 8, 9, 64, 72, 2, 5, (1, 0, 2, 2), (1, 1)),      # ten
+    (2, 7, 8, 128, 70, 3, 3, (1, 1, 1, 1), (2, 2)),     # eighteen
+    (1, 6, 7, 192, 100, 3, 3, (2, 1, 0, 2), (1, 2)),    # three times nine, two rows of padding
+    (1, 4, 5, 64, 48, 5, 6, (4, 4, 5, 5), (1, 1)),      # a window larger than the image
+    (2, 5, 6, 64, 40, 1, 1, (1, 1, 2, 1), (1, 1)),      # one tap, and pixels that lie in the padding
+    (2, 6, 5, 32, 70, 1, 1, (1, 2, 1, 1), (2, 1)),
+    (1, 7, 6, 16, 36, 3, 5, (1, 1, 2, 2), (1, 1)),      # four taps a slice
+]
 POINTWISE = [
     # B, H, W, Ci, Co
     (40, 33, 31, 8, 16), (40, 33, 31, 15, 17), (40, 33, 31, 17, 31), (30, 32, 33, 63, 66), (30, 32, 33, 65, 130),
@@ -54,7 +65,7 @@ def _requant(r, n, bn_bits, relu, bn, K):
 
 @pytest.mark.parametrize("bn_bits", [32, 64])
 @pytest.mark.parametrize("flags", [(1, 1), (1, 0), (0, 0)])
-@pytest.mark.parametrize("geom", CONV + BAND, ids=lambda g: "x".join(map(str, g[:7])))
+@pytest.mark.parametrize("geom", CONV + BAND + TILED, ids=lambda g: "x".join(map(str, g[:7])))
 def test_conv_any_channels(geom, flags, bn_bits):
     B, H, W, Ci, Co, ky, kx, pads, strides = geom
     relu, bn = flags
