@@ -6,7 +6,7 @@
 #include "igemm.h"
 #include "igemm_patch.h"
 #include "igemm_ring.h"
-#include "linear_any.h"
+#include "linear_skinny.h"
 #include "pw_any_geom.h"
 #include "pw_stream.h"
 #include "smallk.h"
@@ -204,15 +204,27 @@ void launch_smallk(int mode, ConvGeom &g, const EpiArgs &e, hipStream_t s)
   }
 }
 
-template <bool ANY>
-void launch_skinny(int mode, const SkinnyGeom &g, const EpiArgs &e, dim3 grid, hipStream_t s)
+template <auto KERN>
+bool launch_skinny_kernel(const SkinnyGeom &g, const EpiArgs &e, dim3 grid, hipStream_t s)
 {
-  const dim3 block(256);
+  if (!raise_lds_limit<KERN>(SKINNY_LDS)) return false;
+  hipLaunchKernelGGL(KERN, grid, dim3(256), SKINNY_LDS, s, g, e);
+  return true;
+}
+template <int MODE, bool ANY>
+bool launch_skinny_mode(const SkinnyGeom &g, const EpiArgs &e, dim3 grid, hipStream_t s)
+{
+  if constexpr (ANY) return launch_skinny_kernel<linear_skinny_any_kernel<MODE>>(g, e, grid, s);
+  else return launch_skinny_kernel<linear_skinny_kernel<MODE>>(g, e, grid, s);
+}
+template <bool ANY>
+bool launch_skinny(int mode, const SkinnyGeom &g, const EpiArgs &e, dim3 grid, hipStream_t s)
+{
   switch (mode) {
-    case EPI_BN: hipLaunchKernelGGL((ANY ? linear_skinny_any_kernel<EPI_BN> : linear_skinny_kernel<EPI_BN>), grid, block, 0, s, g, e); break;
-    case EPI_MULT: hipLaunchKernelGGL((ANY ? linear_skinny_any_kernel<EPI_MULT> : linear_skinny_kernel<EPI_MULT>), grid, block, 0, s, g, e); break;
-    case EPI_RAW: hipLaunchKernelGGL((ANY ? linear_skinny_any_kernel<EPI_RAW> : linear_skinny_kernel<EPI_RAW>), grid, block, 0, s, g, e); break;
-    default: hipLaunchKernelGGL((ANY ? linear_skinny_any_kernel<EPI_OUT32> : linear_skinny_kernel<EPI_OUT32>), grid, block, 0, s, g, e); break;
+    case EPI_BN: return launch_skinny_mode<EPI_BN, ANY>(g, e, grid, s);
+    case EPI_MULT: return launch_skinny_mode<EPI_MULT, ANY>(g, e, grid, s);
+    case EPI_RAW: return launch_skinny_mode<EPI_RAW, ANY>(g, e, grid, s);
+    default: return launch_skinny_mode<EPI_OUT32, ANY>(g, e, grid, s);
   }
 }
 
@@ -404,12 +416,11 @@ void linear_common(const char *fn, int mode, const uint8_t *in, const int8_t *bi
     // K in four parts and a workgroup per block of rows while that still leaves CUs without work
     const bool spread = ngroups * rblocks <= 2 * num_cus();
     const int kparts = spread ? 4 : (rblocks == 1 ? 4 : (rblocks == 2 ? 2 : 1));
-    const SkinnyGeom sg = {in, w, bias, out, rows, (int)num_o_neurons, (int)dim_vec, kparts};
+    const SkinnyGeom sg = {in, w, bias, out, rows, (int)num_o_neurons, (int)dim_vec, kparts, kparts == 4 ? 2 : kparts == 2 ? 1 : 0,
+                           num_o_neurons % 4 == 0 && aligned(out, 4)};
     const dim3 grid(ngroups, spread ? rblocks : 1);
-    if (dim_vec % 16 == 0 && aligned(in, 16) && aligned(w, 16) && aligned(out, 4)) launch_skinny<false>(mode, sg, e, grid, g_stream);
-    else launch_skinny<true>(mode, sg, e, grid, g_stream);
-    check_launch(fn);
-    return;
+    const bool whole = dim_vec % 16 == 0 && aligned(in, 16) && aligned(w, 16);
+    if (whole ? launch_skinny<false>(mode, sg, e, grid, g_stream) : launch_skinny<true>(mode, sg, e, grid, g_stream)) return check_launch(fn);
   }
   ConvGeom g;
   g.in = in;

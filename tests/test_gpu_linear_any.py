@@ -1,4 +1,4 @@
-"""Linear layers whose rows are not whole 16-byte chunks (csrc/linear_any.h): lengths around a chunk, a K slice and
+"""Linear layers whose rows are not whole 16-byte chunks (csrc/linear_skinny.h): lengths around a chunk, a K slice and
 the parts K is dealt in; neurons and rows around their blocks; operands that start at an odd address."""
 import numpy as np
 import pytest
@@ -16,8 +16,12 @@ GEOMS = [
 ]
 
 
+# the ring of four K slices (a wave's part of K shorter, as long, longer), one to four groups of 16 rows, one, two and four parts of K
+RING = [(1, 1024, 20), (17, 1088, 40), (33, 1280, 17), (49, 2560, 36), (64, 4096, 16), (100, 704, 8208), (250, 320, 8224), (40, 1300, 8208)]
+
+
 @pytest.mark.parametrize("bn_bits", [32, 64])
-@pytest.mark.parametrize("geom", GEOMS, ids=lambda g: "x".join(map(str, g)))
+@pytest.mark.parametrize("geom", GEOMS + RING, ids=lambda g: "x".join(map(str, g)))
 def test_linear_any_length(geom, bn_bits):
     M, K, N = geom
     r = rng_for(8300 + K + bn_bits)
