@@ -2,6 +2,14 @@
 // VALU kernels, one thread per output pixel and group of 4 channels (16 for
 // add), so that neighbouring lanes read and write neighbouring bytes.
 #pragma once
+//
+// Bound: small maps by launch and one trip to memory (all taps of a window of up to 4 x 4, or 3 x 3 for the maximum, are asked for
+// together); large ones by HBM.  The place of a thread takes 32-bit divisions by multiplication: written in 64 bits it was some 600
+// instructions.  Whole calls, that and a row of taps per trip / now: average 4x4 on 64 images of 16x16x64 4.2 / 3.2 us, 2x2 on 64 of 32x32x256
+// 11.4 / 8.1 (21 MB), 7x7 on 32 of 7x7x1000 7.6 / 5.6; maximum 3x3 on 112x112x64 3.8 / 3.05, on 64 of 56x56x64 6.0 / 5.9.
+#include <type_traits>
+
+#include "fastdiv.h"
 #include "memops.h"
 #include "requant.h"
 
@@ -26,7 +34,40 @@ struct PoolGeom {
   int cgroups;   // ceil(C / 4)
   int vec4;      // pointers and C are multiples of 4
   long long total;  // B * Ho * Wo * cgroups threads
+  FastDiv d_cg, d_wo, d_ho;  // divisions by cgroups, Wo, Ho
 };
+// (call once cgroups is known)
+static inline void pool_threads(PoolGeom *g)
+{
+  g->total = (long long)g->B * g->Ho * g->Wo * g->cgroups;
+  g->d_cg = fastdiv_make((unsigned)g->cgroups);
+  g->d_wo = fastdiv_make((unsigned)g->Wo);
+  g->d_ho = fastdiv_make((unsigned)g->Ho);
+}
+
+// A thread's channel group and output pixel.
+struct PoolPlace {
+  int cg, ox, oy, b;
+};
+__device__ __forceinline__ PoolPlace pool_place(const PoolGeom &g, long long t)
+{
+  PoolPlace p;
+  if (g.total <= 0xffffffffll) {
+    const unsigned i = (unsigned)t, q = fastdiv(i, g.d_cg), r = fastdiv(q, g.d_wo), b = fastdiv(r, g.d_ho);
+    p.cg = (int)(i - q * (unsigned)g.cgroups);
+    p.ox = (int)(q - r * (unsigned)g.Wo);
+    p.oy = (int)(r - b * (unsigned)g.Ho);
+    p.b = (int)b;
+  } else {
+    p.cg = (int)(t % g.cgroups);
+    t /= g.cgroups;
+    p.ox = (int)(t % g.Wo);
+    t /= g.Wo;
+    p.oy = (int)(t % g.Ho);
+    p.b = (int)(t / g.Ho);
+  }
+  return p;
+}
 
 __device__ __forceinline__ unsigned load4(const uint8_t *p, int n, int vec4)
 {
@@ -51,14 +92,10 @@ __device__ __forceinline__ void store4(uint8_t *p, unsigned v, int n, int vec4)
 // overwrites its input; this kernel reads the input once and leaves it intact.
 __global__ __launch_bounds__(256) void maxpool_kernel(PoolGeom g)
 {
-  long long t = (long long)blockIdx.x * 256 + threadIdx.x;
+  const long long t = (long long)blockIdx.x * 256 + threadIdx.x;
   if (t >= g.total) return;
-  const int cg = (int)(t % g.cgroups);
-  t /= g.cgroups;
-  const int ox = (int)(t % g.Wo);
-  t /= g.Wo;
-  const int oy = (int)(t % g.Ho);
-  const int b = (int)(t / g.Ho);
+  const PoolPlace at = pool_place(g, t);
+  const int cg = at.cg, ox = at.ox, oy = at.oy, b = at.b;
   const int c = cg * 4, n = min(4, g.C - c);
   const int xs = max(ox * g.sx - g.pl, 0), xe = min(ox * g.sx - g.pl + g.kx, g.W);
   const int ys = max(oy * g.sy - g.pt, 0), ye = min(oy * g.sy - g.pt + g.ky, g.H);
@@ -76,14 +113,10 @@ __global__ __launch_bounds__(256) void maxpool_kernel(PoolGeom g)
 template <bool NT, bool LNT>
 __global__ __launch_bounds__(256) void maxpool16_kernel(PoolGeom g)
 {
-  long long t = (long long)blockIdx.x * 256 + threadIdx.x;
+  const long long t = (long long)blockIdx.x * 256 + threadIdx.x;
   if (t >= g.total) return;
-  const int cg = (int)(t % g.cgroups);
-  t /= g.cgroups;
-  const int ox = (int)(t % g.Wo);
-  t /= g.Wo;
-  const int oy = (int)(t % g.Ho);
-  const int b = (int)(t / g.Ho);
+  const PoolPlace at = pool_place(g, t);
+  const int cg = at.cg, ox = at.ox, oy = at.oy, b = at.b;
   const int xs = max(ox * g.sx - g.pl, 0), xe = min(ox * g.sx - g.pl + g.kx, g.W);
   const int ys = max(oy * g.sy - g.pt, 0), ye = min(oy * g.sy - g.pt + g.ky, g.H);
   const uint8_t *img = g.in + (long long)b * g.H * g.W * g.C + cg * 16;
@@ -104,8 +137,15 @@ __global__ __launch_bounds__(256) void maxpool16_kernel(PoolGeom g)
     vmax(m, v2);
     vmax(m, v3);
   } else {
-    for (int y = ys; y < ye; y++)
-      for (int x = xs; x < xe; x++) vmax(m, ld(img + ((long long)y * g.W + x) * g.C));
+    // nine taps at a time (past the window: its last row or column once more)
+    for (int y = ys; y < ye; y += 3)
+      for (int x = xs; x < xe; x += 3) {
+        v4i v[9];
+#pragma unroll
+        for (int i = 0; i < 9; i++) v[i] = ld(img + ((long long)min(y + i / 3, ye - 1) * g.W + min(x + i % 3, xe - 1)) * g.C);
+#pragma unroll
+        for (int i = 0; i < 9; i++) vmax(m, v[i]);
+      }
   }
   store16<NT>(g.out + (((long long)b * g.Ho + oy) * g.Wo + ox) * g.C + cg * 16, m);
 }
@@ -117,40 +157,47 @@ __global__ __launch_bounds__(256) void maxpool16_kernel(PoolGeom g)
 struct AvgArgs {
   long long lambda, out_add;
   int shift, requant;
+  FastDiv d_ks;  // division by kx * ky
 };
 
 __global__ __launch_bounds__(256) void avgpool_kernel(PoolGeom g, AvgArgs a)
 {
-  long long t = (long long)blockIdx.x * 256 + threadIdx.x;
+  const long long t = (long long)blockIdx.x * 256 + threadIdx.x;
   if (t >= g.total) return;
-  const int cg = (int)(t % g.cgroups);
-  t /= g.cgroups;
-  const int ox = (int)(t % g.Wo);
-  t /= g.Wo;
-  const int oy = (int)(t % g.Ho);
-  const int b = (int)(t / g.Ho);
+  const PoolPlace at = pool_place(g, t);
+  const int cg = at.cg, ox = at.ox, oy = at.oy, b = at.b;
   const int c = cg * 4, n = min(4, g.C - c);
   const int ys = max(0, oy * g.sy - g.pb), ye = min(oy * g.sy - g.pt + g.ky, g.H);
   const int xs = max(0, ox * g.sx - g.pl), xe = min(ox * g.sx - g.pr + g.kx, g.W);
   const uint8_t *img = g.in + (long long)b * g.H * g.W * g.C + c;
   unsigned sum[4] = {0, 0, 0, 0};
-  // four taps at a time, their loads issued together (taps past the window re-read its last
-  // column and are not counted): one load per round trip would make the window size the
-  // kernel's latency
-  for (int y = ys; y < ye; y++)
-    for (int x = xs; x < xe; x += 4) {
-      unsigned v[4];
+  // Up to sixteen taps at a time, their loads issued together (taps past the window re-read its last row or column and are not counted): one
+  // load per round trip would make the window size the kernel's latency.  Even and odd bytes are summed in halves of a dword.
+  auto taps = [&](auto side) {
+    constexpr int S = decltype(side)::value;
+    for (int y = ys; y < ye; y += S)
+      for (int x = xs; x < xe; x += S) {
+        unsigned v[S * S], even = 0, odd = 0;
 #pragma unroll
-      for (int i = 0; i < 4; i++) v[i] = load4(img + ((long long)y * g.W + min(x + i, xe - 1)) * g.C, n, g.vec4);
+        for (int i = 0; i < S * S; i++)
+          v[i] = load4(img + ((long long)min(y + i / S, ye - 1) * g.W + min(x + i % S, xe - 1)) * g.C, n, g.vec4);
 #pragma unroll
-      for (int i = 0; i < 4; i++) {
-        if (x + i < xe) {
-#pragma unroll
-          for (int j = 0; j < 4; j++) sum[j] += (v[i] >> (8 * j)) & 0xFF;
+        for (int i = 0; i < S * S; i++) {
+          const unsigned u = y + i / S < ye && x + i % S < xe ? v[i] : 0u;
+          even += u & 0x00FF00FFu;
+          odd += (u >> 8) & 0x00FF00FFu;
         }
+        sum[0] += even & 0xFFFF;
+        sum[1] += odd & 0xFFFF;
+        sum[2] += even >> 16;
+        sum[3] += odd >> 16;
       }
-    }
-  const unsigned ksize = (unsigned)(g.kx * g.ky);
+  };
+  // (no more loads than the window has: 2x2 on 64 images of 32x32x256 12.0 us, 12.7 with sixteen)
+  const int side = max(g.kx, g.ky);
+  if (side <= 2) taps(std::integral_constant<int, 2>{});
+  else if (side == 3) taps(std::integral_constant<int, 3>{});
+  else taps(std::integral_constant<int, 4>{});
   unsigned packed = 0;
 #pragma unroll
   for (int j = 0; j < 4; j++) {
@@ -158,15 +205,16 @@ __global__ __launch_bounds__(256) void avgpool_kernel(PoolGeom g, AvgArgs a)
     if (a.requant) {
 #if PULPNN_BN_BITS == 64
       long long v = (long long)((unsigned long long)sum[j] * (unsigned long long)a.lambda);
-      v = v / (long long)ksize;
+      // (a division by multiplication where 32 bits hold the product)
+      v = (unsigned long long)v <= 0xffffffffull ? (long long)fastdiv((unsigned)v, a.d_ks) : v / (long long)(g.kx * g.ky);
       v = (long long)((unsigned long long)v + (unsigned long long)a.out_add);
       res = (int)(unsigned)(unsigned long long)(v >> a.shift);
 #else
-      unsigned v = sum[j] * (unsigned)(int)a.lambda / ksize + (unsigned)(int)a.out_add;
+      unsigned v = fastdiv(sum[j] * (unsigned)(int)a.lambda, a.d_ks) + (unsigned)(int)a.out_add;
       res = (int)(v >> a.shift);
 #endif
     } else {
-      res = (int)(sum[j] / ksize);
+      res = (int)fastdiv(sum[j], a.d_ks);
     }
     packed |= (unsigned)clipu8(res) << (8 * j);
   }

@@ -89,7 +89,7 @@ bool pool_geom(const char *fn, PoolGeom *g, uint8_t *in, uint8_t *out, uint16_t 
   g->pr = pr;
   g->cgroups = (C + 3) / 4;
   g->vec4 = (C % 4 == 0) && aligned(in, 4) && aligned(out, 4);
-  g->total = (long long)g->B * Ho * Wo * g->cgroups;
+  pool_threads(g);
   if ((g->total + 255) / 256 > 0x7fffffffLL) {
     set_error(PULP_NN_HIP_ERR_ARGUMENT, fn, "batch too large");
     return false;
@@ -388,7 +388,7 @@ void pulp_nn_maxpool(uint8_t *Im_in, uint8_t *Im_out, uint16_t dim_im_in_x, uint
           "left padding this large makes the reference's in-place x pass order dependent");
   if (ch_im_in % 16 == 0 && aligned(Im_in, 16) && aligned(Im_out, 16)) {
     g.cgroups = ch_im_in / 16;
-    g.total = (long long)g.B * g.Ho * g.Wo * g.cgroups;
+    pool_threads(&g);
     const dim3 grid((unsigned)((g.total + 255) / 256));
     // non-temporal loads: windows that do not overlap, on an input too large to find again in a cache
     const bool lnt = stride_x >= dim_kernel_x && stride_y >= dim_kernel_y &&
@@ -416,7 +416,7 @@ void pulp_nn_avgpool(uint8_t *Im_in, uint8_t *Im_out, bn_t lambda, uint16_t out_
     return;
   REQUIRE(!flag_requant || out_shift < PULPNN_BN_BITS, PULP_NN_HIP_ERR_ARGUMENT, "out_shift out of range");
   REQUIRE((long long)dim_kernel_x * dim_kernel_y * 255 < 0xffffffffLL, PULP_NN_HIP_ERR_UNSUPPORTED, "window too large");
-  AvgArgs a = {(long long)lambda, (long long)out_add, (int)out_shift, flag_requant};
+  AvgArgs a = {(long long)lambda, (long long)out_add, (int)out_shift, flag_requant, fastdiv_make((unsigned)dim_kernel_x * dim_kernel_y)};
   hipLaunchKernelGGL(avgpool_kernel, dim3((unsigned)((g.total + 255) / 256)), dim3(256), 0, g_stream, g, a);
   check_launch(__func__);
 }
