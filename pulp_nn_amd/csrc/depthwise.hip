@@ -94,6 +94,14 @@ void depthwise_common(const char *fn, const uint8_t *in, const int8_t *bias, uin
     const DwLayer L = {in, wt, bias, out, (int)g_batch, CH, H, W, Ho, Wo, kx, ky, pt, pl, sx, sy};
     if (launch_dw_hwc(mode, L, e, num_cus(), g_stream)) return check_launch(fn);
   }
+  // Small layers on the matrix cores: up to 2 MB of input and 64 units of an image's 64 channels, where dw3x3_lin_kernel has a long chain of
+  // rows on few workgroups and dw_mfma_kernel splits them (bands / matrix cores: 63x8x64 batch 2 15.1 / 4.5 us, 11x40x64 batch 2 6.7 / 4.3, 51x12x512
+  // batch 5 10.8 / 5.5, 18x28x64 batch 56 6.5 / 4.9; past the line 9x8x64 stride 2 batch 248 5.0 / 8.0, 9x36x64 batch 195 6.3 / 7.5, 23x8x384 batch 73
+  // 8.8 / 11.4; stride 2 on rows of 40 pixels and more 12x40x64 batch 4 4.8 / 5.3, 61x40x64 batch 14 5.4 / 5.9).
+  if (lin && !stream && (long long)g_batch * CH * H * W <= 2 << 20 && (long long)g_batch * (CH / DW_CG) <= 64 && !(sx == 2 && W >= 40)) {
+    const DwLayer L = {in, wt, bias, out, (int)g_batch, CH, H, W, Ho, Wo, kx, ky, pt, pl, sx, sy};
+    if (launch_dw_mfma(mode, L, e, num_cus(), g_stream)) return check_launch(fn);
+  }
   if (plane) {
     const dim3 pgrid((unsigned)(((long long)g.B * g.cgroups + DW_REG_WAVES - 1) / DW_REG_WAVES)), pblock(64 * DW_REG_WAVES);
 #define DWP_LAYOUT(HW, S, HWC)                                                                                            \

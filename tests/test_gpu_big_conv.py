@@ -122,10 +122,14 @@ DW1_GEOMS = [
     (514, 64, 31, 40, (1, 0, 1, 1)),     # no bottom padding: 30 output rows
 ]
 
+# the small ones of these again with more than 64 images, which stay in bands (fewer go to the matrix cores)
+DW1_BANDS = [(70, 64, 20, 20, (1, 1, 1, 1)), (66, 64, 45, 24, (0, 1, 0, 2)), (66, 64, 9, 112, (1, 1, 1, 1)), (90, 64, 6, 8, (1, 1, 1, 1)),
+             (64, 64, 20, 20, (1, 1, 1, 1)), (65, 64, 20, 20, (1, 1, 1, 1))]
+
 
 @pytest.mark.parametrize("bn_bits", [32, 64])
 @pytest.mark.parametrize("flags", [(1, 1), (1, 0), (0, 0)])
-@pytest.mark.parametrize("geom", DW1_GEOMS, ids=lambda g: "x".join(map(str, g[:4])))
+@pytest.mark.parametrize("geom", DW1_GEOMS + DW1_BANDS, ids=lambda g: "x".join(map(str, g[:4])))
 def test_depthwise_stride1_whole_groups(geom, flags, bn_bits):
     from gpu_helpers import depthwise_generic
     B, CH, H, W, pads = geom
