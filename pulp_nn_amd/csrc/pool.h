@@ -1,12 +1,13 @@
 // Max / average pooling and element-wise add on HWC uint8 maps: bandwidth-bound
 // VALU kernels, one thread per output pixel and group of 4 channels (16 for
 // add), so that neighbouring lanes read and write neighbouring bytes.
-#pragma once
 //
 // Bound: small maps by launch and one trip to memory (all taps of a window of up to 4 x 4, or 3 x 3 for the maximum, are asked for
 // together); large ones by HBM.  The place of a thread takes 32-bit divisions by multiplication: written in 64 bits it was some 600
 // instructions.  Whole calls, that and a row of taps per trip / now: average 4x4 on 64 images of 16x16x64 4.2 / 3.2 us, 2x2 on 64 of 32x32x256
-// 11.4 / 8.1 (21 MB), 7x7 on 32 of 7x7x1000 7.6 / 5.6; maximum 3x3 on 112x112x64 3.8 / 3.05, on 64 of 56x56x64 6.0 / 5.9.
+// 11.4 / 8.1 (21 MB), 7x7 on 32 of 7x7x1000 7.6 / 5.6; maximum 3x3 on 112x112x64 3.8 / 3.05, on
+// 64 of 56x56x64 5.35 / 4.4, 2x2 on 64 of 63x63x256 14.7 / 12.9, 7x7 stride 7 29.7 / 16.8 (64 MB).
+#pragma once
 #include <type_traits>
 
 #include "fastdiv.h"
@@ -108,8 +109,8 @@ __global__ __launch_bounds__(256) void maxpool_kernel(PoolGeom g)
 
 // Same, 16 channels per thread with 16-byte accesses (C % 16 == 0, 16-byte aligned maps).
 // g.cgroups counts groups of 16 here.  NT: non-temporal store; LNT: non-temporal loads (windows that do not
-// overlap on an input too large for the caches: every byte is read once).  A whole 2 x 2 window is four loads
-// issued together; other windows go tap by tap.
+// overlap on an input too large for the caches: every byte is read once).  The taps of a window of up to 3 x 3 are
+// asked for together, those of larger ones four of a row at a time.
 template <bool NT, bool LNT>
 __global__ __launch_bounds__(256) void maxpool16_kernel(PoolGeom g)
 {
@@ -128,24 +129,47 @@ __global__ __launch_bounds__(256) void maxpool16_kernel(PoolGeom g)
     m.w = (int)max_u8x4((unsigned)m.w, (unsigned)v.w);
   };
   v4i m = {0, 0, 0, 0};
-  if (ye - ys == 2 && xe - xs == 2) {
+  if (g.kx <= 2 && g.ky <= 2 && ys < ye && xs < xe) {
+    // (where the image ends in the window: its last row or column once more, not a path of its own for the few lanes that are there.  63x63x256
+    // batch 64 18.5 us with one, 14.7 tap by tap at the edges, 12.9 so)
     const uint8_t *p = img + ((long long)ys * g.W + xs) * g.C;
-    const long long row = (long long)g.W * g.C;
-    const v4i v0 = ld(p), v1 = ld(p + g.C), v2 = ld(p + row), v3 = ld(p + row + g.C);
-    m = v0;
-    vmax(m, v1);
-    vmax(m, v2);
-    vmax(m, v3);
+    const long long row = ye - ys > 1 ? (long long)g.W * g.C : 0;
+    const int col = xe - xs > 1 ? g.C : 0;
+    if (g.kx == 2 && g.ky == 2) {
+      const v4i v0 = ld(p), v1 = ld(p + col), v2 = ld(p + row), v3 = ld(p + row + col);
+      m = v0;
+      vmax(m, v1);
+      vmax(m, v2);
+      vmax(m, v3);
+    } else {
+      const v4i v0 = ld(p);
+      m = v0;
+      if (g.kx * g.ky == 2) vmax(m, ld(p + (g.kx == 2 ? col : row)));
+    }
+  } else if (g.kx <= 3 && g.ky <= 3) {
+    // the whole window (past its end: its last row or column once more)
+    if (ys < ye && xs < xe) {
+      v4i v[9];
+#pragma unroll
+      for (int i = 0; i < 9; i++) v[i] = ld(img + ((long long)min(ys + i / 3, ye - 1) * g.W + min(xs + i % 3, xe - 1)) * g.C);
+#pragma unroll
+      for (int i = 0; i < 9; i++) vmax(m, v[i]);
+    }
   } else {
-    // nine taps at a time (past the window: its last row or column once more)
-    for (int y = ys; y < ye; y += 3)
-      for (int x = xs; x < xe; x += 3) {
-        v4i v[9];
+    // four or five taps of a row at a time (nine of three rows re-read too many: 4x4 stride 4 on 64 of 63x63x256 16.4 us, 10.7 so)
+    auto rows = [&](auto side) {
+      constexpr int S = decltype(side)::value;
+      for (int y = ys; y < ye; y++)
+        for (int x = xs; x < xe; x += S) {
+          v4i v[S];
 #pragma unroll
-        for (int i = 0; i < 9; i++) v[i] = ld(img + ((long long)min(y + i / 3, ye - 1) * g.W + min(x + i % 3, xe - 1)) * g.C);
+          for (int i = 0; i < S; i++) v[i] = ld(img + ((long long)y * g.W + min(x + i, xe - 1)) * g.C);
 #pragma unroll
-        for (int i = 0; i < 9; i++) vmax(m, v[i]);
-      }
+          for (int i = 0; i < S; i++) vmax(m, v[i]);
+        }
+    };
+    if (g.kx == 5) rows(std::integral_constant<int, 5>{});
+    else rows(std::integral_constant<int, 4>{});
   }
   store16<NT>(g.out + (((long long)b * g.Ho + oy) * g.Wo + ox) * g.C + cg * 16, m);
 }
