@@ -8,6 +8,7 @@
 #include "igemm_ring.h"
 #include "linear_skinny.h"
 #include "pw_any_geom.h"
+#include "pw_packed.h"
 #include "pw_stream.h"
 #include "smallk.h"
 
@@ -270,6 +271,16 @@ bool launch_pw_stream_ks(int mode, int ks, bool wide, const PwGeom &g, const Epi
   }
 }
 
+template <int K16, int Q>
+void launch_pw_packed(int mode, PwGeom &g, const EpiArgs &e, hipStream_t s)
+{
+  constexpr int PX = 64 / K16;
+  g.units = (g.M + PX - 1) / PX;
+  const dim3 grid(std::min((g.units + 3) / 4, 4 * num_cus())), block(256);
+  if (g.nt) hipLaunchKernelGGL((pw_packed_kernel<K16, Q, true>), grid, block, 0, s, g, e, mode);
+  else hipLaunchKernelGGL((pw_packed_kernel<K16, Q, false>), grid, block, 0, s, g, e, mode);
+}
+
 // Weights-stationary streaming path: a GEMM whose rows are contiguous K-byte pixels,
 // whose weight matrix (at most 256 x 256) fits in LDS and whose channel count is one
 // of 16, 32, 64, 128, 192, 256 (every lane then owns real channels and stores whole
@@ -306,6 +317,17 @@ bool try_pw_stream(int mode, const uint8_t *in, const int8_t *w, const int8_t *b
   // a launch that would leave more than half of the CUs without a workgroup is better off tiled:
   // every CU takes part there, and staging the weights per workgroup no longer pays
   if (2 * need < num_cus()) return false;
+  // Several pixels of 16 or 32 channels in a column of the matrix cores, from a load for every wave on (one pixel a column / so, whole calls,
+  // batches of 64x64: 16 -> 16 batch 64 5.0 / 4.0 us, 200 8.6 / 6.7; 16 -> 32 5.7 / 5.3, 9.65 / 8.5; 32 -> 64 7.8 / 7.1, batch 100 9.2 / 8.6; below the
+  // line alike, but 32 -> 64 batch 32 5.1 / 5.3).  Not where its registers leave too few waves: 16 -> 64 7.6 / 8.0, 32 -> 32 3.9 / 4.5 and 6.8 / 6.9; with
+  // constants of 64 bits 16 -> 32 6.0 / 7.8, 32 -> 64 8.2 / 10.3, but 16 -> 16 batch 200 8.7 / 7.8.
+  if (M >= 64ll * 16 * num_cus()) {
+    if (K == 16 && N == 16) return launch_pw_packed<1, 1>(mode, g, e, s), true;
+    if constexpr (sizeof(bn_t) == 4) {
+      if (K == 16 && N == 32) return launch_pw_packed<1, 2>(mode, g, e, s), true;
+      if (K == 32 && N == 64) return launch_pw_packed<2, 4>(mode, g, e, s), true;
+    }
+  }
   dim3 grid(blocks);
   // (false also if the kernel's LDS limit cannot be raised: the caller then uses the tiled kernel)
   if (tn == 1) return launch_pw_stream_ks<1, 1>(mode, ks, wide, g, e, grid, lds, s);

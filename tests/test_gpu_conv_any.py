@@ -49,6 +49,9 @@ POINTWISE = [
     (30, 32, 33, 130, 255), (24, 33, 33, 257, 64), (24, 33, 33, 500, 100), (24, 33, 33, 512, 260), (40, 32, 32, 48, 424),
     (9, 29, 31, 72, 20), (3, 9, 7, 9, 5), (1, 1, 1, 20, 24), (2, 5, 5, 600, 30),
     (75, 30, 31, 320, 8),  # (band kernel: weights a step at a time)
+    # several pixels of 16 or 32 channels in a column of the matrix cores: whole loads of 64 or 32 pixels, a partial last one, and below the line
+    (64, 64, 64, 16, 16), (70, 61, 63, 16, 16), (65, 64, 64, 16, 32), (67, 63, 63, 16, 32), (130, 32, 64, 32, 64), (131, 31, 67, 32, 64),
+    (63, 64, 65, 16, 32), (41, 29, 31, 32, 64),
 ]
 
 
