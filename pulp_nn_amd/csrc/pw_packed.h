@@ -7,7 +7,7 @@
 // one 16-byte store a lane, 1 KB in memory order, and no exchange between lanes.  Weights and constants live in registers, a wave
 // streams a contiguous run of pixels two loads ahead; no LDS, no barrier.
 //
-// Bound: HBM and the vector ALU, which has half of the instructions of pw_stream_kernel (one pixel a column, three of four lanes of a load
+// Bound: HBM and the vector ALU, which has 125 instructions per 64 pixels of 16 -> 32 where pw_stream_kernel has 213 (one pixel a column, three of four lanes of a load
 // without a part, 8-byte stores).  Whole calls, that / this: 64x64 16 -> 32 batch 256 12.0 / 10.0 us (50 MB; scalar multiplier 11.7 / 9.2), 16 -> 16
 // 10.8 / 7.3 (34 MB, 4.6 TB/s), 32x32 32 -> 64 batch 256 7.8 / 7.1; MobileNet chain at batch 256 166.1 / 163.5.
 #pragma once
