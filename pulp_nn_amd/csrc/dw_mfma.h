@@ -23,7 +23,7 @@
 // Bound: small layers by the instructions of one wave, one after the other: a dependent one takes 8 clocks whichever unit executes it,
 // and nothing covers that with one wave per SIMD (10x8x48: some 9000 clocks from the first instruction to the last).  So: the launch's
 // numbers are read at once; a wave fetches the filters and constants of its own channels and builds the matrix rows while its part of
-// the input is on the way; the input travels by buffer loads whose channel distance is a scalar, and parts of a pass that no channel
+// the input is on the way; the input travels by buffer loads, whose addresses take two instructions, and parts of a pass that no channel
 // needs are left out.  (The same set-up with every array going through LDS behind one barrier and each number read where it is used:
 // 10x8x48 batch 5 5.3 us, now 4.2; 28x7x8 batch 35 5.18, 3.84; 35x29x72 batch 32 8.7, 7.6.)
 // Larger layers by the vector ALU (13x39x408 batch 208 43.6 us, now 38.3, 85 MB).  Measured, whole calls, against the kernels
@@ -101,7 +101,7 @@ __global__ __launch_bounds__(256, CB == 16 ? (NM == 1 ? 5 : NM <= 3 ? 4 : 1) : N
   // exist read as the last one and are not written.)
   const int nq = CB == 16 ? 1 : (ncb + 15) / 16, cw = 4 * nq * wave;
   const int nrow = 4 * nq * g.ky;  // filter rows, those of all channels back to back
-  auto filter_at = [&](int t) { return min((c0 + cw) * g.ky + t, (c0 + ncb) * g.ky - 1) * g.kx; };
+  auto filter_at = [&](int t) { return dwm_filter_at(g, tile, cw, t); };
   const int wlast = g.wt_bytes - 8;
   v2i w_raw = {0, 0};
   if (wlast >= 0) w_raw = *(const v2i_u *)(g.wt + min(filter_at(lane), wlast));
@@ -119,10 +119,9 @@ __global__ __launch_bounds__(256, CB == 16 ? (NM == 1 ? 5 : NM <= 3 ? 4 : 1) : N
   const int slots = g.NR * g.Q;
   const int iy0 = oy0 * g.sy - g.pt, x0 = 16 * xg0 * g.sx - g.pl;
   const int cpi = (int)fastdiv((unsigned)tid, g.d_nper);
-  constexpr int UN = CB == 16 ? 4 : 8;  // loads in flight per thread
+  constexpr int UN = dwm_loads(CB);
   const bool edge = dwm_edge(g, tile, before);  // a load of this tile may leave the tensor
-  // Inside: buffer loads (the channel's distance is a scalar; channels that do not exist are out of range or not used) from 64 bytes
-  // before the tile's first plane, where a row's left padding may begin
+  // Inside: buffer loads (dwm_buffer_off)
   const __amdgpu_buffer_rsrc_t rsrc =
       __builtin_amdgcn_make_buffer_rsrc((void *)(img - 64), 0, (int)min(g.in_bytes - before + 64, 0x7fffffffll), 0x00020000);
   const long long behind = g.in_bytes - before - 16;
@@ -136,7 +135,7 @@ __global__ __launch_bounds__(256, CB == 16 ? (NM == 1 ? 5 : NM <= 3 ? 4 : 1) : N
     const int x = x0 + 16 * q, iy = iy0 + row;
     base = dwm_load_base(g, iy, x);
     lds_at = row * g.pitch + 16 * q + cpi * g.CS;
-    ch = slot < slots ? cpi : CB + 64;
+    ch = dwm_thread_channel(CB, cpi, slot < slots);
     const int n = (unsigned)iy < (unsigned)g.H ? 8 * (g.W - x) : 0;
 #pragma unroll
     for (int d = 0; d < 4; d++) mask[d] = low_bits(n - 32 * d) & high_bits(-8 * x - 32 * d);
@@ -152,10 +151,10 @@ __global__ __launch_bounds__(256, CB == 16 ? (NM == 1 ? 5 : NM <= 3 ? 4 : 1) : N
         v[u] = (v4u){(unsigned)t.x, (unsigned)t.y, (unsigned)t.z, (unsigned)t.w};
       }
     } else {
-      const unsigned at = ch == cpi ? (unsigned)(64 + cpi * plane + base) : 0xffffffffu;
+      const unsigned at = dwm_buffer_first(plane, ch, cpi, base), at_last = dwm_buffer_last(plane, ncb, ch, cpi, base);
 #pragma unroll
       for (int u = 0; u < UN; u++)
-        if (u == 0 || cj + u * g.cpar < ncb) v[u] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, at, (cj + u * g.cpar) * plane, 0);
+        if (u == 0 || cj + u * g.cpar < ncb) v[u] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, dwm_buffer_off(at, at_last, plane, cj + u * g.cpar), 0, 0);
     }
   };
   auto stage = [&](int cj) {

@@ -76,6 +76,32 @@ PULPNN_HD bool dwm_edge(const DwmGeom &g, const DwmTile &t, long long before)
 // start of the plane, masked off).
 PULPNN_HD int dwm_load_base(const DwmGeom &g, int iy, int x) { return (unsigned)iy < (unsigned)g.H ? iy * g.W + x : 0; }
 
+// 16-byte loads that a thread has in flight.
+PULPNN_HD constexpr int dwm_loads(int cb) { return cb == 16 ? 4 : 8; }
+
+// First channel of the thread whose first one is cpi: out of reach of every channel where its pass has no slot for it.
+PULPNN_HD int dwm_thread_channel(int cb, int cpi, bool slot) { return slot ? cpi : cb + 64; }
+
+// Lane's offset of a buffer load of a tile that is no edge, from 64 bytes in front of the tile's first plane, where a row's left padding may
+// begin: chunk `at` of the c-th channel behind the thread's first one, or of the last channel that exists.  The lane's offset says it
+// all and none of it is left to the scalar one, which is not documented to take part in the range check: asked for with the scalar one, the
+// channels past a short last block lay up to 80 KB behind the tensor.  A thread without a slot is out of range.
+// (One addition and one minimum a load.  Out of range by a comparison with the channel, 2 % slower over 114 layers.)
+PULPNN_HD unsigned dwm_buffer_first(int plane, int ch, int cpi, int at) { return ch == cpi ? (unsigned)(64 + cpi * plane + at) : 0xf0000000u; }
+PULPNN_HD unsigned dwm_buffer_last(int plane, int ncb, int ch, int cpi, int at) { return ch == cpi ? (unsigned)(64 + (ncb - 1) * plane + at) : 0xf0000000u; }
+PULPNN_HD unsigned dwm_buffer_off(unsigned first, unsigned last, int plane, int c)
+{
+  const unsigned at = first + (unsigned)(c * plane);
+  return at < last ? at : last;
+}
+
+// First byte of row t of the filters of channel c0 + cw and those behind it; rows of channels that do not exist: the last one.
+PULPNN_HD int dwm_filter_at(const DwmGeom &g, const DwmTile &t, int cw, int row)
+{
+  const int at = (t.c0 + cw) * g.ky + row, last = (t.c0 + t.ncb) * g.ky - 1;
+  return (at < last ? at : last) * g.kx;
+}
+
 // Row of the tile's pixel p, counted row by row.
 PULPNN_HD int dwm_out_row(const DwmGeom &g, const DwmTile &t, int p)
 {

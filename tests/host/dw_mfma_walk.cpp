@@ -1,6 +1,6 @@
 // Walks the tiles of dw_mfma_kernel on the host, with the kernel's own tile arithmetic (csrc/dw_mfma_geom.h), and reports
 // loads that leave the input, LDS ranges that overlap, and output pixels that are written to a wrong place or not at all.
-// Layers on stdin, one a line: B CH H W Ho Wo kx ky pt pl sx sy (bytes of a batch-norm parameter) cus.  One line out per layer: "ok TILES", "no" (not
+// Layers on stdin, one a line: B CH H W Ho Wo kx ky pt pl sx sy cus.  One line out per layer: "ok TILES", "no" (not
 // taken by the kernel) or what is wrong.
 #include <stdio.h>
 #include <stdlib.h>
@@ -40,16 +40,52 @@ static std::string check(const DwLayer &L, int cus)
     const bool edge = dwm_edge(g, t, before);
     const long long behind = g.in_bytes - before - 16;
     const int lo = (int)std::max(-before, -(1ll << 30)), hi = (int)std::min(behind, 0x7fffffffll);
-    for (int row = 0; row < g.NR; row++)
-      for (int q = 0; q < g.Q; q++)
-        for (const int c : {0, t.ncb - 1}) {
-          const int iy = iy0 + row, x = x0 + 16 * q, off = c * (int)plane + dwm_load_base(g, iy, x);
-          const int at = edge ? std::min(std::max(off, lo), hi) : off;
-          if (before + at < 0 || before + at + 16 > bytes) return wrong("load outside the input", t, before + at, bytes);
-          for (int j = 0; j < 16; j++)
-            if (iy >= 0 && iy < L.H && x + j >= 0 && x + j < L.W && (j + off - at < 0 || j + off - at > 15))
-              return wrong("byte of the image not loaded", t, iy, x + j);
-        }
+    // Every load the staging makes: the passes over slots, the threads of a pass, the channels of a thread.  `seen`: slots and channels staged.
+    // (Of the first and the last 48 tiles.)
+    const int slots = id < 48u || id + 48u >= (unsigned)g.total ? g.NR * g.Q : 0, UN = dwm_loads(CB);
+    std::vector<unsigned char> seen(slots * t.ncb);
+    if (g.nper > 256 || g.nper * g.cpar > 256 || g.cpar < 1) return wrong("threads of a pass", t, g.nper, g.cpar);
+    for (int s0 = 0; s0 < slots; s0 += g.nper)
+      for (int tid = 0; tid < 256; tid++) {
+        const int cpi = (int)fastdiv((unsigned)tid, g.d_nper), slot = s0 + tid - cpi * g.nper, row = (int)fastdiv((unsigned)slot, g.d_q), q = slot - row * g.Q;
+        const int iy = iy0 + row, x = x0 + 16 * q, base = dwm_load_base(g, iy, x), ch = dwm_thread_channel(CB, cpi, slot < slots);
+        for (int cj = 0; cj < t.ncb; cj += UN * g.cpar)
+          for (int u = 0; u < UN; u++) {
+            const int c = cj + u * g.cpar;
+            if (u != 0 && c >= t.ncb) break;
+            const bool staged = ch < t.ncb - c;
+            long long at;  // bytes from the tile's first plane
+            if (edge) {
+              at = std::min(std::max(std::min(cpi + c, t.ncb - 1) * (int)plane + base, lo), hi);
+            } else {
+              const unsigned off = dwm_buffer_off(dwm_buffer_first((int)plane, ch, cpi, base), dwm_buffer_last((int)plane, t.ncb, ch, cpi, base), (int)plane, c);
+              if (off >= (unsigned long long)std::min(g.in_bytes - before + 64, 0x7fffffffll)) {  // out of range: zeros
+                if (staged) return wrong("load of a channel out of range", t, cpi + c, off);
+                continue;
+              }
+              at = (long long)off - 64;
+            }
+            if (before + at < 0 || before + at + 16 > bytes) return wrong("load outside the input", t, before + at, bytes);
+            if (!staged) continue;
+            const long long want = (long long)(cpi + c) * plane + base;  // the chunk that the slot is for
+            for (int j = 0; j < 16; j++)
+              if (iy >= 0 && iy < L.H && x + j >= 0 && x + j < L.W && (j + want - at < 0 || j + want - at > 15))
+                return wrong("byte of the image not loaded", t, iy, x + j);
+            seen[slot * t.ncb + cpi + c] = 1;  // (threads past the channels side by side stage some of them once more, alike)
+          }
+      }
+    for (const unsigned char n : seen)
+      if (!n) return wrong("not staged", t, slots, t.ncb);
+    // 8 bytes of filter a lane, from the tensor's last 8 at the most (layers of fewer are read byte by byte)
+    for (int wave = 0; wave < 4; wave++) {
+      const int nq = CB == 16 ? 1 : (t.ncb + 15) / 16, cw = 4 * nq * wave, nrow = 4 * nq * g.ky;
+      if (nrow * DWM_WROW + 8 > dwm_wpart(CB, g.ky)) return wrong("filter rows of a wave", t, nrow, g.ky);
+      for (int r = 0; r < std::max(nrow, 64) && g.wt_bytes >= 8; r++) {
+        const int want = dwm_filter_at(g, t, cw, r), at = std::min(want, g.wt_bytes - 8);
+        if (at < 0) return wrong("load outside the filters", t, cw, r);
+        if (cw + r / g.ky < t.ncb && r < nrow && (want != ((t.c0 + cw) * g.ky + r) * g.kx || want + g.kx > at + 8)) return wrong("filter row not loaded", t, cw, r);
+      }
+    }
     if (g.NR * g.pitch > g.CS || 16 * g.Q > g.pitch || CB * g.CS > g.w_off || g.w_off + 4 * dwm_wpart(CB, L.ky) > g.o_off ||
         g.o_off + (size_t)t.rows * t.wt * (CB + 4) > lds)
       return wrong("LDS ranges", t, g.o_off, (long long)lds);
@@ -64,9 +100,8 @@ static std::string check(const DwLayer &L, int cus)
 int main()
 {
   DwLayer L = {};
-  int bn_bytes, cus;
-  while (scanf("%d %d %d %d %d %d %d %d %d %d %d %d %d %d", &L.B, &L.CH, &L.H, &L.W, &L.Ho, &L.Wo, &L.kx, &L.ky, &L.pt, &L.pl, &L.sx, &L.sy,
-               &bn_bytes, &cus) == 14) {
+  int cus;
+  while (scanf("%d %d %d %d %d %d %d %d %d %d %d %d %d", &L.B, &L.CH, &L.H, &L.W, &L.Ho, &L.Wo, &L.kx, &L.ky, &L.pt, &L.pl, &L.sx, &L.sy, &cus) == 13) {
     std::string s = check<16>(L, cus);
     if (s.compare(0, 2, "ok") == 0 || s == "no") {
       const std::string s64 = (long long)L.Ho * L.Wo <= 64 ? check<64>(L, cus) : "no";

@@ -23,12 +23,12 @@ def walk(tmp_path_factory):
     return run
 
 
-def layer(B, CH, H, W, kx, ky, pads, strides, out_hw=None, bn_bytes=4, cus=256):
+def layer(B, CH, H, W, kx, ky, pads, strides, out_hw=None, cus=256):
     """pads: (top, bottom, left, right)."""
     pt, pb, pl, pr = pads
     sx, sy = strides
     ho, wo = out_hw or ((H + pt + pb - ky) // sy + 1, (W + pl + pr - kx) // sx + 1)
-    return B, CH, H, W, ho, wo, kx, ky, pt, pl, sx, sy, bn_bytes, cus
+    return B, CH, H, W, ho, wo, kx, ky, pt, pl, sx, sy, cus
 
 
 def check(walk, layers, taken=True):
@@ -42,15 +42,20 @@ def test_usual_layers(walk):
     for _ in range(1500):
         k = r.choice([3, 3, 5, 7])
         s = r.choice([1, 1, 2])
-        layers.append(layer(r.choice([1, 2, 33, 256]), r.randint(1, 200), r.randint(k, 70), r.randint(16, 70), k, k, (k // 2,) * 4, (s, s),
-                            bn_bytes=r.choice([4, 8])))
+        layers.append(layer(r.choice([1, 2, 33, 256]), r.randint(1, 200), r.randint(k, 70), r.randint(16, 70), k, k, (k // 2,) * 4, (s, s)))
     check(walk, layers)
+
+
+def test_channels_that_do_not_exist(walk):
+    """The last block of channels is short: what a pass asks for beyond them is out of range by the lane's own offset."""
+    check(walk, [layer(2, 17, 20, 20, 3, 3, (1, 1, 1, 1), (1, 1)), layer(5, 18, 60, 61, 5, 5, (2, 2, 2, 2), (1, 1)),
+                 layer(2, 17, 200, 200, 3, 3, (1, 1, 1, 1), (1, 1)), layer(1100, 65, 7, 7, 3, 3, (1, 1, 1, 1), (1, 1))])
 
 
 def test_narrow_last_column_tile(walk):
     """Several column tiles and several rows per tile: the last tile's rows are shorter, in LDS too."""
     check(walk, [layer(600, 16, 6, 340, 3, 3, (1, 1, 1, 111), (1, 1)), layer(64, 16, 40, 320, 3, 3, (1, 1, 1, 131), (1, 1)),
-                 layer(600, 24, 8, 336, 3, 3, (1, 1, 0, 100), (1, 1), bn_bytes=8)])
+                 layer(600, 24, 8, 336, 3, 3, (1, 1, 0, 100), (1, 1))])
     assert walk([layer(600, 16, 6, 340, 3, 3, (1, 1, 1, 111), (1, 1))]) == ["ok 3600"]  # two column tiles, two rows each
 
 
