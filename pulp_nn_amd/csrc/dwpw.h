@@ -157,6 +157,11 @@ __global__ __launch_bounds__(1024) void dwpw_kernel(DwPwGeom g)
   const int KT = (T.C + 63) / 64;
   unsigned char *xin = dwpw_lds + T.x_off, *par = dwpw_lds + T.par_off;
   const int nblocks = CHAIN ? g.nblocks : 1;
+  // The input's first part (10 registers) and the pointwise constants (9, of 64 bits 17) are asked for ahead of the depthwise stage, unless they do not
+  // fit beside it: in chains with constants of 64 bits that spilled 14 to 22 registers a lane.  There they are asked for where they are used.  Spilled
+  // / so: 8x8x320 two blocks batch 64 21.0 / 18.1 us, four batch 128 36.0 / 31.8; 8x8x64 four batch 256 17.1 / 14.6; 16x16x64 three batch 256
+  // 21.2 / 19.4.  (With 32 bits 8x8x64 two blocks batch 64 7.5 ahead, 7.95 not; 8x8x320 16.1, 16.7.)
+  constexpr bool AHEAD = !CHAIN || sizeof(bn_t) == 4;
 
   // the pointwise stage's blocks of 64 pixels x 16 channels, dealt to the waves
   const int cf_lo = part * T.cf_per, nblk = max(min(T.cf_per, T.Co / 16 - cf_lo), 0) << T.lpxb;
@@ -196,7 +201,7 @@ __global__ __launch_bounds__(1024) void dwpw_kernel(DwPwGeom g)
         v[u] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, c.off >= 0 ? (unsigned)c.off : 0x80000000u, 0, 0);
       }
     };
-    if (first) load_x(0, 64 * wave);
+    if (AHEAD && first) load_x(0, 64 * wave);
     // (many slices of weights behind the input: in front of it they would hold it up)
     if (KP == 1 && wave < nblk) load_w(P, w_cf = cf_first, 0);
     if ((((unsigned)(unsigned long long)P->dw_wt | (unsigned)(unsigned long long)P->dw_bias) & 3) == 0) {
@@ -224,7 +229,8 @@ __global__ __launch_bounds__(1024) void dwpw_kernel(DwPwGeom g)
         l = *(const bn4 *)(P->e_pw.lambda + n);
       }
     };
-    if (wave < nblk) load_pw(cf_first);
+    if constexpr (AHEAD)
+      if (wave < nblk) load_pw(cf_first);
 #pragma unroll 1
     for (int slab = 0; slab < (CHAIN ? 1 : T.slabs); slab++) {
       // ---- input -> LDS ------------------------------------------------------------------------------------------------
@@ -232,7 +238,7 @@ __global__ __launch_bounds__(1024) void dwpw_kernel(DwPwGeom g)
         if (slab) dwpw_barrier();  // everybody is done with the slab before
 #pragma unroll 1
         for (int t0 = 64 * wave; t0 < chunks; t0 += NTH * UN) {
-          if (slab || t0 != 64 * wave) load_x(slab, t0);
+          if (!AHEAD || slab || t0 != 64 * wave) load_x(slab, t0);
 #pragma unroll
           for (int u = 0; u < UN; u++) {
             if (t0 + NTH * u >= chunks) break;
@@ -293,7 +299,13 @@ __global__ __launch_bounds__(1024) void dwpw_kernel(DwPwGeom g)
 #pragma unroll 1
     for (int blk = wave; blk < nblk; blk += NWV) {
       const int cf = cf_lo + (blk >> T.lpxb), px0 = 64 * (blk & ((1 << T.lpxb) - 1));
-      if (blk != wave) load_pw(cf);
+      if constexpr (!AHEAD) {
+        bias = 0;
+        k = l = (bn4){0, 0, 0, 0};
+        load_pw(cf);
+      } else if (blk != wave) {
+        load_pw(cf);
+      }
       const v4i ones = {0x01010101, 0x01010101, 0x01010101, 0x01010101};
       v4i acc[4], wacc = {0, 0, 0, 0};
 #pragma unroll

@@ -32,7 +32,9 @@ bool launch(const DwPwGeom &g)
     // channels or fewer have fewer waves)
     if (g.t.waves == 16 && g.t.kp == DWPW_CHAIN_KP && g.t.C / 16 * g.t.nst <= 16 && g.t.C / 16 << g.t.lpxb <= 16 && launch_chain<W>(g)) return true;
   }
-  return g.t.kp == 1 ? launch_kp<W, S, 1, CHAIN>(g) : g.t.kp == 4 ? launch_kp<W, S, 4, CHAIN>(g) : launch_kp<W, S, 8, CHAIN>(g);
+  if constexpr (!CHAIN)  // (a chain has no eight slices: dwpw_tile)
+    if (g.t.kp == 8) return launch_kp<W, S, 8, CHAIN>(g);
+  return g.t.kp == 1 ? launch_kp<W, S, 1, CHAIN>(g) : launch_kp<W, S, 4, CHAIN>(g);
 }
 template <bool CHAIN>
 bool launch_s1(int W, const DwPwGeom &g)

@@ -245,7 +245,8 @@ inline int dwpw_tile(DwPwTile &g, int W, int S, bool chain, int cus, int bn_byte
   const int want = C > 64 && (chain || (g.whole && W == 16 && S == 2)) ? 16 : dwpw_waves(C, g.TR * WO), par = dwpw_par(C, bn_bytes, true).bytes;
   // LDS: activation operand, input, depthwise parameters, weights.  A slab of the input costs a round trip to memory and two barriers, so
   // there are as few as fit (16x16x256 stride 2, batch 16, two slabs / one: 9.5 / 8.3 us; 8x8x512 10.9 / 9.5).  The weights of a wave are all of
-  // K at once for up to eight slices, if that fits, else four.  More than five slabs of 64 channels only if half as many waves, with room for
+  // K at once for up to eight slices, if that fits, else four (in a chain, where sixteen waves leave no room for eight, always).  More than five
+  // slabs of 64 channels only if half as many waves, with room for
   // fewer weights, do not get along with fewer of them (16x16x640 stride 2, batch 128, 16 waves and ten slabs / 8 and four: 36.8 / 28.9; but
   // 64x64x320, five slabs / two: 61.4 / 76.2), and 4 waves (16x16x768 stride 2 26.2 us, 8 waves 18.7) only where nothing else fits.
   DwPwTile best = {};
@@ -270,7 +271,7 @@ inline int dwpw_tile(DwPwTile &g, int W, int S, bool chain, int cus, int bn_byte
       t.par_off = (int)((t.x_off + x + 1023) & ~1023);
       t.w_off = t.par_off + par;
       const int busy = chain ? t.waves : std::min(t.waves, t.cf_per << t.lpxb);
-      t.kp = C <= 64 ? 1 : C <= 256 || t.w_off + busy * 8 * 1024 > 150 * 1024 ? 4 : 8;
+      t.kp = C <= 64 ? 1 : chain || C <= 256 || t.w_off + busy * 8 * 1024 > 150 * 1024 ? 4 : 8;
       t.lds = t.w_off + busy * t.kp * 1024;
       if (t.lds > 160 * 1024) continue;
       if (!best.lds || t.slabs < best.slabs) best = t, with = waves;
