@@ -158,10 +158,16 @@ __global__ __launch_bounds__(1024) void dwpw_kernel(DwPwGeom g)
   unsigned char *xin = dwpw_lds + T.x_off, *par = dwpw_lds + T.par_off;
   const int nblocks = CHAIN ? g.nblocks : 1;
   // The input's first part (10 registers) and the pointwise constants (9, of 64 bits 17) are asked for ahead of the depthwise stage, unless they do not
-  // fit beside it: in chains with constants of 64 bits that spilled 14 to 22 registers a lane.  There they are asked for where they are used.  Spilled
-  // / so: 8x8x320 two blocks batch 64 21.0 / 18.1 us, four batch 128 36.0 / 31.8; 8x8x64 four batch 256 17.1 / 14.6; 16x16x64 three batch 256
-  // 21.2 / 19.4.  (With 32 bits 8x8x64 two blocks batch 64 7.5 ahead, 7.95 not; 8x8x320 16.1, 16.7.)
-  constexpr bool AHEAD = !CHAIN || sizeof(bn_t) == 4;
+  // fit beside it.  In chains with constants of 64 bits they were spilled, 14 to 22 registers a lane, and in single blocks they left four
+  // waves a SIMD where there had been five; with eight slices of weights they hold those up.  There they are asked for where they are
+  // used.  Ahead / so: chains 8x8x320 two blocks batch 64 21.0 / 18.1 us, four batch 128 36.0 / 31.8; 8x8x64 four batch 256 17.1 / 14.6; blocks
+  // 64x64x16 -> 32 batch 256 33.2 / 30.0, 8x8x256 batch 64 8.3 / 7.5, 4x4x512 11.0 / 10.6; 32 bits, eight slices: 8x8x512 -> 64 stride 2 9.1 /
+  // 8.7.  (With 32 bits otherwise ahead is the better: 8x8x64 two blocks batch 64 7.5 / 7.95; 64x64x16 -> 32 23.2 / 24.6.)
+  constexpr bool WIDE = sizeof(bn_t) == 8, X_AHEAD = !WIDE || (!CHAIN && KP > 1), PW_AHEAD = !WIDE && KP < 8;
+  // Weights: one slice, behind the input; eight, in front of it; four, behind the input and the parameters, where those have been waited for (constants of
+  // 64 bits: at once).  Eight waited for / in front: 8x8x512 -> 64 stride 2 batch 64 9.15 / 8.9; four at once, 32 bits: 8x8x256 -> 512 stride
+  // 2 6.7 / 7.0, 64 bits 7.8 / 7.7.
+  constexpr bool W_FIRST = KP == 8, W_AT_ONCE = WIDE && !CHAIN && KP == 4;
 
   // the pointwise stage's blocks of 64 pixels x 16 channels, dealt to the waves
   const int cf_lo = part * T.cf_per, nblk = max(min(T.cf_per, T.Co / 16 - cf_lo), 0) << T.lpxb;
@@ -201,8 +207,9 @@ __global__ __launch_bounds__(1024) void dwpw_kernel(DwPwGeom g)
         v[u] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, c.off >= 0 ? (unsigned)c.off : 0x80000000u, 0, 0);
       }
     };
-    if (AHEAD && first) load_x(0, 64 * wave);
-    // (many slices of weights behind the input: in front of it they would hold it up)
+    if constexpr (W_FIRST)
+      if (wave < nblk) load_w(P, w_cf = cf_first, 0);
+    if (X_AHEAD && first) load_x(0, 64 * wave);
     if (KP == 1 && wave < nblk) load_w(P, w_cf = cf_first, 0);
     if ((((unsigned)(unsigned long long)P->dw_wt | (unsigned)(unsigned long long)P->dw_bias) & 3) == 0) {
       dwpw_par_load(par, P->dw_wt, P->dw_bias, P->e_dw.k, P->e_dw.lambda, P->mode_dw == EPI_BN, T.C, wave, NWV, lane);
@@ -229,7 +236,9 @@ __global__ __launch_bounds__(1024) void dwpw_kernel(DwPwGeom g)
         l = *(const bn4 *)(P->e_pw.lambda + n);
       }
     };
-    if constexpr (AHEAD)
+    if constexpr (W_AT_ONCE)
+      if (wave < nblk) load_w(P, w_cf = cf_first, 0);
+    if constexpr (PW_AHEAD)
       if (wave < nblk) load_pw(cf_first);
 #pragma unroll 1
     for (int slab = 0; slab < (CHAIN ? 1 : T.slabs); slab++) {
@@ -238,7 +247,7 @@ __global__ __launch_bounds__(1024) void dwpw_kernel(DwPwGeom g)
         if (slab) dwpw_barrier();  // everybody is done with the slab before
 #pragma unroll 1
         for (int t0 = 64 * wave; t0 < chunks; t0 += NTH * UN) {
-          if (!AHEAD || slab || t0 != 64 * wave) load_x(slab, t0);
+          if (!X_AHEAD || slab || t0 != 64 * wave) load_x(slab, t0);
 #pragma unroll
           for (int u = 0; u < UN; u++) {
             if (t0 + NTH * u >= chunks) break;
@@ -248,7 +257,7 @@ __global__ __launch_bounds__(1024) void dwpw_kernel(DwPwGeom g)
       }
       if (slab == 0) {
         __builtin_amdgcn_s_waitcnt(DWPW_WAIT_VM(0));  // (a wave without input has parameters on their way to LDS)
-        if (KP > 1 && wave < nblk) load_w(P, w_cf = cf_first, 0);
+        if (KP == 4 && !W_AT_ONCE && wave < nblk) load_w(P, w_cf = cf_first, 0);
       }
       dwpw_barrier();
 
@@ -299,7 +308,7 @@ __global__ __launch_bounds__(1024) void dwpw_kernel(DwPwGeom g)
 #pragma unroll 1
     for (int blk = wave; blk < nblk; blk += NWV) {
       const int cf = cf_lo + (blk >> T.lpxb), px0 = 64 * (blk & ((1 << T.lpxb) - 1));
-      if constexpr (!AHEAD) {
+      if constexpr (!PW_AHEAD) {
         bias = 0;
         k = l = (bn4){0, 0, 0, 0};
         load_pw(cf);

@@ -1,5 +1,6 @@
 """What the compiler says of the kernels in the built libraries: registers, and scratch memory for those that did not fit."""
 import os
+import re
 import struct
 import subprocess
 
@@ -53,3 +54,12 @@ def test_no_vector_register_is_spilled(bn_bits):
     spilled = {k[".name"]: k[".vgpr_spill_count"] for k in kernels if k[".vgpr_spill_count"] and any(f in k[".name"] for f in FITTED)}
     names = subprocess.run(["c++filt"], input="\n".join(spilled), stdout=subprocess.PIPE, text=True, check=True).stdout.split("\n")
     assert not spilled, "\n".join("%d registers: %s" % (n, s) for n, s in zip(spilled.values(), names))
+
+
+def test_waves_of_single_blocks():
+    """Constants of 64 bits leave the kernels of a single block four waves a SIMD at least, those of one slice of weights five."""
+    kernels = {k[".name"]: k[".vgpr_count"] for elf in _code_objects(build.lib_path(64)) for k in _kernels(elf)}
+    for name, vgprs in kernels.items():
+        m = re.search(r"dwpw_kernelILi(\d+)ELi(\d+)ELi(\d+)ELb0E", name)
+        if m:
+            assert vgprs <= (96 if m[3] == "1" else 128), name
