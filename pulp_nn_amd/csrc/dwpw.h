@@ -127,7 +127,7 @@ __device__ __forceinline__ void dwpw_par_load(unsigned char *par, const int8_t *
 
 // W, S: input width, stride.  KP: slices of K whose weights are in LDS at once.  CHAIN: g.nblocks blocks back to back; otherwise the
 // one block g.blk[0].
-template <int W, int S, int KP, bool CHAIN>
+template <int W, int S, int KP, bool CHAIN, bool LEAN = false>
 __global__ __launch_bounds__(1024) void dwpw_kernel(DwPwGeom g)
 {
   extern __shared__ __attribute__((aligned(16))) unsigned char dwpw_lds[];
@@ -163,7 +163,7 @@ __global__ __launch_bounds__(1024) void dwpw_kernel(DwPwGeom g)
   // used.  Ahead / so: chains 8x8x320 two blocks batch 64 21.0 / 18.1 us, four batch 128 36.0 / 31.8; 8x8x64 four batch 256 17.1 / 14.6; blocks
   // 64x64x16 -> 32 batch 256 33.2 / 30.0, 8x8x256 batch 64 8.3 / 7.5, 4x4x512 11.0 / 10.6; 32 bits, eight slices: 8x8x512 -> 64 stride 2 9.1 /
   // 8.7.  (With 32 bits otherwise ahead is the better: 8x8x64 two blocks batch 64 7.5 / 7.95; 64x64x16 -> 32 23.2 / 24.6.)
-  constexpr bool WIDE = sizeof(bn_t) == 8, X_AHEAD = !WIDE || (!CHAIN && KP > 1), PW_AHEAD = !WIDE && KP < 8;
+  constexpr bool WIDE = sizeof(bn_t) == 8, X_AHEAD = !WIDE || (!CHAIN && KP > 1), PW_AHEAD = !WIDE && KP < 8 && !LEAN;
   // Weights: one slice, behind the input; eight, in front of it; four, behind the input and the parameters, where those have been waited for (constants of
   // 64 bits: at once).  Eight waited for / in front: 8x8x512 -> 64 stride 2 batch 64 9.15 / 8.9; four at once, 32 bits: 8x8x256 -> 512 stride
   // 2 6.7 / 7.0, 64 bits 7.8 / 7.7.

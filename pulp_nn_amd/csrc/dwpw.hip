@@ -6,11 +6,11 @@
 
 namespace {
 
-template <int W, int S, int KP, bool CHAIN>
+template <int W, int S, int KP, bool CHAIN, bool LEAN = false>
 bool launch_kp(const DwPwGeom &g)
 {
-  if (!raise_lds_limit<dwpw_kernel<W, S, KP, CHAIN>>((size_t)g.t.lds)) return false;
-  hipLaunchKernelGGL((dwpw_kernel<W, S, KP, CHAIN>), dim3((unsigned)g.t.tiles << g.t.lsplit), dim3(64 * g.t.waves), (size_t)g.t.lds, g_stream, g);
+  if (!raise_lds_limit<dwpw_kernel<W, S, KP, CHAIN, LEAN>>((size_t)g.t.lds)) return false;
+  hipLaunchKernelGGL((dwpw_kernel<W, S, KP, CHAIN, LEAN>), dim3((unsigned)g.t.tiles << g.t.lsplit), dim3(64 * g.t.waves), (size_t)g.t.lds, g_stream, g);
   return true;
 }
 template <int W>
@@ -34,6 +34,8 @@ bool launch(const DwPwGeom &g)
   }
   if constexpr (!CHAIN)  // (a chain has no eight slices: dwpw_tile)
     if (g.t.kp == 8) return launch_kp<W, S, 8, CHAIN>(g);
+  if constexpr (!CHAIN && sizeof(bn_t) == 4)  // (with 64 bits every kernel of a single block is as lean)
+    if (g.t.kp == 4 && dwpw_lean(g.t, num_cus())) return launch_kp<W, S, 4, CHAIN, true>(g);
   return g.t.kp == 1 ? launch_kp<W, S, 1, CHAIN>(g) : launch_kp<W, S, 4, CHAIN>(g);
 }
 template <bool CHAIN>

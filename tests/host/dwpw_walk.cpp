@@ -122,7 +122,7 @@ static std::string check(int B, int C, int H, int Co, int chained, int bn_bytes,
         if (p < 0 || p + C > x_bytes || src[p / 16] != (at.b0 * H) * W + px) return "next block's input";
       }
   }
-  return "ok " + std::to_string(g.waves);
+  return "ok " + std::to_string(g.waves) + (!chained && g.kp == 4 && dwpw_lean(g, cus) ? " lean" : "");
 }
 
 // every W, S, C and bn, heights up to three tiles of 256 pixels, and channels out and batches on both sides of every line

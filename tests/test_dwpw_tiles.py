@@ -31,5 +31,11 @@ def test_tiles_on_the_host(tmp_path):
     for b, s in zip(blocks, said):
         assert s.startswith("ok") or s == "no", "block %s: %s" % (b, s)
     assert res.returncode == 0, res.stderr
+    # (the line of the kernel with five waves a SIMD: a second workgroup that LDS holds and that can begin beside the pointwise stage of the first)
+    lean = [(268, 256, 16, 16, 64, 1), (300, 192, 16, 16, 64, 1), (500, 128, 16, 16, 32, 1), (64, 128, 32, 32, 32, 1)]
+    not_lean = [(64, 256, 16, 16, 64, 1), (268, 256, 16, 16, 128, 1), (268, 128, 16, 16, 64, 1), (64, 256, 8, 8, 512, 2), (268, 64, 16, 16, 64, 1)]
+    text = "\n".join("%d %d %d %d %d %d 0 4 256" % b for b in lean + not_lean)
+    line = subprocess.run([exe], input=text, stdout=subprocess.PIPE, text=True, timeout=110).stdout.split("\n")[:-1]
+    assert [s.endswith("lean") for s in line] == [True] * len(lean) + [False] * len(not_lean), line
     taken = [b for b, s in zip(blocks, said) if s != "no"]
     assert len(said) == len(blocks) and len(taken) > 200 and sum(b[6] for b in taken) > 30

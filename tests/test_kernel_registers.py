@@ -56,10 +56,13 @@ def test_no_vector_register_is_spilled(bn_bits):
     assert not spilled, "\n".join("%d registers: %s" % (n, s) for n, s in zip(spilled.values(), names))
 
 
-def test_waves_of_single_blocks():
-    """Constants of 64 bits leave the kernels of a single block four waves a SIMD at least, those of one slice of weights five."""
-    kernels = {k[".name"]: k[".vgpr_count"] for elf in _code_objects(build.lib_path(64)) for k in _kernels(elf)}
-    for name, vgprs in kernels.items():
-        m = re.search(r"dwpw_kernelILi(\d+)ELi(\d+)ELi(\d+)ELb0E", name)
-        if m:
-            assert vgprs <= (96 if m[3] == "1" else 128), name
+@pytest.mark.parametrize("bn_bits", [32, 64])
+def test_waves_of_single_blocks(bn_bits):
+    """Constants of 64 bits leave the kernels of a single block four waves a SIMD at least, those of one slice of weights five; so
+    are the lean ones of the 32-bit library."""
+    kernels = {k[".name"]: k[".vgpr_count"] for elf in _code_objects(build.lib_path(bn_bits)) for k in _kernels(elf)}
+    blocks = [(m[1], m[2] == "1", vgprs) for name, vgprs in kernels.items()
+              if (m := re.search(r"dwpw_kernelILi\d+ELi\d+ELi(\d+)ELb0ELb([01])E", name))]
+    assert any(lean for _, lean, _ in blocks) == (bn_bits == 32)
+    for slices, lean, vgprs in blocks:
+        assert vgprs <= (96 if lean or (bn_bits == 64 and slices == "1") else 128), (slices, lean)
