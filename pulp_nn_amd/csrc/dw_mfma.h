@@ -77,7 +77,7 @@ __device__ __forceinline__ bn_t readlane_bn(bn_t v, int l)
 
 // MODE: requantisation branch; NM: MFMAs per (channel, 16 units) = ceil(ky * ND / 16); CB: channels per workgroup
 template <int CB, int NM, int MODE>
-__global__ __launch_bounds__(256, CB == 16 ? (NM == 1 ? 5 : NM <= 3 ? 4 : 1) : NM == 1 ? 3 : 1) void dw_mfma_kernel(DwmGeom g, EpiArgs e)
+__global__ __launch_bounds__(256, CB == 16 ? (NM == 1 ? 5 : NM <= 3 ? 4 : 1) : NM <= 2 ? 4 : NM == 3 ? 3 : 1) void dw_mfma_kernel(DwmGeom g, EpiArgs e)
 {
   extern __shared__ __attribute__((aligned(16))) unsigned char dwm_lds[];
   // The launch's numbers, all at once: left to itself the compiler asks for each where it is first needed (and again where it is
@@ -119,7 +119,7 @@ __global__ __launch_bounds__(256, CB == 16 ? (NM == 1 ? 5 : NM <= 3 ? 4 : 1) : N
   const int slots = g.NR * g.Q;
   const int iy0 = oy0 * g.sy - g.pt, x0 = 16 * xg0 * g.sx - g.pl;
   const int cpi = (int)fastdiv((unsigned)tid, g.d_nper);
-  constexpr int UN = dwm_loads(CB);
+  constexpr int UN = DWM_LOADS;
   const bool edge = dwm_edge(g, tile, before);  // a load of this tile may leave the tensor
   // Inside: buffer loads (dwm_buffer_off)
   const __amdgpu_buffer_rsrc_t rsrc =

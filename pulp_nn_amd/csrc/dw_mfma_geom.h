@@ -76,8 +76,9 @@ PULPNN_HD bool dwm_edge(const DwmGeom &g, const DwmTile &t, long long before)
 // start of the plane, masked off).
 PULPNN_HD int dwm_load_base(const DwmGeom &g, int iy, int x) { return (unsigned)iy < (unsigned)g.H ? iy * g.W + x : 0; }
 
-// 16-byte loads that a thread has in flight.
-PULPNN_HD constexpr int dwm_loads(int cb) { return cb == 16 ? 4 : 8; }
+// 16-byte loads that a thread has in flight.  (Eight with 64 channels a workgroup: 50 registers more, three waves a SIMD and, from two MFMAs a
+// unit on, two.  Eight / four: 7x7x512 batch 256 24.0 / 19.7 us, 64 bits 28.0 / 24.0, 5x5x512 22.8 / 17.6; 5x5 filters on 7x7x256 20.6 / 17.9.)
+enum { DWM_LOADS = 4 };
 
 // First channel of the thread whose first one is cpi: out of reach of every channel where its pass has no slot for it.
 PULPNN_HD int dwm_thread_channel(int cb, int cpi, bool slot) { return slot ? cpi : cb + 64; }

@@ -210,7 +210,7 @@ inline bool dwpw_small16(long long B, int C, int W, int Ho, int Co, int S, int c
 
 // Whether four slices of weights take the kernel that asks for the pointwise constants where they are used and has five waves a SIMD, not four: where LDS
 // holds a second workgroup of sixteen waves, and so few of them have a part in the pointwise stage that the next one can begin beside them.
-// Constants ahead / lean: 16x16x256 -> 64 batch 268 27.1 / 22.8 us, 16x16x192 -> 64 26.9 / 23.5, 16x16x128 -> 32 batch 500 21.5 / 19.4; elsewhere ahead is the better: 8x8x256 -> 512
+// Constants ahead / lean: 16x16x256 -> 64 batch 268 27.1 / 22.8 us, 16x16x192 -> 64 26.9 / 23.1, 16x16x128 -> 32 batch 500 21.5 / 18.9; elsewhere ahead is the better: 8x8x256 -> 512
 // stride 2 batch 64 6.7 / 6.8, 16x16x640 -> 1024 stride 2 batch 128 31.9 / 32.9, 8x8x128 -> 256 stride 2 batch 18 4.7 / 4.9.
 inline bool dwpw_lean(const DwPwTile &t, int cus)
 {

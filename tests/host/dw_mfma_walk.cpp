@@ -42,7 +42,7 @@ static std::string check(const DwLayer &L, int cus)
     const int lo = (int)std::max(-before, -(1ll << 30)), hi = (int)std::min(behind, 0x7fffffffll);
     // Every load the staging makes: the passes over slots, the threads of a pass, the channels of a thread.  `seen`: slots and channels staged.
     // (Of the first and the last 48 tiles.)
-    const int slots = id < 48u || id + 48u >= (unsigned)g.total ? g.NR * g.Q : 0, UN = dwm_loads(CB);
+    const int slots = id < 48u || id + 48u >= (unsigned)g.total ? g.NR * g.Q : 0, UN = DWM_LOADS;
     std::vector<unsigned char> seen(slots * t.ncb);
     if (g.nper > 256 || g.nper * g.cpar > 256 || g.cpar < 1) return wrong("threads of a pass", t, g.nper, g.cpar);
     for (int s0 = 0; s0 < slots; s0 += g.nper)
