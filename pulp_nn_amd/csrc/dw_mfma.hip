@@ -22,7 +22,7 @@ bool launch_cb(int mode, const DwLayer &L, const EpiArgs &e, int cus, hipStream_
   DwmGeom g;
   int nm;
   size_t lds;
-  if (!dwm_shape<CB>(L, cus, &g, &nm, &lds)) return false;
+  if (!dwm_shape<CB>(L, cus, &g, &nm, &lds) || (CB == 64 && !dwm_wide(L, g, cus))) return false;
   if (nm == 1) launch_mode<CB, 1>(mode, g, e, lds, s);
   else if (nm == 2) launch_mode<CB, 2>(mode, g, e, lds, s);
   else if (nm == 3) launch_mode<CB, 3>(mode, g, e, lds, s);
@@ -34,10 +34,5 @@ bool launch_cb(int mode, const DwLayer &L, const EpiArgs &e, int cus, hipStream_
 
 bool launch_dw_mfma(int mode, const DwLayer &L, const EpiArgs &e, int cus, hipStream_t s)
 {
-  // 64 channels per workgroup instead of 16 where a plane is so small (up to 64 output pixels) that the set-up of a
-  // workgroup, some 400 instructions per wave, is most of its work, and enough workgroups remain.  Measured, kernel time
-  // at 16 / 64 channels: 7x7x512 batch 256 33.8 / 23.8 us, 8x8x256 18.9 / 14.5; but 17x17x408 batch 85 18.8 / 27.9,
-  // 28x28x256 batch 64 11.8 / 17.9 (fewer workgroups to cover each other's load, multiply and store phases).
-  if (L.Ho * L.Wo <= 64 && (long long)L.B * ((L.CH + 63) / 64) >= 4ll * cus && launch_cb<64>(mode, L, e, cus, s)) return true;
-  return launch_cb<16>(mode, L, e, cus, s);
+  return (L.Ho * L.Wo <= 64 && launch_cb<64>(mode, L, e, cus, s)) || launch_cb<16>(mode, L, e, cus, s);
 }

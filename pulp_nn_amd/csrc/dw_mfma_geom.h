@@ -66,6 +66,16 @@ PULPNN_HD DwmTile dwm_tile(const DwmGeom &g, unsigned id)
   return t;
 }
 
+// Whether a layer of this tile shape, with 64 channels a workgroup, takes that rather than 16.
+// A workgroup's set-up is most of its work on planes of up to 64 output pixels, and with 64 channels it is paid once instead of four times, as long as
+// enough workgroups remain and LDS holds whole planes: cut in bands, the planes' rows are staged again and the set-up is paid again.  Whole calls, 16 /
+// 64 channels: 7x7x512 batch 256 28.1 / 19.7 us, 5x5x512 26.9 / 17.9, 4x4x130 batch 700 21.4 / 16.8, 5x5 filters on 7x7x256 20.9 / 17.9; in bands stride 2 on
+// 13x13x256 22.0 / 25.6, 7x7 filters on 7x7x256 25.0 / 34.2.
+inline bool dwm_wide(const DwLayer &L, const DwmGeom &g64, int cus)
+{
+  return L.Ho * L.Wo <= 64 && (long long)L.B * ((L.CH + 63) / 64) >= 4ll * cus && g64.bands == 1;
+}
+
 // Whether a 16-byte load of the tile may leave the tensor (before: bytes of the tensor in front of the tile's first plane).
 PULPNN_HD bool dwm_edge(const DwmGeom &g, const DwmTile &t, long long before)
 {

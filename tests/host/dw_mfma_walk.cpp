@@ -94,7 +94,7 @@ static std::string check(const DwLayer &L, int cus)
     outputs += (long long)t.rows * t.wt * t.ncb;
   }
   if (all && outputs != (long long)L.B * L.CH * L.Ho * L.Wo) return "outputs left out";
-  return "ok " + std::to_string(g.total);
+  return "ok " + std::to_string(g.total) + (CB == 64 && dwm_wide(L, g, cus) ? " wide" : "");
 }
 
 int main()
@@ -106,6 +106,7 @@ int main()
     if (s.compare(0, 2, "ok") == 0 || s == "no") {
       const std::string s64 = (long long)L.Ho * L.Wo <= 64 ? check<64>(L, cus) : "no";
       if (s64.compare(0, 2, "ok") != 0 && s64 != "no") s = "64 channels: " + s64;
+      else if (s64.find("wide") != std::string::npos) s = s64;
     }
     puts(s.c_str());
   }

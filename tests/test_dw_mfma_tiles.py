@@ -52,6 +52,15 @@ def test_channels_that_do_not_exist(walk):
                  layer(2, 17, 200, 200, 3, 3, (1, 1, 1, 1), (1, 1)), layer(1100, 65, 7, 7, 3, 3, (1, 1, 1, 1), (1, 1))])
 
 
+def test_64_channels_a_workgroup_where_planes_are_whole(walk):
+    wide = [layer(256, 512, 7, 7, 3, 3, (1, 1, 1, 1), (1, 1)), layer(256, 256, 7, 7, 5, 5, (2, 2, 2, 2), (1, 1)),
+            layer(700, 130, 4, 4, 3, 3, (1, 1, 1, 1), (1, 1)), layer(1024, 64, 8, 8, 3, 3, (1, 1, 1, 1), (1, 1))]
+    not_wide = [layer(256, 256, 13, 13, 3, 3, (1, 1, 1, 1), (2, 2)), layer(256, 256, 7, 7, 7, 7, (3, 3, 3, 3), (1, 1)),   # cut in bands
+                layer(1023, 64, 8, 8, 3, 3, (1, 1, 1, 1), (1, 1)), layer(1024, 64, 8, 9, 3, 3, (1, 1, 1, 1), (1, 1))]
+    assert all(s.startswith("ok") and s.endswith("wide") for s in walk(wide))
+    assert all(s.startswith("ok") and not s.endswith("wide") for s in walk(not_wide))
+
+
 def test_narrow_last_column_tile(walk):
     """Several column tiles and several rows per tile: the last tile's rows are shorter, in LDS too."""
     check(walk, [layer(600, 16, 6, 340, 3, 3, (1, 1, 1, 111), (1, 1)), layer(64, 16, 40, 320, 3, 3, (1, 1, 1, 131), (1, 1)),
