@@ -188,6 +188,9 @@ __global__ __launch_bounds__(256, CB == 16 ? (NM == 1 ? 5 : NM <= 3 ? 4 : 1) : N
       const bool ok = r < g.ky;
       boff[mm][i] = ok ? r * g.pitch + 4 * xd : 0;
       woff[mm][i] = ok ? r * DWM_WROW + 4 * min(max(xd - wq + 2, 0), 4) : 0;
+      // (here, not where it is used: the compiler would keep r and xd until then, and spill with three MFMAs a unit.  With two it has registers to spare,
+      // and the 64-bit kernels are up to 14 % slower with this.)
+      if constexpr (NM == 3) asm volatile("" : "+v"(boff[mm][i]));
     }
   __builtin_amdgcn_sched_barrier(0);
 

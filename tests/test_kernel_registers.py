@@ -10,7 +10,7 @@ import pytest
 from pulp_nn_amd import build
 
 # kernels that hold more at once than one wave's registers would take if it were asked for all at the same place
-FITTED = ("dwpw_kernel", "dwpw_chain_kernel")
+FITTED = ("dwpw_kernel", "dwpw_chain_kernel", "dw_mfma_kernel")
 MAGIC = b"__CLANG_OFFLOAD_BUNDLE__"
 
 
