@@ -57,7 +57,6 @@ def test_no_vector_register_is_spilled(bn_bits):
 
 
 @pytest.mark.parametrize("bn_bits", [32, 64])
-@pytest.mark.parametrize("bn_bits", [32, 64])
 def test_waves_of_small_depthwise_planes(bn_bits):
     """64 channels a workgroup: four workgroups share a compute unit with one or two MFMAs a unit, three with three."""
     kernels = {k[".name"]: k[".vgpr_count"] for elf in _code_objects(build.lib_path(bn_bits)) for k in _kernels(elf)}
@@ -66,6 +65,7 @@ def test_waves_of_small_depthwise_planes(bn_bits):
     assert len(found) == 12 and not [f for f in found if f[0] > f[1]]
 
 
+@pytest.mark.parametrize("bn_bits", [32, 64])
 def test_waves_of_single_blocks(bn_bits):
     """Constants of 64 bits leave the kernels of a single block four waves a SIMD at least, those of one slice of weights five; so
     are the lean ones of the 32-bit library."""
