@@ -411,12 +411,9 @@ void conv_common(const char *fn, bool pointwise, const uint8_t *in, const int8_t
     // 32 -> 24 7.7 / 5.3; 64x32x32 16 -> 32 6.9 / 6.4; but 133x28x28 16 -> 32 7.7 / 8.3): a line at 32 channels that this rule
     // does not draw.
     const bool whole16 = ch_in % 16 == 0 && aligned(in, 16) && aligned(w, 16);
-    // Up to 128 output channels it is also the faster one for channel counts that are no multiples of 64, which the tiled kernel gathers
-    // chunk by chunk, on images of up to some 60000 pixels in all (tiled / band: 12x12 112 -> 71 batch 146 16.5 / 10.3 us, 41x11 160 -> 100 batch 2
-    // 12.9 / 9.1, 59x17 96 -> 128 batch 7 8.7 / 8.2; but 42x31 48 -> 96 batch 54 14.4 / 18.3, 34x53 176 -> 128 batch 36 29.1 / 34.9; the mean over 52
-    // layers is 0.88, over the 44 on this side of the line 0.85, two of them slower: 63x21 96 -> 96 stride 2 batch 39 9.3 / 11.0), as long as a tile's
-    // input leaves LDS to a second workgroup (5x5 on 208 channels 66 / 124), and not for pointwise layers (12x11 48 -> 112 batch 5 4.0 / 5.0).
-    const bool odd64 = ch_in % 64 && g.N <= 128 && g.M <= 60000 && kx * ky > 1 && (kx * ky <= 9 || ch_in <= 96);
+    // Up to 128 output channels it is also the faster one for many layers whose channel count is no multiple of 64, which the tiled kernel gathers
+    // chunk by chunk (band_for_odd_channels).
+    const bool odd64 = g.N > 64 && band_for_odd_channels(L, num_cus(), (int)sizeof(bn_t));
     const bool few = ch_in == 16 || ch_in == 32 ? false : ch_in % 64 == 0 ? g.N <= 32 : g.N <= 64 || odd64;
     if (!whole16 || few) {
       if (launch_conv_band(mode, L, e, num_cus(), g_stream)) return check_launch(fn);

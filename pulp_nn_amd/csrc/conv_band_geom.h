@@ -163,3 +163,28 @@ inline bool band_shape(const ConvLayer &L, int cus, int bn_bytes, BandGeom *out,
   *lds_out = (size_t)lds;
   return true;
 }
+
+// Whether a layer of 65 to 128 output channels on a channel count of whole 16-byte chunks but no multiple of 64 takes this kernel, not the tiled one, which
+// gathers such inputs chunk by chunk in tiles of 128 pixels x 64 channels.  Whole calls, tiled / band: 12x12 112 -> 71 batch 146 16.5 / 10.3 us, 27x8
+// 176 -> 120 batch 177 19.7 / 11.7, 48x18 96 -> 100 stride 2 batch 101 9.7 / 6.2.  Not
+// - up to five K slices, which the tiled kernel fetches at once (2x2 on 41x54 48 -> 72 batch 9 5.8 / 7.0);
+// - where LDS holds one workgroup (20x53 176 -> 112 stride 2 batch 119 19.9 / 36.5), or from stride 2 on, where a pixel's input is four pixels, in more than
+//   two a compute unit or in tiles of eight groups of pixels or a third empty (24x48 176 -> 96 stride 2 batch 182 26.3 / 36.9);
+// - where the tiled kernel's tiles are one for almost every compute unit, which is what it does best, and these are more (63x21 96 -> 96 stride 2 batch 39
+//   8.7 / 10.5, 10x17 96 -> 120 batch 92 8.8 / 10.3);
+// - on more than some 60000 pixels in all (42x31 48 -> 96 batch 54 14.4 / 18.3), nor, with large filters, on more than 96 channels.
+// Over 190 layers drawn for it the mean is 0.867 of the tiled kernel's time, of the 137 that it takes 0.82; four of those are more than 2 % slower, the worst
+// 18x51 112 -> 80 batch 34 13.1 / 16.2.
+inline bool band_for_odd_channels(const ConvLayer &L, int cus, int bn_bytes)
+{
+  const long long m = (long long)L.B * L.Ho * L.Wo, tiled = (m + 127) / 128 * ((L.N + 63) / 64);
+  const int taps = L.kx * L.ky;
+  if (L.N > 128 || L.Ci % 64 == 0 || taps == 1 || (taps > 9 && L.Ci > 96) || taps * L.Ci <= 320 || m > 60000) return false;
+  BandGeom g;
+  int tn, tm;
+  size_t lds;
+  if (!band_shape(L, cus, bn_bytes, &g, &tn, &tm, &lds) || lds > 80 * 1024) return false;
+  if (tm > 2 && g.total > cus && tiled <= cus && 5 * tiled >= 4 * cus) return false;
+  if (L.sx == 1 && L.sy == 1) return true;
+  return g.total <= 2 * cus && (tm == 2 || (tm == 4 && 10 * g.R * g.PC >= 7 * 16 * tm * (4 / g.WN)));
+}

@@ -1,6 +1,7 @@
 // Walks the tiles of conv_band_kernel on the host with the launcher's own tile shape (csrc/conv_band_geom.h) and reports
 // tiles whose staged input or fragments leave their LDS range, and output pixels that no tile or more than one computes.
-// Layers on stdin, one a line: B H W Ci Ho Wo N kx ky pt pl sx sy bn_bytes cus.  One line out per layer: "ok LDS TILES", "no"
+// Layers on stdin, one a line: B H W Ci Ho Wo N kx ky pt pl sx sy bn_bytes cus.  One line out per layer: "ok LDS TILES", with "odd" behind it where
+// band_for_odd_channels says so, "no"
 // (not taken by the kernel) or what is wrong.
 #include <stdio.h>
 
@@ -30,7 +31,7 @@ static std::string check(const ConvLayer &L, int bn_bytes, int cus)
   if ((ll)g.xtiles * g.PC < g.Wo || (ll)(g.xtiles - 1) * g.PC >= g.Wo || (ll)g.bands * g.R < g.Ho || (ll)(g.bands - 1) * g.R >= g.Ho ||
       g.nblocks * nch < g.N || (g.nblocks - 1) * nch >= g.N || B * g.bands * g.xtiles * g.nblocks != g.total)
     return "tiles: " + std::to_string(g.total);
-  return "ok " + std::to_string(lds) + " " + std::to_string(g.total);
+  return "ok " + std::to_string(lds) + " " + std::to_string(g.total) + (L.N > 64 && band_for_odd_channels(L, cus, bn_bytes) ? " odd" : "");
 }
 
 int main()

@@ -41,6 +41,19 @@ def test_usual_layers(walk):
     assert sum(s != "no" for s in said) > 3500
 
 
+def test_odd_channel_counts_up_to_128_outputs(walk):
+    """The line between this kernel and the tiled one, from both sides."""
+    def conv(B, H, W, Ci, N, k, s, bn_bytes=4):
+        return layer(B, H, W, Ci, (H + k // 2 * 2 - k) // s + 1, (W + k // 2 * 2 - k) // s + 1, N, k, k, k // 2, k // 2, s, s, bn_bytes=bn_bytes)
+    band = [conv(146, 12, 12, 112, 71, 3, 1), conv(177, 27, 8, 176, 120, 3, 1), conv(101, 48, 18, 96, 100, 3, 2), conv(2, 37, 30, 80, 65, 7, 2, 8),
+            conv(48, 9, 9, 96, 128, 3, 1), conv(40, 32, 31, 208, 128, 3, 2)]
+    tiled = [conv(9, 41, 54, 48, 72, 2, 1), conv(119, 20, 53, 176, 112, 3, 2, 8), conv(182, 24, 48, 176, 96, 3, 2), conv(39, 63, 21, 96, 96, 3, 2),
+             conv(92, 10, 17, 96, 120, 3, 1, 8), conv(54, 42, 31, 48, 96, 3, 1), conv(2, 20, 20, 208, 100, 5, 1), conv(8, 16, 16, 96, 128, 1, 1),
+             conv(8, 16, 16, 128, 128, 3, 1), conv(8, 16, 16, 96, 129, 3, 1), conv(19, 62, 50, 240, 120, 2, 2)]
+    assert all(s.endswith("odd") for s in walk(band))
+    assert not any(s.endswith("odd") for s in walk(tiled))
+
+
 def test_lds_past_an_int(walk):
     """Strides and filters whose staged input would take more bytes than an int counts: not taken, or in tiles that fit."""
     layers = [layer(1, 60, 60, 57, 15292, 50, 6, 4, 1, sx=34257, sy=35775), layer(1, 60, 60, 53, 11955, 1, 10, 4, 2, sx=1, sy=37077),
