@@ -2,8 +2,7 @@
 // VALU kernels, one thread per output pixel and group of 4 channels (16 for
 // add), so that neighbouring lanes read and write neighbouring bytes.
 //
-// Bound: small maps by launch and one trip to memory (all taps of a window of up to 4 x 4, or 3 x 3 for the maximum, are asked for
-// together); large ones by HBM.  The place of a thread takes 32-bit divisions by multiplication: written in 64 bits it was some 600
+// Bound: small maps by launch and one trip to memory (the taps of a window are asked for in blocks, pool_blocks.h); large ones by HBM.  The place of a thread takes 32-bit divisions by multiplication: written in 64 bits it was some 600
 // instructions.  Whole calls, that and a row of taps per trip / now: average 4x4 on 64 images of 16x16x64 4.2 / 3.2 us, 2x2 on 64 of 32x32x256
 // 11.4 / 8.1 (21 MB), 7x7 on 32 of 7x7x1000 7.6 / 5.6; maximum 3x3 on 112x112x64 3.8 / 3.05, on
 // 64 of 56x56x64 5.35 / 4.4, 2x2 on 64 of 63x63x256 14.7 / 12.9, 7x7 stride 7 29.7 / 16.8 (64 MB).
@@ -12,6 +11,7 @@
 
 #include "fastdiv.h"
 #include "memops.h"
+#include "pool_blocks.h"
 #include "requant.h"
 
 typedef unsigned short ushort2v __attribute__((ext_vector_type(2)));
@@ -109,9 +109,9 @@ __global__ __launch_bounds__(256) void maxpool_kernel(PoolGeom g)
 
 // Same, 16 channels per thread with 16-byte accesses (C % 16 == 0, 16-byte aligned maps).
 // g.cgroups counts groups of 16 here.  NT: non-temporal store; LNT: non-temporal loads (windows that do not
-// overlap on an input too large for the caches: every byte is read once).  The taps of a window of up to 3 x 3 are
-// asked for together, those of larger ones four of a row at a time.
-template <bool NT, bool LNT>
+// overlap on an input too large for the caches: every byte is read once).
+// BW, BH: columns and rows of taps whose loads are issued together (pool_blocks.h).
+template <bool NT, bool LNT, int BW, int BH>
 __global__ __launch_bounds__(256) void maxpool16_kernel(PoolGeom g)
 {
   const long long t = (long long)blockIdx.x * 256 + threadIdx.x;
@@ -129,24 +129,26 @@ __global__ __launch_bounds__(256) void maxpool16_kernel(PoolGeom g)
     m.w = (int)max_u8x4((unsigned)m.w, (unsigned)v.w);
   };
   v4i m = {0, 0, 0, 0};
-  if (g.kx <= 2 && g.ky <= 2 && ys < ye && xs < xe) {
-    // (where the image ends in the window: its last row or column once more, not a path of its own for the few lanes that are there.  63x63x256
-    // batch 64 18.5 us with one, 14.7 tap by tap at the edges, 12.9 so)
-    const uint8_t *p = img + ((long long)ys * g.W + xs) * g.C;
-    const long long row = ye - ys > 1 ? (long long)g.W * g.C : 0;
-    const int col = xe - xs > 1 ? g.C : 0;
-    if (g.kx == 2 && g.ky == 2) {
-      const v4i v0 = ld(p), v1 = ld(p + col), v2 = ld(p + row), v3 = ld(p + row + col);
-      m = v0;
-      vmax(m, v1);
-      vmax(m, v2);
-      vmax(m, v3);
-    } else {
-      const v4i v0 = ld(p);
-      m = v0;
-      if (g.kx * g.ky == 2) vmax(m, ld(p + (g.kx == 2 ? col : row)));
+  if constexpr (BW * BH == 4 && BW == BH) {
+    // A window of up to 2 x 2.  (Where the image ends in it: its last row or column once more, not a path of its own for the few lanes that are there.
+    // 63x63x256 batch 64 18.5 us with one, 14.7 tap by tap at the edges, 12.9 so)
+    if (ys < ye && xs < xe) {
+      const uint8_t *p = img + ((long long)ys * g.W + xs) * g.C;
+      const long long row = ye - ys > 1 ? (long long)g.W * g.C : 0;
+      const int col = xe - xs > 1 ? g.C : 0;
+      if (g.kx == 2 && g.ky == 2) {
+        const v4i v0 = ld(p), v1 = ld(p + col), v2 = ld(p + row), v3 = ld(p + row + col);
+        m = v0;
+        vmax(m, v1);
+        vmax(m, v2);
+        vmax(m, v3);
+      } else {
+        const v4i v0 = ld(p);
+        m = v0;
+        if (g.kx * g.ky == 2) vmax(m, ld(p + (g.kx == 2 ? col : row)));
+      }
     }
-  } else if (g.kx <= 3 && g.ky <= 3) {
+  } else if constexpr (BW * BH == 9) {
     // the whole window (past its end: its last row or column once more)
     if (ys < ye && xs < xe) {
       v4i v[9];
@@ -156,20 +158,14 @@ __global__ __launch_bounds__(256) void maxpool16_kernel(PoolGeom g)
       for (int i = 0; i < 9; i++) vmax(m, v[i]);
     }
   } else {
-    // four or five taps of a row at a time (nine of three rows re-read too many: 4x4 stride 4 on 64 of 63x63x256 16.4 us, 10.7 so)
-    auto rows = [&](auto side) {
-      constexpr int S = decltype(side)::value;
-      for (int y = ys; y < ye; y++)
-        for (int x = xs; x < xe; x += S) {
-          v4i v[S];
+    for (int y = ys; y < ye; y += BH)
+      for (int x = xs; x < xe; x += BW) {
+        v4i v[BW * BH];
 #pragma unroll
-          for (int i = 0; i < S; i++) v[i] = ld(img + ((long long)y * g.W + min(x + i, xe - 1)) * g.C);
+        for (int i = 0; i < BW * BH; i++) v[i] = ld(img + ((long long)min(y + i / BW, ye - 1) * g.W + min(x + i % BW, xe - 1)) * g.C);
 #pragma unroll
-          for (int i = 0; i < S; i++) vmax(m, v[i]);
-        }
-    };
-    if (g.kx == 5) rows(std::integral_constant<int, 5>{});
-    else rows(std::integral_constant<int, 4>{});
+        for (int i = 0; i < BW * BH; i++) vmax(m, v[i]);
+      }
   }
   store16<NT>(g.out + (((long long)b * g.Ho + oy) * g.Wo + ox) * g.C + cg * 16, m);
 }
@@ -184,6 +180,8 @@ struct AvgArgs {
   FastDiv d_ks;  // division by kx * ky
 };
 
+// BW, BH: columns and rows of taps whose loads are issued together (pool_blocks.h)
+template <int BW, int BH>
 __global__ __launch_bounds__(256) void avgpool_kernel(PoolGeom g, AvgArgs a)
 {
   const long long t = (long long)blockIdx.x * 256 + threadIdx.x;
@@ -195,33 +193,25 @@ __global__ __launch_bounds__(256) void avgpool_kernel(PoolGeom g, AvgArgs a)
   const int xs = max(0, ox * g.sx - g.pl), xe = min(ox * g.sx - g.pr + g.kx, g.W);
   const uint8_t *img = g.in + (long long)b * g.H * g.W * g.C + c;
   unsigned sum[4] = {0, 0, 0, 0};
-  // Up to sixteen taps at a time, their loads issued together (taps past the window re-read its last row or column and are not counted): one
-  // load per round trip would make the window size the kernel's latency.  Even and odd bytes are summed in halves of a dword.
-  auto taps = [&](auto side) {
-    constexpr int S = decltype(side)::value;
-    for (int y = ys; y < ye; y += S)
-      for (int x = xs; x < xe; x += S) {
-        unsigned v[S * S], even = 0, odd = 0;
+  // A block's loads are issued together (taps past the window re-read its last row or column and are not counted): one load per round trip
+  // would make the window size the kernel's latency.  Even and odd bytes are summed in halves of a dword.
+  for (int y = ys; y < ye; y += BH)
+    for (int x = xs; x < xe; x += BW) {
+      unsigned v[BW * BH], even = 0, odd = 0;
 #pragma unroll
-        for (int i = 0; i < S * S; i++)
-          v[i] = load4(img + ((long long)min(y + i / S, ye - 1) * g.W + min(x + i % S, xe - 1)) * g.C, n, g.vec4);
+      for (int i = 0; i < BW * BH; i++)
+        v[i] = load4(img + ((long long)min(y + i / BW, ye - 1) * g.W + min(x + i % BW, xe - 1)) * g.C, n, g.vec4);
 #pragma unroll
-        for (int i = 0; i < S * S; i++) {
-          const unsigned u = y + i / S < ye && x + i % S < xe ? v[i] : 0u;
-          even += u & 0x00FF00FFu;
-          odd += (u >> 8) & 0x00FF00FFu;
-        }
-        sum[0] += even & 0xFFFF;
-        sum[1] += odd & 0xFFFF;
-        sum[2] += even >> 16;
-        sum[3] += odd >> 16;
+      for (int i = 0; i < BW * BH; i++) {
+        const unsigned u = y + i / BW < ye && x + i % BW < xe ? v[i] : 0u;
+        even += u & 0x00FF00FFu;
+        odd += (u >> 8) & 0x00FF00FFu;
       }
-  };
-  // (no more loads than the window has: 2x2 on 64 images of 32x32x256 12.0 us, 12.7 with sixteen)
-  const int side = max(g.kx, g.ky);
-  if (side <= 2) taps(std::integral_constant<int, 2>{});
-  else if (side == 3) taps(std::integral_constant<int, 3>{});
-  else taps(std::integral_constant<int, 4>{});
+      sum[0] += even & 0xFFFF;
+      sum[1] += odd & 0xFFFF;
+      sum[2] += even >> 16;
+      sum[3] += odd >> 16;
+    }
   unsigned packed = 0;
 #pragma unroll
   for (int j = 0; j < 4; j++) {

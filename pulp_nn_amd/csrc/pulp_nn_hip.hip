@@ -62,6 +62,21 @@ int num_cus()
 
 namespace {
 
+template <int BW, int BH>
+void launch_maxpool16(const PoolGeom &g, bool nt, bool lnt)
+{
+  const dim3 grid((unsigned)((g.total + 255) / 256)), block(256);
+  if (nt && lnt) hipLaunchKernelGGL((maxpool16_kernel<true, true, BW, BH>), grid, block, 0, g_stream, g);
+  else if (nt) hipLaunchKernelGGL((maxpool16_kernel<true, false, BW, BH>), grid, block, 0, g_stream, g);
+  else if (lnt) hipLaunchKernelGGL((maxpool16_kernel<false, true, BW, BH>), grid, block, 0, g_stream, g);
+  else hipLaunchKernelGGL((maxpool16_kernel<false, false, BW, BH>), grid, block, 0, g_stream, g);
+}
+template <int BW, int BH>
+void launch_avgpool(const PoolGeom &g, const AvgArgs &a)
+{
+  hipLaunchKernelGGL((avgpool_kernel<BW, BH>), dim3((unsigned)((g.total + 255) / 256)), dim3(256), 0, g_stream, g, a);
+}
+
 bool pool_geom(const char *fn, PoolGeom *g, uint8_t *in, uint8_t *out, uint16_t W, uint16_t H, uint16_t C,
                uint16_t Wo, uint16_t Ho, uint16_t kx, uint16_t ky, uint16_t pt, uint16_t pb, uint16_t pl,
                uint16_t pr, uint16_t sx, uint16_t sy)
@@ -389,15 +404,19 @@ void pulp_nn_maxpool(uint8_t *Im_in, uint8_t *Im_out, uint16_t dim_im_in_x, uint
   if (ch_im_in % 16 == 0 && aligned(Im_in, 16) && aligned(Im_out, 16)) {
     g.cgroups = ch_im_in / 16;
     pool_threads(&g);
-    const dim3 grid((unsigned)((g.total + 255) / 256));
     // non-temporal loads: windows that do not overlap, on an input too large to find again in a cache
     const bool lnt = stride_x >= dim_kernel_x && stride_y >= dim_kernel_y &&
                      (long long)g.B * g.H * g.W * g.C >= PULPNN_NT_BYTES;
     const bool snt = g.total * 16 >= PULPNN_NT_BYTES;
-    if (snt && lnt) hipLaunchKernelGGL((maxpool16_kernel<true, true>), grid, dim3(256), 0, g_stream, g);
-    else if (snt) hipLaunchKernelGGL((maxpool16_kernel<true, false>), grid, dim3(256), 0, g_stream, g);
-    else if (lnt) hipLaunchKernelGGL((maxpool16_kernel<false, true>), grid, dim3(256), 0, g_stream, g);
-    else hipLaunchKernelGGL((maxpool16_kernel<false, false>), grid, dim3(256), 0, g_stream, g);
+    switch (pool_max_block(g.kx, g.ky)) {
+      case PB_2x2: launch_maxpool16<2, 2>(g, snt, lnt); break;
+      case PB_3x3: launch_maxpool16<3, 3>(g, snt, lnt); break;
+      case PB_3x1: launch_maxpool16<3, 1>(g, snt, lnt); break;
+      case PB_1x3: launch_maxpool16<1, 3>(g, snt, lnt); break;
+      case PB_4x1: launch_maxpool16<4, 1>(g, snt, lnt); break;
+      case PB_1x4: launch_maxpool16<1, 4>(g, snt, lnt); break;
+      case PB_5x1: launch_maxpool16<5, 1>(g, snt, lnt); break;
+    }
   } else {
     hipLaunchKernelGGL(maxpool_kernel, dim3((unsigned)((g.total + 255) / 256)), dim3(256), 0, g_stream, g);
   }
@@ -417,7 +436,20 @@ void pulp_nn_avgpool(uint8_t *Im_in, uint8_t *Im_out, bn_t lambda, uint16_t out_
   REQUIRE(!flag_requant || out_shift < PULPNN_BN_BITS, PULP_NN_HIP_ERR_ARGUMENT, "out_shift out of range");
   REQUIRE((long long)dim_kernel_x * dim_kernel_y * 255 < 0xffffffffLL, PULP_NN_HIP_ERR_UNSUPPORTED, "window too large");
   AvgArgs a = {(long long)lambda, (long long)out_add, (int)out_shift, flag_requant, fastdiv_make((unsigned)dim_kernel_x * dim_kernel_y)};
-  hipLaunchKernelGGL(avgpool_kernel, dim3((unsigned)((g.total + 255) / 256)), dim3(256), 0, g_stream, g, a);
+  switch (pool_avg_block(g.kx, g.ky)) {
+    case PB_1x1: launch_avgpool<1, 1>(g, a); break;
+    case PB_2x1: launch_avgpool<2, 1>(g, a); break;
+    case PB_1x2: launch_avgpool<1, 2>(g, a); break;
+    case PB_2x2: launch_avgpool<2, 2>(g, a); break;
+    case PB_3x1: launch_avgpool<3, 1>(g, a); break;
+    case PB_1x3: launch_avgpool<1, 3>(g, a); break;
+    case PB_3x3: launch_avgpool<3, 3>(g, a); break;
+    case PB_4x1: launch_avgpool<4, 1>(g, a); break;
+    case PB_1x4: launch_avgpool<1, 4>(g, a); break;
+    case PB_5x1: launch_avgpool<5, 1>(g, a); break;
+    case PB_5x3: launch_avgpool<5, 3>(g, a); break;
+    case PB_4x4: launch_avgpool<4, 4>(g, a); break;
+  }
   check_launch(__func__);
 }
 

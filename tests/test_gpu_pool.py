@@ -9,7 +9,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("channels", [16, 48, 20, 7])
-@pytest.mark.parametrize("kernel", [(1, 1), (2, 2), (3, 3), (2, 3), (4, 3), (4, 4), (5, 2), (7, 7)], ids=str)
+@pytest.mark.parametrize("kernel", [(1, 1), (2, 2), (3, 3), (2, 3), (4, 3), (4, 4), (5, 2), (7, 7), (2, 1), (1, 2), (3, 1), (1, 3), (1, 4), (5, 1),
+                                    (5, 3), (6, 6), (7, 1), (1, 8), (10, 11)], ids=str)
 def test_windows(kernel, channels):
     r = rng_for(8500 + 10 * kernel[0] + kernel[1] + channels)
     x = rand_u8(r, (3, 11, 13, channels))
