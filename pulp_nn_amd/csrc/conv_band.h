@@ -49,7 +49,7 @@ __device__ __forceinline__ v4i bytes_up(v4i v, int n)
 
 // TN: 16-channel groups per wave; TM: 16-pixel groups per wave; PF: K steps of a group of weights
 template <int TN, int TM, int PF>
-__global__ __launch_bounds__(256, TN * TM <= 4 ? 4 : TN * TM == 8 ? 3 : TN * TM == 16 ? 2 : 1) void conv_band_kernel(BandGeom g, EpiArgs e)
+__global__ __launch_bounds__(256, TN * TM <= 4 ? 4 : TN * TM == 8 ? 3 : 2) void conv_band_kernel(BandGeom g, EpiArgs e)
 {
   extern __shared__ __attribute__((aligned(16))) unsigned char band_lds[];
   typedef unsigned v4u __attribute__((ext_vector_type(4)));
@@ -114,7 +114,7 @@ __global__ __launch_bounds__(256, TN * TM <= 4 ? 4 : TN * TM == 8 ? 3 : TN * TM 
 
   // ---- ... the constants of the thread's channel -----------------------------------------------------------------------
   int p_bias = 0;
-  bn_t p_k = g.mode == EPI_MULT ? (bn_t)e.mult : (bn_t)1, p_l = 0;
+  bn_t p_k = 0, p_l = 0;  // (of batch-norm, and read in that mode alone)
   if (tid < nch && n0 + tid < g.N) {
     if (g.bias) p_bias = (int)g.bias[n0 + tid];
     if (g.mode == EPI_BN) {

@@ -17,8 +17,9 @@ bool launch_tm(int tm, int pf, const BandGeom &g, const EpiArgs &e, size_t lds, 
 {
   if constexpr (TN == 1)
     if (tm == 2 && pf != 2) return pf == 4 ? launch<1, 2, 4>(g, e, lds, s) : launch<1, 2, 1>(g, e, lds, s);
-  return tm == 2 ? launch<TN, 2, band_pf(TN, 2)>(g, e, lds, s) : tm == 4 ? launch<TN, 4, band_pf(TN, 4)>(g, e, lds, s)
-                                                                               : launch<TN, 8, band_pf(TN, 8)>(g, e, lds, s);
+  if constexpr (TN < 4)  // (64 channels a wave: four groups of pixels at the most)
+    if (tm == 8) return launch<TN, 8, band_pf(TN, 8)>(g, e, lds, s);
+  return tm == 2 ? launch<TN, 2, band_pf(TN, 2)>(g, e, lds, s) : launch<TN, 4, band_pf(TN, 4)>(g, e, lds, s);
 }
 
 }  // namespace
