@@ -122,7 +122,7 @@ DW1_GEOMS = [
     (514, 64, 31, 40, (1, 0, 1, 1)),     # no bottom padding: 30 output rows
 ]
 
-# the small ones of these again with more than 64 images, which stay in bands (fewer go to the matrix cores)
+# the small ones of these again on both sides of the line: with more than 64 images they stay in bands, up to 64 they go to the matrix cores
 DW1_BANDS = [(70, 64, 20, 20, (1, 1, 1, 1)), (66, 64, 45, 24, (0, 1, 0, 2)), (66, 64, 9, 112, (1, 1, 1, 1)), (90, 64, 6, 8, (1, 1, 1, 1)),
              (64, 64, 20, 20, (1, 1, 1, 1)), (65, 64, 20, 20, (1, 1, 1, 1))]
 

@@ -102,8 +102,8 @@ def test_random_depthwise(case, bn_bits):
 
 
 def _dw_group_cases(n, seed):
-    """Whole 64-channel groups with rows of whole dwords and output columns in whole groups of four: the shapes whose
-    bands are staged by LDS-direct loads (16-byte pieces that may straddle the image's first and last row)."""
+    """Whole 64-channel groups with rows of whole dwords and output columns in whole groups of four.  With few images most of them go to
+    the matrix cores, some at stride 2 to the bands that are staged by LDS-direct loads."""
     r = rng_for(seed)
     cases = []
     while len(cases) < n:
@@ -117,6 +117,31 @@ def _dw_group_cases(n, seed):
             continue
         cases.append((int(r.choice([1, 2, 5])), ch, h, w, pads, s))
     return cases
+
+
+def _dw_band_cases(seed):
+    """The same with more than 64 times an image's 64 channels, and too few for the streamed kernel: all in bands staged by LDS-direct loads (16-byte
+    pieces that may straddle the image's first and last row), at both strides, with and without left padding, one to three groups."""
+    r = rng_for(seed)
+    cases = []
+    for s in (1, 2):
+        for pl in (0, 1):
+            for groups in (1, 2, 3):
+                for _ in range(2):
+                    while True:
+                        h, w = int(r.integers(3, 41)), 4 * int(r.integers(2, 16))
+                        pads = (int(r.integers(0, 2)), int(r.integers(0, 2)), pl, int(r.integers(0, 3)))
+                        ho, wo = (h + pads[0] + pads[1] - 3) // s + 1, (w + pads[2] + pads[3] - 3) // s + 1
+                        if ho >= 1 and wo >= 4 and wo % 4 == 0 and (w not in (16, 32, 64) or not (pl and pads[0])) and not (h == w == 8):
+                            break
+                    cases.append((64 // groups + int(r.integers(1, 9)), 64 * groups, h, w, pads, s))
+    return cases + [(22, 192, 45, 24, (0, 1, 0, 2), 1)]
+
+
+@pytest.mark.parametrize("bn_bits", [32, 64])
+@pytest.mark.parametrize("case", _dw_band_cases(9103), ids=lambda c: "x".join(map(str, c[:4])) + "p%d%d%d%ds%d" % (c[4] + (c[5],)))
+def test_random_depthwise_in_bands(case, bn_bits):
+    test_random_depthwise_whole_groups(case, bn_bits)
 
 
 @pytest.mark.parametrize("bn_bits", [32, 64])
