@@ -172,9 +172,11 @@ inline bool band_shape(const ConvLayer &L, int cus, int bn_bytes, BandGeom *out,
 //   two a compute unit or in tiles of eight groups of pixels or a third empty (24x48 176 -> 96 stride 2 batch 182 26.3 / 36.9);
 // - where the tiled kernel's tiles are one for almost every compute unit, which is what it does best, and these are more (63x21 96 -> 96 stride 2 batch 39
 //   8.7 / 10.5, 10x17 96 -> 120 batch 92 8.8 / 10.3);
+// - where two workgroups of eight groups of pixels, which is what a compute unit holds, are not all it gets (16x28 176 -> 128 batch 133 24.7 / 32.6, 33x15
+//   48 -> 128 batch 119 9.3 / 14.2);
 // - on more than some 60000 pixels in all (42x31 48 -> 96 batch 54 14.4 / 18.3), nor, with large filters, on more than 96 channels.
-// Over 190 layers drawn for it the mean is 0.867 of the tiled kernel's time, of the 137 that it takes 0.82; four of those are more than 2 % slower, the worst
-// 18x51 112 -> 80 batch 34 13.1 / 16.2.
+// Over 300 layers drawn for it the mean is 0.857 of the tiled kernel's time; of the 231 that it takes fourteen are more than 3 % slower, the worst 18x51 112 -> 80
+// batch 34 13.1 / 16.2, 48x34 208 -> 128 batch 13 1.23.
 inline bool band_for_odd_channels(const ConvLayer &L, int cus, int bn_bytes)
 {
   const long long m = (long long)L.B * L.Ho * L.Wo, tiled = (m + 127) / 128 * ((L.N + 63) / 64);
@@ -185,6 +187,7 @@ inline bool band_for_odd_channels(const ConvLayer &L, int cus, int bn_bytes)
   size_t lds;
   if (!band_shape(L, cus, bn_bytes, &g, &tn, &tm, &lds) || lds > 80 * 1024) return false;
   if (tm > 2 && g.total > cus && tiled <= cus && 5 * tiled >= 4 * cus) return false;
+  if (tm == 8 && g.total > 2 * cus) return false;
   if (L.sx == 1 && L.sy == 1) return true;
   return g.total <= 2 * cus && (tm == 2 || (tm == 4 && 10 * g.R * g.PC >= 7 * 16 * tm * (4 / g.WN)));
 }

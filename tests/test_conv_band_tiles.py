@@ -49,7 +49,8 @@ def test_odd_channel_counts_up_to_128_outputs(walk):
             conv(48, 9, 9, 96, 128, 3, 1), conv(40, 32, 31, 208, 128, 3, 2)]
     tiled = [conv(9, 41, 54, 48, 72, 2, 1), conv(119, 20, 53, 176, 112, 3, 2, 8), conv(182, 24, 48, 176, 96, 3, 2), conv(39, 63, 21, 96, 96, 3, 2),
              conv(92, 10, 17, 96, 120, 3, 1, 8), conv(54, 42, 31, 48, 96, 3, 1), conv(2, 20, 20, 208, 100, 5, 1), conv(8, 16, 16, 96, 128, 1, 1),
-             conv(8, 16, 16, 128, 128, 3, 1), conv(8, 16, 16, 96, 129, 3, 1), conv(19, 62, 50, 240, 120, 2, 2)]
+             conv(8, 16, 16, 128, 128, 3, 1), conv(8, 16, 16, 96, 129, 3, 1), conv(19, 62, 50, 240, 120, 2, 2),
+             conv(133, 16, 28, 176, 128, 3, 1), conv(119, 33, 15, 48, 128, 3, 1)]
     assert all(s.endswith("odd") for s in walk(band))
     assert not any(s.endswith("odd") for s in walk(tiled))
 
