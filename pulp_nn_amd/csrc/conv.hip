@@ -317,10 +317,11 @@ bool try_pw_stream(int mode, const uint8_t *in, const int8_t *w, const int8_t *b
   // a launch that would leave more than half of the CUs without a workgroup is better off tiled:
   // every CU takes part there, and staging the weights per workgroup no longer pays
   if (2 * need < num_cus()) return false;
-  // Several pixels of 16 or 32 channels in a column of the matrix cores, from a load for every wave on (one pixel a column / so, whole calls,
-  // batches of 64x64: 16 -> 16 batch 64 5.0 / 4.0 us, 200 8.6 / 6.7; 16 -> 32 5.7 / 5.3, 9.65 / 8.5; 32 -> 64 7.8 / 7.1, batch 100 9.2 / 8.6; below the
-  // line alike, but 32 -> 64 batch 32 5.1 / 5.3).  Not where its registers leave too few waves: 16 -> 64 7.6 / 8.0, 32 -> 32 3.9 / 4.5 and 6.8 / 6.9; with
-  // constants of 64 bits 16 -> 32 6.0 / 7.8, 32 -> 64 8.2 / 10.3, but 16 -> 16 batch 200 8.7 / 7.8.
+  // Several pixels of 16 or 32 channels in a column of the matrix cores, from a load of 16 channels for every wave on (of 32 that is two loads a wave).  One pixel a
+  // column / so, kernel times, batches of 64x64: batch 64 16 -> 16 5.3 / 4.1 us, 16 -> 32 6.0 / 5.4, 32 -> 64 7.4 / 6.7; batch 128 7.2 / 5.1, 8.2 / 6.6, 10.2 / 8.4; below
+  // the line batch 56 5.0 / 4.0, 5.6 / 5.2, 7.3 / 6.5; batch 48 4.8 / 3.7, 5.4 / 4.7, 7.0 / 6.2; batch 32 3.7 / 3.2, 4.1 / 3.9, 5.2 / 5.4; with 64 bits 16 -> 16 batch 64 5.4 / 5.1,
+  // 56 5.0 / 5.0, 32 3.7 / 3.9: with 32 bits a line at three quarters of it, for 16 channels lower still, that this rule does not draw.  Not where its
+  // registers leave too few waves: 16 -> 64 7.6 / 8.0, 32 -> 32 3.9 / 4.5 and 6.8 / 6.9; with constants of 64 bits 16 -> 32 6.0 / 7.8, 32 -> 64 8.2 / 10.3.
   if (M >= 64ll * 16 * num_cus()) {
     if (K == 16 && N == 16) return launch_pw_packed<1, 1>(mode, g, e, s), true;
     if constexpr (sizeof(bn_t) == 4) {
@@ -403,13 +404,13 @@ void conv_common(const char *fn, bool pointwise, const uint8_t *in, const int8_t
   } else {
     // Channel counts that are not whole 16-byte chunks: from a band of the input in LDS (conv_band.h).  So are layers of
     // few output channels, which leave most of the tiled kernel's 128 x 64 tile empty and its many waves waiting for each
-    // other (kernel times, tiled / band: 8x38x9 240 -> 32 s2 21.9 / 12.6 us; 2x8x13 48 -> 16 5x5 14.2 / 7.2; 31x19 80 -> 16
-    // 10.6 / 6.8; 23x14 144 -> 35 12.0 / 8.8; but 133x16x28 176 -> 128 28.6 / 34.2, 252x12x29 64 -> 40 s2 7.3 / 8.4).
+    // other (kernel times, tiled / band: 8x38x9 240 -> 32 s2 21.9 / 10.8 us; 2x8x13 48 -> 16 5x5 14.2 / 6.6; 31x19 80 -> 16
+    // 9.8 / 5.6; 23x14 144 -> 35 11.2 / 7.2, batch 23 11.4 / 8.3; 37x19 48 -> 20 batch 22 8.7 / 5.8; but 252x12x29 64 -> 40 s2 5.9 / 7.3).
     // 16 and 32 input channels stay with the tiled kernel, which takes two or four taps per K slice there.  It is the faster one
-    // from 40 output channels on (tiled / band, 32 -> 64 at batch 256 16x16 6.7 / 8.5, batch 133 28x28 10.8 / 14.5, batch 64 64x64
-    // 18.4 / 24.1; 8x57x43 32 -> 40 5.2 / 9.3) and the slower one below (256x16x16 32 -> 32 7.3 / 6.8, 32 -> 16 6.9 / 5.7; 256x8x8
-    // 32 -> 24 7.7 / 5.3; 64x32x32 16 -> 32 6.9 / 6.4; but 133x28x28 16 -> 32 7.7 / 8.3): a line at 32 channels that this rule
-    // does not draw.
+    // from 40 output channels on (tiled / band, 32 -> 64 at batch 256 16x16 6.1 / 8.0, batch 133 28x28 9.9 / 13.0, batch 64 64x64
+    // 16.2 / 22.6; 8x57x43 32 -> 40 4.8 / 6.2) and the slower one below on small layers (16x16 32 -> 24 batch 1 6.7 / 4.6, 32x32 32 -> 32 batch 16
+    // 6.3 / 5.0, 8x57x43 16 -> 24 6.4 / 5.0, 256x16x16 32 -> 16 5.8 / 5.6; but 256x16x16 32 -> 32 6.4 / 7.0, 133x28x28 16 -> 32 6.6 / 7.7, 64x64x64
+    // 32 -> 32 10.6 / 14.2): a line by output channels and size that this rule does not draw.
     const bool whole16 = ch_in % 16 == 0 && aligned(in, 16) && aligned(w, 16);
     // Up to 128 output channels it is also the faster one for many layers whose channel count is no multiple of 64, which the tiled kernel gathers
     // chunk by chunk (band_for_odd_channels).
