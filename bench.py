@@ -51,7 +51,7 @@ KERNELS = {
     "cfg2_dw_s1": "dw3x3_lin_kernel<1, 1, 0>",
     "cfg2_dw_s2": "dw3x3_stream_kernel<2, 1, 0>",
     "cfg4_conv": "igemm_patch_kernel<0, 0>",
-    "cfg4_maxpool": "maxpool16_kernel<false, true>",
+    "cfg4_maxpool": "maxpool16_kernel<false, true, 2, 2>",
     "cfg4_linear": "linear_skinny_kernel<0>",
 }
 

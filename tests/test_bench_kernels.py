@@ -9,6 +9,8 @@ import sys
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 sys.path.insert(0, ROOT)
 import bench  # noqa: E402
+from pulp_nn_amd import build  # noqa: E402
+from test_kernel_registers import kernel_names  # noqa: E402
 
 
 def test_every_named_kernel_is_in_the_committed_trace():
@@ -24,3 +26,14 @@ def test_every_named_kernel_has_one_traffic_figure():
     for workload, kernel in bench.KERNELS.items():
         got = bench.traffic_for(table, kernel)
         assert got is not None and got > 0, "%s: no single traffic row for %s" % (workload, kernel)
+
+
+def test_every_named_kernel_is_in_a_built_library():
+    """(A kernel renamed since the trace was taken would be in that trace still.)"""
+    found = set()
+    for bn_bits in (32, 64):
+        if not os.path.exists(build.lib_path(bn_bits)):
+            build.build(bn_bits)
+        found |= set(kernel_names(bn_bits))
+    for workload, kernel in bench.KERNELS.items():
+        assert kernel in found, "%s: no library has %s" % (workload, kernel)

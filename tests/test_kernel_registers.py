@@ -43,6 +43,13 @@ def _kernels(elf):
             off = desc + (descsz + 3) // 4 * 4
 
 
+def kernel_names(bn_bits):
+    """Names of a library's kernels as a profiler prints them, without arguments."""
+    names = [k[".name"] for elf in _code_objects(build.lib_path(bn_bits)) for k in _kernels(elf)]
+    plain = subprocess.run(["c++filt"], input="\n".join(names), stdout=subprocess.PIPE, text=True, check=True).stdout.split("\n")
+    return [n.removeprefix("void ").split("(")[0] for n in plain]
+
+
 @pytest.mark.parametrize("bn_bits", [32, 64])
 def test_no_vector_register_is_spilled(bn_bits):
     lib = build.lib_path(bn_bits)
