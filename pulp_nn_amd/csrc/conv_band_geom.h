@@ -107,7 +107,15 @@ inline bool band_shape(const ConvLayer &L, int cus, int bn_bytes, BandGeom *out,
     while (tr > 1 && lds_for(tr, tpc, t) > 80 * 1024) tr--;
     while (t == 2 && tpc > 1 && lds_for(tr, tpc, t) > MOST) tpc = (tpc + 1) / 2;
     if (t > 2 && lds_for(tr, tpc, t) > 80 * 1024) continue;
-    const long long wgs = (long long)B * ((g.Ho + tr - 1) / tr) * ((g.Wo + tpc - 1) / tpc) * ((g.N + 16 * tn * g.WN - 1) / (16 * tn * g.WN));
+    auto count = [&](int n) { return (long long)B * ((g.Ho + tr - 1) / tr) * ((g.Wo + n - 1) / n) * ((g.N + 16 * tn * g.WN - 1) / (16 * tn * g.WN)); };
+    // A row of which LDS holds one workgroup, however few weights are in flight, in halves where the busiest compute unit then has less than a whole
+    // one's rounds to do (whole rows / halves, 64 bits: 28x13x53 256 -> 32 5x5 43.6 / 31.7 us, 109x15x51 256 -> 32 5x5 stride 2 86.3 / 78.5; where the rounds
+    // come out even halves lose: 125x8x57 224 -> 48 5x5 stride 2 40.5 / 48.2).
+    const int half = (tpc + 1) / 2;
+    if (tn == 1 && t == 2 && tr == 1 && count(tpc) > cus && lds_for(tr, tpc, t) - 4 * band_wbytes(1, 1) > MOST / 2 && lds_for(tr, half, t) <= MOST / 2 &&
+        (count(half) + cus - 1) / cus < 2 * ((count(tpc) + cus - 1) / cus))
+      tpc = half;
+    const long long wgs = count(tpc);
     if (t > 2 && wgs < cus) continue;
     const long long work = (wgs + cus - 1) / cus * ((tn == 4 ? 1 : 4 - tn) + (tr * tpc + 16 * wm - 1) / (16 * wm));
     if (tm && work >= least) continue;
@@ -149,12 +157,15 @@ inline bool band_shape(const ConvLayer &L, int cus, int bn_bytes, BandGeom *out,
   *tm_out = tm;
   // Groups of weights: four steps for long filters in launches of few workgroups, which wait for their weights; one where that lets another
   // workgroup share a compute unit (call times, two / four steps: 8x38x9 240 -> 32 stride 2 11.4 / 11.0; 57x43 24 -> 40 stride 2 batch 32
-  // 8.0 / 8.5, 19x33 85 -> 8 batch 123 11.1 / 13.7; two / one: 27x39 pointwise 320 -> 8 batch 215 25.7 / 20.7).
+  // 8.0 / 8.5, 19x33 85 -> 8 batch 123 11.1 / 13.7; two / one: 27x39 pointwise 320 -> 8 batch 215 25.7 / 20.7; in
+  // no more than two workgroups a compute unit 16x55x64 178 -> 64 5x5 stride 2 38.7 / 24.2, 12x41x28 250 -> 32 7x7 81.8 / 50.6, 73x14x54 224 -> 32 5x5 stride 2
+  // 39.8 / 26.9).  (Without weights in LDS there was room for a second one in some where now there is none: 125x8x57 224 -> 48 5x5 stride 2 23.7 / 40.5,
+  // 109x15x51 256 -> 32 59.9 / 78.3.)
   int pf = band_pf(tn, tm);
   if (tn == 1 && tm == 2) {
     const auto with = [&](int n) { return lds + 4 * (band_wbytes(1, n) - band_wbytes(1, pf)); };
     const int to = g.NK > 8 && total <= 2ll * cus && with(4) <= (total <= cus ? MOST : 80 * 1024) ? 4
-                   : total > 2ll * cus && MOST / with(1) > MOST / with(2) && MOST / with(2) < 3    ? 1
+                   : total > MOST / with(2) * cus && MOST / with(1) > MOST / with(2) && MOST / with(2) < 3 ? 1
                                                                                                    : 2;
     lds = with(to);
     pf = to;

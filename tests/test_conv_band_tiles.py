@@ -55,6 +55,21 @@ def test_odd_channel_counts_up_to_128_outputs(walk):
     assert not any(s.endswith("odd") for s in walk(tiled))
 
 
+def _conv(B, H, W, Ci, N, k, s, bn_bytes=4):
+    return layer(B, H, W, Ci, (H + k // 2 * 2 - k) // s + 1, (W + k // 2 * 2 - k) // s + 1, N, k, k, k // 2, k // 2, s, s, bn_bytes=bn_bytes)
+
+
+def test_room_for_a_second_workgroup(walk):
+    """More workgroups than compute units, of which LDS would hold one with two steps of weights: one step, or halves of rows."""
+    one_step = [_conv(10, 55, 63, 178, 33, 5, 2), _conv(16, 55, 64, 178, 64, 5, 2, 8), _conv(73, 14, 54, 224, 32, 5, 2, 8)]
+    halves = [_conv(21, 13, 53, 256, 17, 5, 1), _conv(28, 13, 53, 256, 32, 5, 1, 8)]
+    whole = [_conv(36, 25, 57, 250, 48, 5, 2), _conv(29, 15, 51, 224, 32, 7, 1)]  # (halves would come out even)
+    for l, said in zip(one_step + halves + whole, walk(one_step + halves + whole)):
+        lds, tiles = map(int, said.split()[1:3])
+        rows = l[0] * l[4]
+        assert (lds <= 80 * 1024) == (l not in whole) and tiles == (2 * rows if l in halves else rows), l
+
+
 def test_lds_past_an_int(walk):
     """Strides and filters whose staged input would take more bytes than an int counts: not taken, or in tiles that fit."""
     layers = [layer(1, 60, 60, 57, 15292, 50, 6, 4, 1, sx=34257, sy=35775), layer(1, 60, 60, 53, 11955, 1, 10, 4, 2, sx=1, sy=37077),

@@ -31,6 +31,8 @@ BAND = [
     (260, 6, 7, 24, 100, 3, 3, (1, 1, 1, 1), (1, 1)),   # two groups a wave, eight of pixels
     (40, 21, 26, 8, 150, 3, 3, (1, 1, 1, 1), (1, 1)),   # four and four
     (1, 5, 150, 256, 20, 5, 5, (2, 2, 2, 2), (2, 1)),   # a tile that LDS holds part of a row for
+    (10, 55, 63, 178, 33, 5, 5, (2, 2, 2, 2), (2, 2)),  # weights one step at a time: two workgroups a compute unit
+    (21, 13, 53, 256, 17, 5, 5, (2, 2, 2, 2), (1, 1)),  # halves of rows, the second one shorter
 ]
 # small layers of the tiled kernel: nine K slices at a time, taps outside the image on every side
 TILED = [
