@@ -413,9 +413,9 @@ void conv_common(const char *fn, bool pointwise, const uint8_t *in, const int8_t
     // 32 -> 32 10.6 / 14.2): a line by output channels and size that this rule does not draw.
     const bool whole16 = ch_in % 16 == 0 && aligned(in, 16) && aligned(w, 16);
     // Up to 128 output channels it is also the faster one for many layers whose channel count is no multiple of 64, which the tiled kernel gathers
-    // chunk by chunk (band_for_odd_channels).
-    const bool odd64 = g.N > 64 && band_for_odd_channels(L, num_cus(), (int)sizeof(bn_t));
-    const bool few = ch_in == 16 || ch_in == 32 ? false : ch_in % 64 == 0 ? g.N <= 32 : g.N <= 64 || odd64;
+    // chunk by chunk (band_for_odd_channels; up to 64 band_for_up_to_64).
+    auto odd64 = [&] { return g.N > 64 ? band_for_odd_channels(L, num_cus(), (int)sizeof(bn_t)) : band_for_up_to_64(L, num_cus(), (int)sizeof(bn_t)); };
+    const bool few = ch_in == 16 || ch_in == 32 ? false : g.N <= 32 || (ch_in % 64 && odd64());
     if (!whole16 || few) {
       if (launch_conv_band(mode, L, e, num_cus(), g_stream)) return check_launch(fn);
     }

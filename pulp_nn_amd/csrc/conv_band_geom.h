@@ -175,6 +175,22 @@ inline bool band_shape(const ConvLayer &L, int cus, int bn_bytes, BandGeom *out,
   return true;
 }
 
+// Whether a layer of 33 to 64 output channels on a channel count of whole 16-byte chunks but no multiple of 64 takes this kernel, not the tiled one: it
+// does, over 60 layers in 0.73 of the time, but for
+// - eight groups of pixels a wave, of which a compute unit holds two workgroups and gets more (tiled / band: 144x41x32 144 -> 48 stride 2 18.7 / 26.3 us,
+//   183x36x44 160 -> 39 28.1 / 38.2, 81x15x60 224 -> 41 31.8 / 31.6; four or two groups, or room for a third, are mixed: 94x48x39 144 -> 63 23.0 / 20.9);
+// - halves of rows, with larger filters, in more than four workgroups a compute unit (144x12x61 224 -> 48 5x5 stride 2 51.2 / 70.6; 48x11x50 224 -> 40 7x7
+//   stride 2 86.1 / 63.8).
+inline bool band_for_up_to_64(const ConvLayer &L, int cus, int bn_bytes)
+{
+  BandGeom g;
+  int tn, tm;
+  size_t lds;
+  if (!band_shape(L, cus, bn_bytes, &g, &tn, &tm, &lds)) return false;
+  if (L.kx * L.ky <= 9) return L.kx * L.ky == 1 || !(tm == 8 && lds > 53 * 1024 && g.total > 2 * cus);
+  return !(g.xtiles > 1 && 2 * g.R * g.PC <= 16 * tm * (4 / g.WN) && g.total > 4 * cus);
+}
+
 // Whether a layer of 65 to 128 output channels on a channel count of whole 16-byte chunks but no multiple of 64 takes this kernel, not the tiled one, which
 // gathers such inputs chunk by chunk in tiles of 128 pixels x 64 channels.  Whole calls, tiled / band: 12x12 112 -> 71 batch 146 16.5 / 10.3 us, 27x8
 // 176 -> 120 batch 177 19.7 / 11.7, 48x18 96 -> 100 stride 2 batch 101 9.7 / 6.2.  Not

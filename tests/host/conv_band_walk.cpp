@@ -3,7 +3,7 @@
 // computes, and, for the first, the last and some tiles between of layers that are not large, chunks of the band that a workgroup stages twice or
 // not at all and loads inside the image that leave the input.
 // Layers on stdin, one a line: B H W Ci Ho Wo N kx ky pt pl sx sy bn_bytes cus.  One line out per layer: "ok LDS TILES", with "odd" behind it where
-// band_for_odd_channels says so, "no"
+// band_for_odd_channels (up to 64 output channels: band_for_up_to_64) says so, "no"
 // (not taken by the kernel) or what is wrong.
 #include <stdio.h>
 
@@ -81,7 +81,7 @@ static std::string check(const ConvLayer &L, int bn_bytes, int cus)
       const std::string s = staging(g, (unsigned)id);
       if (!s.empty()) return "tile " + std::to_string(id) + ": " + s;
     }
-  return "ok " + std::to_string(lds) + " " + std::to_string(g.total) + (L.N > 64 && band_for_odd_channels(L, cus, bn_bytes) ? " odd" : "");
+  return "ok " + std::to_string(lds) + " " + std::to_string(g.total) + ((L.N > 64 ? band_for_odd_channels(L, cus, bn_bytes) : band_for_up_to_64(L, cus, bn_bytes)) ? " odd" : "");
 }
 
 int main()

@@ -70,6 +70,15 @@ def test_room_for_a_second_workgroup(walk):
         assert (lds <= 80 * 1024) == (l not in whole) and tiles == (2 * rows if l in halves else rows), l
 
 
+def test_33_to_64_outputs(walk):
+    """The line between this kernel and the tiled one, from both sides."""
+    band = [_conv(32, 42, 61, 80, 40, 3, 1), _conv(94, 48, 39, 144, 63, 3, 2), _conv(47, 39, 45, 240, 40, 5, 2), _conv(48, 11, 50, 224, 40, 7, 2), _conv(163, 15, 54, 48, 40, 3, 1),
+            _conv(36, 41, 32, 144, 48, 3, 2)]
+    tiled = [_conv(144, 41, 32, 144, 48, 3, 2), _conv(183, 36, 44, 160, 39, 3, 2, 8), _conv(144, 12, 61, 224, 48, 5, 2, 8), _conv(28, 38, 57, 224, 48, 7, 2)]
+    assert all(s.endswith("odd") for s in walk(band))
+    assert not any(s.endswith("odd") for s in walk(tiled))
+
+
 def test_lds_past_an_int(walk):
     """Strides and filters whose staged input would take more bytes than an int counts: not taken, or in tiles that fit."""
     layers = [layer(1, 60, 60, 57, 15292, 50, 6, 4, 1, sx=34257, sy=35775), layer(1, 60, 60, 53, 11955, 1, 10, 4, 2, sx=1, sy=37077),
