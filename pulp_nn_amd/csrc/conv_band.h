@@ -25,8 +25,9 @@
 // the vector instructions around each MFMA and by LDS, which holds input, weights and with them the workgroups that share a compute
 // unit.  Whole calls, weights in registers in operand layout and tiles for two workgroups a compute unit / now: 57x43 24 -> 40 stride 2 batch 32
 // 9.8 / 6.7 us; 15x31 168 -> 16 batch 19 11.3 / 9.7; 56x56 100 -> 100 batch 16 25.9 / 16.7; 40x30 250 -> 250 stride 2 batch 60 115 / 47;
-// 13x19 90 -> 192 5x5 batch 70 125 / 36; 24x27 168 -> 176 5x5 stride 2 batch 72 47.4 / 44.6; over 380 layers the mean is 0.90; slower by
-// more than 2 %: 23x14 144 -> 35 batch 23 8.3 / 8.6 and 37x19 48 -> 20 batch 22 5.7 / 5.9.  (The 128 x 64 tile with a byte gather,
+// 13x19 90 -> 192 5x5 batch 70 125 / 36; 24x27 168 -> 176 5x5 stride 2 batch 72 47.4 / 44.6; over 380 layers the mean is 0.90, two of them
+// slower by more than 2 % (23x14 144 -> 35 batch 23 8.3 / 8.6, 37x19 48 -> 20 batch 22 5.7 / 5.9); over 60 others of 33 to 64 outputs 0.91, five of them slower by
+// 2 to 7 % (10x38 224 -> 48 batch 32 11.4 / 12.3, 34x10 208 -> 62 batch 58 11.9 / 12.7, 15x54 48 -> 40 batch 163 16.8 / 17.6).  (The 128 x 64 tile with a byte gather,
 // which these shapes took before: 19.3, 236 and 409 us for the first, the second and the last.)
 #pragma once
 #include <type_traits>
